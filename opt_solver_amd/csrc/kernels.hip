@@ -481,104 +481,155 @@ void launch_assemble(hipStream_t st, const DevPtrs &d, const AsmTask *tasks, int
 // NotPositiveDefinite.
 constexpr int kNb = 64;
 
-// kPotrfWaves wavefronts per diagonal block, each owning kPotrfCols = 64 /
-// kPotrfWaves columns: thread (r, h), r the lane and h the wave, holds row r
-// of the block's lower triangle in columns [C h, C h + C) (a[i] =
-// A[r][C h + i], C = kPotrfCols) and rows [C h, C h + C) of column r of W,
-// the identity turned into the unit lower inverse by the same row
-// operations (w[i] = W[C h + i][r]). Step j: the wave owning column j puts
-// the multipliers g_c = A[c][j] / d_jj, the column A[.][j] and the row
-// W[j][.] in LDS (two alternating buffers: one barrier per step); then each
-// thread updates A[r][c] -= A[r][j] g_c for c > j and W[i][r] -= g_i W[j][r]
-// for i > j in its columns. inv(L_kk) = D^-1/2 W. Rows and columns past kb
-// are the identity. The 64 steps are a dependent chain; more waves shorten
-// each step's update (2 C FMAs per thread).
-constexpr int kPotrfWaves = 8;
-constexpr int kPotrfCols = kNb / kPotrfWaves;
+// One workgroup of four wavefronts per diagonal block, in four 16-column
+// panels. The block is stacked over the identity: the column operations that
+// turn A into L turn I into inv(L)^T, so one full 64 x 64 square S holds both,
+// 16 x 16 blocks (g, p) with g > p being A / L and g < p being inv(L)^T (the
+// diagonal blocks' inverses go to their strict upper parts, and for the
+// update whole to X).
+// Panel p, wavefront 0: row r of block (g, p) in lane r of row g of 16 lanes
+// (the identity block for g = p), and beside it row r of the diagonal block
+// (p, p), so the 16 dependent pivots run in registers without a barrier or
+// an exchange between rows of lanes; the multipliers are broadcast inside a
+// row of lanes (DPP: 14.5 cycles for the broadcast and its two FMAs, readlane
+// took 24 for one).
+// Then the blocks right of the panel are updated on FP64 MFMA,
+// (i, c) -= (i, p) (c, p)^T for c > p, i <= p or i >= c: the next panel's
+// column (p + 1) by all four wavefronts first, the rest by wavefronts 1 to 3
+// beside the next panel's pivots. Rows and columns past kb are the identity;
+// panels past kb are skipped. Bound by wavefront 0's instructions (about 6
+// cycles each in FP64, 17 for the rsqrt estimate): 20.0 us a block with one
+// column at a time over eight wavefronts, 10.6 us now.
+constexpr int kPB = 16;       // panel width
+constexpr int kPLd = kNb + 16;  // column stride of S: the two lane rows of a half wavefront's MFMA operand read fall on different banks
 
-__device__ __forceinline__ void potrf_steps(double (&a)[kPotrfCols], double (&w)[kPotrfCols], int r, int h, int kb,
-                                            double (*gl)[kNb], double (*cola)[kNb], double (*colw)[kNb], double *rsv,
-                                            bool &bad) {
-    constexpr int C = kPotrfCols;
-    for (int jb = 0; jb < kPotrfWaves; ++jb) {
-#pragma unroll
-        for (int jj = 0; jj < C; ++jj) {
-            const int j = C * jb + jj;
-            const int bs = j & 1;
-            if (h == jb) {
-                const double ajj = a[jj];
-                const double djj = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(ajj), j),
-                                                    __builtin_amdgcn_readlane(__double2loint(ajj), j));
-                // 1 / sqrt(djj): the hardware estimate refined by two
-                // Newton steps (y <- y (3 - d y^2) / 2)
-                double rs = __builtin_amdgcn_rsq(djj);
-                rs = rs * (1.5 - 0.5 * djj * rs * rs);
-                rs = rs * (1.5 - 0.5 * djj * rs * rs);
-                gl[bs][r] = r > j ? ajj * (rs * rs) : 0.0;
-                cola[bs][r] = ajj;
-                colw[bs][r] = w[jj];
-                if (r == 0) rsv[j] = rs;
-                bad = bad || (j < kb && !(djj > 0.0 && djj <= DBL_MAX));
-                a[jj] = r > j ? ajj * rs : (r == j ? djj * rs : ajj);
-            }
-            __syncthreads();
-            const double arj = cola[bs][r], wjr = colw[bs][r];
-            if (h == jb) {
-#pragma unroll
-                for (int i = jj + 1; i < C; ++i) {
-                    a[i] -= arj * gl[bs][C * jb + i];
-                    w[i] -= gl[bs][C * jb + i] * wjr;
-                }
-            } else if (h > jb) {
-#pragma unroll
-                for (int i = 0; i < C; ++i) {
-                    a[i] -= arj * gl[bs][C * h + i];
-                    w[i] -= gl[bs][C * h + i] * wjr;
-                }
-            }
+// v of lane C of the lane's row of 16 lanes
+template <int C>
+__device__ __forceinline__ double row_bcast(double v) {
+    return __builtin_amdgcn_update_dpp(0.0, v, 0x150 + C, 0xf, 0xf, true);
+}
+// 1 / sqrt(d): the hardware estimate y (better than 2^-20) and one third-order
+// step in e = 1 - d y^2, y (1 + e / 2 + 3 e^2 / 8), its error of order e^3
+__device__ __forceinline__ double pivot_rsqrt(double d) {
+    const double y = __builtin_amdgcn_rsq(d);
+    const double e = fma(-d * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+// Pivot J of a panel: a the diagonal block's row, b the lane's own block's
+// row, rs 1 / sqrt of the pivot. The next pivot's column goes first.
+template <int J, int C>
+__device__ __forceinline__ void potrf_cols(double (&a)[kPB], double (&b)[kPB], double na, double nb) {
+    if constexpr (C < kPB) {
+        const double m = row_bcast<C>(a[J]);
+        a[C] = fma(m, na, a[C]);
+        b[C] = fma(m, nb, b[C]);
+        potrf_cols<J, C + 1>(a, b, na, nb);
+    }
+}
+template <int J>
+__device__ __forceinline__ void potrf_pivots(double (&a)[kPB], double (&b)[kPB], double rs) {
+    if constexpr (J < kPB) {
+        a[J] *= rs;
+        b[J] *= rs;
+        double rn = 0.0;
+        if constexpr (J + 1 < kPB) {
+            const double m = row_bcast<J + 1>(a[J]);
+            a[J + 1] = fma(-m, a[J], a[J + 1]);
+            rn = pivot_rsqrt(row_bcast<J + 1>(a[J + 1]));
+            b[J + 1] = fma(-m, b[J], b[J + 1]);
         }
+        potrf_cols<J, J + 2>(a, b, -a[J], -b[J]);
+        potrf_pivots<J + 1>(a, b, rn);
     }
 }
 
-__global__ __launch_bounds__(kNb * kPotrfWaves) void k_potrf(DevPtrs d, const PotrfItem *__restrict__ items) {
-    constexpr int C = kPotrfCols;
-    __shared__ double gl[2][kNb];
-    __shared__ double cola[2][kNb];
-    __shared__ double colw[2][kNb];
-    __shared__ double rsv[kNb];
+// Block (i, c) of S -= block (i, p) (X when i = p) times block (c, p)^T.
+__device__ __forceinline__ void potrf_update(double *S, const double *X, int p, int i, int c) {
+    const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+    v4d acc;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[v] = S[(kPB * c + 4 * v + lk) * kPLd + kPB * i + lr];
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+        const double o = i == p ? X[(4 * kk + lk) * kPB + lr] : S[(kPB * p + 4 * kk + lk) * kPLd + kPB * i + lr];
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(S[(kPB * p + 4 * kk + lk) * kPLd + kPB * c + lr], -o, acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) S[(kPB * c + 4 * v + lk) * kPLd + kPB * i + lr] = acc[v];
+}
+
+__global__ __launch_bounds__(kThreads) void k_potrf(DevPtrs d, const PotrfItem *__restrict__ items) {
+    __shared__ double S[kNb * kPLd];     // column-major
+    __shared__ double X[2][kPB * kPB];   // panels' diagonal inverse transposed, whole, column-major
     __shared__ int flag_bad;
     const PotrfItem it = items[blockIdx.x];
     const FrontDev F = d.fronts[it.s];
     const int f = F.f, k = it.k, kb = it.kb;
     double *base = d.L + F.lofs;
-    const int r = threadIdx.x & 63;
-    const int h = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (threadIdx.x == 0) flag_bad = 0;
-    bool bad = false;
-    double a[C], w[C];
+    {
+        double v[kNb / 4];
 #pragma unroll
-    for (int i = 0; i < C; ++i) {
-        const int c = C * h + i;
-        a[i] = base[static_cast<int64_t>(k + min(c, kb - 1)) * f + k + min(r, kb - 1)];
-    }
+        for (int i = 0; i < kNb / 4; ++i)
+            v[i] = base[static_cast<int64_t>(k + min(w + 4 * i, kb - 1)) * f + k + min(lane, kb - 1)];
 #pragma unroll
-    for (int i = 0; i < C; ++i) {
-        const int c = C * h + i;
-        const bool in = r < kb && c < kb && r >= c;
-        a[i] = masked(a[i], in) + ((!in && r == c) ? 1.0 : 0.0);
-        w[i] = (c == r) ? 1.0 : 0.0;
+        for (int i = 0; i < kNb / 4; ++i) {
+            const int c = w + 4 * i;
+            S[c * kPLd + lane] = (lane < kb && c < kb && lane >= c) ? v[i] : (lane == c ? 1.0 : 0.0);
+        }
     }
-    potrf_steps(a, w, r, h, kb, gl, cola, colw, rsv, bad);
-    if (bad) flag_bad = 1;
+    const int nblk = (kb + kPB - 1) / kPB;
+    const int lr = lane & 15, lk = lane >> 4;
+    __syncthreads();
+    for (int p = 0; p < nblk; ++p) {
+        if (w == 0) {
+            double a[kPB], b[kPB];
+#pragma unroll
+            for (int c = 0; c < kPB; ++c) {
+                a[c] = S[(kPB * p + c) * kPLd + kPB * p + lr];
+                b[c] = lk == p ? (c == lr ? 1.0 : 0.0) : S[(kPB * p + c) * kPLd + lane];
+            }
+            potrf_pivots<0>(a, b, pivot_rsqrt(row_bcast<0>(a[0])));
+            if (lk == p) {
+#pragma unroll
+                for (int c = 0; c < kPB; ++c) {
+                    X[p & 1][c * kPB + lr] = b[c];
+                    b[c] = c <= lr ? a[c] : b[c];
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < kPB; ++c) S[(kPB * p + c) * kPLd + lane] = b[c];
+        } else if (p > 0) {
+            // the rest of panel p - 1's update: columns from p + 1 on
+            int t = 0;
+            for (int c = p + 1; c < nblk; ++c)
+                for (int i = 0; i < nblk; ++i)
+                    if ((i < p || i >= c) && t++ % 3 == w - 1) potrf_update(S, X[(p - 1) & 1], p - 1, i, c);
+        }
+        __syncthreads();
+        if (p + 1 < nblk) {
+            // column p + 1 of this panel's update (row w of it)
+            if (w < nblk) potrf_update(S, X[p & 1], p, w, p + 1);
+            __syncthreads();
+        }
+    }
+    // a pivot that is not positive and finite leaves a NaN in its L_jj (its
+    // rsqrt is a NaN, or the step from it multiplies 0 by infinity)
+    if (w == 0 && lane < kb) {
+        const double ljj = S[lane * kPLd + lane];
+        if (!(ljj > 0.0 && ljj <= DBL_MAX)) flag_bad = 1;
+    }
     __syncthreads();
     if (threadIdx.x == 0 && flag_bad) atomicMin(d.flag, it.s + 1);
-    // lower (c <= r): L_kk; strict upper (r < c): M[r][c] = inv(L_kk)[c][r]
-    // = W[c][r] / L_cc
-    if (r < kb) {
+    // lower: L_kk; strict upper: M[r][c] = inv(L_kk)[c][r]
+    if (lane < kb) {
 #pragma unroll
-        for (int i = 0; i < C; ++i) {
-            const int c = C * h + i;
-            if (c < kb) base[static_cast<int64_t>(k + c) * f + k + r] = c <= r ? a[i] : w[i] * rsv[c];
+        for (int i = 0; i < kNb / 4; ++i) {
+            const int c = w + 4 * i;
+            if (c < kb) base[static_cast<int64_t>(k + c) * f + k + lane] = S[c * kPLd + lane];
         }
     }
 }
@@ -586,7 +637,7 @@ __global__ __launch_bounds__(kNb * kPotrfWaves) void k_potrf(DevPtrs d, const Po
 void launch_potrf(hipStream_t st, const DevPtrs &d, const PotrfItem *it, int64_t n) {
     if (n <= 0) return;
     for (int64_t o = 0; o < n; o += kMaxLaunchGroups)
-        k_potrf<<<dim3(static_cast<unsigned>(std::min(kMaxLaunchGroups, n - o))), kNb * kPotrfWaves, 0, st>>>(d, it + o);
+        k_potrf<<<dim3(static_cast<unsigned>(std::min(kMaxLaunchGroups, n - o))), kThreads, 0, st>>>(d, it + o);
 }
 
 // Panel TRSM: rows [r0, r0 + 64) of columns [k, k + kb): X = A M, with

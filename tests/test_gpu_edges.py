@@ -1,0 +1,56 @@
+"""Kernels at the sizes where their tiles and remainders begin and end,
+against the oracle's factor of the same analysis and known solutions."""
+import numpy as np
+import pytest
+
+from tests.conftest import gpu_available
+from tests.helpers import matvec
+
+pytestmark = pytest.mark.gpu
+
+if not gpu_available():
+    pytest.skip("no GPU", allow_module_level=True)
+
+from opt_solver_amd import generators as g  # noqa: E402
+from opt_solver_amd.solver import Plan, analyse  # noqa: E402
+from tests.test_gpu_spd import block_rel_err  # noqa: E402
+
+
+def dense_spd(n, seed):
+    """A dense symmetric positive definite matrix (one supernode): G G^T / n
+    + I has a condition number of about 5."""
+    rng = np.random.default_rng([n, seed])
+    G = rng.standard_normal((n, n))
+    M = G @ G.T / n + np.eye(n)
+    r, c = np.tril_indices(n)
+    return g.coo_lower_to_csc(n, r, c, M[r, c])
+
+
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 31, 33, 47, 48, 49, 63, 64, 65, 81, 128, 129, 200])
+def test_dense_cholesky_panel_edges(oracle_lib, n):
+    """One front of n pivots: diagonal blocks of every remainder modulo 16
+    and 64. Both factors are within n eps cond (200 x 2.2e-16 x 5 = 2e-13)
+    of the exact one."""
+    print("case dense", n, flush=True)
+    A = dense_spd(n, 1)
+    an = analyse(A)
+    assert an.nsup == 1
+    fac = Plan(an, posdef=True).factor(A[3])
+    orc = oracle_lib.Factor(an.arrays(), A[3], posdef=True)
+    assert fac.status == 0
+    assert block_rel_err(fac.export(), orc.export()) < 4e-13
+    x = np.random.default_rng(n).uniform(-1, 1, n)
+    assert np.abs(fac.solve(matvec(A, x)) - x).max() < 1e-12
+
+
+@pytest.mark.parametrize("n,bad", [(1, 0), (16, 15), (40, 16), (64, 63), (70, 65)])
+def test_dense_cholesky_bad_pivot(n, bad):
+    """A pivot that is zero or negative at the edge of a panel is reported."""
+    for shift in (0.0, -1.0):
+        n_, cp, ri, v = dense_spd(n, 2)
+        M = g.csc_to_dense(n, cp, ri, v)
+        L = np.linalg.cholesky(M)
+        v = v.copy()
+        v[cp[bad]] += shift * 1e-3 - L[bad, bad] ** 2 * (1.0 if shift else 1.0 + 1e-9)
+        fac = Plan(analyse((n, cp, ri, v)), posdef=True).factor(v)
+        assert fac.status == 1
