@@ -2449,14 +2449,16 @@ void launch_ldlt_store(hipStream_t st, const LdltDev &d, const int32_t *flist, i
 // ---------------------------------------------------------------------------
 // D^-1 step of the LDL^T solve (apply_dinv, solve_backward.cpp:156-173): per pivot,
 // kind 1 scales, kind 2 applies the 2x2 inverse, kind 0 (second column of a
-// 2x2) is skipped. The L sweeps are in kernels_solve.hip.
+// 2x2) is skipped. The L sweeps are in kernels_solve.hip. gridDim.y
+// workgroups share a front's pivots (a front of 14,000 pivots is 200 us of
+// scattered reads for one).
 __global__ void k_ldlt_diag(LdltDev d, const int32_t *__restrict__ flist, int32_t nf, double *__restrict__ y,
                             int32_t n, int32_t nrhs) {
     const int fi = blockIdx.x;
     if (fi >= nf) return;
     const FrontLd F = d.fronts[flist[fi]];
     const int32_t *rows = d.rows + F.rofs;
-    for (int c = threadIdx.x; c < F.pstore; c += blockDim.x) {
+    for (int c = blockIdx.y * blockDim.x + threadIdx.x; c < F.pstore; c += gridDim.y * blockDim.x) {
         const int8_t kd = d.dkind[F.dofs + c];
         const double *dv = d.dinv + 3 * (F.dofs + c);
         for (int r = 0; r < nrhs; ++r) {
@@ -2538,12 +2540,14 @@ void launch_ldlt_diag_div(hipStream_t st, const LdltDev &d, const int32_t *flist
     }
 }
 
-void launch_ldlt_diag(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, double *y, int32_t n,
-                      int32_t nrhs) {
+void launch_ldlt_diag(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, int32_t max_p, double *y,
+                      int32_t n, int32_t nrhs) {
     if (nf <= 0) return;
+    const int32_t threads = max_p > 64 ? kLT : 64;
+    const int32_t parts = std::max(1, std::min(16, (max_p + threads - 1) / threads));
     for (int64_t o = 0; o < nf; o += kMaxLaunchGroups) {
         const int32_t m = static_cast<int32_t>(std::min<int64_t>(kMaxLaunchGroups, nf - o));
-        k_ldlt_diag<<<dim3(static_cast<unsigned>(m)), 64, 0, st>>>(d, flist + o, m, y, n, nrhs);
+        k_ldlt_diag<<<dim3(static_cast<unsigned>(m), parts), threads, 0, st>>>(d, flist + o, m, y, n, nrhs);
     }
 }
 

@@ -421,40 +421,97 @@ __global__ void k_zero_i32(int32_t *p, int32_t n) {
 // ---------------------------------------------------------------------------
 // Sweeps of an LDL^T factor (unit L with D on the stored diagonal; the D^-1
 // step runs between them): steps of kLS pivots (a large front's dense
-// triangle costs a launch per kLS pivots), each solved inside its triangle
-// item as up to four 64-pivot sub-blocks whose unit triangles go through
-// LDS. Items: forward triangle {k, kb: the block solved in the step before;
-// tk, tkb: this block}, forward chunk {rows [a0, a1), update by [k, k+kb)},
-// backward chunk {columns [a0, a1), contributions of rows [k, k+kb); flags
-// bit 0: atomic}, backward triangle {k, kb: block solved before (or the
-// rows below the pivots); tk, tkb}.
+// triangle costs two launches per kLS pivots), each solved by its triangle
+// item as up to four 64-pivot sub-blocks. Items: forward triangle {tk, tkb:
+// this block; kItemFused: then the rows [a0, a1) below it}, forward chunk
+// {rows [a0, a1), update by the block [k, k+kb)}, backward chunk {columns
+// [a0, a1), contributions of rows [k, k+kb); kItemAtomic}, backward
+// triangle {tk, tkb; k, kb: rows below the pivots whose contributions it
+// takes itself}. Triangles of more than kLB pivots (kItemWide) have kernels
+// of their own. Every item takes NR right-hand sides at a time, so L is read
+// once for all of them.
 constexpr int kLB = 64;    // sub-block: a unit triangle in LDS, substituted by one wave
 constexpr int kLS = 256;   // pivots per step
 constexpr int kLThreads = 256;
-constexpr int kLSeg = 512;  // rows of a backward tail item
-constexpr int32_t kItemTri = 2;
-constexpr int32_t kItemFused = 4;  // forward: the triangle, then the rows [a0, a1) below it in the same workgroup
+constexpr int kLWide = 512;   // threads of a wide triangle item
+constexpr int kLSeg = 512;    // rows of a backward tail item
 
-__device__ __forceinline__ double lwave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+__device__ __forceinline__ double lane_value(double v, int l) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
 }
 
-// sum_{c < kb} L(i, k + c) xs[c] (kb <= kLS) for row i = r0 + (tid & 63)
+// Sum over the wavefront of M (8 or 16) values per lane. Each halving step
+// exchanges half of the values with a partner lane, so the M sums end up in
+// different lanes: value e(lane) = the lane's top log2(M) bits. 32: the two
+// halves of the wavefront (v_permlane32_swap: {a.lo, b.lo}, {a.hi, b.hi}),
+// 16: rows of 16 lanes, 8 and 4: inside a row (rotation by 8, mirror of 8
+// lanes); the lanes that share e are then added.
+template <int ROW>
+__device__ __forceinline__ double swap_add(double a, double b) {
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    const unsigned al = __double2loint(a), ah = __double2hiint(a), bl = __double2loint(b), bh = __double2hiint(b);
+    u2 l, h;
+    if constexpr (ROW == 32) {
+        l = __builtin_amdgcn_permlane32_swap(al, bl, false, false);
+        h = __builtin_amdgcn_permlane32_swap(ah, bh, false, false);
+    } else {
+        l = __builtin_amdgcn_permlane16_swap(al, bl, false, false);
+        h = __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
+    }
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, false),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, false));
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppRor8 = 0x128;
+template <int M>
+__device__ __forceinline__ double wave_sums(double (&v)[M]) {
+    static_assert(M == 8 || M == 16, "values per lane");
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int k = 0; k < M / 2; ++k) v[k] = swap_add<32>(v[k], v[k + M / 2]);
+#pragma unroll
+    for (int k = 0; k < M / 4; ++k) v[k] = swap_add<16>(v[k], v[k + M / 4]);
+#pragma unroll
+    for (int k = 0; k < M / 8; ++k) {
+        const double keep = lane & 8 ? v[k + M / 8] : v[k], give = lane & 8 ? v[k] : v[k + M / 8];
+        v[k] = keep + dpp_move<kDppRor8>(give);
+    }
+    double t = v[0];
+    if constexpr (M == 16) {
+        const double keep = lane & 4 ? v[1] : v[0], give = lane & 4 ? v[0] : v[1];
+        t = keep + dpp_move<kDppHalfMirror>(give);
+    }
+    t += dpp_move<kDppXor1>(t);
+    t += dpp_move<kDppXor2>(t);
+    if constexpr (M == 8) t += dpp_move<kDppHalfMirror>(t);
+    return t;
+}
+template <int M>
+__device__ __forceinline__ int wave_sums_index() {
+    return (threadIdx.x & 63) >> (M == 16 ? 2 : 3);
+}
+
+// sum_{c < kb} L(i, k + c) xs[r][c] (kb <= kLS) for row i = r0 + (tid & 63)
 // (< r1), wave w taking the columns [w q, (w + 1) q), q = ceil(kb / 4),
-// in order; the total ((w0 + w1) + (w2 + w3)) lands in part[0][row]. The
+// in order; the total ((w0 + w1) + (w2 + w3)) lands in part[r][0][row]. The
 // loads go out 16 columns at a time (clamped addresses, masked values), so
 // a workgroup waits on a column group's latency, not each column's.
+template <int NR, int XS>
 __device__ __forceinline__ void rows_times_block(const double *L, int f, int k, int kb, int r0, int r1,
-                                                 const double *xs, double (*part)[kLB]) {
+                                                 const double (*xs)[XS], double (*part)[4][kLB]) {
     constexpr int kG = 16;
     const int row = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int i = min(r0 + row, r1 - 1);
     const int q = (kb + 3) >> 2;
     const int cb = w * q, ce = min(kb, cb + q);
-    double acc = 0.0;
-    if (r0 + row < r1 && ce > cb) {
+    double acc[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) acc[r] = 0.0;
+    if (ce > cb) {
         const double *Lc = L + static_cast<int64_t>(k) * f + i;
         for (int c = cb; c < ce; c += kG) {
             double lv[kG];
@@ -462,12 +519,19 @@ __device__ __forceinline__ void rows_times_block(const double *L, int f, int k, 
             for (int j = 0; j < kG; ++j) lv[j] = Lc[static_cast<int64_t>(min(c + j, ce - 1)) * f];
 #pragma unroll
             for (int j = 0; j < kG; ++j)
-                if (c + j < ce) acc += lv[j] * xs[c + j];
+                if (c + j < ce) {
+#pragma unroll
+                    for (int r = 0; r < NR; ++r) acc[r] += lv[j] * xs[r][c + j];
+                }
         }
     }
-    part[w][row] = acc;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) part[r][w][row] = acc[r];
     __syncthreads();
-    if (w == 0) part[0][row] = (part[0][row] + part[1][row]) + (part[2][row] + part[3][row]);
+    if (w < NR) {
+        double(*p)[kLB] = part[w];
+        p[0][row] = (p[0][row] + p[1][row]) + (p[2][row] + p[3][row]);
+    }
     __syncthreads();
 }
 
@@ -479,68 +543,242 @@ __device__ __forceinline__ void load_unit_triangle(const double *L, int f, int c
     }
 }
 
+// One wavefront's substitution with the unit triangle T (zero on and above
+// the diagonal and past the block): lane l holds y_l. Bound by the 64
+// dependent steps; T's values are read 16 steps ahead of the chain, the
+// solved value is broadcast through scalar registers (through LDS a step
+// took about 150 cycles, here about 30).
+__device__ __forceinline__ double unit_forward(const double (*T)[kLB + 1], double yv, int nc) {
+    const int l = threadIdx.x & 63;
+#pragma unroll
+    for (int c0 = 0; c0 < kLB; c0 += 16) {
+        if (c0 >= nc) break;
+        double t[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) t[u] = T[c0 + u][l];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) yv -= t[u] * lane_value(yv, c0 + u);
+    }
+    return yv;
+}
+__device__ __forceinline__ double unit_backward(const double (*T)[kLB + 1], double yv, int nc) {
+    const int l = threadIdx.x & 63;
+#pragma unroll
+    for (int c0 = kLB - 16; c0 >= 0; c0 -= 16) {
+        if (c0 >= nc) continue;
+        double t[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) t[u] = T[l][c0 + u];
+#pragma unroll
+        for (int u = 15; u >= 0; --u) yv -= t[u] * lane_value(yv, c0 + u);
+    }
+    return yv;
+}
+
+template <int NR>
 __global__ __launch_bounds__(kLThreads) void k_ldlt_fwd_step(LdltDev d, const SolveItem *__restrict__ items,
                                                             double *__restrict__ y, int32_t n, int32_t nrhs) {
-    __shared__ double xs[kLS];  // the block solved in the step before
-    __shared__ double xc[kLS];  // this item's block as it is solved
-    __shared__ double part[4][kLB];
-    __shared__ double part2[4][kLB];
+    static_assert(NR <= kLThreads / 64, "one wave per right-hand side in the triangles");
+    __shared__ double xs[NR][kLS];  // the block solved (in the step before, or here)
+    __shared__ double part[NR][4][kLB];
     __shared__ double T[kLB][kLB + 1];
     const SolveItem it = items[blockIdx.x];
     const FrontLd F = d.fronts[it.s];
     const int f = F.f, p = F.pstore;
     const double *L = d.fac + F.lofs;
     const int32_t *rows = d.rows + F.rofs;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const bool tri = (it.flags & kItemTri) != 0;
-    for (int r = 0; r < nrhs; ++r) {
-        double *yr = y + static_cast<int64_t>(r) * n;
-        for (int t = tid; t < it.kb; t += kLThreads) xs[t] = yr[rows[it.k + t]];
-        __syncthreads();
+    if (tri) load_unit_triangle(L, f, it.tk, it.tkb, T);
+    for (int r0 = 0; r0 < nrhs; r0 += NR) {
+        const int nr = min(NR, nrhs - r0);
+        double *yr = y + static_cast<int64_t>(r0) * n;
         if (tri) {
-            const int nsub = (it.tkb + kLB - 1) / kLB;
-            for (int sb = 0; sb < nsub; ++sb) {
-                const int c0 = it.tk + sb * kLB, nc = min(kLB, it.tkb - sb * kLB);
-                load_unit_triangle(L, f, c0, nc, T);
-                // the sub-block's rows: by the block before (when the item
-                // carries it), then by this block's solved sub-blocks
-                if (it.kb > 0) rows_times_block(L, f, it.k, it.kb, c0, c0 + nc, xs, part);
-                if (sb > 0) rows_times_block(L, f, it.tk, sb * kLB, c0, c0 + nc, xc, part2);
-                else __syncthreads();  // the triangle in LDS
-                if (tid < 64) {
-                    const int l = tid;
-                    double yv = l < nc ? yr[rows[c0 + l]] : 0.0;
-                    if (it.kb > 0) yv -= part[0][l];
-                    if (sb > 0) yv -= part2[0][l];
-                    for (int c = 0; c < nc; ++c) {
-                        const double xv = __shfl(yv, c, 64);
-                        if (l > c) yv -= T[c][l] * xv;
-                    }
-                    if (l < nc) {
-                        yr[rows[c0 + l]] = yv;
-                        xc[sb * kLB + l] = yv;
-                    }
-                }
-                __syncthreads();
+            __syncthreads();  // the triangle in LDS
+            if (w < nr) {
+                double *yw = yr + static_cast<int64_t>(w) * n;
+                const bool in = lane < it.tkb;
+                const int32_t g = rows[it.tk + min(lane, it.tkb - 1)];
+                const double yv = unit_forward(T, in ? yw[g] : 0.0, it.tkb);
+                if (in) yw[g] = yv;
+                xs[w][lane] = in ? yv : 0.0;
+            } else if (w < NR) {
+                xs[w][lane] = 0.0;
             }
+            __syncthreads();
             if (it.flags & kItemFused) {
-                // the rows below, with the block just solved (the same sums
-                // as the separate row items of the next step)
+                // the rows below, with the block just solved
                 for (int rb = it.a0; rb < it.a1; rb += kLB) {
                     const int re = min(rb + kLB, it.a1);
-                    rows_times_block(L, f, it.tk, it.tkb, rb, re, xc, part);
-                    if (tid < 64 && rb + tid < re) atomicAdd(&yr[rows[rb + tid]], -part[0][tid]);
+                    rows_times_block<NR>(L, f, it.tk, it.tkb, rb, re, xs, part);
+                    if (w < nr && rb + lane < re)
+                        unsafeAtomicAdd(&yr[static_cast<int64_t>(w) * n + rows[rb + lane]], -part[w][0][lane]);
                     __syncthreads();
                 }
             }
         } else {
-            rows_times_block(L, f, it.k, it.kb, it.a0, it.a1, xs, part);
-            if (tid < 64) {
-                const int i = it.a0 + tid;
-                if (i < it.a1) {
-                    if (i >= p) atomicAdd(&yr[rows[i]], -part[0][tid]);
-                    else yr[rows[i]] -= part[0][tid];
+            for (int e = tid; e < NR * kLS; e += kLThreads) {
+                const int r = e / kLS, t = e % kLS;
+                xs[r][t] = (r < nr && t < it.kb) ? yr[static_cast<int64_t>(r) * n + rows[it.k + t]] : 0.0;
+            }
+            __syncthreads();
+            rows_times_block<NR>(L, f, it.k, it.kb, it.a0, it.a1, xs, part);
+            const int i = it.a0 + lane;
+            if (w < nr && i < it.a1) {
+                double *dst = &yr[static_cast<int64_t>(w) * n + rows[i]];
+                if (i >= p) unsafeAtomicAdd(dst, -part[w][0][lane]);
+                else *dst -= part[w][0][lane];
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// Wide triangles (kLB < tkb <= kLS), one workgroup of 512: the whole
+// triangle is read into registers up front (its ten 64 x 64 blocks, eight
+// columns of each per wave, lane = row: one memory latency instead of one
+// per sub-block), then per sub-block one wave per right-hand side
+// substitutes with the block's unit triangle from LDS and every wave applies
+// its columns to the rows below. Bound by the substitution chains and the
+// read of the triangle by one CU. One step of a 43,245-row KKT's sweeps took
+// 54 us forward and 67 us backward with the blocks read in turn and the
+// right-hand sides one after the other.
+constexpr int kTriBlocks = 10;
+__host__ __device__ constexpr int tri_block(int i, int j) { return i * (i + 1) / 2 + j; }
+
+__device__ __forceinline__ void load_wide_triangle(const double *L, int f, int tk, int tkb,
+                                                   double (&R)[kTriBlocks][8]) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (64 * i >= tkb) break;
+        const int row = tk + min(64 * i + lane, tkb - 1);
+#pragma unroll
+        for (int j = 0; j <= i; ++j)
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                R[tri_block(i, j)][e] = L[static_cast<int64_t>(tk + min(64 * j + 8 * w + e, tkb - 1)) * f + row];
+    }
+}
+// sub-block j's unit triangle to LDS
+__device__ __forceinline__ void put_unit_triangle(const double (&v)[8], int nc, double (*T)[kLB + 1]) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) T[8 * w + e][lane] = (lane > 8 * w + e && lane < nc) ? v[e] : 0.0;
+}
+
+template <int NR>
+__global__ __launch_bounds__(kLWide) void k_ldlt_fwd_tri(LdltDev d, const SolveItem *__restrict__ items,
+                                                         double *__restrict__ y, int32_t n, int32_t nrhs) {
+    __shared__ double T[kLB][kLB + 1];
+    __shared__ double Y[NR][kLS];
+    __shared__ double part[NR][8][kLS - kLB];
+    const SolveItem it = items[blockIdx.x];
+    const FrontLd F = d.fronts[it.s];
+    const int f = F.f, tk = it.tk, tkb = it.tkb;
+    const int32_t *rows = d.rows + F.rofs + tk;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    double R[kTriBlocks][8];
+    load_wide_triangle(d.fac + F.lofs, f, tk, tkb, R);
+    for (int r0 = 0; r0 < nrhs; r0 += NR) {
+        const int nr = min(NR, nrhs - r0);
+        double *yr = y + static_cast<int64_t>(r0) * n;
+        for (int e = tid; e < NR * kLS; e += kLWide) {
+            const int r = e / kLS, t = e % kLS;
+            Y[r][t] = (r < nr && t < tkb) ? yr[static_cast<int64_t>(r) * n + rows[t]] : 0.0;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (64 * j >= tkb) break;
+            put_unit_triangle(R[tri_block(j, j)], tkb - 64 * j, T);
+            __syncthreads();
+            if (w < nr) {
+                const double yv = unit_forward(T, Y[w][64 * j + lane], tkb - 64 * j);
+                Y[w][64 * j + lane] = yv;
+                if (64 * j + lane < tkb) yr[static_cast<int64_t>(w) * n + rows[64 * j + lane]] = yv;
+            }
+            __syncthreads();
+            if (j == 3 || 64 * (j + 1) >= tkb) break;
+            const int nbelow = tkb - 64 * (j + 1);
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                double x[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = Y[r][64 * j + 8 * w + e];
+#pragma unroll
+                for (int i = j + 1; i < 4; ++i) {
+                    if (64 * i >= tkb) break;
+                    double acc = 0.0;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) acc += R[tri_block(i, j)][e] * x[e];
+                    part[r][w][64 * (i - j - 1) + lane] = acc;
                 }
+            }
+            __syncthreads();
+            for (int e = tid; e < NR * (kLS - kLB); e += kLWide) {
+                const int r = e / (kLS - kLB), t = e % (kLS - kLB);
+                if (t < nbelow) {
+                    double acc = 0.0;
+#pragma unroll
+                    for (int g = 0; g < 8; ++g) acc += part[r][g][t];
+                    Y[r][64 * (j + 1) + t] -= acc;
+                }
+            }
+        }
+        __syncthreads();
+    }
+}
+
+template <int NR>
+__global__ __launch_bounds__(kLWide) void k_ldlt_bwd_tri(LdltDev d, const SolveItem *__restrict__ items,
+                                                         double *__restrict__ y, int32_t n, int32_t nrhs) {
+    __shared__ double T[kLB][kLB + 1];
+    __shared__ double X[NR][kLS];
+    __shared__ double U[NR][kLB];
+    const SolveItem it = items[blockIdx.x];
+    const FrontLd F = d.fronts[it.s];
+    const int f = F.f, tk = it.tk, tkb = it.tkb;
+    const int32_t *rows = d.rows + F.rofs + tk;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    double R[kTriBlocks][8];
+    load_wide_triangle(d.fac + F.lofs, f, tk, tkb, R);
+    for (int r0 = 0; r0 < nrhs; r0 += NR) {
+        const int nr = min(NR, nrhs - r0);
+        double *yr = y + static_cast<int64_t>(r0) * n;
+        for (int e = tid; e < NR * kLS; e += kLWide) {
+            const int r = e / kLS, t = e % kLS;
+            X[r][t] = (r < nr && t < tkb) ? yr[static_cast<int64_t>(r) * n + rows[t]] : 0.0;
+        }
+#pragma unroll
+        for (int j = 3; j >= 0; --j) {
+            if (64 * j >= tkb) continue;
+            __syncthreads();  // the sub-block solved before (or X) in LDS, its triangle read
+            const bool below = j < 3 && 64 * (j + 1) < tkb;
+            put_unit_triangle(R[tri_block(j, j)], tkb - 64 * j, T);
+            if (below) {
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    double acc[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) acc[e] = 0.0;
+#pragma unroll
+                    for (int i = j + 1; i < 4; ++i) {
+                        if (64 * i >= tkb) break;
+                        const double x = X[r][64 * i + lane];
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) acc[e] += R[tri_block(i, j)][e] * x;
+                    }
+                    const double v = wave_sums<8>(acc);
+                    if ((lane & 7) == 0) U[r][8 * w + wave_sums_index<8>()] = v;
+                }
+            }
+            __syncthreads();
+            if (w < nr) {
+                double yv = X[w][64 * j + lane];
+                if (below) yv -= U[w][lane];
+                yv = unit_backward(T, yv, tkb - 64 * j);
+                X[w][64 * j + lane] = yv;
+                if (64 * j + lane < tkb) yr[static_cast<int64_t>(w) * n + rows[64 * j + lane]] = yv;
             }
         }
         __syncthreads();
@@ -550,111 +788,123 @@ __global__ __launch_bounds__(kLThreads) void k_ldlt_fwd_step(LdltDev d, const So
 // Backward contributions of rows [k, k + kb) (values xs) to the columns
 // [c0, c1): each wave takes 16 columns at a time, its lanes the rows t =
 // lane + 64 m in order, the 16 columns' loads of one m in flight together;
-// out(c, sum) from lane 0.
-template <class Out>
-__device__ __forceinline__ void cols_times_rows(const double *L, int f, int k, int kb, int c0, int c1, const double *xs,
-                                                Out &&out) {
+// out(r, c, sum) once per column and right-hand side.
+template <int NR, class Out>
+__device__ __forceinline__ void cols_times_rows(const double *L, int f, int k, int kb, int c0, int c1,
+                                                const double (*xs)[kLSeg], Out &&out) {
     constexpr int kG = 16;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     for (int cb = c0 + w * kG; cb < c1; cb += 4 * kG) {
-        double acc[kG];
+        double acc[NR][kG];
 #pragma unroll
-        for (int j = 0; j < kG; ++j) acc[j] = 0.0;
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+            for (int j = 0; j < kG; ++j) acc[r][j] = 0.0;
         for (int t0 = 0; t0 < kb; t0 += 64) {
-            const int t = t0 + lane;
-            const bool tin = t < kb;
-            const double xv = tin ? xs[t] : 0.0;
-            const int tc = min(t, kb - 1);
+            const int t = min(t0 + lane, kb - 1);
             double lv[kG];
 #pragma unroll
-            for (int j = 0; j < kG; ++j) lv[j] = L[static_cast<int64_t>(min(cb + j, c1 - 1)) * f + k + tc];
+            for (int j = 0; j < kG; ++j) lv[j] = L[static_cast<int64_t>(min(cb + j, c1 - 1)) * f + k + t];
 #pragma unroll
-            for (int j = 0; j < kG; ++j)
-                if (tin) acc[j] += lv[j] * xv;
+            for (int r = 0; r < NR; ++r) {
+                const double xv = t0 + lane < kb ? xs[r][t] : 0.0;
+#pragma unroll
+                for (int j = 0; j < kG; ++j) acc[r][j] += lv[j] * xv;
+            }
         }
 #pragma unroll
-        for (int j = 0; j < kG; ++j) {
-            const double v = lwave_sum(acc[j]);
-            if (lane == 0 && cb + j < c1) out(cb + j, v);
+        for (int r = 0; r < NR; ++r) {
+            const double v = wave_sums<kG>(acc[r]);
+            const int c = cb + wave_sums_index<kG>();
+            if ((lane & 3) == 0 && c < c1) out(r, c, v);
         }
     }
 }
 
+template <int NR>
 __global__ __launch_bounds__(kLThreads) void k_ldlt_bwd_step(LdltDev d, const SolveItem *__restrict__ items,
                                                             double *__restrict__ y, int32_t n, int32_t nrhs) {
-    __shared__ double xs[kLSeg];
-    __shared__ double xc[kLS];
-    __shared__ double upd[kLS];
-    __shared__ double upd2[kLB];
+    static_assert(NR <= kLThreads / 64, "one wave per right-hand side in the triangles");
+    __shared__ double xs[NR][kLSeg];
+    __shared__ double upd[NR][kLB];
     __shared__ double T[kLB][kLB + 1];
     const SolveItem it = items[blockIdx.x];
     const FrontLd F = d.fronts[it.s];
     const int f = F.f;
     const double *L = d.fac + F.lofs;
     const int32_t *rows = d.rows + F.rofs;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const bool tri = (it.flags & kItemTri) != 0;
-    for (int r = 0; r < nrhs; ++r) {
-        double *yr = y + static_cast<int64_t>(r) * n;
-        for (int t = tid; t < it.kb; t += kLThreads) xs[t] = yr[rows[it.k + t]];
+    if (tri) load_unit_triangle(L, f, it.tk, it.tkb, T);
+    for (int r0 = 0; r0 < nrhs; r0 += NR) {
+        const int nr = min(NR, nrhs - r0);
+        double *yr = y + static_cast<int64_t>(r0) * n;
+        for (int e = tid; e < NR * kLSeg; e += kLThreads) {
+            const int r = e / kLSeg, t = e % kLSeg;
+            if (t < it.kb) xs[r][t] = r < nr ? yr[static_cast<int64_t>(r) * n + rows[it.k + t]] : 0.0;
+        }
         __syncthreads();
         if (!tri) {
-            cols_times_rows(L, f, it.k, it.kb, it.a0, it.a1, xs, [&](int c, double acc) {
-                if (it.flags & 1) atomicAdd(&yr[rows[c]], -acc);
-                else yr[rows[c]] -= acc;
+            cols_times_rows<NR>(L, f, it.k, it.kb, it.a0, it.a1, xs, [&](int r, int c, double acc) {
+                if (r >= nr) return;
+                double *dst = &yr[static_cast<int64_t>(r) * n + rows[c]];
+                if (it.flags & kItemAtomic) unsafeAtomicAdd(dst, -acc);
+                else *dst -= acc;
             });
             __syncthreads();
             continue;
         }
-        // the block's columns: contributions of the rows solved before
+        // the block's columns: contributions of the rows below the pivots
         // (when the item carries them)
-        if (it.kb > 0)
-            cols_times_rows(L, f, it.k, it.kb, it.tk, it.tk + it.tkb, xs,
-                            [&](int c, double acc) { upd[c - it.tk] = acc; });
-        else
-            for (int c = tid; c < it.tkb; c += kLThreads) upd[c] = 0.0;
-        __syncthreads();
-        const int nsub = (it.tkb + kLB - 1) / kLB;
-        for (int sb = nsub - 1; sb >= 0; --sb) {
-            const int c0 = it.tk + sb * kLB, nc = min(kLB, it.tkb - sb * kLB);
-            const int e0 = c0 + nc, e1 = it.tk + it.tkb;  // this block's sub-blocks solved so far
-            load_unit_triangle(L, f, c0, nc, T);
-            cols_times_rows(L, f, e0, e1 - e0, c0, c0 + nc, xc + (e0 - it.tk),
-                            [&](int c, double acc) { upd2[c - c0] = acc; });
-            __syncthreads();
-            if (tid < 64) {
-                const int l = tid;
-                double yv = l < nc ? (yr[rows[c0 + l]] - upd[sb * kLB + l]) - (e1 > e0 ? upd2[l] : 0.0) : 0.0;
-                for (int c = nc - 1; c >= 0; --c) {
-                    const double xv = __shfl(yv, c, 64);
-                    if (l < c) yv -= T[l][c] * xv;
-                }
-                if (l < nc) {
-                    yr[rows[c0 + l]] = yv;
-                    xc[sb * kLB + l] = yv;
-                }
-            }
+        if (it.kb > 0) {
+            cols_times_rows<NR>(L, f, it.k, it.kb, it.tk, it.tk + it.tkb, xs,
+                                [&](int r, int c, double acc) { upd[r][c - it.tk] = acc; });
             __syncthreads();
         }
+        if (w < nr) {
+            double *yw = yr + static_cast<int64_t>(w) * n;
+            const bool in = lane < it.tkb;
+            const int32_t g = rows[it.tk + min(lane, it.tkb - 1)];
+            double yv = in ? yw[g] : 0.0;
+            if (it.kb > 0 && in) yv -= upd[w][lane];
+            yv = unit_backward(T, yv, it.tkb);
+            if (in) yw[g] = yv;
+        }
+        __syncthreads();
     }
 }
 
 }  // namespace
 
-void launch_ldlt_fwd_step(hipStream_t st, const LdltDev &d, const SolveItem *items, int64_t count, double *y,
-                          int32_t n, int32_t nrhs) {
-    if (count <= 0) return;
-    for (int64_t o = 0; o < count; o += kMaxLaunchGroups)
-        k_ldlt_fwd_step<<<dim3(static_cast<unsigned>(std::min(kMaxLaunchGroups, count - o))), kLThreads, 0, st>>>(
-            d, items + o, y, n, nrhs);
+// right-hand sides per pass of an item: the smallest of 1, 2, 4 that covers
+// them, 4 when there are more (a triangle's waves; accumulators in registers)
+template <class Go>
+static void by_rhs(int32_t nrhs, Go &&go) {
+    if (nrhs == 1) go(std::integral_constant<int, 1>{});
+    else if (nrhs == 2) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, 4>{});
 }
 
-void launch_ldlt_bwd_step(hipStream_t st, const LdltDev &d, const SolveItem *items, int64_t count, double *y,
-                          int32_t n, int32_t nrhs) {
-    if (count <= 0) return;
-    for (int64_t o = 0; o < count; o += kMaxLaunchGroups)
-        k_ldlt_bwd_step<<<dim3(static_cast<unsigned>(std::min(kMaxLaunchGroups, count - o))), kLThreads, 0, st>>>(
-            d, items + o, y, n, nrhs);
+void launch_ldlt_fwd_step(hipStream_t st, const LdltDev &d, const SolveItem *items, int64_t count, bool wide,
+                          double *y, int32_t n, int32_t nrhs) {
+    for (int64_t o = 0; o < count; o += kMaxLaunchGroups) {
+        const dim3 grid(static_cast<unsigned>(std::min(kMaxLaunchGroups, count - o)));
+        by_rhs(nrhs, [&](auto nr) {
+            if (wide) k_ldlt_fwd_tri<decltype(nr)::value><<<grid, kLWide, 0, st>>>(d, items + o, y, n, nrhs);
+            else k_ldlt_fwd_step<decltype(nr)::value><<<grid, kLThreads, 0, st>>>(d, items + o, y, n, nrhs);
+        });
+    }
+}
+
+void launch_ldlt_bwd_step(hipStream_t st, const LdltDev &d, const SolveItem *items, int64_t count, bool wide,
+                          double *y, int32_t n, int32_t nrhs) {
+    for (int64_t o = 0; o < count; o += kMaxLaunchGroups) {
+        const dim3 grid(static_cast<unsigned>(std::min(kMaxLaunchGroups, count - o)));
+        by_rhs(nrhs, [&](auto nr) {
+            if (wide) k_ldlt_bwd_tri<decltype(nr)::value><<<grid, kLWide, 0, st>>>(d, items + o, y, n, nrhs);
+            else k_ldlt_bwd_step<decltype(nr)::value><<<grid, kLThreads, 0, st>>>(d, items + o, y, n, nrhs);
+        });
+    }
 }
 
 void launch_sweep(hipStream_t st, const DevPtrs &d, bool forward, const SolveItem *items, const int32_t *step_of,

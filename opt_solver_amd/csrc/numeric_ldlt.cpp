@@ -427,38 +427,43 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
 }
 
 // Step lists of the blocked sweeps from the realized fronts (pivots per
-// front known after the factorization): 64-pivot blocks; forward steps
-// solve block t after block t-1's update of its rows, while chunk items
-// apply that update to the rest of the front (64-row chunks, rows past the
-// pivots by atomic add); backward steps first take the contributions of
-// the rows past the pivots (512-row segments, atomic), then solve the
-// blocks last to first, chunk items applying each solved block to the
-// columns before it. One launch per step covers every front of a level.
+// front known after the factorization): 256-pivot blocks; forward: each
+// block's triangle, then row items applying it to the rest of the front
+// (64-row chunks, rows past the pivots by atomic add); backward: the
+// contributions of the rows past the pivots (512-row segments, atomic), then
+// the blocks last to first, column items applying each solved block to the
+// columns before it. One launch per step and kind of item covers every
+// front of a level.
 // The items of one front's forward (bwd = false) or backward sweep, step
 // by step: emit(step, item).
 template <class Emit>
 static void front_solve_items(int32_t f, int32_t p, int32_t s, bool bwd, Emit &&emit) {
     // B pivots per step (the kernels solve them as 64-pivot sub-blocks),
     // chunks of C rows (forward) or columns (backward)
-    constexpr int32_t B = 256, C = 64, Seg = 512, Tri = 2;
+    // a triangle of more than C pivots is wide: a kernel of its own, and the
+    // rows below it items of their own (one workgroup would read them alone)
+    constexpr int32_t B = 256, C = 64, Seg = 512;
+    const auto tri = [&](int32_t tk, int32_t tkb) {
+        return SolveItem{s, 0, 0, 0, 0, tk, tkb, kItemTri | (tkb > C ? kItemWide : 0)};
+    };
     if (p <= 0) return;
     const int32_t nb = (p + B - 1) / B;
     if (!bwd) {
-        constexpr int32_t Fused = 4, FusedRows = 512;
-        if (nb == 1 && f > p && f - p <= FusedRows) {
+        constexpr int32_t FusedRows = 512;
+        if (p <= C && f > p && f - p <= FusedRows) {
             // one workgroup: the triangle, then the rows below it
-            emit(0, SolveItem{s, 0, 0, p, f, 0, p, Tri | Fused});
+            emit(0, SolveItem{s, 0, 0, p, f, 0, p, kItemTri | kItemFused});
             return;
         }
         // block b: a step of row items applying block b - 1 to every row
         // from block b down, then a step of its triangle item alone (so the
         // triangle's one workgroup does no more than the block's own work)
         int32_t t = 0;
-        emit(t++, SolveItem{s, 0, 0, 0, 0, 0, std::min(B, p), Tri});
+        emit(t++, tri(0, std::min(B, p)));
         for (int32_t b = 1; b < nb; ++b, ++t) {
             const int32_t tk = b * B, tkb = std::min(B, p - tk), k = tk - B;
             for (int32_t r = tk; r < f; r += C) emit(t, SolveItem{s, k, B, r, std::min(r + C, f), 0, 0, 0});
-            emit(++t, SolveItem{s, 0, 0, 0, 0, tk, tkb, Tri});
+            emit(++t, tri(tk, tkb));
         }
         if (f > p) {
             const int32_t k = (nb - 1) * B;
@@ -466,26 +471,26 @@ static void front_solve_items(int32_t f, int32_t p, int32_t s, bool bwd, Emit &&
         }
         return;
     }
-    if (nb == 1 && f > p && f - p <= Seg) {
+    if (p <= C && f > p && f - p <= Seg) {
         // one workgroup: the rows below (one segment) folded into the
         // triangle item's own column sums, then the triangle
-        emit(0, SolveItem{s, p, f - p, 0, 0, 0, p, Tri});
+        emit(0, SolveItem{s, p, f - p, 0, 0, 0, p, kItemTri});
         return;
     }
     int32_t t = 0;
     if (f > p) {
         for (int32_t r = p; r < f; r += Seg)
-            for (int32_t c = 0; c < p; c += C) emit(0, SolveItem{s, r, std::min(Seg, f - r), c, std::min(c + C, p), 0, 0, 1});
+            for (int32_t c = 0; c < p; c += C) emit(0, SolveItem{s, r, std::min(Seg, f - r), c, std::min(c + C, p), 0, 0, kItemAtomic});
         t = 1;
     }
     const int32_t kL = (nb - 1) * B;
-    emit(t++, SolveItem{s, 0, 0, 0, 0, kL, p - kL, Tri});
+    emit(t++, tri(kL, p - kL));
     // block j: a step of column items applying block j + 1 to every column
     // up to block j's last, then a step of its triangle item alone
     for (int32_t j = nb - 2; j >= 0; --j, ++t) {
         const int32_t tk = j * B, k = tk + B, kb = std::min(B, p - k);
         for (int32_t c = 0; c < tk + B; c += C) emit(t, SolveItem{s, k, kb, c, c + C, 0, 0, 0});
-        emit(++t, SolveItem{s, 0, 0, 0, 0, tk, B, Tri});
+        emit(++t, tri(tk, B));
     }
 }
 
@@ -503,14 +508,20 @@ static int ldlt_solve_lists(smfgpu_plan_s *P) {
     // front array; the passes below read these compact arrays
     const size_t ns = P->fronts.size();
     std::vector<int32_t> lf(ns), lp(ns);
+    P->max_pstore = 0;
     for (size_t s = 0; s < ns; ++s) {
         lf[s] = P->fl[s].f;
         lp[s] = P->fl[s].pstore;
+        P->max_pstore = std::max(P->max_pstore, lp[s]);
     }
     // counts per level and step give the steps' offsets; the items are then
     // written in place into pinned staging and uploaded once
+    // a step's wide triangles and its other items are two launches
+    const auto slot = [](int32_t t, const SolveItem &it) { return 2 * t + ((it.flags & kItemWide) ? 0 : 1); };
     auto build = [&](bool bwd, PinnedArr<SolveItem> &items, DBuf<SolveItem> &dev,
-                     std::vector<std::pair<int64_t, int64_t>> &steps, std::vector<int32_t> &lvs) -> int {
+                     std::vector<std::pair<int64_t, int64_t>> &steps, std::vector<uint8_t> &wide,
+                     std::vector<int32_t> &lvs) -> int {
+        wide.clear();
         std::vector<int32_t> lv_nstep(nlev, 0);
         std::vector<int64_t> lv_t0(nlev, 0), tfirst;
         int64_t total = 0;
@@ -518,15 +529,17 @@ static int ldlt_solve_lists(smfgpu_plan_s *P) {
             lvs[lv] = static_cast<int32_t>(steps.size());
             cnt.clear();
             for (int32_t s : P->level_fronts[lv])
-                front_solve_items(lf[s], lp[s], s, bwd, [&](int32_t t, const SolveItem &) {
-                    if (cnt.size() <= static_cast<size_t>(t)) cnt.resize(t + 1, 0);
-                    ++cnt[t];
+                front_solve_items(lf[s], lp[s], s, bwd, [&](int32_t t, const SolveItem &it) {
+                    const size_t e = slot(t, it);
+                    if (cnt.size() <= e) cnt.resize(e + 1, 0);
+                    ++cnt[e];
                 });
             lv_t0[lv] = static_cast<int64_t>(tfirst.size());
             for (size_t t = 0; t < cnt.size(); ++t) {
                 tfirst.push_back(total);  // first item of step index t (none if cnt[t] == 0)
                 if (cnt[t] > 0) {
                     steps.emplace_back(total, cnt[t]);
+                    wide.push_back(t % 2 == 0);
                     total += cnt[t];
                 }
             }
@@ -540,7 +553,7 @@ static int ldlt_solve_lists(smfgpu_plan_s *P) {
             // counting pass
             pos.assign(tfirst.begin() + lv_t0[lv], tfirst.begin() + lv_t0[lv] + lv_nstep[lv]);
             for (int32_t s : P->level_fronts[lv])
-                front_solve_items(lf[s], lp[s], s, bwd, [&](int32_t t, const SolveItem &it) { items[pos[t]++] = it; });
+                front_solve_items(lf[s], lp[s], s, bwd, [&](int32_t t, const SolveItem &it) { items[pos[slot(t, it)]++] = it; });
         }
         for (const auto &st : steps)
             if (st.second > INT32_MAX) return set_error(SMFGPU_ERR_ALLOC, "factor: solve step too large");
@@ -553,8 +566,8 @@ static int ldlt_solve_lists(smfgpu_plan_s *P) {
         return SMFGPU_OK;
     };
     int rc;
-    if ((rc = build(false, P->h_fwd_items, P->d_fwd_items, P->fwd_steps, P->fwd_lv)) ||
-        (rc = build(true, P->h_bwd_items, P->d_bwd_items, P->bwd_steps, P->bwd_lv)))
+    if ((rc = build(false, P->h_fwd_items, P->d_fwd_items, P->fwd_steps, P->fwd_wide, P->fwd_lv)) ||
+        (rc = build(true, P->h_bwd_items, P->d_bwd_items, P->bwd_steps, P->bwd_wide, P->bwd_lv)))
         return rc;
     HIP_OK(hipStreamSynchronize(P->stream));
     return SMFGPU_OK;
@@ -959,7 +972,7 @@ int ldlt_solve(smfgpu_plan_s *P, const double *b_dev, int64_t ldb, double *out_d
             for (int32_t lv = 0; lv < nl; ++lv)
                 for (int32_t i = P->fwd_lv[lv]; i < P->fwd_lv[lv + 1]; ++i)
                     launch_ldlt_fwd_step(st, d, P->d_fwd_items.p + P->fwd_steps[i].first, P->fwd_steps[i].second,
-                                         y, n, nr);
+                                         P->fwd_wide[i] != 0, y, n, nr);
         if (job == 2) launch_ldlt_diag_div(st, d, P->d_flist.p, static_cast<int32_t>(P->lv_flist_ofs[nl]), y, n, nr);
         if (job == 1 || job == 2) {
             // the permuted-order result
@@ -968,12 +981,12 @@ int ldlt_solve(smfgpu_plan_s *P, const double *b_dev, int64_t ldb, double *out_d
             continue;
         }
         if (job == 0 || job == 4)
-            launch_ldlt_diag(st, d, P->d_flist.p, static_cast<int32_t>(P->lv_flist_ofs[nl]), y, n, nr);
+            launch_ldlt_diag(st, d, P->d_flist.p, static_cast<int32_t>(P->lv_flist_ofs[nl]), P->max_pstore, y, n, nr);
         if (tm) HIP_OK(hipEventRecord(P->sev[1], st));
         for (int32_t lv = nl - 1; lv >= 0; --lv)
             for (int32_t i = P->bwd_lv[lv]; i < P->bwd_lv[lv + 1]; ++i)
                 launch_ldlt_bwd_step(st, d, P->d_bwd_items.p + P->bwd_steps[i].first, P->bwd_steps[i].second,
-                                     y, n, nr);
+                                     P->bwd_wide[i] != 0, y, n, nr);
         if (tm) {
             HIP_OK(hipEventRecord(P->sev[2], st));
             HIP_OK(hipStreamSynchronize(st));

@@ -153,18 +153,24 @@ void launch_ldlt_assemble(hipStream_t st, const LdltDev &d, const AsmTask *tasks
 // the rest (many workgroups per front)
 void launch_ldlt_epilogue(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, int32_t n_inline);
 void launch_ldlt_store(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, int32_t max_cols);
-void launch_ldlt_diag(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, double *y, int32_t n,
-                      int32_t nrhs);
+void launch_ldlt_diag(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, int32_t max_p, double *y,
+                      int32_t n, int32_t nrhs);
 // the diagonal-only solve job: D from the stored columns, by division
 void launch_ldlt_diag_div(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, double *y, int32_t n,
                           int32_t nrhs);
 void launch_front_patch(hipStream_t st, FrontLd *fronts, const FrontLd *patch, const int32_t *ids, int32_t np);
+// flags of the LDL^T sweeps' items
+constexpr int32_t kItemAtomic = 1;  // backward chunk: several items add to its columns
+constexpr int32_t kItemTri = 2;     // a block's triangle, else a chunk
+constexpr int32_t kItemFused = 4;   // forward: the triangle, then the rows [a0, a1) below it in the same workgroup
+constexpr int32_t kItemWide = 8;    // a triangle of more than 64 pivots
 // one step of the blocked forward / backward sweep (items of all fronts of
-// a level; SolveItem flags bit 1: triangle item)
-void launch_ldlt_fwd_step(hipStream_t st, const LdltDev &d, const SolveItem *items, int64_t count, double *y,
-                          int32_t n, int32_t nrhs);
-void launch_ldlt_bwd_step(hipStream_t st, const LdltDev &d, const SolveItem *items, int64_t count, double *y,
-                          int32_t n, int32_t nrhs);
+// a level); wide: the step's triangles of more than 64 pivots, else its
+// other items (the two are independent)
+void launch_ldlt_fwd_step(hipStream_t st, const LdltDev &d, const SolveItem *items, int64_t count, bool wide,
+                          double *y, int32_t n, int32_t nrhs);
+void launch_ldlt_bwd_step(hipStream_t st, const LdltDev &d, const SolveItem *items, int64_t count, bool wide,
+                          double *y, int32_t n, int32_t nrhs);
 // one iteration's pivot logic; with gpart set it first decides on the group
 // the stats launch evaluated (nch workgroups per front)
 void launch_big_panel(hipStream_t st, const LdltDev &d, BigLd *states, int32_t nbig, double u, double eff_small,

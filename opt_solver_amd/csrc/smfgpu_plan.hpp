@@ -237,6 +237,8 @@ struct smfgpu_plan_s {
     PinnedArr<SolveItem> h_fwd_items, h_bwd_items;  // LDL^T: staging of the solve items
     std::vector<std::pair<int64_t, int64_t>> fwd_steps, bwd_steps;
     std::vector<int32_t> fwd_lv, bwd_lv;
+    int32_t max_pstore = 0;                   // LDL^T: most stored pivots of a front
+    std::vector<uint8_t> fwd_wide, bwd_wide;  // LDL^T: per step, whether its items are wide triangles
     // SPD sweeps as one persistent launch each: the items in the order the
     // sweep takes them (forward: as stored; backward: levels from the root
     // down), the step of each, the item count of each step, and the

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from tests.conftest import gpu_available
-from tests.helpers import matvec
+from tests.helpers import dense_front_problem, matvec
 
 pytestmark = pytest.mark.gpu
 
@@ -54,3 +54,27 @@ def test_dense_cholesky_bad_pivot(n, bad):
         v[cp[bad]] += shift * 1e-3 - L[bad, bad] ** 2 * (1.0 if shift else 1.0 + 1e-9)
         fac = Plan(analyse((n, cp, ri, v)), posdef=True).factor(v)
         assert fac.status == 1
+
+
+@pytest.mark.parametrize("p,q", [(1, 0), (63, 65), (64, 512), (64, 513), (65, 1), (128, 64), (129, 700), (191, 3),
+                                 (192, 0), (193, 40), (255, 600), (256, 1), (257, 512), (320, 0), (513, 65)])
+def test_indefinite_sweep_edges(p, q):
+    """Sweeps of an LDL^T factor whose first front has p pivots and q rows
+    below them (a dense front of p + q rows split in two supernodes):
+    sub-blocks of 64, steps of 256, the fused limits of 64 pivots and 512
+    rows, every number of right-hand sides a pass holds. The matrix is a
+    random symmetric one plus an alternating diagonal of +-2 n, so its
+    solution is known to about n eps."""
+    n = p + q
+    print("case sweep", p, q, flush=True)
+    rng = np.random.default_rng([p, q])
+    M = rng.uniform(-1, 1, (n, n))
+    M = M + M.T + np.diag(2.0 * n * np.where(np.arange(n) % 3 == 0, -1.0, 1.0))
+    A, arrays = dense_front_problem(M, p)
+    fac = Plan(arrays, posdef=False).factor(A[3])
+    assert fac.status == 0
+    X = rng.uniform(-1, 1, (n, 7))
+    B = M @ X
+    for nr in (1, 2, 3, 7):
+        xs = fac.solve(B[:, :nr] if nr > 1 else B[:, 0]).reshape(n, nr)
+        assert np.abs(xs - X[:, :nr]).max() < 1e-13 * max(n, 10)
