@@ -38,7 +38,7 @@ KNOBS = [
     ("LDL^T device levels: largest symbolic front laid out on the device (rows)",
      "LDLT_DEVICE_FRONTS", [95, 64, 48], 95, ("batch", "kkt")),
     ("LDL^T fronts from this many rows take the multi-workgroup path (below: one workgroup)",
-     "LDLT_BIG_MIN", [256, 192, 384, 512], 256, ("kkt", "kkt_bf16x3")),
+     "LDLT_BIG_MIN", [96, 128, 192, 256], 96, ("kkt", "kkt_bf16x3")),
     ("LDL^T large fronts: workgroups of the MFMA update launches",
      "LDLT_UPDATE_WG", [1024, 512, 2048], 1024, ("kkt", "kkt_bf16x3")),
     ("LDL^T large fronts on bf16 planes: outer block (columns per flush)",

@@ -1076,17 +1076,17 @@ __device__ __forceinline__ void big_tile(const LdltDev &d, const FrontLd &F, con
 
 // Tiles [lo, hi) of a launch's range of nt for this workgroup's XCD, which
 // its workgroups stride over: workgroups are dispatched to the 8 XCDs round
-// robin by linear index, so with a multiple of 8 per front, blockIdx.x % 8
+// robin by linear index, so with a multiple of 8 per front, part % 8
 // is the XCD. Each XCD then works through a contiguous run of tiles (one
 // column block's operand panel stays in its L2) instead of every eighth.
 struct XcdRange {
     int lo, hi, step;
 };
-__device__ __forceinline__ XcdRange xcd_range(int nt) {
-    const int x = blockIdx.x & 7, per = gridDim.x >> 3;
+__device__ __forceinline__ XcdRange xcd_range(const BigPart &g, int nt) {
+    const int x = g.part & 7, per = g.parts >> 3;
     const int lo = static_cast<int>(static_cast<int64_t>(nt) * x / 8);
     const int hi = static_cast<int>(static_cast<int64_t>(nt) * (x + 1) / 8);
-    return XcdRange{lo + static_cast<int>(blockIdx.x >> 3), hi, per};
+    return XcdRange{lo + (g.part >> 3), hi, per};
 }
 
 __device__ __forceinline__ int big_tiles(int f, int c0, int c1) {
@@ -1346,28 +1346,30 @@ __global__ __launch_bounds__(64) void k_big_gdiag(LdltDev d, const BigLd *__rest
 // column maxima per pivot to the group buffer, each row's unscaled column
 // entries to W (the columns the panel kernel's pivots will have: W column
 // ps - pend0 + t, pend0 being the W base the panel kernel starts from) and
-// its final group entries to W's speculation columns [kGroupSpec,
-// kGroupSpec + 64). Nothing of the front square changes: a rejected panel
+// its final group entries to W's speculation columns [big_spec,
+// big_spec + 64). Nothing of the front square changes: a rejected panel
 // finds its columns as they were. W columns of rejected pivots are
 // rewritten (rows below the pivot) when those positions get their pivots.
 __global__ __launch_bounds__(kLT) void k_big_group(LdltDev d, const BigLd *__restrict__ states,
-                                                   double *__restrict__ gpart, int32_t nch) {
+                                                   const BigPart *__restrict__ grid, double *__restrict__ gpart,
+                                                   int32_t nch) {
     __shared__ double Wd[kGroupCols][kGroupCols + 1];
     __shared__ double Lm[kGroupCols][16];
     __shared__ double invd[kGroupCols], wgmax[kGroupCols];
     __shared__ double red[16][kLT + 1];
     __shared__ double red2[16][16];
-    const BigLd B = states[blockIdx.y];
+    const BigPart g = grid[blockIdx.x];
+    const BigLd B = states[g.front];
     const int ps = B.k, ncols = group_cols(B, 16);
     if (ncols <= 0) return;
     const FrontLd F = d.fronts[B.s];
     const int f = F.f;
     const int gend = ps + ncols;
-    const int bx = blockIdx.x;
+    const int bx = g.part;
     if (bx >= max(1, (f - gend + kGroupRows - 1) / kGroupRows)) return;
     const double *G = d.arena + F.fofs;
     double *W = d.work + F.wofs;
-    const double *gp = gpart + blockIdx.y * gpart_stride(nch);
+    const double *gp = gpart + g.front * gpart_stride(nch);
     const int64_t wcol0 = ps - B.pend0;  // W column of the group's first pivot
     const int tid = threadIdx.x;
     for (int e = tid; e < kGroupCols * kGroupCols; e += kLT) Wd[e >> 6][e & 63] = gp[kGdWd + e];
@@ -1385,11 +1387,11 @@ __global__ __launch_bounds__(kLT) void k_big_group(LdltDev d, const BigLd *__res
     // workgroup has)
     grow_run<true, false>(a, ncols, Wd, Lm, invd, red, red2, wgmax, W, wcol0, f, i, rowok);
     __syncthreads();
-    if (tid < ncols) gpart[blockIdx.y * gpart_stride(nch) + kGMax + bx * kGroupCols + tid] = wgmax[tid];
+    if (tid < ncols) gpart[g.front * gpart_stride(nch) + kGMax + bx * kGroupCols + tid] = wgmax[tid];
     if (rowok) {
 #pragma unroll
         for (int c = 0; c < kGroupCols; ++c)
-            if (c < ncols) W[static_cast<int64_t>(kGroupSpec + c) * f + i] = a[c];
+            if (c < ncols) W[static_cast<int64_t>(big_spec(F.ne) + c) * f + i] = a[c];
     }
 }
 
@@ -1401,18 +1403,20 @@ __global__ __launch_bounds__(kLT) void k_big_group(LdltDev d, const BigLd *__res
 // went through the same operations on the accepted columns as a row below
 // it would have.
 __global__ __launch_bounds__(kLT) void k_big_gapply(LdltDev d, const BigLd *__restrict__ states,
+                                                    const BigPart *__restrict__ grid,
                                                     const double *__restrict__ gpart, int32_t nch) {
-    const BigLd B = states[blockIdx.y];
+    const BigPart g = grid[blockIdx.x];
+    const BigLd B = states[g.front];
     if (!B.g_apply) return;
     const int ps = B.g_ps, nacc = B.g_n, ncols = B.g_cols;
     const FrontLd F = d.fronts[B.s];
     const int f = F.f;
     const int gend = ps + ncols;
-    const int bx = blockIdx.x;
+    const int bx = g.part;
     if (bx >= max(1, (f - gend + kGroupRows - 1) / kGroupRows)) return;
     double *G = d.arena + F.fofs;
     double *W = d.work + F.wofs;
-    const double *gp = gpart + blockIdx.y * gpart_stride(nch);
+    const double *gp = gpart + g.front * gpart_stride(nch);
     const int64_t wcol0 = ps - B.w_base;
     const int tid = threadIdx.x;
     if (bx == 0) {
@@ -1427,7 +1431,7 @@ __global__ __launch_bounds__(kLT) void k_big_gapply(LdltDev d, const BigLd *__re
     const int i = gend + bx * kGroupRows + tid;
     if (i < f) {
         // eight columns' loads in flight at a time
-        const double *src = W + static_cast<int64_t>(kGroupSpec) * f + i;
+        const double *src = W + static_cast<int64_t>(big_spec(F.ne)) * f + i;
         double *dst = G + static_cast<int64_t>(ps) * f + i;
         for (int c0 = 0; c0 < nacc; c0 += 8) {
             double v[8];
@@ -1636,6 +1640,9 @@ __global__ __launch_bounds__(kLT) void k_big_panel(LdltDev d, BigLd *states, Prm
             pend0 = k;
         }
     }
+    // every eligible column is a pivot: no second pass, and this iteration's
+    // updates are the last
+    if (pass == 0 && k >= ne) npass = 2;
     __syncthreads();
     if (tid == 0) {
         B.k = k;
@@ -1667,12 +1674,14 @@ __global__ __launch_bounds__(kLT) void k_big_panel(LdltDev d, BigLd *states, Prm
     }
 }
 
-// The requested update and flush of every front: grid (per_front, nbig),
-// tiles by grid stride.
+// The requested update and flush of every front, its tiles by stride over
+// its workgroups.
 template <int MODE>
-__global__ __launch_bounds__(kLT, 2) void k_big_update(LdltDev d, const BigLd *__restrict__ states) {
+__global__ __launch_bounds__(kLT, 2) void k_big_update(LdltDev d, const BigLd *__restrict__ states,
+                                                       const BigPart *__restrict__ grid) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[big_lds_bytes<MODE>()];
-    const BigLd B = states[blockIdx.y];
+    const BigPart g = grid[blockIdx.x];
+    const BigLd B = states[g.front];
     if (B.prec != MODE) return;  // another precision's launch
     const FrontLd F = d.fronts[B.s];
     const double *W = d.work + F.wofs;
@@ -1680,7 +1689,7 @@ __global__ __launch_bounds__(kLT, 2) void k_big_update(LdltDev d, const BigLd *_
     // BF16 modes on planes: the flush is k_big_wide's
     const bool wide = MODE >= 2 && d.xpl != nullptr;
     const int t2 = (!wide && B.x_p1 > B.x_p0) ? big_tiles(F.f, B.x_c0, F.ne) : 0;
-    const XcdRange xr = xcd_range(t1 + t2);
+    const XcdRange xr = xcd_range(g, t1 + t2);
     for (int tile = xr.lo; tile < xr.hi; tile += xr.step) {
         const bool u = tile < t1;
         big_tile<MODE>(d, F, W, B.w_base, u ? B.u_c0 : B.x_c0, u ? B.u_c1 : F.ne, u ? B.u_p0 : B.x_p0,
@@ -1730,9 +1739,11 @@ __global__ __launch_bounds__(kLT) void k_big_stall(LdltDev d, BigLd *states, int
 
 // L*D columns [c0, c1) of every done front, rows [ne, f), into W (the
 // column order of schur_update's fill_ld_column, ldlt_kernel.cpp:764-816)
-__global__ __launch_bounds__(kLT) void k_big_ld(LdltDev d, const BigLd *__restrict__ states, int32_t c0,
-                                               int32_t width, int32_t wide) {
-    const BigLd B = states[blockIdx.y];
+__global__ __launch_bounds__(kLT) void k_big_ld(LdltDev d, const BigLd *__restrict__ states,
+                                               const BigPart *__restrict__ grid, int32_t c0, int32_t width,
+                                               int32_t wide) {
+    const BigPart g = grid[blockIdx.x];
+    const BigLd B = states[g.front];
     if ((B.prec >= 2 && d.xpl != nullptr) != (wide != 0)) return;  // the other chunk width's fronts
     const FrontLd F = d.fronts[B.s];
     const int f = F.f, ne = F.ne, p = B.k;
@@ -1743,8 +1754,8 @@ __global__ __launch_bounds__(kLT) void k_big_ld(LdltDev d, const BigLd *__restri
     double *W = d.work + F.wofs;
     const int q = f - ne;
     const int64_t tot = static_cast<int64_t>(c1 - c0) * q;
-    for (int64_t idx = static_cast<int64_t>(blockIdx.x) * kLT + threadIdx.x; idx < tot;
-         idx += static_cast<int64_t>(gridDim.x) * kLT) {
+    for (int64_t idx = static_cast<int64_t>(g.part) * kLT + threadIdx.x; idx < tot;
+         idx += static_cast<int64_t>(g.parts) * kLT) {
         const int c = c0 + static_cast<int>(idx / q);
         const int j = ne + static_cast<int>(idx % q);
         const int8_t tg = tags[c];
@@ -1763,23 +1774,25 @@ __global__ __launch_bounds__(kLT) void k_big_ld(LdltDev d, const BigLd *__restri
 }
 
 template <int MODE>
-__global__ __launch_bounds__(kLT, 2) void k_big_cbupdate(LdltDev d, const BigLd *__restrict__ states, int32_t c0,
-                                                     int32_t width) {
+__global__ __launch_bounds__(kLT, 2) void k_big_cbupdate(LdltDev d, const BigLd *__restrict__ states,
+                                                         const BigPart *__restrict__ grid, int32_t c0,
+                                                         int32_t width) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[big_lds_bytes<MODE>()];
-    const BigLd B = states[blockIdx.y];
+    const BigPart g = grid[blockIdx.x];
+    const BigLd B = states[g.front];
     if (B.prec != MODE) return;
     const FrontLd F = d.fronts[B.s];
     const int c1 = min(B.k, c0 + width);
     if (c1 <= c0 || F.ne >= F.f) return;
     const double *W = d.work + F.wofs;
-    const XcdRange xr = xcd_range(big_tiles(F.f, F.ne, F.f));
+    const XcdRange xr = xcd_range(g, big_tiles(F.f, F.ne, F.f));
     for (int tile = xr.lo; tile < xr.hi; tile += xr.step) {
         big_tile<MODE>(d, F, W, c0, F.ne, F.f, c0, c1, tile, smem);
         __syncthreads();
     }
 }
 
-// 256 x 256 tile of the rank-kBigWork updates on the bf16 planes (modes 2,
+// 256 x 256 tile of the outer-block updates on the bf16 planes (modes 2,
 // 3): C[i][j] -= sum_c A[i][c] B[j][c] over plane columns [0, np), lower
 // part of rows [c0, f) x columns [c0, c1) of front F, tile `tile` in
 // super-block order.
@@ -1799,7 +1812,7 @@ __device__ __forceinline__ void big_tile_w(const LdltDev &d, const FrontLd &F, c
     for (int a = 0; a < 8; ++a)
 #pragma unroll
         for (int b = 0; b < 4; ++b) acc[a][b] = v4f_t{0.f, 0.f, 0.f, 0.f};
-    const int64_t ps = static_cast<int64_t>(kBigWork) * f;
+    const int64_t ps = static_cast<int64_t>(big_work(F.ne)) * f;
     tile_loop_bf16p_w<MODE == 3, kBigKcBf>(pl, pl + ps, pl + 2 * ps, pl + 3 * ps, f, i0, j0, f, c1, 0, np, active, smem,
                                            acc);
     if (!active) return;
@@ -1863,15 +1876,17 @@ __device__ __forceinline__ int big_tiles_w(int f, int c0, int c1) {
     return nc * nr - nc * (nc - 1) / 2;
 }
 
-// The rank-kBigWork updates of BF16 / split-BF16 fronts on their planes, in
+// The outer-block updates of BF16 / split-BF16 fronts on their planes, in
 // 256 x 256 tiles: CB, the contribution block's chunk at c0 (after
 // k_big_ld and k_big_pack<true>); else the flush request (after
 // k_big_pack<false>).
 template <int MODE, bool CB>
-__global__ __launch_bounds__(kWideThreads) void k_big_wide(LdltDev d, const BigLd *__restrict__ states, int32_t c0,
+__global__ __launch_bounds__(kWideThreads) void k_big_wide(LdltDev d, const BigLd *__restrict__ states,
+                                                           const BigPart *__restrict__ grid, int32_t c0,
                                                            int32_t width) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[bfw_lds_bytes<MODE == 3, kBigKcBf>()];
-    const BigLd B = states[blockIdx.y];
+    const BigPart g = grid[blockIdx.x];
+    const BigLd B = states[g.front];
     if (B.prec != MODE) return;
     const FrontLd F = d.fronts[B.s];
     int r0, rc, np;
@@ -1888,23 +1903,24 @@ __global__ __launch_bounds__(kWideThreads) void k_big_wide(LdltDev d, const BigL
         np = B.x_p1 - B.x_p0;
     }
     const uint16_t *pl = d.xpl + 4 * F.wofs;
-    const XcdRange xr = xcd_range(big_tiles_w(F.f, r0, rc));
+    const XcdRange xr = xcd_range(g, big_tiles_w(F.f, r0, rc));
     for (int tile = xr.lo; tile < xr.hi; tile += xr.step) {
         big_tile_w<MODE>(d, F, pl, r0, rc, np, tile, smem);
         __syncthreads();
     }
 }
 
-// bf16 planes of a rank-kBigWork update's operands in the packed layout of
+// bf16 planes of an outer-block update's operands in the packed layout of
 // tile_loop_bf16p (row i, plane column c at (c / 8) f 8 + 8 i + c % 8), for
 // the fronts of BF16 (high part) or split-BF16 (both parts) precision:
 // A = front columns [p0, p0 + np), rows [r0, f); B = W columns from p0 - w0,
 // rows [r0, rb); plane columns [np, np rounded up to 8) zero. CB: the
 // contribution-block chunk at c0 (W from k_big_ld), else the flush request.
 template <bool CB>
-__global__ __launch_bounds__(kLT) void k_big_pack(LdltDev d, const BigLd *__restrict__ states, int32_t c0,
-                                                  int32_t width) {
-    const BigLd B = states[blockIdx.y];
+__global__ __launch_bounds__(kLT) void k_big_pack(LdltDev d, const BigLd *__restrict__ states,
+                                                  const BigPart *__restrict__ grid, int32_t c0, int32_t width) {
+    const BigPart gr = grid[blockIdx.x];
+    const BigLd B = states[gr.front];
     if (B.prec < 2) return;
     const FrontLd F = d.fronts[B.s];
     const int f = F.f;
@@ -1929,12 +1945,12 @@ __global__ __launch_bounds__(kLT) void k_big_pack(LdltDev d, const BigLd *__rest
     const double *G = d.arena + F.fofs;
     const double *W = d.work + F.wofs;
     uint16_t *pl = d.xpl + 4 * F.wofs;
-    const int64_t ps = static_cast<int64_t>(kBigWork) * f;
+    const int64_t ps = static_cast<int64_t>(big_work(F.ne)) * f;
     const int ng = (np + 7) / 8;
     const int nr = f - r0;
     const int64_t tot = 2 * static_cast<int64_t>(ng) * nr;
-    for (int64_t idx = static_cast<int64_t>(blockIdx.x) * kLT + threadIdx.x; idx < tot;
-         idx += static_cast<int64_t>(gridDim.x) * kLT) {
+    for (int64_t idx = static_cast<int64_t>(gr.part) * kLT + threadIdx.x; idx < tot;
+         idx += static_cast<int64_t>(gr.parts) * kLT) {
         const int i = r0 + static_cast<int>(idx % nr);
         const int64_t q = idx / nr;
         const int g = static_cast<int>(q % ng);
@@ -1977,33 +1993,28 @@ void launch_big_panel(hipStream_t st, const LdltDev &d, BigLd *states, int32_t n
     k_big_panel<<<dim3(nbig), kLT, 0, st>>>(d, states, prm, nb, gpart, nch);
 }
 
-void launch_big_group_stats(hipStream_t st, const LdltDev &d, const BigLd *states, int32_t nbig, double *gpart,
-                            int32_t nch) {
+void launch_big_group_stats(hipStream_t st, const LdltDev &d, const BigLd *states, int32_t nbig, const BigGrid &g,
+                            double *gpart, int32_t nch) {
     k_big_gdiag<<<dim3(nbig), 64, 0, st>>>(d, states, gpart, nch);
-    k_big_group<<<dim3(nch, nbig), kLT, 0, st>>>(d, states, gpart, nch);
+    k_big_group<<<dim3(g.nrows), kLT, 0, st>>>(d, states, g.rows, gpart, nch);
 }
 
-void launch_big_group_apply(hipStream_t st, const LdltDev &d, const BigLd *states, int32_t nbig, double *gpart,
+void launch_big_group_apply(hipStream_t st, const LdltDev &d, const BigLd *states, const BigGrid &g, double *gpart,
                             int32_t nch) {
-    k_big_gapply<<<dim3(nch, nbig), kLT, 0, st>>>(d, states, gpart, nch);
+    k_big_gapply<<<dim3(g.nrows), kLT, 0, st>>>(d, states, g.rows, gpart, nch);
 }
 
-// workgroups per front of the 256 x 256 tiles (one per CU; a multiple of 8)
-static int32_t wide_per_front(int32_t per_front) { return std::max(8, per_front / 16 * 8); }
-
-void launch_big_update(hipStream_t st, const LdltDev &d, const BigLd *states, int32_t nbig, int32_t per_front,
+void launch_big_update(hipStream_t st, const LdltDev &d, const BigLd *states, const BigGrid &g,
                        const int32_t *nmode) {
-    if (nbig <= 0) return;
-    const dim3 g(per_front, nbig);
-    if (d.xpl != nullptr && nmode[2] + nmode[3] > 0) k_big_pack<false><<<g, kLT, 0, st>>>(d, states, 0, 0);
-    if (nmode[0] > 0) k_big_update<0><<<g, kLT, 0, st>>>(d, states);
-    if (nmode[1] > 0) k_big_update<1><<<g, kLT, 0, st>>>(d, states);
-    if (nmode[2] > 0) k_big_update<2><<<g, kLT, 0, st>>>(d, states);
-    if (nmode[3] > 0) k_big_update<3><<<g, kLT, 0, st>>>(d, states);
+    const dim3 nt(g.ntiles);
+    if (d.xpl != nullptr && nmode[2] + nmode[3] > 0) k_big_pack<false><<<nt, kLT, 0, st>>>(d, states, g.tiles, 0, 0);
+    if (nmode[0] > 0) k_big_update<0><<<nt, kLT, 0, st>>>(d, states, g.tiles);
+    if (nmode[1] > 0) k_big_update<1><<<nt, kLT, 0, st>>>(d, states, g.tiles);
+    if (nmode[2] > 0) k_big_update<2><<<nt, kLT, 0, st>>>(d, states, g.tiles);
+    if (nmode[3] > 0) k_big_update<3><<<nt, kLT, 0, st>>>(d, states, g.tiles);
     if (d.xpl != nullptr) {
-        const dim3 gw(wide_per_front(per_front), nbig);
-        if (nmode[2] > 0) k_big_wide<2, false><<<gw, kWideThreads, 0, st>>>(d, states, 0, 0);
-        if (nmode[3] > 0) k_big_wide<3, false><<<gw, kWideThreads, 0, st>>>(d, states, 0, 0);
+        if (nmode[2] > 0) k_big_wide<2, false><<<dim3(g.nwide), kWideThreads, 0, st>>>(d, states, g.wide, 0, 0);
+        if (nmode[3] > 0) k_big_wide<3, false><<<dim3(g.nwide), kWideThreads, 0, st>>>(d, states, g.wide, 0, 0);
     }
 }
 
@@ -2012,24 +2023,22 @@ void launch_big_stall(hipStream_t st, const LdltDev &d, BigLd *states, int32_t n
     k_big_stall<<<dim3(nbig), kLT, 0, st>>>(d, states, nb);
 }
 
-void launch_big_cb(hipStream_t st, const LdltDev &d, const BigLd *states, int32_t nbig, int32_t c0, int32_t width,
-                   int32_t per_front, const int32_t *nmode, bool wide) {
-    if (nbig <= 0) return;
-    const dim3 g(per_front, nbig);
-    k_big_ld<<<g, kLT, 0, st>>>(d, states, c0, width, wide ? 1 : 0);
+void launch_big_cb(hipStream_t st, const LdltDev &d, const BigLd *states, const BigGrid &g, int32_t c0, int32_t width,
+                   const int32_t *nmode, bool wide) {
+    const dim3 nt(g.ntiles);
+    k_big_ld<<<nt, kLT, 0, st>>>(d, states, g.tiles, c0, width, wide ? 1 : 0);
     if (wide) {
         // the BF16 modes' fronts on planes
-        const dim3 gw(wide_per_front(per_front), nbig);
-        k_big_pack<true><<<g, kLT, 0, st>>>(d, states, c0, width);
-        if (nmode[2] > 0) k_big_wide<2, true><<<gw, kWideThreads, 0, st>>>(d, states, c0, width);
-        if (nmode[3] > 0) k_big_wide<3, true><<<gw, kWideThreads, 0, st>>>(d, states, c0, width);
+        k_big_pack<true><<<nt, kLT, 0, st>>>(d, states, g.tiles, c0, width);
+        if (nmode[2] > 0) k_big_wide<2, true><<<dim3(g.nwide), kWideThreads, 0, st>>>(d, states, g.wide, c0, width);
+        if (nmode[3] > 0) k_big_wide<3, true><<<dim3(g.nwide), kWideThreads, 0, st>>>(d, states, g.wide, c0, width);
         return;
     }
-    if (nmode[0] > 0) k_big_cbupdate<0><<<g, kLT, 0, st>>>(d, states, c0, width);
-    if (nmode[1] > 0) k_big_cbupdate<1><<<g, kLT, 0, st>>>(d, states, c0, width);
+    if (nmode[0] > 0) k_big_cbupdate<0><<<nt, kLT, 0, st>>>(d, states, g.tiles, c0, width);
+    if (nmode[1] > 0) k_big_cbupdate<1><<<nt, kLT, 0, st>>>(d, states, g.tiles, c0, width);
     if (d.xpl == nullptr) {
-        if (nmode[2] > 0) k_big_cbupdate<2><<<g, kLT, 0, st>>>(d, states, c0, width);
-        if (nmode[3] > 0) k_big_cbupdate<3><<<g, kLT, 0, st>>>(d, states, c0, width);
+        if (nmode[2] > 0) k_big_cbupdate<2><<<nt, kLT, 0, st>>>(d, states, g.tiles, c0, width);
+        if (nmode[3] > 0) k_big_cbupdate<3><<<nt, kLT, 0, st>>>(d, states, g.tiles, c0, width);
     }
 }
 
@@ -2120,6 +2129,7 @@ __device__ __forceinline__ double stored_entry(const double *G, int f, int c, in
 // global memory or LDS; store: also write its stored factor columns.
 template <int NT = kLT>
 __device__ void finish_front_wg(const LdltDev &d, FrontLd &F, const double *G, bool store) {
+    __shared__ int n2;
     const int f = F.f;
     int p = F.p;
     int8_t *tags = d.tags + F.rofs;
@@ -2134,11 +2144,15 @@ __device__ void finish_front_wg(const LdltDev &d, FrontLd &F, const double *G, b
     if (tid == 0) {
         F.pstore = ps;
         if (root && p < F.ne) F.nzero += F.ne - p;
-        int n2 = 0;
-        for (int c = 0; c < ps; ++c) n2 += tags[c] == 2;
-        F.n2x2 = n2;
         F.delayed = root ? 0 : F.ne - p;
+        n2 = 0;
     }
+    __syncthreads();
+    int mine = 0;
+    for (int c = tid; c < ps; c += NT) mine += tags[c] == 2;
+    if (mine) atomicAdd(&n2, mine);
+    __syncthreads();
+    if (tid == 0) F.n2x2 = n2;
     for (int c = tid; c < ps; c += NT) {
         const double *Lc = G + static_cast<int64_t>(c) * f;
         const int8_t tg = tags[c];
@@ -2443,7 +2457,9 @@ void launch_ldlt_epilogue(hipStream_t st, const LdltDev &d, const int32_t *flist
 
 void launch_ldlt_store(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, int32_t max_cols) {
     if (nf <= 0 || max_cols <= 0) return;
-    k_ldlt_store<<<dim3(max_cols < 2048 ? max_cols : 2048, nf), kLT, 0, st>>>(d, flist);
+    // about 8192 workgroups over the launch's fronts, at least 16 a front
+    const int32_t per = std::min(max_cols, std::max(16, 8192 / nf));
+    k_ldlt_store<<<dim3(per, nf), kLT, 0, st>>>(d, flist);
 }
 
 // ---------------------------------------------------------------------------

@@ -690,7 +690,7 @@ SMFGPU_API int smfgpu_plan_stats(smfgpu_plan_t P, double *out) {
              P->d_L16h.bytes() + P->d_L16l.bytes() +
              P->d_fwd_items.bytes() + P->d_bwd_items.bytes() + P->d_bwd_seq.bytes() + P->d_fwd_step_of.bytes() +
              P->d_bwd_step_of.bytes() + P->d_fwd_step_cnt.bytes() + P->d_bwd_step_cnt.bytes() +
-             P->d_sweep_ctr.bytes() + P->d_sweep_err.bytes() + P->d_gpart.bytes() + P->d_big.bytes() +
+             P->d_sweep_ctr.bytes() + P->d_sweep_err.bytes() + P->d_gpart.bytes() + P->d_big.bytes() + P->d_parts.bytes() +
              P->d_fr_ptr.bytes();
     // solve and refinement work buffers (allocated on first use)
     bytes += P->d_y.bytes() + P->d_b.bytes() + P->d_r.bytes() + P->d_rowstat.bytes() + P->d_x.bytes() +

@@ -16,7 +16,9 @@ namespace smfgpu {
 void launch_front_gather(hipStream_t st, const FrontLd *fronts, FrontLd *out, const int32_t *ids, int32_t np);
 
 constexpr int kBlockedMinFront = 96;  // ldlt_kernel.hpp:15 (blocked_min_front)
-constexpr int64_t kStoreWide = int64_t{1} << 20;  // stored entries from which a front gets the store kernel
+// stored entries from which a front gets the store kernel (one workgroup
+// stores about 30 GB/s: 16 us for a front at the limit)
+constexpr int64_t kStoreWide = int64_t{1} << 15;
 
 namespace {
 
@@ -260,13 +262,17 @@ static int ldlt_dev_levels(smfgpu_plan_s *P, int32_t lv0, double u, double eff_s
 }
 
 // Large fronts of one level (multi-workgroup blocked LDL^T): the panel,
-// update and stall kernels in turn until every front is done (the state
-// read back every kBigCheck rounds), then the contribution blocks' update
-// in chunks of an outer block's pivots and the fronts' results.
+// update and stall kernels in turn until every front is done, then the
+// contribution blocks' update in chunks of an outer block's pivots and the
+// fronts' results. The state is read back after as many rounds as the
+// fronts need when every panel group is accepted (a round then takes 64
+// pivots of each), and again after what is left by the same count, at most
+// kBigCheck rounds at a time: an idle round costs its six launches (about
+// 20 us), a read-back about as much.
 static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vector<int32_t> &big,
                            const smfgpu_factor_options &opt, double eff_small, double small, int32_t nb,
                            std::vector<BigLd> &h, int32_t &reduced) {
-    constexpr int kBigCheck = 16;
+    constexpr int32_t kBigCheck = 16;
     hipStream_t st = P->stream;
     LdltDev d = d0;
     d.xpl = nullptr;
@@ -336,38 +342,71 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
     }
     reduced += nbig - nmode[0];
     if ((rc = ensure(P->d_big, static_cast<size_t>(nbig), false, "large-front states"))) return rc;
-    // bf16 planes of the rank-kBigWork updates' operands (BF16 and split-BF16
+    // bf16 planes of the outer-block updates' operands (BF16 and split-BF16
     // fronts, and the training pairs' split-BF16 and BF16 runs)
     if (P->ldlt_planes != 0 && (nmode[2] + nmode[3] > 0 || (collect && !sf.empty()))) {
         int64_t planes = 0;
-        for (int32_t s : big) planes = std::max(planes, 4 * (P->fl[s].wofs + static_cast<int64_t>(P->fl[s].f) * kBigWork));
+        for (int32_t s : big)
+            planes = std::max(planes, 4 * (P->fl[s].wofs + static_cast<int64_t>(P->fl[s].f) * big_work(P->fl[s].ne)));
         if ((rc = ensure(P->d_xpl, static_cast<size_t>(planes), false, "update planes"))) return rc;
         d.xpl = P->d_xpl.p;
     }
     HIP_OK(hipMemcpyAsync(P->d_big.p, h.data(), nbig * sizeof(BigLd), hipMemcpyHostToDevice, st));
-    // update workgroups per front: a multiple of 8 (one run of tiles per XCD)
+    // workgroups of each launch, by front: 256-row chunks for the group
+    // kernels; for the updates as many workgroups as the front has tiles of
+    // its lower triangle, at most its share of ldlt_update_wg (at least 64),
+    // rounded up to a multiple of 8
     const int32_t per_front = std::max(64, P->ldlt_update_wg / nbig) / 8 * 8;
-    // speculative groups: workgroups per front over the rows below a
-    // group's diagonal region, and their column maxima
+    const int32_t wide_per_front = std::max(8, per_front / 16 * 8);
     int32_t maxf = 0;
+    std::vector<BigPart> parts;
+    const auto add_parts = [&](auto &&count) {
+        const size_t first = parts.size();
+        for (int32_t b = 0; b < nbig; ++b) {
+            const int32_t n = count(P->fl[big[b]].f);
+            for (int32_t i = 0; i < n; ++i) parts.push_back(BigPart{b, i, n});
+        }
+        return static_cast<int32_t>(parts.size() - first);
+    };
+    const auto tile_parts = [](int32_t f, int32_t tile, int32_t cap) {
+        const int64_t m = (f + tile - 1) / tile;
+        return static_cast<int32_t>(std::min<int64_t>(cap, (m * (m + 1) / 2 + 7) / 8 * 8));
+    };
     for (int32_t s : big) maxf = std::max(maxf, P->fl[s].f);
     const int32_t nch = (maxf + kGroupRows - 1) / kGroupRows + 1;
+    BigGrid grid{};
+    grid.nrows = add_parts([&](int32_t f) { return (f + kGroupRows - 1) / kGroupRows; });
+    grid.ntiles = add_parts([&](int32_t f) { return tile_parts(f, 128, per_front); });
+    grid.nwide = add_parts([&](int32_t f) { return tile_parts(f, 256, wide_per_front); });
+    if ((rc = ensure(P->d_parts, parts.size(), false, "large-front workgroups"))) return rc;
+    HIP_OK(hipMemcpyAsync(P->d_parts.p, parts.data(), parts.size() * sizeof(BigPart), hipMemcpyHostToDevice, st));
+    grid.rows = P->d_parts.p;
+    grid.tiles = grid.rows + grid.nrows;
+    grid.wide = grid.tiles + grid.ntiles;
     const size_t gstride = static_cast<size_t>(nch) * kGroupCols + kGroupBuf;
     if (group && (rc = ensure(P->d_gpart, static_cast<size_t>(nbig) * gstride, false, "group buffer"))) return rc;
     double *gpart = group ? P->d_gpart.p : nullptr;
-    for (int64_t it = 0;; ++it) {
-        if (group) launch_big_group_stats(st, d, P->d_big.p, nbig, gpart, nch);
+    const auto rounds_left = [&]() {
+        int32_t left = 0;
+        for (const BigLd &B : h)
+            if (B.pass != 2) left = std::max(left, (P->fl[B.s].ne - B.k + (group ? kGroupCols : nb) - 1) / (group ? kGroupCols : nb));
+        return std::max(left, 1);
+    };
+    int64_t check = rounds_left();
+    for (int64_t it = 1;; ++it) {
+        if (group) launch_big_group_stats(st, d, P->d_big.p, nbig, grid, gpart, nch);
         launch_big_panel(st, d, P->d_big.p, nbig, opt.pivot_u, eff_small, small, nb, gpart, nch);
-        if (group) launch_big_group_apply(st, d, P->d_big.p, nbig, gpart, nch);
-        launch_big_update(st, d, P->d_big.p, nbig, per_front, nmode);
+        if (group) launch_big_group_apply(st, d, P->d_big.p, grid, gpart, nch);
+        launch_big_update(st, d, P->d_big.p, grid, nmode);
         launch_big_stall(st, d, P->d_big.p, nbig, nb);
-        if (it % kBigCheck == kBigCheck - 1) {
+        if (it == check) {
             HIP_OK(hipMemcpyAsync(h.data(), P->d_big.p, nbig * sizeof(BigLd), hipMemcpyDeviceToHost, st));
             HIP_OK(hipStreamSynchronize(st));
             bool done = true;
             for (const BigLd &B : h) done = done && B.pass == 2;
             if (done) break;
             if (it > cap) return set_error(SMFGPU_ERR_DEVICE, "factor: a large front did not finish");
+            check = it + std::min(rounds_left(), kBigCheck);
         }
     }
     HIP_OK(hipGetLastError());
@@ -378,10 +417,10 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
     auto cb_update = [&](const int32_t *nm) {
         if (nm[0] + nm[1] > 0 || (d.xpl == nullptr && nm[2] + nm[3] > 0))
             for (int32_t c0 = 0; c0 < pmax; c0 += kBigOuter)
-                launch_big_cb(st, d, P->d_big.p, nbig, c0, kBigOuter, per_front, nm, false);
+                launch_big_cb(st, d, P->d_big.p, grid, c0, kBigOuter, nm, false);
         if (d.xpl != nullptr && nm[2] + nm[3] > 0)
             for (int32_t c0 = 0; c0 < pmax; c0 += P->ldlt_outer_wide)
-                launch_big_cb(st, d, P->d_big.p, nbig, c0, P->ldlt_outer_wide, per_front, nm, true);
+                launch_big_cb(st, d, P->d_big.p, grid, c0, P->ldlt_outer_wide, nm, true);
     };
     const bool labels = collect && !sf.empty() && maxq > 0;
     if (labels) {
@@ -708,7 +747,7 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
             const bool stat = front_static_value(spr, F.root, F.nd, F.psym) > 0.0;
             if (F.f >= P->ldlt_big_min && F.ne > 0 && !stat) {
                 F.wofs = work_used;
-                work_used += static_cast<int64_t>(F.f) * kBigWork;
+                work_used += static_cast<int64_t>(F.f) * big_work(F.ne);
                 big_list.push_back(s);
             } else if (F.f >= kBlockedMinFront) {
                 F.wofs = work_used;

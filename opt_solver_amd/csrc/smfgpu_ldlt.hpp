@@ -51,8 +51,8 @@ struct LdltDev {
     const int32_t *amap;      // per permuted entry: position among its front's symbolic rows
     const double *av;
     double *junk;             // target of masked-out stores of the MFMA updates (contents meaningless)
-    uint16_t *xpl;            // bf16 operand planes of the large fronts' rank-kBigWork updates (BF16 / split BF16):
-                              // per front at 4 wofs, planes A hi, A lo, B hi, B lo of kBigWork f entries each
+    uint16_t *xpl;            // bf16 operand planes of the large fronts' outer-block updates (BF16 / split BF16):
+                              // per front at 4 wofs, planes A hi, A lo, B hi, B lo of big_work(ne) f entries each
 };
 
 // Large fronts (multi-workgroup blocked LDL^T): one state per front,
@@ -71,10 +71,11 @@ struct LdltDev {
 // twice as many products).
 constexpr int32_t kBigOuter = 512;
 constexpr int32_t kBigOuterMax = 1024;
-// W columns per front: an outer block's pivots (L*D chunks of the final
-// update), then a speculative group's final entries (kGroupSpec)
-constexpr int32_t kBigWork = kBigOuterMax + 64;
-constexpr int32_t kGroupSpec = kBigOuterMax;
+// W columns of a front with ne eligible columns: an outer block's pivots
+// (L*D chunks of the final update), then a speculative group's final
+// entries, from column big_spec on
+__host__ __device__ constexpr int32_t big_spec(int32_t ne) { return ne < kBigOuterMax ? ne : kBigOuterMax; }
+__host__ __device__ constexpr int32_t big_work(int32_t ne) { return big_spec(ne) + 64; }
 static_assert(kBigOuterMax >= kBigOuter, "W holds the pivots of an outer block");
 struct BigLd {
     int32_t s;                  // supernode
@@ -97,9 +98,23 @@ struct BigLd {
     int32_t prec;               // precision code of the MFMA updates: 0 FP64, 1 FP32, 2 BF16, 3 split BF16
     double flops;
 };
+// Workgroup `part` of the `parts` a launch gives front `front` of the level's
+// large fronts. A level's launches share one list per kind of work, sized by
+// each front: a list entry per workgroup instead of the largest front's
+// number for every front (a level mixes fronts of 96 rows with fronts of
+// thousands, and an empty workgroup still costs its dispatch).
+struct BigPart {
+    int32_t front, part, parts;
+};
+struct BigGrid {
+    const BigPart *rows;    // 256-row chunks (group kernels)
+    const BigPart *tiles;   // 128 x 128 update tiles, a multiple of 8 per front (one run of tiles per XCD)
+    const BigPart *wide;    // 256 x 256 update tiles, likewise
+    int32_t nrows, ntiles, nwide;
+};
 constexpr int32_t kGroupCols = 64;   // columns of a speculative group (four panels of 16)
 constexpr int32_t kGroupRows = 256;  // rows per workgroup below a group's diagonal region
-static_assert(kBigWork - kGroupSpec == kGroupCols, "W holds a group's speculative columns");
+static_assert(big_work(1) - big_spec(1) == kGroupCols, "W holds a group's speculative columns");
 constexpr int64_t kGroupBuf = 192 + 64 * 16 + 2 * 64 * 64;  // group buffer per front before the per-workgroup maxima
 
 // Static pivoting (control.hpp:333-364): sp = static_pivot_tol * max|A|
@@ -176,19 +191,18 @@ void launch_ldlt_bwd_step(hipStream_t st, const LdltDev &d, const SolveItem *ite
 void launch_big_panel(hipStream_t st, const LdltDev &d, BigLd *states, int32_t nbig, double u, double eff_small,
                       double small_pivot, int32_t nb, const double *gpart, int32_t nch);
 // speculative group: column maxima (stats) and the accepted panels' rows (apply)
-void launch_big_group_stats(hipStream_t st, const LdltDev &d, const BigLd *states, int32_t nbig, double *gpart,
-                            int32_t nch);
-void launch_big_group_apply(hipStream_t st, const LdltDev &d, const BigLd *states, int32_t nbig, double *gpart,
+void launch_big_group_stats(hipStream_t st, const LdltDev &d, const BigLd *states, int32_t nbig, const BigGrid &g,
+                            double *gpart, int32_t nch);
+void launch_big_group_apply(hipStream_t st, const LdltDev &d, const BigLd *states, const BigGrid &g, double *gpart,
                             int32_t nch);
 // nmode[m]: fronts of the level whose updates run in precision code m
 // (0 FP64, 1 FP32, 2 BF16, 3 split BF16); a launch per code in use
-void launch_big_update(hipStream_t st, const LdltDev &d, const BigLd *states, int32_t nbig, int32_t per_front,
-                       const int32_t *nmode);
+void launch_big_update(hipStream_t st, const LdltDev &d, const BigLd *states, const BigGrid &g, const int32_t *nmode);
 void launch_big_stall(hipStream_t st, const LdltDev &d, BigLd *states, int32_t nbig, int32_t nb);
 // final contribution-block update with pivots [c0, c0 + width) of every
 // front (L*D of the chunk into W first); then the fronts' results
-void launch_big_cb(hipStream_t st, const LdltDev &d, const BigLd *states, int32_t nbig, int32_t c0, int32_t width,
-                   int32_t per_front, const int32_t *nmode, bool wide);
+void launch_big_cb(hipStream_t st, const LdltDev &d, const BigLd *states, const BigGrid &g, int32_t c0, int32_t width,
+                   const int32_t *nmode, bool wide);
 void launch_big_finish(hipStream_t st, const LdltDev &d, const BigLd *states, int32_t nbig);
 
 }  // namespace smfgpu

@@ -253,8 +253,9 @@ struct smfgpu_plan_s {
     int32_t panel_outer_red = kPanelOuterRed;      // the same for reduced-precision factorizations
     std::vector<int64_t> asm_first;                // SPD: first assembly task of each level
     int32_t cb_seg = 4096;                         // SPD: pivot columns per contribution-block update
-    int32_t ldlt_big_min = 256;                    // LDL^T: fronts with at least this many rows take the large-front path
+    int32_t ldlt_big_min = 96;                     // LDL^T: fronts with at least this many rows take the large-front path
     DBuf<BigLd> d_big;                             // LDL^T: large-front states of the level
+    DBuf<BigPart> d_parts;                         // the level's launches: workgroup -> front
     int32_t ldlt_planes = 1;                       // LDL^T: bf16 operand planes for the large fronts' outer-block updates
     int32_t ldlt_outer_wide = 1024;                // LDL^T: outer block of the fronts updated on planes
     int32_t ldlt_group = 1;                        // LDL^T: speculative panel groups on the large-front path
