@@ -1103,16 +1103,16 @@ __device__ __forceinline__ int big_tiles(int f, int c0, int c1) {
 // goes through a fixed sequence of row-local operations: eliminate_1x1's
 // rank-1 updates within the panel (ldlt_kernel.cpp:350-432) and the deferred
 // update of the later columns (705-761). A group of up to four panels of 16
-// is evaluated under that assumption. The stats launch factors the group's
-// diagonal region in one wave of every workgroup (the multipliers and the
-// unscaled columns go to LDS), lets every thread carry one row below it
-// through the same operations, and records per pivot the largest entry of
-// its column. The panel kernel then applies the first test to each pivot in
-// order and accepts the leading panels that pass; the apply launch redoes the
-// accepted panels and writes their columns and W. A panel that fails is
-// factored by the panel kernel's full search. Per row, the operations and
-// their order are those of the one-panel path, so are the accepted values
-// and the pivot decisions.
+// is evaluated under that assumption, a round of four launches: the region
+// launch (one workgroup per front; it first moves the rows of a panel that
+// stalled in the round before) factors the group's 64 x 64 diagonal region;
+// the rows launch carries the rows below it through the same pivots and
+// records per pivot the largest entry of its column; the panel launch applies
+// the first test to each pivot in order, accepts the leading panels that pass
+// and writes their columns; the update launch applies the deferred updates. A
+// panel that fails is factored by the panel launch's full search. A row's
+// operations are those of the one-panel path with each multiply and subtract
+// fused.
 // Guarded loads are unconditional loads from clamped (in-front) addresses
 // times a 0 / 1 mask, so the compiler keeps every load of a row in flight
 // (inputs are finite: the factorization rejects non-finite values).
@@ -1141,386 +1141,477 @@ __device__ __forceinline__ int group_cols(const BigLd &B, int nb) {
     return pos - B.k;
 }
 
-// Group buffer per front (doubles): the diagonal region's results, written
-// by the region launch and read by the stats, panel and apply launches,
-// then 64 column maxima per workgroup of the stats launch.
-constexpr int64_t kGdMax = 0;                               // 64: largest |entry| below each pivot in the region
-constexpr int64_t kGdPiv = 64;                              // 64: pivots
-constexpr int64_t kGdInv = 128;                             // 64: 1 / pivot
-constexpr int64_t kGdLm = 192;                              // 64 x 16: multipliers of each pivot for its panel
-constexpr int64_t kGdWd = kGdLm + 64 * 16;                  // 64 x 64: [t][r] row r of the region at pivot t, unscaled
-constexpr int64_t kGdFin = kGdWd + 64 * 64;                 // 64 x 64: [c][r] the region's final entries
-constexpr int64_t kGMax = kGdFin + 64 * 64;
-static_assert(kGMax == kGroupBuf, "group buffer layout");
-__device__ __forceinline__ int64_t gpart_stride(int nch) { return kGMax + static_cast<int64_t>(nch) * kGroupCols; }
+// Group buffer per front (doubles).
+constexpr int64_t kGMax = 0;                    // 64: per pivot the bits of the largest |entry| below it in its column
+constexpr int64_t kGdPiv = 64;                  // 64: pivots
+constexpr int64_t kGdInv = 128;                 // 64: 1 / pivot
+constexpr int64_t kGdWd = 192;                  // 64 x 64: [t][r] row r of the region at pivot t, unscaled
+constexpr int64_t kGdFin = kGdWd + 64 * 64;     // 64 x 64: [c][r] the region's final entries (r > c: row r's multiplier)
+static_assert(kGdFin + 64 * 64 == kGroupBuf, "group buffer layout");
 
-// Per-panel steps of a group (panel M: columns [16 M, 16 M + 16) of the
-// group), templated so that every index into a row's registers is a
-// constant; FULL: the group has all 64 columns (no column guards). A
-// skipped update (multiplier 0, or a row above the column) is a select,
-// the same value as the reference's skip. Diagonal region: lane r of
-// wave 0 holds row ps + r.
-template <int M, bool FULL>
-__device__ __forceinline__ void gdiag_pivots(double (&a)[kGroupCols], int r, int ncols,
-                                             double (*Wd)[kGroupCols + 1], double (*Lm)[16], double *invd,
-                                             double *dd) {
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int kk = 16 * M + q;
-        if (FULL || kk < ncols) {
-            // stores without conditions: every lane writes the same value
-            // to dd, invd and Lm; Wd[kk][r] for r <= kk is never read
-            const double v = a[kk];
-            const double dk = rdlane(v, kk);
-            const double inv = 1.0 / dk;
-            dd[kk] = dk;
-            invd[kk] = inv;
-            Wd[kk][r] = v;
-#pragma unroll
-            for (int jq = q + 1; jq < 16; ++jq) {
-                const int j = 16 * M + jq;
-                if (FULL || j < ncols) {
-                    const double lj = __dmul_rn(rdlane(v, j), inv);
-                    Lm[kk][jq] = lj;
-                    const double t = __dsub_rn(a[j], __dmul_rn(v, lj));
-                    a[j] = (lj != 0.0 && r >= j) ? t : a[j];
-                }
-            }
-            const double sc = __dmul_rn(v, inv);
-            a[kk] = r > kk ? sc : a[kk];
+// 1 / d: the hardware estimate (better than 2^-20), a third-order step in
+// the residual e = 1 - d y, and one Newton step for the last bit
+__device__ __forceinline__ double pivot_rcp(double d) {
+    double y = __builtin_amdgcn_rcp(d);
+    double e = fma(-d, y, 1.0);
+    y = fma(y, fma(e, e, e), y);
+    e = fma(-d, y, 1.0);
+    return fma(y, e, y);
+}
+// v of lane C of the lane's row of 16 lanes
+template <int C>
+__device__ __forceinline__ double row_bcast(double v) {
+    return __builtin_amdgcn_update_dpp(0.0, v, 0x150 + C, 0xf, 0xf, true);
+}
+
+// Pivot J of a 16-column panel of the region: a the diagonal block's row,
+// x the lane's own row, inv 1 / pivot. l receives the scaled column (rows
+// past the pivot), a and x keep theirs unscaled. The next pivot's column
+// goes first.
+template <int J, int C>
+__device__ __forceinline__ void region_cols(double (&a)[16], double (&x)[16], double la) {
+    if constexpr (C < 16) {
+        const double m = row_bcast<C>(la);
+        a[C] = fma(-a[J], m, a[C]);
+        x[C] = fma(-x[J], m, x[C]);
+        region_cols<J, C + 1>(a, x, la);
+    }
+}
+template <int J>
+__device__ __forceinline__ void region_pivots(double (&a)[16], double (&x)[16], double (&l)[16], double (&dv)[16],
+                                              double (&iv)[16], double dj, double inv) {
+    if constexpr (J < 16) {
+        dv[J] = dj;
+        iv[J] = inv;
+        const double la = a[J] * inv;
+        l[J] = x[J] * inv;
+        double dn = 0.0, in = 0.0;
+        if constexpr (J + 1 < 16) {
+            const double m = row_bcast<J + 1>(la);
+            a[J + 1] = fma(-a[J], m, a[J + 1]);
+            dn = row_bcast<J + 1>(a[J + 1]);
+            in = pivot_rcp(dn);
+            x[J + 1] = fma(-x[J], m, x[J + 1]);
         }
+        region_cols<J, J + 2>(a, x, la);
+        region_pivots<J + 1>(a, x, l, dv, iv, dn, in);
     }
 }
 
-// Rows below the region (one per thread): the same pivots with the
-// multipliers from LDS; STATS keeps |entry| per pivot in red[q][tid].
-template <int M, bool STATS, bool FULL>
-__device__ __forceinline__ void grow_pivots(double (&a)[kGroupCols], int ncols, const double (*Lm)[16],
-                                            const double *invd, double (*red)[kLT + 1], double *W, int64_t wcol0,
-                                            int f, int i, bool rowok) {
+constexpr int kRLd = 81;  // column stride of the region's LDS squares (odd: a column scan by 64 lanes spreads over the banks)
+
+// Block (i, c) of the region -= W block (i, p) times L block (c, p)^T
+__device__ __forceinline__ void region_update(double *S, const double *Ls, int p, int i, int c) {
+    const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+    v4d_t acc;
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int kk = 16 * M + q;
-        if (FULL || kk < ncols) {
-            const double v = a[kk];
-            if (STATS) red[q][threadIdx.x] = fabs(v);
-            if (rowok) W[(wcol0 + kk) * f + i] = v;
+    for (int v = 0; v < 4; ++v) acc[v] = S[(16 * c + 4 * v + lk) * kRLd + 16 * i + lr];
 #pragma unroll
-            for (int jq = q + 1; jq < 16; ++jq) {
-                const int j = 16 * M + jq;
-                if (FULL || j < ncols) {
-                    const double lj = Lm[kk][jq];
-                    const double t = __dsub_rn(a[j], __dmul_rn(v, lj));
-                    a[j] = lj != 0.0 ? t : a[j];
-                }
-            }
-            a[kk] = __dmul_rn(v, invd[kk]);
-        }
-    }
+    for (int kk = 0; kk < 4; ++kk)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(Ls[(16 * p + 4 * kk + lk) * kRLd + 16 * c + lr],
+                                                   -S[(16 * p + 4 * kk + lk) * kRLd + 16 * i + lr], acc, 0, 0, 0);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) S[(16 * c + 4 * v + lk) * kRLd + 16 * i + lr] = acc[v];
 }
 
-// Deferred update of the group's columns after panel M by its pivots
-// (below = true for every row under the region, else rows at or below the
-// column).
-template <int M, bool FULL>
-__device__ __forceinline__ void gdeferred(double (&a)[kGroupCols], int ncols, const double (*Wd)[kGroupCols + 1],
-                                          int r, bool below) {
-#pragma unroll
-    for (int j = 16 * M + 16; j < kGroupCols; ++j) {
-        if (FULL || j < ncols) {
-            double sacc = 0.0;
-#pragma unroll
-            for (int t = 0; t < 16; ++t) sacc = __dadd_rn(sacc, __dmul_rn(a[16 * M + t], Wd[16 * M + t][j]));
-            const double u = __dsub_rn(a[j], sacc);
-            a[j] = (below || r >= j) ? u : a[j];
-        }
-    }
-}
-
-// Column maxima of panel M's pivots over the workgroup's rows (red holds
-// |entry| per pivot and thread).
-template <int M>
-__device__ __forceinline__ void gpanel_max(double (*red)[kLT + 1], double (*red2)[16], double *wgmax) {
+// Partner pulls or rotation of a stalled first-pass panel
+// (ldlt_kernel.cpp:1052-1097); every column is current (flushed).
+__device__ void big_stall_wg(const LdltDev &d, BigLd &B, int32_t nb, RedScratch &rs, int32_t *order) {
+    FrontLd &Fd = d.fronts[B.s];
+    const int f = Fd.f, ne = Fd.ne;
+    int32_t *rows = d.rows + Fd.rofs;
+    FV A{d.arena + Fd.fofs, f, f};
     const int tid = threadIdx.x;
-    __syncthreads();
-    {
-        const int q = tid & 15, part = tid >> 4;
-        double mx = 0.0;
-#pragma unroll
-        for (int rw = 0; rw < 16; ++rw) mx = fmax(mx, red[q][part * 16 + rw]);
-        red2[part][q] = mx;
+    const int k = B.k, pl = B.pl;
+    const int live = B.live;
+    if (k != B.k_paired) {
+        const int np = partner_pairs_wg(A, k, pl, ne, nb, rows, order, rs);
+        if (np > 0) {
+            place_rows_wg(A, k, ne, np, order, rows, rs);
+            if (tid == 0) {
+                B.live = max(live, k + np);
+                B.k_paired = k;
+                B.stalled = 0;
+                B.stalls += 1;
+                B.pulls += np / 2;
+            }
+            return;
+        }
     }
-    __syncthreads();
-    if (tid < 16) {
-        double mx = 0.0;
-#pragma unroll
-        for (int pp = 0; pp < 16; ++pp) mx = fmax(mx, red2[pp][tid]);
-        wgmax[16 * M + tid] = mx;
-    }
-}
-
-// The four panels of the diagonal region in turn (FULL: 64 columns).
-template <bool FULL>
-__device__ __forceinline__ void gdiag_run(double (&a)[kGroupCols], int r, int ncols, double (*Wd)[kGroupCols + 1],
-                                          double (*Lm)[16], double *invd, double *dd) {
-    gdiag_pivots<0, FULL>(a, r, ncols, Wd, Lm, invd, dd);
-    __syncthreads();
-    if (FULL || 16 < ncols) {
-        gdeferred<0, FULL>(a, ncols, Wd, r, false);
-        gdiag_pivots<1, FULL>(a, r, ncols, Wd, Lm, invd, dd);
-    }
-    __syncthreads();
-    if (FULL || 32 < ncols) {
-        gdeferred<1, FULL>(a, ncols, Wd, r, false);
-        gdiag_pivots<2, FULL>(a, r, ncols, Wd, Lm, invd, dd);
-    }
-    __syncthreads();
-    if (FULL || 48 < ncols) {
-        gdeferred<2, FULL>(a, ncols, Wd, r, false);
-        gdiag_pivots<3, FULL>(a, r, ncols, Wd, Lm, invd, dd);
-    }
-    __syncthreads();
-}
-
-// The rows below the region (one per thread) through the four panels.
-template <bool STATS, bool FULL>
-__device__ __forceinline__ void grow_run(double (&a)[kGroupCols], int ncols, const double (*Wd)[kGroupCols + 1],
-                                         const double (*Lm)[16], const double *invd, double (*red)[kLT + 1],
-                                         double (*red2)[16], double *wgmax, double *W, int64_t wcol0, int f, int i,
-                                         bool rowok) {
-    grow_pivots<0, STATS, FULL>(a, ncols, Lm, invd, red, W, wcol0, f, i, rowok);
-    if (STATS) gpanel_max<0>(red, red2, wgmax);
-    if (FULL || 16 < ncols) {
-        gdeferred<0, FULL>(a, ncols, Wd, 0, true);
-        grow_pivots<1, STATS, FULL>(a, ncols, Lm, invd, red, W, wcol0, f, i, rowok);
-        if (STATS) gpanel_max<1>(red, red2, wgmax);
-    }
-    if (FULL || 32 < ncols) {
-        gdeferred<1, FULL>(a, ncols, Wd, 0, true);
-        grow_pivots<2, STATS, FULL>(a, ncols, Lm, invd, red, W, wcol0, f, i, rowok);
-        if (STATS) gpanel_max<2>(red, red2, wgmax);
-    }
-    if (FULL || 48 < ncols) {
-        gdeferred<2, FULL>(a, ncols, Wd, 0, true);
-        grow_pivots<3, STATS, FULL>(a, ncols, Lm, invd, red, W, wcol0, f, i, rowok);
-        if (STATS) gpanel_max<3>(red, red2, wgmax);
+    const int m = pl - k;
+    const int mv = min(m, live - pl);
+    for (int t = 0; t < mv; ++t) sym_swap_wg(A, k + t, live - mv + t, rows, nullptr, 0, 0, 0);
+    if (tid == 0) {
+        B.live = live - m;
+        B.stalled = 0;
+        B.stalls += 1;
+        B.rotated += m;
     }
 }
 
-// The group's diagonal region [ps, ps + ncols), one wave per front: lane r
-// holds row ps + r. Results to the group buffer.
-__global__ __launch_bounds__(64) void k_big_gdiag(LdltDev d, const BigLd *__restrict__ states,
-                                                  double *__restrict__ gpart, int32_t nch) {
-    __shared__ double Wd[kGroupCols][kGroupCols + 1];
-    __shared__ double Lm[kGroupCols][16];
-    __shared__ double invd[kGroupCols], dd[kGroupCols];
+// One workgroup per front: the pulls or rotation of a panel that stalled in
+// the round before, then the next group's diagonal region [ps, ps + ncols)
+// (padded to 64 with the identity) in 16-column panels: wavefront 0 runs a
+// panel's pivots in registers, one row of the region per lane and beside it
+// the diagonal block's row (multipliers broadcast inside each row of 16
+// lanes by DPP), then the columns right of it are updated on FP64 MFMA, the
+// next panel's by every wavefront, the rest by wavefronts 1 to 3 beside the
+// next panel's pivots. Bound by wavefront 0's chain of 64 pivots: 42 us with
+// one wavefront and every multiplier through readlane, 12.8 us now.
+__global__ __launch_bounds__(kLT) void k_big_region(LdltDev d, BigLd *__restrict__ states, double *__restrict__ gpart,
+                                                    int32_t nb) {
+    __shared__ double S[64 * kRLd];   // the region, columns unscaled once factored
+    __shared__ double Ls[64 * kRLd];  // final entries: multipliers below the pivots, pivots on the diagonal
+    __shared__ double dd[64], invd[64];
+    __shared__ RedScratch rs;
+    __shared__ int32_t order[128];
+    if (states[blockIdx.x].pass == 0 && states[blockIdx.x].stalled) {
+        big_stall_wg(d, states[blockIdx.x], nb, rs, order);
+        __syncthreads();
+    }
+    if (gpart == nullptr) return;
     const BigLd B = states[blockIdx.x];
-    const int ps = B.k, ncols = group_cols(B, 16);
+    const int ps = B.k, ncols = group_cols(B, nb);
     if (ncols <= 0) return;
     const FrontLd F = d.fronts[B.s];
     const int f = F.f;
     const double *G = d.arena + F.fofs;
-    double *gp = gpart + blockIdx.x * gpart_stride(nch);
-    const int r = threadIdx.x;
-    double a[kGroupCols];
-    const bool mine = r < ncols;
-    const int rr = ps + min(r, ncols - 1);
+    double *gp = gpart + blockIdx.x * kGroupBuf;
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    {
+        double v[16];
 #pragma unroll
-    for (int c = 0; c < kGroupCols; ++c)
-        a[c] = masked(G[static_cast<int64_t>(ps + min(c, ncols - 1)) * f + rr], mine && c <= r);
-    if (ncols == kGroupCols) gdiag_run<true>(a, r, ncols, Wd, Lm, invd, dd);
-    else gdiag_run<false>(a, r, ncols, Wd, Lm, invd, dd);
+        for (int i = 0; i < 16; ++i)
+            v[i] = G[static_cast<int64_t>(ps + min(w + 4 * i, ncols - 1)) * f + ps + min(lane, ncols - 1)];
 #pragma unroll
-    for (int c = 0; c < kGroupCols; ++c) gp[kGdFin + c * kGroupCols + r] = a[c];
-    for (int e = r; e < kGroupCols * kGroupCols; e += 64) gp[kGdWd + e] = Wd[e >> 6][e & 63];
-    for (int e = r; e < kGroupCols * 16; e += 64) gp[kGdLm + e] = Lm[e >> 4][e & 15];
-    gp[kGdPiv + r] = dd[r];
-    gp[kGdInv + r] = invd[r];
-    double mx = 0.0;
-    for (int rw = r + 1; rw < ncols; ++rw) mx = fmax(mx, fabs(Wd[r][rw]));
-    gp[kGdMax + r] = mx;
-}
-
-// Rows of a group below its diagonal region, [ps + ncols, f), in chunks of
-// kGroupRows per workgroup, one row per thread, with the region's tables:
-// column maxima per pivot to the group buffer, each row's unscaled column
-// entries to W (the columns the panel kernel's pivots will have: W column
-// ps - pend0 + t, pend0 being the W base the panel kernel starts from) and
-// its final group entries to W's speculation columns [big_spec,
-// big_spec + 64). Nothing of the front square changes: a rejected panel
-// finds its columns as they were. W columns of rejected pivots are
-// rewritten (rows below the pivot) when those positions get their pivots.
-__global__ __launch_bounds__(kLT) void k_big_group(LdltDev d, const BigLd *__restrict__ states,
-                                                   const BigPart *__restrict__ grid, double *__restrict__ gpart,
-                                                   int32_t nch) {
-    __shared__ double Wd[kGroupCols][kGroupCols + 1];
-    __shared__ double Lm[kGroupCols][16];
-    __shared__ double invd[kGroupCols], wgmax[kGroupCols];
-    __shared__ double red[16][kLT + 1];
-    __shared__ double red2[16][16];
-    const BigPart g = grid[blockIdx.x];
-    const BigLd B = states[g.front];
-    const int ps = B.k, ncols = group_cols(B, 16);
-    if (ncols <= 0) return;
-    const FrontLd F = d.fronts[B.s];
-    const int f = F.f;
-    const int gend = ps + ncols;
-    const int bx = g.part;
-    if (bx >= max(1, (f - gend + kGroupRows - 1) / kGroupRows)) return;
-    const double *G = d.arena + F.fofs;
-    double *W = d.work + F.wofs;
-    const double *gp = gpart + g.front * gpart_stride(nch);
-    const int64_t wcol0 = ps - B.pend0;  // W column of the group's first pivot
-    const int tid = threadIdx.x;
-    for (int e = tid; e < kGroupCols * kGroupCols; e += kLT) Wd[e >> 6][e & 63] = gp[kGdWd + e];
-    for (int e = tid; e < kGroupCols * 16; e += kLT) Lm[e >> 4][e & 15] = gp[kGdLm + e];
-    if (tid < kGroupCols) invd[tid] = gp[kGdInv + tid];
+        for (int i = 0; i < 16; ++i) {
+            const int c = w + 4 * i;
+            S[c * kRLd + lane] = (lane < ncols && c <= lane) ? v[i] : (lane == c ? 1.0 : 0.0);
+        }
+    }
+    const int nblk = (ncols + 15) / 16;
     __syncthreads();
-    const int i = gend + bx * kGroupRows + tid;
-    const bool rowok = i < f;
-    const int il = min(i, f - 1);
-    double a[kGroupCols];
+    for (int p = 0; p < nblk; ++p) {
+        if (w == 0) {
+            double a[16], x[16], l[16], dv[16], iv[16];
 #pragma unroll
-    for (int c = 0; c < kGroupCols; ++c)
-        a[c] = masked(G[static_cast<int64_t>(ps + min(c, ncols - 1)) * f + il], rowok && c < ncols);
-    // (the unguarded form unrolls into more registers than a 256-thread
-    // workgroup has)
-    grow_run<true, false>(a, ncols, Wd, Lm, invd, red, red2, wgmax, W, wcol0, f, i, rowok);
+            for (int c = 0; c < 16; ++c) {
+                a[c] = S[(16 * p + c) * kRLd + 16 * p + lr];
+                x[c] = S[(16 * p + c) * kRLd + lane];
+            }
+            const double d0 = row_bcast<0>(a[0]);
+            region_pivots<0>(a, x, l, dv, iv, d0, pivot_rcp(d0));
+#pragma unroll
+            for (int c = 0; c < 16; ++c) {
+                const int col = 16 * p + c;
+                S[col * kRLd + lane] = x[c];
+                Ls[col * kRLd + lane] = lane > col ? l[c] : x[c];
+                dd[col] = dv[c];
+                invd[col] = iv[c];
+            }
+        } else if (p > 0) {
+            // the rest of panel p - 1's update: columns from p + 1 on
+            int t = 0;
+            for (int c = p + 1; c < nblk; ++c)
+                for (int i = c; i < nblk; ++i)
+                    if (t++ % 3 == w - 1) region_update(S, Ls, p - 1, i, c);
+        }
+        __syncthreads();
+        if (p + 1 < nblk) {
+            if (w + p + 1 < nblk) region_update(S, Ls, p, w + p + 1, p + 1);
+            __syncthreads();
+        }
+    }
+    // the largest entry below each pivot, one quarter of the rows per wave
+    {
+        double mx = 0.0;
+        if (lane < ncols)
+            for (int r = max(16 * w, lane + 1); r < min(16 * w + 16, ncols); ++r) mx = fmax(mx, fabs(S[lane * kRLd + r]));
+        rs.v[tid] = mx;
+    }
     __syncthreads();
-    if (tid < ncols) gpart[g.front * gpart_stride(nch) + kGMax + bx * kGroupCols + tid] = wgmax[tid];
-    if (rowok) {
-#pragma unroll
-        for (int c = 0; c < kGroupCols; ++c)
-            if (c < ncols) W[static_cast<int64_t>(big_spec(F.ne) + c) * f + i] = a[c];
+    if (tid < 64) {
+        reinterpret_cast<unsigned long long *>(gp + kGMax)[tid] = static_cast<unsigned long long>(
+            __double_as_longlong(fmax(fmax(rs.v[tid], rs.v[tid + 64]), fmax(rs.v[tid + 128], rs.v[tid + 192]))));
+        if (tid < ncols) {
+            gp[kGdPiv + tid] = dd[tid];
+            gp[kGdInv + tid] = invd[tid];
+        }
+    }
+    for (int e = tid; e < 64 * 64; e += kLT) {
+        const int c = e >> 6, r = e & 63;
+        if (c < 16 * nblk) {
+            gp[kGdWd + e] = S[c * kRLd + r];
+            gp[kGdFin + e] = Ls[c * kRLd + r];
+        }
     }
 }
 
-// The accepted panels of a group, columns [ps, ps + nacc): the region's
-// final entries and W rows (its rows [ps, ps + ncols), from the region
-// launch's tables) and the rows below it from W's speculation columns.
-// Per row, the region launch and k_big_group carried out the operations
-// of the one-panel path in its order; a row of the region at or past nacc
-// went through the same operations on the accepted columns as a row below
-// it would have.
-__global__ __launch_bounds__(kLT) void k_big_gapply(LdltDev d, const BigLd *__restrict__ states,
-                                                    const BigPart *__restrict__ grid,
-                                                    const double *__restrict__ gpart, int32_t nch) {
+// Largest of 8 values per lane over the wavefront, value e in the lanes
+// whose top three bits are e: three halving exchanges (halves of the
+// wavefront, rows of 16 lanes, rotation by 8), then the 8 lanes that share e.
+__device__ __forceinline__ double wave_max8(double (&v)[8]) {
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    const auto pick = [](u2 lo, u2 hi) {
+        return fmax(__hiloint2double(hi[0], lo[0]), __hiloint2double(hi[1], lo[1]));
+    };
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        v[k] = pick(__builtin_amdgcn_permlane32_swap(__double2loint(v[k]), __double2loint(v[k + 4]), false, false),
+                    __builtin_amdgcn_permlane32_swap(__double2hiint(v[k]), __double2hiint(v[k + 4]), false, false));
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+        v[k] = pick(__builtin_amdgcn_permlane16_swap(__double2loint(v[k]), __double2loint(v[k + 2]), false, false),
+                    __builtin_amdgcn_permlane16_swap(__double2hiint(v[k]), __double2hiint(v[k + 2]), false, false));
+    const bool up = (threadIdx.x & 8) != 0;
+    double t = fmax(up ? v[1] : v[0], dpp_d<0x128>(up ? v[0] : v[1]));
+    t = fmax(t, dpp_d<kDppXor1>(t));
+    t = fmax(t, dpp_d<kDppXor2>(t));
+    return fmax(t, dpp_d<kDppHalfMirror>(t));
+}
+
+// Rows of a group below its diagonal region, [ps + ncols, f), kGroupRows
+// (one wavefront, a row per lane) per workgroup: column maxima per pivot to
+// the group buffer (atomic maxima of the bits of |entry|), each row's
+// unscaled column entries to W (the columns the panel kernel's pivots will
+// have: W column ps - pend0 + t, pend0 being the W base the panel kernel
+// starts from) and its final group entries to W's speculation columns
+// [big_spec, big_spec + 64). Nothing of the front square changes: a rejected
+// panel finds its columns as they were. W columns of rejected pivots are
+// rewritten (rows below the pivot) when those positions get their pivots.
+// A row's 64 columns stay in its lane's registers. Panel by panel: the
+// earlier panels' update on FP64 MFMA (operands and result through LDS, which
+// turns the tile's layout into rows per lane), then the panel's 16 pivots,
+// their multipliers broadcast inside each row of 16 lanes by DPP. Bound by
+// latency: the columns' loads, then wavefront-serial work (384 MFMAs of 64
+// cycles' issue, 480 FMAs with a broadcast each). 58 us with separate
+// multiplies and subtracts, multipliers from LDS and 256 rows a workgroup;
+// 32 us with all 2016 FMAs of a row on the vector unit; 16.8 us now.
+constexpr int kGLd = 80;  // LDS column stride: the two lane rows of a half wavefront fall on different banks
+
+template <int P, int T, int J>
+__device__ __forceinline__ void group_cols_fma(double (&a)[kGroupCols], double na, double l) {
+    if constexpr (J < 16) {
+        a[16 * P + J] = fma(na, row_bcast<J>(l), a[16 * P + J]);
+        group_cols_fma<P, T, J + 1>(a, na, l);
+    }
+}
+template <int P, int T>
+__device__ __forceinline__ void group_pivots(double (&a)[kGroupCols], const double (&l)[16]) {
+    if constexpr (T < 15) {
+        group_cols_fma<P, T, T + 1>(a, -a[16 * P + T], l[T]);
+        group_pivots<P, T + 1>(a, l);
+    }
+}
+// Panel P of the rows' columns; Lc[t][j]: multiplier of column j by pivot t;
+// X: the earlier panels' columns (slot per panel), D in a slot not needed any
+// more.
+template <int P>
+__device__ __forceinline__ void group_panel(double (&a)[kGroupCols], const double (*Lc)[kGLd], double (*X)[16][kGLd]) {
+    const int lane = threadIdx.x, lr = lane & 15, lk = lane >> 4;
+    if constexpr (P > 0) {
+        v4d_t acc[4];
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) acc[rt] = v4d_t{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < P; ++i)
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) {
+                const double l = Lc[16 * i + 4 * kk + lk][16 * P + lr];
+#pragma unroll
+                for (int rt = 0; rt < 4; ++rt)
+                    acc[rt] = __builtin_amdgcn_mfma_f64_16x16x4f64(l, X[i][4 * kk + lk][16 * rt + lr], acc[rt], 0, 0, 0);
+            }
+        double (*D)[kGLd] = X[P < 2 ? P : 2];
+        __syncthreads();
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) D[4 * v + lk][16 * rt + lr] = acc[rt][v];
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < 16; ++c) a[16 * P + c] -= D[c][lane];
+    }
+    double l[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) l[t] = Lc[16 * P + t][16 * P + lr];
+    group_pivots<P, 0>(a, l);
+    if constexpr (P < 3) {
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < 16; ++c) X[P][c][lane] = a[16 * P + c];
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(kGroupRows) void k_big_group(LdltDev d, const BigLd *__restrict__ states,
+                                                          const BigPart *__restrict__ grid,
+                                                          double *__restrict__ gpart) {
+    static_assert(kGroupRows == 64, "one wavefront, a row per lane");
+    __shared__ double Lc[kGroupCols][kGLd];
+    __shared__ double X[3][16][kGLd];
+    __shared__ double invs[kGroupCols];
     const BigPart g = grid[blockIdx.x];
     const BigLd B = states[g.front];
-    if (!B.g_apply) return;
-    const int ps = B.g_ps, nacc = B.g_n, ncols = B.g_cols;
+    const int ps = B.k, ncols = group_cols(B, 16);
+    if (ncols <= 0) return;
     const FrontLd F = d.fronts[B.s];
     const int f = F.f;
-    const int gend = ps + ncols;
-    const int bx = g.part;
-    if (bx >= max(1, (f - gend + kGroupRows - 1) / kGroupRows)) return;
-    double *G = d.arena + F.fofs;
+    const int lane = threadIdx.x;
+    const int i = ps + ncols + g.part * kGroupRows + lane;
+    if (ps + ncols + g.part * kGroupRows >= f) return;
+    const bool rowok = i < f;
+    const double *Gi = d.arena + F.fofs + static_cast<int64_t>(ps) * f + min(i, f - 1);
+    const double *__restrict__ gp = gpart + g.front * kGroupBuf;
+    double a[kGroupCols];
+#pragma unroll
+    for (int c = 0; c < kGroupCols; ++c) a[c] = Gi[static_cast<int64_t>(min(c, ncols - 1)) * f];
+    invs[lane] = gp[kGdInv + min(lane, ncols - 1)];
+    // the multipliers (columns past the region's panels are not read)
+#pragma unroll
+    for (int t0 = 0; t0 < kGroupCols; t0 += 16) {
+        if (t0 < ncols) {
+            double v[16];
+#pragma unroll
+            for (int t = 0; t < 16; ++t) v[t] = gp[kGdFin + (t0 + t) * 64 + lane];
+#pragma unroll
+            for (int t = 0; t < 16; ++t) Lc[t0 + t][lane] = v[t];
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < kGroupCols; ++c) a[c] = masked(a[c], rowok && c < ncols);
+    __syncthreads();
+    group_panel<0>(a, Lc, X);
+    if (ncols > 16) group_panel<1>(a, Lc, X);
+    if (ncols > 32) group_panel<2>(a, Lc, X);
+    if (ncols > 48) group_panel<3>(a, Lc, X);
     double *W = d.work + F.wofs;
-    const double *gp = gpart + g.front * gpart_stride(nch);
-    const int64_t wcol0 = ps - B.w_base;
-    const int tid = threadIdx.x;
-    if (bx == 0) {
-        for (int e = tid; e < kGroupCols * kGroupCols; e += kLT) {
-            const int c = e >> 6, rw = e & 63;
-            if (c < nacc && rw < ncols && c <= rw) {
-                G[static_cast<int64_t>(ps + c) * f + ps + rw] = gp[kGdFin + e];
-                if (c < rw) W[(wcol0 + c) * f + ps + rw] = gp[kGdWd + e];
+    double *Wu = W + static_cast<int64_t>(ps - B.pend0) * f + i;    // from the W column of the group's first pivot
+    double *Wf = W + static_cast<int64_t>(big_spec(F.ne)) * f + i;
+    auto *gmax = reinterpret_cast<unsigned long long *>(gpart + g.front * kGroupBuf + kGMax);
+#pragma unroll
+    for (int c0 = 0; c0 < kGroupCols; c0 += 8) {
+        if (c0 >= ncols) break;
+        double m[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int c = c0 + u;
+            m[u] = fabs(a[c]);
+            if (rowok && c < ncols) {
+                Wu[static_cast<int64_t>(c) * f] = a[c];
+                Wf[static_cast<int64_t>(c) * f] = a[c] * invs[c];
             }
         }
-    }
-    const int i = gend + bx * kGroupRows + tid;
-    if (i < f) {
-        // eight columns' loads in flight at a time
-        const double *src = W + static_cast<int64_t>(big_spec(F.ne)) * f + i;
-        double *dst = G + static_cast<int64_t>(ps) * f + i;
-        for (int c0 = 0; c0 < nacc; c0 += 8) {
-            double v[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = src[static_cast<int64_t>(min(c0 + u, nacc - 1)) * f];
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (c0 + u < nacc) dst[static_cast<int64_t>(c0 + u) * f] = v[u];
-        }
+        const double mx = wave_max8(m);
+        const int c = c0 + (lane >> 3);
+        if ((lane & 7) == 0 && c < ncols)
+            atomicMax(gmax + c, static_cast<unsigned long long>(__double_as_longlong(mx)));
     }
 }
 
-__global__ __launch_bounds__(kLT) void k_big_panel(LdltDev d, BigLd *states, Prm prm, int32_t nb,
-                                                  const double *__restrict__ gpart, int32_t nch) {
+// Leading panels of a group that pass the first test: the number of accepted
+// columns, from the pivots and column maxima the region and rows launches
+// left (lane c of every wavefront tests column c). A NaN maximum fails.
+__device__ __forceinline__ int group_accepted(const double *gp, int gcols, const Prm &prm, double &piv) {
+    const int c = threadIdx.x & 63;
+    bool ok = true;
+    piv = 0.0;
+    if (c < gcols) {
+        piv = gp[kGdPiv + c];
+        const double a0 = fabs(piv), cm = gp[kGMax + c];
+        ok = a0 >= prm.eff_small && prm.u * cm <= a0 && !(a0 < kWeakPivotRatio * cm);
+    }
+    const unsigned long long bad = __ballot(!ok);
+    if (bad == 0) return gcols;
+    return (__ffsll(bad) - 1) / 16 * 16;
+}
+
+// The panel launch, a workgroup per kGroupRows rows of a front: every
+// workgroup judges the group and copies the accepted panels' columns of its
+// rows from W's speculation columns to the front; the first one also writes
+// the region's own entries and does the pivot logic: what to update and
+// flush, or, without an accepted group, one panel with the full pivot
+// search. It reads the round's states and writes the next ones (other
+// workgroups still read the old).
+__global__ __launch_bounds__(kLT) void k_big_panel(LdltDev d, const BigLd *__restrict__ states,
+                                                  BigLd *__restrict__ next, const BigPart *__restrict__ grid,
+                                                  Prm prm, int32_t nb, const double *__restrict__ gpart) {
     __shared__ RedScratch rs;
     __shared__ int cnt[3];
-    BigLd &B = states[blockIdx.x];
+    const BigPart g = grid[blockIdx.x];
+    BigLd B = states[g.front];
     const int pass = B.pass;
+    const int gcols = gpart ? group_cols(B, nb) : 0;
+    const int tid = threadIdx.x;
     if (pass == 2) {
-        // done: nothing for this iteration's update kernel
-        if (threadIdx.x == 0) {
+        // done: nothing for this round's update launch
+        if (g.part == 0 && tid == 0) {
             B.u_p1 = B.u_p0;
             B.x_p1 = B.x_p0;
             B.stalled = 0;
-            B.g_apply = 0;
+            next[g.front] = B;
         }
         return;
     }
+    if (gcols <= 0 && g.part > 0) return;
     FrontLd &Fd = d.fronts[B.s];
     const int f = Fd.f, ne = Fd.ne;
     int32_t *rows = d.rows + Fd.rofs;
     int8_t *tags = d.tags + Fd.rofs;
     double *W = d.work + Fd.wofs;
     FV A{d.arena + Fd.fofs, f, f};
-    const int tid = threadIdx.x;
     int k = B.k, oe = B.oe, pend0 = B.pend0, full = B.full;
     const int live = B.live;
-    if (tid < 3) cnt[tid] = B.cnt[tid];
     double flops = B.flops;
-    __syncthreads();
     int u_c0 = 0, u_c1 = 0, u_p0 = 0, u_p1 = 0, x_c0 = ne, x_p0 = 0, x_p1 = 0, w_base = pend0;
     int stalled = 0, npass = pass, ps = k, pl = k;
-    int spec = B.spec, g_apply = 0, g_ps = 0, g_n = 0, g_cols = 0, searched = 0;
+    int spec = B.spec, searched = 0;
     bool group_done = false;
-    const int gcols = gpart ? group_cols(B, nb) : 0;
+    int nacc = 0, npos = 0, nzero = 0;
     if (gcols > 0) {
-        // decide on the group the stats launch evaluated: column maxima over
-        // its workgroups and the diagonal region, then the first test per
-        // pivot in order; whole panels are accepted
-        __shared__ double gmax[kGroupCols], gd[kGroupCols];
-        __shared__ int acc_s;
-        const int nact = max(1, (f - (k + gcols) + kGroupRows - 1) / kGroupRows);
-        const double *gp = gpart + blockIdx.x * gpart_stride(nch);
-        {
-            const int c = tid & 63, part = tid >> 6;
-            double mx = 0.0;
-            if (c < gcols)
-                for (int w = part; w < nact; w += 4) mx = fmax(mx, gp[kGMax + w * kGroupCols + c]);
-            rs.v[tid] = mx;
-        }
-        __syncthreads();
-        if (tid < kGroupCols) {
-            const double pm = fmax(fmax(rs.v[tid], rs.v[tid + 64]), fmax(rs.v[tid + 128], rs.v[tid + 192]));
-            gmax[tid] = tid < gcols ? fmax(pm, gp[kGdMax + tid]) : 0.0;
-            gd[tid] = tid < gcols ? gp[kGdPiv + tid] : 0.0;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            int nacc = 0;
-            for (int c0 = 0; c0 < gcols; c0 += 16) {
-                const int c1 = min(c0 + 16, gcols);
-                bool ok = true;
-                for (int kk = c0; kk < c1 && ok; ++kk) {
-                    const double a0 = fabs(gd[kk]), cm = gmax[kk];
-                    ok = a0 >= prm.eff_small && !(prm.u * cm > a0) && !(a0 < kWeakPivotRatio * cm);
+        const double *gp = gpart + g.front * kGroupBuf;
+        double piv;
+        nacc = group_accepted(gp, gcols, prm, piv);
+        if (nacc > 0) {
+            // rows below the region: eight columns' loads in flight
+            const int i = k + gcols + g.part * kGroupRows + (tid & 63);
+            if (i < f) {
+                const double *src = W + static_cast<int64_t>(big_spec(ne)) * f + i;
+                double *dst = A.F + static_cast<int64_t>(k) * f + i;
+                for (int c0 = 16 * (tid >> 6); c0 < min(nacc, 16 * (tid >> 6) + 16); c0 += 8) {
+                    double v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) v[u] = src[static_cast<int64_t>(min(c0 + u, nacc - 1)) * f];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        if (c0 + u < nacc) dst[static_cast<int64_t>(c0 + u) * f] = v[u];
                 }
-                if (!ok) break;
-                nacc = c1;
             }
-            acc_s = nacc;
+        }
+        if (g.part > 0) return;
+        if (nacc > 0) {
+            // the region's entries; a row of it at or past nacc went through
+            // the same operations on the accepted columns as a row below it
+            const int64_t wcol0 = k - pend0;
+            for (int e = tid; e < kGroupCols * kGroupCols; e += kLT) {
+                const int c = e >> 6, rw = e & 63;
+                if (c < nacc && rw < gcols && c <= rw) {
+                    A.at(k + rw, k + c) = gp[kGdFin + e];
+                    if (c < rw) W[(wcol0 + c) * f + k + rw] = gp[kGdWd + e];
+                }
+            }
+            // inertia of the accepted pivots, as inertia_1x1; flops in exact
+            // integers
+            const bool in = (tid & 63) < nacc;
+            const bool zero = in && (!isfinite(piv) || fabs(piv) < prm.eff_small);
+            const bool pos = in && !zero && piv > 0.0;
+            nzero = __popcll(__ballot(zero));
+            npos = __popcll(__ballot(pos));
             for (int kk = 0; kk < nacc; ++kk) {
-                inertia_1x1(gd[kk], prm.eff_small, cnt);
                 const double rem = static_cast<double>(f - (k + kk + 1));
                 flops += rem + rem * (rem + 1.0);
             }
-        }
-        __syncthreads();
-        const int nacc = acc_s;
-        if (nacc > 0) {
             for (int c = tid; c < nacc; c += kLT) tags[k + c] = 1;
             const int kn = k + nacc;
             if (kn < oe) {
@@ -1538,10 +1629,6 @@ __global__ __launch_bounds__(kLT) void k_big_panel(LdltDev d, BigLd *states, Prm
                 pend0 = kn;
                 oe = min(ne, kn + B.outer);
             }
-            g_apply = 1;
-            g_ps = k;
-            g_n = nacc;
-            g_cols = gcols;
             spec = nacc == gcols ? 1 : 0;  // a panel failed inside: the next panel goes the one-panel way
             ps = k + ((nacc - 1) / 16) * 16;
             pl = kn;
@@ -1549,6 +1636,8 @@ __global__ __launch_bounds__(kLT) void k_big_panel(LdltDev d, BigLd *states, Prm
             group_done = true;
         }
     }
+    if (tid < 3) cnt[tid] = states[g.front].cnt[tid] + (tid == 0 ? npos : (tid == 1 ? nacc - npos - nzero : nzero));
+    __syncthreads();
     if (group_done) {
     } else if (pass == 0) {
         spec = 1;
@@ -1667,10 +1756,7 @@ __global__ __launch_bounds__(kLT) void k_big_panel(LdltDev d, BigLd *states, Prm
         B.flops = flops;
         B.searches += searched;
         B.spec = spec;
-        B.g_apply = g_apply;
-        B.g_ps = g_ps;
-        B.g_n = g_n;
-        B.g_cols = g_cols;
+        next[g.front] = B;
     }
 }
 
@@ -1695,45 +1781,6 @@ __global__ __launch_bounds__(kLT, 2) void k_big_update(LdltDev d, const BigLd *_
         big_tile<MODE>(d, F, W, B.w_base, u ? B.u_c0 : B.x_c0, u ? B.u_c1 : F.ne, u ? B.u_p0 : B.x_p0,
                     u ? B.u_p1 : B.x_p1, u ? tile : tile - t1, smem);
         __syncthreads();
-    }
-}
-
-// Partner pulls or rotation of a stalled first-pass panel
-// (ldlt_kernel.cpp:1052-1097); every column is current (flushed).
-__global__ __launch_bounds__(kLT) void k_big_stall(LdltDev d, BigLd *states, int32_t nb) {
-    __shared__ RedScratch rs;
-    __shared__ int32_t order[128];
-    BigLd &B = states[blockIdx.x];
-    if (B.pass != 0 || !B.stalled) return;
-    FrontLd &Fd = d.fronts[B.s];
-    const int f = Fd.f, ne = Fd.ne;
-    int32_t *rows = d.rows + Fd.rofs;
-    FV A{d.arena + Fd.fofs, f, f};
-    const int tid = threadIdx.x;
-    const int k = B.k, pl = B.pl;
-    int live = B.live;
-    if (k != B.k_paired) {
-        const int np = partner_pairs_wg(A, k, pl, ne, nb, rows, order, rs);
-        if (np > 0) {
-            place_rows_wg(A, k, ne, np, order, rows, rs);
-            if (tid == 0) {
-                B.live = max(live, k + np);
-                B.k_paired = k;
-                B.stalled = 0;
-                B.stalls += 1;
-                B.pulls += np / 2;
-            }
-            return;
-        }
-    }
-    const int m = pl - k;
-    const int mv = min(m, live - pl);
-    for (int t = 0; t < mv; ++t) sym_swap_wg(A, k + t, live - mv + t, rows, nullptr, 0, 0, 0);
-    if (tid == 0) {
-        B.live = live - m;
-        B.stalled = 0;
-        B.stalls += 1;
-        B.rotated += m;
     }
 }
 
@@ -1987,23 +2034,6 @@ __global__ void k_big_finish(LdltDev d, const BigLd *__restrict__ states, int32_
     F.searches = B.searches;
 }
 
-void launch_big_panel(hipStream_t st, const LdltDev &d, BigLd *states, int32_t nbig, double u, double eff_small,
-                      double small_pivot, int32_t nb, const double *gpart, int32_t nch) {
-    Prm prm{u, eff_small, small_pivot};
-    k_big_panel<<<dim3(nbig), kLT, 0, st>>>(d, states, prm, nb, gpart, nch);
-}
-
-void launch_big_group_stats(hipStream_t st, const LdltDev &d, const BigLd *states, int32_t nbig, const BigGrid &g,
-                            double *gpart, int32_t nch) {
-    k_big_gdiag<<<dim3(nbig), 64, 0, st>>>(d, states, gpart, nch);
-    k_big_group<<<dim3(g.nrows), kLT, 0, st>>>(d, states, g.rows, gpart, nch);
-}
-
-void launch_big_group_apply(hipStream_t st, const LdltDev &d, const BigLd *states, const BigGrid &g, double *gpart,
-                            int32_t nch) {
-    k_big_gapply<<<dim3(g.nrows), kLT, 0, st>>>(d, states, g.rows, gpart, nch);
-}
-
 void launch_big_update(hipStream_t st, const LdltDev &d, const BigLd *states, const BigGrid &g,
                        const int32_t *nmode) {
     const dim3 nt(g.ntiles);
@@ -2018,9 +2048,14 @@ void launch_big_update(hipStream_t st, const LdltDev &d, const BigLd *states, co
     }
 }
 
-void launch_big_stall(hipStream_t st, const LdltDev &d, BigLd *states, int32_t nbig, int32_t nb) {
-    if (nbig <= 0) return;
-    k_big_stall<<<dim3(nbig), kLT, 0, st>>>(d, states, nb);
+void launch_big_round(hipStream_t st, const LdltDev &d, BigLd *states, BigLd *next, int32_t nbig, const BigGrid &g,
+                      double u, double eff_small, double small_pivot, int32_t nb, double *gpart,
+                      const int32_t *nmode) {
+    const Prm prm{u, eff_small, small_pivot};
+    k_big_region<<<dim3(nbig), kLT, 0, st>>>(d, states, gpart, nb);
+    if (gpart != nullptr) k_big_group<<<dim3(g.nrows), kGroupRows, 0, st>>>(d, states, g.rows, gpart);
+    k_big_panel<<<dim3(g.nrows), kLT, 0, st>>>(d, states, next, g.rows, prm, nb, gpart);
+    launch_big_update(st, d, next, g, nmode);
 }
 
 void launch_big_cb(hipStream_t st, const LdltDev &d, const BigLd *states, const BigGrid &g, int32_t c0, int32_t width,

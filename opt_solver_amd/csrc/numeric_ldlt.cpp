@@ -267,8 +267,8 @@ static int ldlt_dev_levels(smfgpu_plan_s *P, int32_t lv0, double u, double eff_s
 // fronts' results. The state is read back after as many rounds as the
 // fronts need when every panel group is accepted (a round then takes 64
 // pivots of each), and again after what is left by the same count, at most
-// kBigCheck rounds at a time: an idle round costs its six launches (about
-// 20 us), a read-back about as much.
+// kBigCheck rounds at a time: an idle round costs its four launches (about
+// 13 us), a read-back about as much.
 static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vector<int32_t> &big,
                            const smfgpu_factor_options &opt, double eff_small, double small, int32_t nb,
                            std::vector<BigLd> &h, int32_t &reduced) {
@@ -341,7 +341,9 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
         cap += 4 * (static_cast<int64_t>(F.ne) / std::max(nb, 1) + 2) + 2 * static_cast<int64_t>(F.ne);
     }
     reduced += nbig - nmode[0];
-    if ((rc = ensure(P->d_big, static_cast<size_t>(nbig), false, "large-front states"))) return rc;
+    // two sets of states: a round reads one and writes the other
+    if ((rc = ensure(P->d_big, 2 * static_cast<size_t>(nbig), false, "large-front states"))) return rc;
+    BigLd *cur = P->d_big.p, *nxt = P->d_big.p + nbig;
     // bf16 planes of the outer-block updates' operands (BF16 and split-BF16
     // fronts, and the training pairs' split-BF16 and BF16 runs)
     if (P->ldlt_planes != 0 && (nmode[2] + nmode[3] > 0 || (collect && !sf.empty()))) {
@@ -351,14 +353,13 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
         if ((rc = ensure(P->d_xpl, static_cast<size_t>(planes), false, "update planes"))) return rc;
         d.xpl = P->d_xpl.p;
     }
-    HIP_OK(hipMemcpyAsync(P->d_big.p, h.data(), nbig * sizeof(BigLd), hipMemcpyHostToDevice, st));
-    // workgroups of each launch, by front: 256-row chunks for the group
-    // kernels; for the updates as many workgroups as the front has tiles of
+    HIP_OK(hipMemcpyAsync(cur, h.data(), nbig * sizeof(BigLd), hipMemcpyHostToDevice, st));
+    // workgroups of each launch, by front: 64-row chunks for the group
+    // and panel kernels; for the updates as many workgroups as the front has tiles of
     // its lower triangle, at most its share of ldlt_update_wg (at least 64),
     // rounded up to a multiple of 8
     const int32_t per_front = std::max(64, P->ldlt_update_wg / nbig) / 8 * 8;
     const int32_t wide_per_front = std::max(8, per_front / 16 * 8);
-    int32_t maxf = 0;
     std::vector<BigPart> parts;
     const auto add_parts = [&](auto &&count) {
         const size_t first = parts.size();
@@ -372,8 +373,6 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
         const int64_t m = (f + tile - 1) / tile;
         return static_cast<int32_t>(std::min<int64_t>(cap, (m * (m + 1) / 2 + 7) / 8 * 8));
     };
-    for (int32_t s : big) maxf = std::max(maxf, P->fl[s].f);
-    const int32_t nch = (maxf + kGroupRows - 1) / kGroupRows + 1;
     BigGrid grid{};
     grid.nrows = add_parts([&](int32_t f) { return (f + kGroupRows - 1) / kGroupRows; });
     grid.ntiles = add_parts([&](int32_t f) { return tile_parts(f, 128, per_front); });
@@ -383,8 +382,7 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
     grid.rows = P->d_parts.p;
     grid.tiles = grid.rows + grid.nrows;
     grid.wide = grid.tiles + grid.ntiles;
-    const size_t gstride = static_cast<size_t>(nch) * kGroupCols + kGroupBuf;
-    if (group && (rc = ensure(P->d_gpart, static_cast<size_t>(nbig) * gstride, false, "group buffer"))) return rc;
+    if (group && (rc = ensure(P->d_gpart, static_cast<size_t>(nbig) * kGroupBuf, false, "group buffer"))) return rc;
     double *gpart = group ? P->d_gpart.p : nullptr;
     const auto rounds_left = [&]() {
         int32_t left = 0;
@@ -394,13 +392,10 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
     };
     int64_t check = rounds_left();
     for (int64_t it = 1;; ++it) {
-        if (group) launch_big_group_stats(st, d, P->d_big.p, nbig, grid, gpart, nch);
-        launch_big_panel(st, d, P->d_big.p, nbig, opt.pivot_u, eff_small, small, nb, gpart, nch);
-        if (group) launch_big_group_apply(st, d, P->d_big.p, grid, gpart, nch);
-        launch_big_update(st, d, P->d_big.p, grid, nmode);
-        launch_big_stall(st, d, P->d_big.p, nbig, nb);
+        launch_big_round(st, d, cur, nxt, nbig, grid, opt.pivot_u, eff_small, small, nb, gpart, nmode);
+        std::swap(cur, nxt);
         if (it == check) {
-            HIP_OK(hipMemcpyAsync(h.data(), P->d_big.p, nbig * sizeof(BigLd), hipMemcpyDeviceToHost, st));
+            HIP_OK(hipMemcpyAsync(h.data(), cur, nbig * sizeof(BigLd), hipMemcpyDeviceToHost, st));
             HIP_OK(hipStreamSynchronize(st));
             bool done = true;
             for (const BigLd &B : h) done = done && B.pass == 2;
@@ -417,10 +412,10 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
     auto cb_update = [&](const int32_t *nm) {
         if (nm[0] + nm[1] > 0 || (d.xpl == nullptr && nm[2] + nm[3] > 0))
             for (int32_t c0 = 0; c0 < pmax; c0 += kBigOuter)
-                launch_big_cb(st, d, P->d_big.p, grid, c0, kBigOuter, nm, false);
+                launch_big_cb(st, d, cur, grid, c0, kBigOuter, nm, false);
         if (d.xpl != nullptr && nm[2] + nm[3] > 0)
             for (int32_t c0 = 0; c0 < pmax; c0 += P->ldlt_outer_wide)
-                launch_big_cb(st, d, P->d_big.p, grid, c0, P->ldlt_outer_wide, nm, true);
+                launch_big_cb(st, d, cur, grid, c0, P->ldlt_outer_wide, nm, true);
     };
     const bool labels = collect && !sf.empty() && maxq > 0;
     if (labels) {
@@ -449,18 +444,18 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
                 h[b].prec = is_cand[b] ? m : -1;  // -1: no update kernel touches the front
                 if (is_cand[b]) ++nm[m];
             }
-            HIP_OK(hipMemcpyAsync(P->d_big.p, h.data(), nbig * sizeof(BigLd), hipMemcpyHostToDevice, st));
+            HIP_OK(hipMemcpyAsync(cur, h.data(), nbig * sizeof(BigLd), hipMemcpyHostToDevice, st));
             cb_update(nm);
             if ((rc = copy_sq(true, kSelOutOfCode[m])) || (rc = copy_sq(false, 3))) return rc;
         }
         for (BigLd &B : h) B.prec = 0;
-        HIP_OK(hipMemcpyAsync(P->d_big.p, h.data(), nbig * sizeof(BigLd), hipMemcpyHostToDevice, st));
+        HIP_OK(hipMemcpyAsync(cur, h.data(), nbig * sizeof(BigLd), hipMemcpyHostToDevice, st));
     }
     cb_update(nmode);
     if (labels)
         launch_label_sq(st, P->d_arena.p, P->d_snap.p, snap_total, P->d_selfr.p, static_cast<int32_t>(sf.size()), maxq,
                         P->d_lab.p);
-    launch_big_finish(st, d, P->d_big.p, nbig);
+    launch_big_finish(st, d, cur, nbig);
     HIP_OK(hipGetLastError());
     return SMFGPU_OK;
 }

@@ -56,10 +56,11 @@ struct LdltDev {
 };
 
 // Large fronts (multi-workgroup blocked LDL^T): one state per front,
-// advanced by a panel kernel (one workgroup per front: the blocked
-// algorithm's pivot logic on a panel of nb columns), an update kernel (many
-// workgroups, MFMA) and a stall kernel (partner pulls / rotation), launched
-// in turn by the host until every front is done. The per-panel deferred
+// advanced in rounds by a region kernel (one workgroup per front: a stalled
+// panel's partner pulls / rotation, a speculative group's diagonal region),
+// the group's rows kernel, a panel kernel (the blocked algorithm's pivot
+// logic on the group or on a panel of nb columns) and an update kernel (many
+// workgroups, MFMA), launched in turn by the host until every front is done. The per-panel deferred
 // updates go to the columns of a kBigOuter-wide outer block; the pivots'
 // updates of the columns beyond it are held back (their unscaled columns
 // kept in W) and applied in one flush when the outer block ends, before a
@@ -93,8 +94,6 @@ struct BigLd {
     int32_t cnt[3];
     int32_t stalls, pulls, rotated, searches;  // as FrontLd's
     int32_t spec;               // 1: the next first-pass iteration tries a speculative group
-    int32_t g_apply, g_ps, g_n; // accepted group to write: columns [g_ps, g_ps + g_n)
-    int32_t g_cols;             // the group's width (its diagonal region's rows)
     int32_t prec;               // precision code of the MFMA updates: 0 FP64, 1 FP32, 2 BF16, 3 split BF16
     double flops;
 };
@@ -107,15 +106,15 @@ struct BigPart {
     int32_t front, part, parts;
 };
 struct BigGrid {
-    const BigPart *rows;    // 256-row chunks (group kernels)
+    const BigPart *rows;    // kGroupRows-row chunks (group and panel kernels)
     const BigPart *tiles;   // 128 x 128 update tiles, a multiple of 8 per front (one run of tiles per XCD)
     const BigPart *wide;    // 256 x 256 update tiles, likewise
     int32_t nrows, ntiles, nwide;
 };
 constexpr int32_t kGroupCols = 64;   // columns of a speculative group (four panels of 16)
-constexpr int32_t kGroupRows = 256;  // rows per workgroup below a group's diagonal region
+constexpr int32_t kGroupRows = 64;   // rows per workgroup below a group's diagonal region
 static_assert(big_work(1) - big_spec(1) == kGroupCols, "W holds a group's speculative columns");
-constexpr int64_t kGroupBuf = 192 + 64 * 16 + 2 * 64 * 64;  // group buffer per front before the per-workgroup maxima
+constexpr int64_t kGroupBuf = 192 + 2 * 64 * 64;  // group buffer per front (doubles)
 
 // Static pivoting (control.hpp:333-364): sp = static_pivot_tol * max|A|
 // (0: off), fallback = fallback_static_pivot_tol * max|A| for roots and
@@ -186,19 +185,14 @@ void launch_ldlt_fwd_step(hipStream_t st, const LdltDev &d, const SolveItem *ite
                           double *y, int32_t n, int32_t nrhs);
 void launch_ldlt_bwd_step(hipStream_t st, const LdltDev &d, const SolveItem *items, int64_t count, bool wide,
                           double *y, int32_t n, int32_t nrhs);
-// one iteration's pivot logic; with gpart set it first decides on the group
-// the stats launch evaluated (nch workgroups per front)
-void launch_big_panel(hipStream_t st, const LdltDev &d, BigLd *states, int32_t nbig, double u, double eff_small,
-                      double small_pivot, int32_t nb, const double *gpart, int32_t nch);
-// speculative group: column maxima (stats) and the accepted panels' rows (apply)
-void launch_big_group_stats(hipStream_t st, const LdltDev &d, const BigLd *states, int32_t nbig, const BigGrid &g,
-                            double *gpart, int32_t nch);
-void launch_big_group_apply(hipStream_t st, const LdltDev &d, const BigLd *states, const BigGrid &g, double *gpart,
-                            int32_t nch);
+// one round of the level's large fronts: the states of the round and,
+// written by the panel launch, the next ones; gpart: the group buffers (null:
+// one panel per round)
+void launch_big_round(hipStream_t st, const LdltDev &d, BigLd *states, BigLd *next, int32_t nbig, const BigGrid &g,
+                      double u, double eff_small, double small_pivot, int32_t nb, double *gpart,
+                      const int32_t *nmode);
 // nmode[m]: fronts of the level whose updates run in precision code m
 // (0 FP64, 1 FP32, 2 BF16, 3 split BF16); a launch per code in use
-void launch_big_update(hipStream_t st, const LdltDev &d, const BigLd *states, const BigGrid &g, const int32_t *nmode);
-void launch_big_stall(hipStream_t st, const LdltDev &d, BigLd *states, int32_t nbig, int32_t nb);
 // final contribution-block update with pivots [c0, c0 + width) of every
 // front (L*D of the chunk into W first); then the fronts' results
 void launch_big_cb(hipStream_t st, const LdltDev &d, const BigLd *states, const BigGrid &g, int32_t c0, int32_t width,
