@@ -755,28 +755,32 @@ constexpr int kSyrkKc32 = 32;
 constexpr int kSyrkKcBf = 64;
 constexpr int kSyrkKcBf3 = 32;
 
-template <int MODE, int kAhead>
-__device__ __forceinline__ void syrk_tile(const DevPtrs &d, const SyrkItem &it, unsigned char *smem) {
+template <int MODE, int kAhead, int TILE = kT>
+__device__ __forceinline__ void syrk_tile(const DevPtrs &d, const SyrkItem &it, int i0, int j0, unsigned char *smem) {
+    static_assert(TILE == kT || MODE == 0, "64 x 64 tiles are FP64 only");
     typedef typename std::conditional<MODE == 0, double, float>::type E;
     typedef SyrkMfma<E> M;
+    constexpr int kNB = TILE / 32, kW = TILE / 2;
     const FrontDev F = d.fronts[it.s];
     const int f = F.f;
-    const int i0 = it.i0, j0 = it.j0;
     const int j1 = min(it.j1, f);
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int w = tid >> 6;
     const int wr = w >> 1, wc = w & 1;
-    const bool active = (i0 + wr * 64 + 63) >= (j0 + wc * 64);
-    typename M::acc_t acc[4][4];
+    const bool active = (i0 + wr * kW + kW - 1) >= (j0 + wc * kW);
+    typename M::acc_t acc[kNB][kNB];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < kNB; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = M::zero();
+        for (int b = 0; b < kNB; ++b) acc[a][b] = M::zero();
     if constexpr (MODE == 0) {
+        if (TILE < kT && (i0 + TILE <= j0 || i0 >= f || j0 >= j1)) return;  // a quarter outside the lower part
         const double *Lb = d.L + F.lofs;
-        if (active) tile_loop<double, true, kSyrkKc64, kAhead>(Lb, Lb, f, 0, i0, j0, f, j1, it.t0, it.t1, smem, acc);
-        else tile_loop<double, false, kSyrkKc64, kAhead>(Lb, Lb, f, 0, i0, j0, f, j1, it.t0, it.t1, smem, acc);
+        if (active)
+            tile_loop<double, true, kSyrkKc64, kAhead, double, TILE>(Lb, Lb, f, 0, i0, j0, f, j1, it.t0, it.t1, smem, acc);
+        else
+            tile_loop<double, false, kSyrkKc64, kAhead, double, TILE>(Lb, Lb, f, 0, i0, j0, f, j1, it.t0, it.t1, smem, acc);
     } else if constexpr (MODE == 1) {
         const float *Lb = d.L32 + F.lofs;
         if (active) tile_loop<float, true, kSyrkKc32, kAhead>(Lb, Lb, f, 0, i0, j0, f, j1, it.t0, it.t1, smem, acc);
@@ -790,32 +794,32 @@ __device__ __forceinline__ void syrk_tile(const DevPtrs &d, const SyrkItem &it, 
         else tile_loop_bf16p<kSplit, false, kKc>(Lh, Ll, Lh, Ll, f, i0, j0, f, j1, it.t0, it.t1, smem, acc);
     }
     if (!active) return;
-    // C -= acc, 16 elements at a time: all 16 loads issued before the
+    // C -= acc, a column block at a time: all its loads issued before the
     // stores; elements outside the tile's lower part read and write a junk
     // slot instead, so loads and stores are unconditional
     double *junk = d.junk + threadIdx.x;
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        double *dst[4][4];
-        double old[4][4];
+    for (int m = 0; m < kNB; ++m) {
+        double *dst[kNB][4];
+        double old[kNB][4];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int j = j0 + wc * 64 + m * 16 + M::row(v, lane);
+            const int j = j0 + wc * kW + m * 16 + M::row(v, lane);
             double *cb = col_base(d, F, min(j, j1 - 1));
 #pragma unroll
-            for (int nn = 0; nn < 4; ++nn) {
-                const int i = i0 + wr * 64 + nn * 16 + (lane & 15);
+            for (int nn = 0; nn < kNB; ++nn) {
+                const int i = i0 + wr * kW + nn * 16 + (lane & 15);
                 dst[nn][v] = (i < f && j < j1 && i >= j) ? cb + i : junk;
             }
         }
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
-            for (int nn = 0; nn < 4; ++nn) old[nn][v] = *dst[nn][v];
+            for (int nn = 0; nn < kNB; ++nn) old[nn][v] = *dst[nn][v];
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
-            for (int nn = 0; nn < 4; ++nn) *dst[nn][v] = old[nn][v] - static_cast<double>(acc[m][nn][v]);
+            for (int nn = 0; nn < kNB; ++nn) *dst[nn][v] = old[nn][v] - static_cast<double>(acc[m][nn][v]);
     }
 }
 
@@ -836,7 +840,24 @@ __global__ __launch_bounds__(kThreads) void k_syrk64(DevPtrs d, const SyrkItem *
     __shared__ __attribute__((aligned(16))) unsigned char smem[tile_lds_bytes<double, kSyrkKc64>()];
     const SyrkItem it = items[xcd_contiguous(blockIdx.x, gridDim.x)];
     if (d.prec != nullptr && d.prec[it.s] != 0) return;
-    syrk_tile<0, kAhead>(d, it, smem);
+    syrk_tile<0, kAhead>(d, it, it.i0, it.j0, smem);
+}
+
+// The same items in four 64 x 64 tiles each (a workgroup per quarter, 32 KB
+// of LDS): launches of few items, whose 128 x 128 tiles would leave CUs idle
+// for the length of one tile. Fewer than 128 items: a 64-column update 13 us
+// against 22, a 512-column one 40 against 87. Up to 512 items (two of the
+// larger tiles per CU): 24 against 29 us, and 104-115 against 118-132 us at
+// 512 columns; deeper updates read too much twice (465 items of 2000 columns
+// 523 against 455 us).
+constexpr int64_t kSyrkSmall = 512, kSyrkSmallDeep = 256;
+constexpr int32_t kSyrkSmallDepth = 512;
+__global__ __launch_bounds__(kThreads) void k_syrk64_small(DevPtrs d, const SyrkItem *__restrict__ items) {
+    __shared__ __attribute__((aligned(16))) unsigned char smem[tile_lds_bytes<double, kSyrkKc64, 64>()];
+    const int b = xcd_contiguous(blockIdx.x, gridDim.x);
+    const SyrkItem it = items[b >> 2];
+    if (d.prec != nullptr && d.prec[it.s] != 0) return;
+    syrk_tile<0, 2, 64>(d, it, it.i0 + 64 * (b & 1), it.j0 + 32 * (b & 2), smem);
 }
 
 template <int MODE>
@@ -853,7 +874,7 @@ __global__ __launch_bounds__(kThreads) void k_syrk_red(DevPtrs d, const SyrkItem
     __shared__ __attribute__((aligned(16))) unsigned char smem[RedLds<MODE>::bytes];
     const SyrkItem it = items[xcd_contiguous(blockIdx.x, gridDim.x)];
     if (d.prec == nullptr || d.prec[it.s] != MODE) return;
-    syrk_tile<MODE, kAhead>(d, it, smem);
+    syrk_tile<MODE, kAhead>(d, it, it.i0, it.j0, smem);
 }
 
 // all three reduced precisions in one kernel, for the learned selector's
@@ -868,19 +889,21 @@ __global__ __launch_bounds__(kThreads) void k_syrk_red_any(DevPtrs d, const Syrk
     __shared__ __attribute__((aligned(16))) unsigned char smem[RedMax<0>::bytes];
     const SyrkItem it = items[xcd_contiguous(blockIdx.x, gridDim.x)];
     const int pc = d.prec == nullptr ? 0 : d.prec[it.s];
-    if (pc == 1) syrk_tile<1, 1>(d, it, smem);
-    else if (pc == 2) syrk_tile<2, 1>(d, it, smem);
-    else if (pc == 3) syrk_tile<3, 1>(d, it, smem);
+    if (pc == 1) syrk_tile<1, 1>(d, it, it.i0, it.j0, smem);
+    else if (pc == 2) syrk_tile<2, 1>(d, it, it.i0, it.j0, smem);
+    else if (pc == 3) syrk_tile<3, 1>(d, it, it.i0, it.j0, smem);
 }
 
 // n items; the reduced kernels cover the last n_red of them (the items of
 // fronts that may run below FP64), one launch per precision code in
 // red_modes (bit c: code c), or one launch of the combined kernel when
 // several codes are possible
-void launch_syrk(hipStream_t st, const DevPtrs &d, const SyrkItem *it, int64_t n, int64_t n_red, int ahead,
-                 int red_modes) {
+void launch_syrk(hipStream_t st, const DevPtrs &d, const SyrkItem *it, int64_t n, int64_t n_red, int32_t depth,
+                 int ahead, int red_modes) {
     if (n <= 0) return;
-    for (int64_t o = 0; o < n; o += kMaxLaunchGroups) {
+    const bool small = n < (depth <= kSyrkSmallDepth ? kSyrkSmall : kSyrkSmallDeep);
+    if (small) k_syrk64_small<<<dim3(static_cast<unsigned>(4 * n)), kThreads, 0, st>>>(d, it);
+    for (int64_t o = 0; o < n && !small; o += kMaxLaunchGroups) {
         const dim3 grid(static_cast<unsigned>(std::min(kMaxLaunchGroups, n - o)));
         if (ahead == 1) k_syrk64<1><<<grid, kThreads, 0, st>>>(d, it + o);
         else k_syrk64<2><<<grid, kThreads, 0, st>>>(d, it + o);

@@ -62,14 +62,16 @@ __device__ __forceinline__ double buffer_load<double>(__amdgpu_buffer_rsrc_t r, 
 // LDS row length of a staged chunk: FP32 rows are padded by 16 floats so
 // that the four panel columns a wave reads at once (lanes 16 k .. 16 k + 15
 // take column k) fall on different banks; FP64 reads do not conflict.
-template <typename E>
-__host__ __device__ constexpr int tile_lds_ld() { return kT + (sizeof(E) == 4 ? 16 : 0); }
+template <typename E, int TILE = kT>
+__host__ __device__ constexpr int tile_lds_ld() { return TILE + (sizeof(E) == 4 ? 16 : 0); }
 // LDS bytes of the two stages of both operands
-template <typename E, int kKc>
-__host__ __device__ constexpr int tile_lds_bytes() { return 4 * kKc * tile_lds_ld<E>() * static_cast<int>(sizeof(E)); }
+template <typename E, int kKc, int TILE = kT>
+__host__ __device__ constexpr int tile_lds_bytes() { return 4 * kKc * tile_lds_ld<E, TILE>() * static_cast<int>(sizeof(E)); }
 
-// One 128 x 128 tile, operands of type E staged in a double-buffered LDS
-// ring. kAhead = 1: the global loads of chunk k+1 are in flight during the
+// One TILE x TILE tile (128, or 64 where a launch has too few of the larger
+// ones to fill the chip: a quarter of the serial work per workgroup), each of
+// the four waves a quarter of it in TILE / 32 x TILE / 32 MFMA blocks.
+// Operands of type E are staged in a double-buffered LDS ring. kAhead = 1: the global loads of chunk k+1 are in flight during the
 // MFMAs of chunk k; kAhead = 2: those of chunk k+2 (two register sets, the
 // loads get two MFMA phases to arrive). Loads are branch-free buffer loads
 // (out-of-range rows and columns read 0); waves
@@ -80,14 +82,15 @@ __host__ __device__ constexpr int tile_lds_bytes() { return 4 * kKc * tile_lds_l
 // valid, panel columns [t0, t1). GE is the operands' type in global memory:
 // GE = double with E = float rounds FP64 operands to FP32 as they are
 // written to LDS (FP32 MFMA on FP64 data).
-template <typename E, bool ACTIVE, int kKc, int kAhead, typename GE = E>
+template <typename E, bool ACTIVE, int kKc, int kAhead, typename GE = E, int TILE = kT>
 __device__ __forceinline__ void tile_loop(const GE *Ab, const GE *Bb, int ld, int boff, int i0, int j0, int f, int j1,
                                           int t0, int t1, unsigned char *smem,
-                                          typename SyrkMfma<E>::acc_t (&acc)[4][4]) {
+                                          typename SyrkMfma<E>::acc_t (&acc)[TILE / 32][TILE / 32]) {
     typedef SyrkMfma<E> M;
     constexpr int kThreads = kTileThreads;
-    constexpr int kLoadPer = (kKc * kT) / kThreads;  // elements of A (and of B) per thread per chunk
-    constexpr int kLd = tile_lds_ld<E>();
+    constexpr int kNB = TILE / 32;                     // MFMA blocks of a wave, each way
+    constexpr int kLoadPer = (kKc * TILE) / kThreads;  // elements of A (and of B) per thread per chunk
+    constexpr int kLd = tile_lds_ld<E, TILE>();
     E (*As)[kKc][kLd] = reinterpret_cast<E (*)[kKc][kLd]>(smem);                             // [2][kKc][kLd]
     E (*Bs)[kKc][kLd] = reinterpret_cast<E (*)[kKc][kLd]>(smem + 2 * kKc * kLd * sizeof(E));  // [2][kKc][kLd]
     const int tid = threadIdx.x;
@@ -100,9 +103,9 @@ __device__ __forceinline__ void tile_loop(const GE *Ab, const GE *Bb, int ld, in
     // t1, and rows past the front (A) or past j1 (B), whose offsets are
     // pushed past the descriptor's end, read 0 without a branch, a clamp or
     // a mask (the range check covers the lane offset).
-    constexpr int kPass = kThreads / kT;  // panel columns of one load instruction
+    constexpr int kPass = kThreads / TILE;  // panel columns of one load instruction
     constexpr uint32_t kOut = 0x80000000u;
-    const int rl = tid % kT, th = tid / kT;
+    const int rl = tid % TILE, th = tid / TILE;
     const uint32_t colb = static_cast<uint32_t>(ld) * static_cast<uint32_t>(sizeof(GE));
     const uint32_t voa = (i0 + rl < f) ? th * colb + static_cast<uint32_t>(i0 + rl) * sizeof(GE) : kOut;
     const uint32_t vob = (j0 + rl < j1) ? th * colb + static_cast<uint32_t>(j0 + rl) * sizeof(GE) : kOut;
@@ -132,16 +135,16 @@ __device__ __forceinline__ void tile_loop(const GE *Ab, const GE *Bb, int ld, in
         if (!ACTIVE) return;
 #pragma unroll
         for (int kk = 0; kk < kKc; kk += 4) {
-            E a[4], b[4];
+            E a[kNB], b[kNB];
             const int kr = kk + (lane >> 4);
 #pragma unroll
-            for (int m = 0; m < 4; ++m) a[m] = Bs[stg][kr][wc * 64 + m * 16 + (lane & 15)];
+            for (int m = 0; m < kNB; ++m) a[m] = Bs[stg][kr][wc * 16 * kNB + m * 16 + (lane & 15)];
 #pragma unroll
-            for (int nn = 0; nn < 4; ++nn) b[nn] = As[stg][kr][wr * 64 + nn * 16 + (lane & 15)];
+            for (int nn = 0; nn < kNB; ++nn) b[nn] = As[stg][kr][wr * 16 * kNB + nn * 16 + (lane & 15)];
 #pragma unroll
-            for (int m = 0; m < 4; ++m)
+            for (int m = 0; m < kNB; ++m)
 #pragma unroll
-                for (int nn = 0; nn < 4; ++nn) acc[m][nn] = M::mfma(a[m], b[nn], acc[m][nn]);
+                for (int nn = 0; nn < kNB; ++nn) acc[m][nn] = M::mfma(a[m], b[nn], acc[m][nn]);
         }
     };
     int stg = 0;

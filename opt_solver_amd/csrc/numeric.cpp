@@ -251,7 +251,9 @@ int dense_schedule(smfgpu_plan_s *P) {
         for (int32_t s : fl)
             if (P->fronts[s].f >= red_min) emit(s);
         const int64_t y1 = static_cast<int64_t>(syrk.size());
-        launches.push_back(Launch{K_SYRK, lv, y0, y1 - y0, y1 - yr});
+        int32_t depth = 0;
+        for (int64_t i = y0; i < y1; ++i) depth = std::max(depth, syrk[i].t1 - syrk[i].t0);
+        launches.push_back(Launch{K_SYRK, lv, y0, y1 - y0, y1 - yr, depth});
     };
     for (int32_t lv = 0; lv < nlev; ++lv) {
         const auto &fl = P->level_fronts[lv];
@@ -1038,7 +1040,8 @@ SMFGPU_API int smfgpu_factor(smfgpu_plan_t P, const double *values, int64_t nval
             case K_POTRF: launch_potrf(st, d, P->d_potrf.p + l.first, l.count); break;
             case K_TRSM: launch_trsm(st, d, P->d_trsm.p + l.first, l.count); break;
             case K_SYRK:
-                launch_syrk(st, d, P->d_syrk.p + l.first, l.count, gi ? l.red : 0, P->syrk_ahead, red_modes);
+                launch_syrk(st, d, P->d_syrk.p + l.first, l.count, gi ? l.red : 0, l.depth, P->syrk_ahead,
+                            red_modes);
                 break;
             case K_SELECT:
                 if (sel_on) launch_select(st, P->d_selfr.p + l.first, static_cast<int32_t>(l.count), P->d_colstat.p, sprm,

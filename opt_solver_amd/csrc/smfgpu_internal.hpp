@@ -99,6 +99,7 @@ struct Launch {
     int64_t first;  // first item in the kind's item array
     int64_t count;  // number of items (= workgroups)
     int64_t red;    // K_SYRK: the last `red` items belong to fronts that may run below FP64
+    int32_t depth = 0;  // K_SYRK: most panel columns of an item
 };
 
 // ---------------------------------------------------------------------
@@ -148,10 +149,11 @@ void launch_assemble(hipStream_t st, const DevPtrs &d, const AsmTask *tasks, int
                      int32_t fmax, int32_t chunk_cap, int32_t wave_rows);
 void launch_potrf(hipStream_t st, const DevPtrs &d, const PotrfItem *it, int64_t n);
 void launch_trsm(hipStream_t st, const DevPtrs &d, const TrsmItem *it, int64_t n);
-// n items; the reduced-precision kernels run the last n_red of them, one
-// launch per precision code in red_modes (bit c: code c)
-void launch_syrk(hipStream_t st, const DevPtrs &d, const SyrkItem *it, int64_t n, int64_t n_red, int ahead,
-                 int red_modes);
+// n items of at most depth panel columns; the reduced-precision kernels run
+// the last n_red of them, one launch per precision code in red_modes (bit c:
+// code c)
+void launch_syrk(hipStream_t st, const DevPtrs &d, const SyrkItem *it, int64_t n, int64_t n_red, int32_t depth,
+                 int ahead, int red_modes);
 void launch_zero_upper(hipStream_t st, const DevPtrs &d, const PotrfItem *it, int64_t n);
 
 // Solves: y is the permuted right-hand side block, n x nrhs (ld n).
