@@ -314,7 +314,7 @@ SMFGPU_API int smfgpu_solve(smfgpu_factor_t f, double *b, int32_t nrhs, int32_t 
  * fixed 64 MiB device array per GPU (resolved when a plan is created on that
  * device, held until the process ends) instead of a plan buffer allocated on
  * first use; right-hand sides pass through the sweeps in groups of at most
- * min(4 (Cholesky) / 16 (LDL^T), 2^23 / n) columns. Plans with n > 2^23
+ * min(16, 2^23 / n) columns. Plans with n > 2^23
  * rows are refused with SMFGPU_ERR_INVALID_ARG. Every call on one GPU
  * shares that array: calls that overlap on one GPU (from several threads or
  * plans) race. Returns after the solve has finished. */

@@ -27,32 +27,91 @@ namespace {
 constexpr int kSB = 128;        // pivot columns per step
 constexpr int kSD = 64;         // diagonal block (stored inverse)
 constexpr int kSThreads = 512;  // eight waves
-constexpr int kSeg = 512;       // rows per backward update item
 
-struct TriRegs {
-    double a[8], b[8], c[8];  // Dg_a, L_ba, Dg_b of the triangle, element (rl, g + 8 e)
+typedef double v4d __attribute__((ext_vector_type(4)));
+typedef double v2du __attribute__((ext_vector_type(2), aligned(8)));  // two rows of a column (8-byte aligned)
+
+// a of the lane's half plus b of the other's: lanes of the first half (ROW 32:
+// of the wavefront, 16: of each pair of rows of 16 lanes) get a + a of their
+// partner lane, the others b + b of theirs
+template <int ROW>
+__device__ __forceinline__ double swap_add(double a, double b) {
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    const unsigned al = __double2loint(a), ah = __double2hiint(a), bl = __double2loint(b), bh = __double2hiint(b);
+    u2 l, h;
+    if constexpr (ROW == 32) {
+        l = __builtin_amdgcn_permlane32_swap(al, bl, false, false);
+        h = __builtin_amdgcn_permlane32_swap(ah, bh, false, false);
+    } else {
+        l = __builtin_amdgcn_permlane16_swap(al, bl, false, false);
+        h = __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
+    }
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+
+// Products of 16 rows or columns of L (lane lr = lane % 16) with the
+// right-hand sides, the sum's index split over the four rows of lanes lk =
+// lane / 16. More than four right-hand sides: FP64 MFMA 16x16x4, the
+// right-hand sides as the 16 rows of the result (A operand: lane lr holds
+// right-hand side lr, lanes past NR zeros); one takes 64 entries of L for up
+// to 16 of them in 64 cycles, 19 TB/s over the chip, so a sweep stays bound by
+// reading L, once for all 16. Up to four: FMAs (an item's 512 MFMAs are 3.4
+// us of its CU, the FMAs of one right-hand side 0.3) and a sum over lk.
+template <int NR>
+struct Acc {
+    double a[NR];
+    __device__ __forceinline__ Acc() {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) a[r] = 0.0;
+    }
+    __device__ __forceinline__ void add(const double (*v)[NR], int t, double l) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) a[r] += v[t][r] * l;
+    }
+    __device__ __forceinline__ void put(double (*part)[NR], int col) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            const double s = swap_add<32>(a[r], a[r]);
+            const double q = swap_add<16>(s, s);
+            if ((threadIdx.x & 48) == 0) part[col][r] = q;
+        }
+    }
+};
+template <>
+struct Acc<16> {
+    v4d a = {0.0, 0.0, 0.0, 0.0};
+    __device__ __forceinline__ void add(const double (*v)[16], int t, double l) {
+        a = __builtin_amdgcn_mfma_f64_16x16x4f64(v[t][threadIdx.x & 15], l, a, 0, 0, 0);
+    }
+    // accumulator: right-hand side 4 v + lk, column lr
+    __device__ __forceinline__ void put(double (*part)[16], int col) {
+        const int lk = (threadIdx.x & 63) >> 4;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) part[col][4 * v + lk] = a[v];
+    }
 };
 
-// Element (t = rl, c = g + 8 e) of the triangle's three 64 x 64 blocks:
-// a: upper part of the first diagonal block (t <= c: inverse rows and the
-// diagonal), b: rows 64.. of the block below it, c: second diagonal block.
+// The triangle's three 64 x 64 blocks, element (t = rl, c = g + 8 e): BLK 0:
+// upper part of the first diagonal block (t <= c: inverse rows and the
+// diagonal), 1: rows 64.. of the block below it, 2: second diagonal block.
+// The first one needed is read before the item's update, the others after it
+// (their 32 registers would leave one workgroup per CU).
 // Guarded loads are unconditional loads from clamped (in-front) addresses
 // times a 0 / 1 mask: a select around a load lets the compiler move the
 // load into a branch that waits for every load in flight.
 __device__ __forceinline__ double masked(double v, bool keep) { return v * (keep ? 1.0 : 0.0); }
 
-__device__ __forceinline__ void tri_prefetch(TriRegs &R, const double *Lb, int f, int tk, int tkb, int rl, int g) {
+template <int BLK>
+__device__ __forceinline__ void tri_load(double (&R)[8], const double *Lb, int f, int tk, int tkb, int rl, int g) {
     const int na = min(kSD, tkb), nb = tkb - kSD;
-    const int ra = tk + min(rl, na - 1);                     // rows of block a
-    const int rb = nb > 0 ? tk + kSD + min(rl, nb - 1) : ra;  // rows of block b (a's when there is none)
+    const int nr = BLK == 0 ? na : max(nb, 1), nc = BLK == 2 ? max(nb, 1) : na;
+    const int row = tk + min((BLK > 0 && nb > 0 ? kSD : 0) + min(rl, nr - 1), tkb - 1);
+    const int col = tk + (BLK == 2 && nb > 0 ? kSD : 0);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         const int c = g + 8 * e;
-        const int ca = tk + min(c, na - 1);
-        const int cb = nb > 0 ? tk + kSD + min(c, nb - 1) : ca;
-        R.a[e] = masked(Lb[static_cast<int64_t>(ca) * f + ra], rl <= c && c < na);
-        R.b[e] = masked(Lb[static_cast<int64_t>(ca) * f + rb], rl < nb && c < na);
-        R.c[e] = masked(Lb[static_cast<int64_t>(cb) * f + rb], rl <= c && c < nb);
+        R[e] = masked(Lb[static_cast<int64_t>(col + min(c, nc - 1)) * f + row],
+                      BLK == 1 ? rl < nb && c < na : rl <= c && c < (BLK == 0 ? na : nb));
     }
 }
 
@@ -61,70 +120,89 @@ __device__ __forceinline__ void put_block(double (*Dg)[kSD + 1], const double (&
     for (int e = 0; e < 8; ++e) Dg[rl][g + 8 * e] = v[e];
 }
 
-// z[c] = y[c] / L_cc + sum_{t<c} M[t][c] y[t]  (M[t][c] = inv(L)[c][t])
-template <int NR>
-__device__ __forceinline__ void tri_fwd(const double (*Dg)[kSD + 1], const double (*yb)[NR], double (*z)[NR], int nb,
-                                        int nrhs) {
-    const int c = threadIdx.x & 63, r = threadIdx.x >> 6;
-    if (r < NR && r < nrhs && c < nb) {
-        double s = yb[c][r] / Dg[c][c];
-        for (int t = 0; t < c; ++t) s += Dg[t][c] * yb[t][r];
-        z[c][r] = s;
+// 1 / d: the hardware estimate (better than 2^-20), a third-order step and
+// one Newton step for the last bit
+__device__ __forceinline__ double recip(double d) {
+    double y = __builtin_amdgcn_rcp(d);
+    double e = fma(-d, y, 1.0);
+    y = fma(y, fma(e, e, e), y);
+    e = fma(-d, y, 1.0);
+    return fma(y, e, y);
+}
+
+// a diagonal block: the inverse's transpose, its diagonal 1 / L_cc (columns
+// past n zero)
+__device__ __forceinline__ void put_diag(double (*Dg)[kSD + 1], const double (&v)[8], int rl, int g, int n) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int c = g + 8 * e;
+        Dg[rl][c] = (rl == c && c < n) ? recip(v[e]) : v[e];
     }
 }
 
-// x[c] = v[c] / L_cc + sum_{t>c} M[c][t] v[t]
-template <int NR>
-__device__ __forceinline__ void tri_bwd(const double (*Dg)[kSD + 1], const double (*v)[NR], double (*x)[NR], int nb,
-                                        int nrhs) {
-    const int c = threadIdx.x & 63, r = threadIdx.x >> 6;
-    if (r < NR && r < nrhs && c < nb) {
-        double s = v[c][r] / Dg[c][c];
-        for (int t = c + 1; t < nb; ++t) s += Dg[c][t] * v[t][r];
-        x[c][r] = s;
+// part[h][i][r] = sum over half h of k of D(i, k) v[k][r], D(i, k) =
+// TR ? Dg[k][i] : Dg[i][k], 64 x 64; wave w: 16 of i (w % 4), half w / 4
+template <int NR, bool TR>
+__device__ __forceinline__ void block_times(const double (*Dg)[kSD + 1], const double (*v)[NR],
+                                            double (*part)[kSD][NR]) {
+    const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4, w = threadIdx.x >> 6;
+    const int i = 16 * (w & 3) + lr, h = w >> 2;
+    Acc<NR> acc;
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) {
+        const int k = 32 * h + 4 * kk + lk;
+        acc.add(v, k, TR ? Dg[k][i] : Dg[i][k]);
     }
+    acc.put(part[h], i);
 }
 
-// Forward update of rows [lo, hi): y[row] -= sum_{t < kb} L[row][k + t] zs[t].
-// Rows in the triangle [tk, tk + tkb) go to yb (LDS), other own pivot rows
-// in place, ancestor rows by atomic add.
-template <int NR>
+// Forward update of rows [lo, hi): y[row] -= sum_{t < kb} L[row][k + t] zs[t]
+// (zs zero past kb). Rows in the triangle [tk, tk + tkb) go to yb (LDS),
+// other own pivot rows in place, ancestor rows by atomic add. ROWS rows at a
+// time: a lane takes two rows (16-byte loads), the waves 32 rows each and
+// shares of the kSB columns.
+template <int NR, int ROWS>
 __device__ void fwd_update(const double *Lb, const int32_t *frows, int f, int p, int col0, int k, int kb, int lo,
-                           int hi, const double (*zs)[NR], double (*part)[64][NR], double (*yb)[NR], int tk, int tkb,
+                           int hi, const double (*zs)[NR], double (*part)[kSD][NR], double (*yb)[NR], int tk, int tkb,
                            double *y, int n, int nrhs) {
-    const int tid = threadIdx.x, rl = tid & 63, g = tid >> 6;
-    for (int r0 = lo; r0 < hi; r0 += 64) {
-        const int row = r0 + rl;
-        const int rowc = min(row, hi - 1);
-        double acc[NR];
+    constexpr int kTiles = ROWS / 32, kSplit = 8 / kTiles, kCols = kSB / kSplit;
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lk = lane >> 4, w = tid >> 6;
+    const int pt = w % kTiles, c0 = w / kTiles * kCols;
+    double (*pp)[NR] = reinterpret_cast<double (*)[NR]>(part);  // kSplit x ROWS
+    for (int r0 = lo; r0 < hi; r0 += ROWS) {
+        const int row = r0 + 32 * pt + 2 * lr;
+        const double *Lr = Lb + static_cast<int64_t>(k) * f + min(row, f - 2);
+        Acc<NR> acc0, acc1;
+        v2du l[kCols / 4];
 #pragma unroll
-        for (int r = 0; r < NR; ++r) acc[r] = 0.0;
-        double l[16];
-#pragma unroll
-        for (int tt = 0; tt < 16; ++tt)
-            l[tt] = Lb[static_cast<int64_t>(k + min(g * 16 + tt, kb - 1)) * f + rowc];
-#pragma unroll
-        for (int tt = 0; tt < 16; ++tt) {
-            const double lv = masked(l[tt], row < hi && g * 16 + tt < kb);
-#pragma unroll
-            for (int r = 0; r < NR; ++r) acc[r] += lv * zs[g * 16 + tt][r];
+        for (int kk = 0; kk < kCols / 4; ++kk) {
+            if (c0 + 4 * kk >= kb) break;
+            l[kk] = *reinterpret_cast<const v2du *>(Lr + static_cast<int64_t>(min(c0 + 4 * kk + lk, kb - 1)) * f);
         }
 #pragma unroll
-        for (int r = 0; r < NR; ++r) part[g][rl][r] = acc[r];
+        for (int kk = 0; kk < kCols / 4; ++kk) {
+            if (c0 + 4 * kk >= kb) break;
+            const double l0 = row > f - 2 ? l[kk][1] : l[kk][0];  // the front's last row alone
+            acc0.add(zs, c0 + 4 * kk + lk, l0);
+            acc1.add(zs, c0 + 4 * kk + lk, l[kk][1]);
+        }
+        double (*q)[NR] = pp + w / kTiles * ROWS + 32 * pt;
+        acc0.put(q, 2 * lr);
+        acc1.put(q, 2 * lr + 1);
         __syncthreads();
-        if (tid < 64 * NR) {
-            const int rr = tid & 63, r = tid >> 6;
+        for (int e = tid; e < ROWS * NR; e += kSThreads) {
+            const int rr = e % ROWS, r = e / ROWS;
             const int i = r0 + rr;
             if (i < hi && r < nrhs) {
-                double s = 0.0;
+                double sum = 0.0;
 #pragma unroll
-                for (int g2 = 0; g2 < 8; ++g2) s += part[g2][rr][r];
+                for (int g = 0; g < kSplit; ++g) sum += pp[g * ROWS + rr][r];
                 if (i >= tk && i < tk + tkb) {
-                    yb[i - tk][r] = y[col0 + i + static_cast<int64_t>(r) * n] - s;
+                    yb[i - tk][r] = y[col0 + i + static_cast<int64_t>(r) * n] - sum;
                 } else if (i < p) {
-                    y[col0 + i + static_cast<int64_t>(r) * n] -= s;
+                    y[col0 + i + static_cast<int64_t>(r) * n] -= sum;
                 } else {
-                    unsafeAtomicAdd(&y[static_cast<int64_t>(frows[i]) + static_cast<int64_t>(r) * n], -s);
+                    unsafeAtomicAdd(&y[static_cast<int64_t>(frows[i]) + static_cast<int64_t>(r) * n], -sum);
                 }
             }
         }
@@ -134,12 +212,25 @@ __device__ void fwd_update(const double *Lb, const int32_t *frows, int f, int p,
 
 template <int NR>
 struct FwdLds {
-    static_assert(NR * 64 <= kSThreads, "one wave per right-hand side in the triangles");
     double Dg[kSD][kSD + 1];
     double zs[kSB][NR];
     double yb[kSB][NR];
-    double part[8][64][NR];
+    double part[4][kSD][NR];  // partial sums: 4 x 64 or 2 x 128 rows, 2 x 64 in the triangles
 };
+
+// out[i][r] = base[i][r] - (or without base: =) part[0] + part[1], i < n
+template <int NR, bool SUB>
+__device__ __forceinline__ void add_halves(double (*out)[NR], const double (*part)[kSD][NR], int n) {
+    for (int e = threadIdx.x; e < kSD * NR; e += kSThreads) {
+        const int i = e / NR, r = e % NR;
+        const double v = part[0][i][r] + part[1][i][r];
+        if (SUB) {
+            if (i < n) out[i][r] -= v;
+        } else {
+            out[i][r] = i < n ? v : 0.0;
+        }
+    }
+}
 
 template <int NR>
 __device__ void fwd_item(const DevPtrs &d, const SolveItem &it, double *__restrict__ y, int32_t n, int32_t nrhs,
@@ -153,139 +244,142 @@ __device__ void fwd_item(const DevPtrs &d, const SolveItem &it, double *__restri
     const double *Lb = d.L + F.lofs;
     const int32_t *frows = d.rows + F.rofs;
     const int tid = threadIdx.x, rl = tid & 63, g = tid >> 6;
-    TriRegs R;
-    if (it.tkb > 0) tri_prefetch(R, Lb, f, it.tk, it.tkb, rl, g);
+    double Ra[8], Rb[8], Rc[8];
+    if (it.tkb > 0) tri_load<0>(Ra, Lb, f, it.tk, it.tkb, rl, g);
     for (int idx = tid; idx < kSB * NR; idx += kSThreads) {
         const int t = idx % kSB, r = idx / kSB;
         zs[t][r] = (t < it.kb && r < nrhs) ? y[F.col0 + it.k + t + static_cast<int64_t>(r) * n] : 0.0;
-        if (it.tkb > 0 && it.kb == 0) yb[t][r] = (t < it.tkb && r < nrhs) ? y[F.col0 + it.tk + t + static_cast<int64_t>(r) * n] : 0.0;
+        if (it.tkb > 0) yb[t][r] = (it.kb == 0 && t < it.tkb && r < nrhs) ? y[F.col0 + it.tk + t + static_cast<int64_t>(r) * n] : 0.0;
     }
     __syncthreads();
     if (it.kb > 0)
-        fwd_update<NR>(Lb, frows, f, p, F.col0, it.k, it.kb, it.a0, it.a1, zs, part, yb, it.tk, it.tkb, y, n, nrhs);
+        fwd_update<NR, 64>(Lb, frows, f, p, F.col0, it.k, it.kb, it.a0, it.a1, zs, part, yb, it.tk, it.tkb, y, n, nrhs);
     if (it.tkb <= 0) return;
     // the triangle: z_a = inv(L_a) y_a; y_b -= L_ba z_a; z_b = inv(L_b) y_b
     const int na = min(kSD, it.tkb), nb = it.tkb - kSD;
-    put_block(Dg, R.a, rl, g);
+    if (nb > 0) {
+        tri_load<1>(Rb, Lb, f, it.tk, it.tkb, rl, g);
+        tri_load<2>(Rc, Lb, f, it.tk, it.tkb, rl, g);
+    }
+    put_diag(Dg, Ra, rl, g, na);
     __syncthreads();
-    tri_fwd<NR>(Dg, yb, zs, na, nrhs);
+    block_times<NR, true>(Dg, yb, part);
+    __syncthreads();
+    add_halves<NR, false>(zs, part, na);
+    if (nb > 0) put_block(Dg, Rb, rl, g);
     __syncthreads();
     if (nb > 0) {
-        double acc[NR];
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-            acc[r] = 0.0;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) acc[r] += R.b[e] * zs[g + 8 * e][r];
-            part[g][rl][r] = acc[r];
-        }
-        put_block(Dg, R.c, rl, g);
+        block_times<NR, false>(Dg, zs, part);
         __syncthreads();
-        if (tid < 64 * NR) {
-            const int rr = tid & 63, r = tid >> 6;
-            if (rr < nb && r < nrhs) {
-                double s = 0.0;
-#pragma unroll
-                for (int g2 = 0; g2 < 8; ++g2) s += part[g2][rr][r];
-                yb[kSD + rr][r] -= s;
-            }
-        }
+        add_halves<NR, true>(yb + kSD, part, nb);
+        put_diag(Dg, Rc, rl, g, nb);
         __syncthreads();
-        tri_fwd<NR>(Dg, yb + kSD, zs + kSD, nb, nrhs);
+        block_times<NR, true>(Dg, yb + kSD, part);
+        __syncthreads();
+        add_halves<NR, false>(zs + kSD, part, nb);
+        __syncthreads();
+    } else if (it.kb > 0) {
+        // zs past the block still holds the block before
+        for (int e = tid; e < kSD * NR; e += kSThreads) zs[kSD + e / NR][e % NR] = 0.0;
         __syncthreads();
     }
-    // zs now holds z of the whole block (entries past tkb are still zero)
+    // zs now holds z of the whole block, zeros past tkb
     for (int idx = tid; idx < it.tkb * nrhs; idx += kSThreads) {
         const int t = idx % it.tkb, r = idx / it.tkb;
         y[F.col0 + it.tk + t + static_cast<int64_t>(r) * n] = zs[t][r];
     }
     if (it.flags & 2)  // the rows below the last block, by this workgroup
-        fwd_update<NR>(Lb, frows, f, p, F.col0, it.tk, it.tkb, it.tk + it.tkb, f, zs, part, yb, -1, 0, y, n, nrhs);
+        fwd_update<NR, 128>(Lb, frows, f, p, F.col0, it.tk, it.tkb, it.tk + it.tkb, f, zs, part, yb, -1, 0, y, n, nrhs);
 }
 
 template <int NR>
-__global__ __launch_bounds__(kSThreads) void k_fwd_step(DevPtrs d, const SolveItem *__restrict__ items,
+__global__ __launch_bounds__(kSThreads, NR == 1 ? 4 : 1) void k_fwd_step(DevPtrs d, const SolveItem *__restrict__ items,
                                                        double *__restrict__ y, int32_t n, int32_t nrhs) {
     __shared__ FwdLds<NR> S;
     fwd_item<NR>(d, items[blockIdx.x], y, n, nrhs, S);
 }
 
+template <int NR>
+constexpr int kXs = NR > 4 ? 256 : kSolveSeg;  // rows of x a backward update stages at a time
+
 // Backward update of columns [c0, c1): y[col0 + c] -= sum_{i in [r0, r1)}
-// L[i][c] x_i, x_i = y[col0 + i] for own pivot rows, y[rows[i]] else.
-// Lanes: 16 rows x 4 columns; wave g owns columns 8 g + {cq, cq + 4} of
-// each 64-column tile. Columns of the triangle go to v (LDS).
+// L[i][c] x_i, x_i = y[col0 + i] for own pivot rows, y[rows[i]] else. 64
+// columns at a time: wave w takes 16 of them (w % 4) and half of the rows; a
+// lane takes 4 consecutive rows of its column (two 16-byte loads, whole cache
+// lines across the lanes), 64 rows of loads in flight and the next 64 behind
+// them. Columns of the triangle go to v (LDS).
 template <int NR>
 __device__ void bwd_update(const double *Lb, const int32_t *frows, int f, int p, int col0, int r0, int r1, int c0,
-                           int c1, bool atomic, double (*xs)[NR], double (*v)[NR], int tk, int tkb,
-                           double *y, int n, int nrhs) {
+                           int c1, bool atomic, double (*xs)[NR], double (*part)[kSD][NR], double (*v)[NR], int tk,
+                           int tkb, double *y, int n, int nrhs) {
+    constexpr int kX = kXs<NR>, kU = 4;
     const int tid = threadIdx.x;
-    const int lane = tid & 63, g = tid >> 6, rq = lane & 15, cq = lane >> 4;
+    const int lane = tid & 63, lr = lane & 15, lk = lane >> 4, w = tid >> 6, h = w >> 2;
     const int nr = r1 - r0;
-    for (int idx = tid; idx < kSeg * NR; idx += kSThreads) {
-        const int i = idx % kSeg, r = idx / kSeg;
-        double xv = 0.0;
-        if (i < nr && r < nrhs) {
-            const int row = r0 + i;
-            const int64_t gi = row < p ? static_cast<int64_t>(col0 + row) : static_cast<int64_t>(frows[row]);
-            xv = y[gi + static_cast<int64_t>(r) * n];
-        }
-        xs[i][r] = xv;
-    }
-    __syncthreads();
     for (int cb = c0; cb < c1; cb += 64) {
-        const int ca = cb + 8 * g + cq, cbb = ca + 4;
-        const bool va = ca < c1, vb = cbb < c1;
-        const double *La = Lb + static_cast<int64_t>(va ? ca : c0) * f + r0;
-        const double *Lbb = Lb + static_cast<int64_t>(vb ? cbb : c0) * f + r0;
-        double acc0[NR], acc1[NR];
+        const int c = min(cb + 16 * (w & 3) + lr, c1 - 1);
+        const double *Lc = Lb + static_cast<int64_t>(c) * f + r0;
+        Acc<NR> acc;
+        for (int s0 = 0; s0 < nr; s0 += kX) {
+            const int ns = min(kX, nr - s0);
+            const int half = (ns + 31) / 32 * 16;  // rows of a wave, a multiple of 16
+            const int g0 = s0 + h * half, ge = min(s0 + ns, g0 + half);
+            v2du l[2][kU][2];
+            const auto load = [&](v2du (&q)[kU][2], int g) {
 #pragma unroll
-        for (int r = 0; r < NR; ++r) acc0[r] = acc1[r] = 0.0;
-        for (int i0 = 0; i0 < nr; i0 += 128) {
-            double la[8], lb[8];
+                for (int u = 0; u < kU; ++u) {
+                    const int i = g + 16 * u + 4 * lk;
+                    if (g + 16 * u >= ge) break;
+                    if (g + 16 * u + 16 <= nr) {
+                        q[u][0] = *reinterpret_cast<const v2du *>(Lc + i);
+                        q[u][1] = *reinterpret_cast<const v2du *>(Lc + i + 2);
+                    } else {
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int i = min(i0 + 16 * u + rq, nr - 1);
-                la[u] = La[i];
-                lb[u] = Lbb[i];
-            }
+                        for (int j = 0; j < 4; ++j) q[u][j >> 1][j & 1] = Lc[min(i + j, nr - 1)];
+                    }
+                }
+            };
+            const auto mul = [&](const v2du (&q)[kU][2], int g) {
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const bool in = i0 + 16 * u + rq < nr;
-                la[u] = masked(la[u], va && in);
-                lb[u] = masked(lb[u], vb && in);
-            }
+                for (int u = 0; u < kU; ++u) {
+                    if (g + 16 * u >= ge) break;
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int i = min(i0 + 16 * u + rq, kSeg - 1);
-#pragma unroll
-                for (int r = 0; r < NR; ++r) {
-                    acc0[r] += la[u] * xs[i][r];
-                    acc1[r] += lb[u] * xs[i][r];
+                    for (int j = 0; j < 4; ++j) acc.add(xs, g - s0 + 16 * u + 4 * lk + j, q[u][j >> 1][j & 1]);
+                }
+            };
+            load(l[0], g0);
+            if (cb > c0 || s0 > 0) __syncthreads();
+            if (cb == c0 || nr > kX) {
+                for (int idx = tid; idx < kX * NR; idx += kSThreads) {
+                    const int i = idx % kX, r = idx / kX;
+                    double xv = 0.0;
+                    if (i < ns && r < nrhs) {
+                        const int row = r0 + s0 + i;
+                        const int64_t gi = row < p ? static_cast<int64_t>(col0 + row) : static_cast<int64_t>(frows[row]);
+                        xv = y[gi + static_cast<int64_t>(r) * n];
+                    }
+                    xs[i][r] = xv;
                 }
             }
-        }
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-#pragma unroll
-            for (int o = 8; o >= 1; o >>= 1) {
-                acc0[r] += __shfl_xor(acc0[r], o);
-                acc1[r] += __shfl_xor(acc1[r], o);
+            __syncthreads();
+            for (int g = g0; g < ge; g += 32 * kU) {
+                load(l[1], g + 16 * kU);
+                mul(l[0], g);
+                if (g + 16 * kU >= ge) break;
+                load(l[0], g + 32 * kU);
+                mul(l[1], g + 16 * kU);
             }
         }
-        if (rq == 0) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int c = h ? cbb : ca;
-                if (!(h ? vb : va)) continue;
-#pragma unroll
-                for (int r = 0; r < NR; ++r) {
-                    if (r >= nrhs) break;
-                    const double s = h ? acc1[r] : acc0[r];
-                    double *dst = &y[col0 + c + static_cast<int64_t>(r) * n];
-                    if (c >= tk && c < tk + tkb) v[c - tk][r] = *dst - s;
-                    else if (atomic) unsafeAtomicAdd(dst, -s);
-                    else *dst -= s;
-                }
+        acc.put(part[h], 16 * (w & 3) + lr);
+        __syncthreads();
+        for (int e = tid; e < kSD * NR; e += kSThreads) {
+            const int cc = cb + e % kSD, r = e / kSD;
+            if (cc < c1 && r < nrhs) {
+                const double s = part[0][e % kSD][r] + part[1][e % kSD][r];
+                double *dst = &y[col0 + cc + static_cast<int64_t>(r) * n];
+                if (cc >= tk && cc < tk + tkb) v[cc - tk][r] = *dst - s;
+                else if (atomic) unsafeAtomicAdd(dst, -s);
+                else *dst -= s;
             }
         }
     }
@@ -295,9 +389,10 @@ __device__ void bwd_update(const double *Lb, const int32_t *frows, int f, int p,
 template <int NR>
 struct BwdLds {
     double Dg[kSD][kSD + 1];
-    double xs[kSeg][NR];
+    double xs[kXs<NR>][NR];
     double v[kSB][NR];
     double xo[kSB][NR];
+    double part[2][kSD][NR];
 };
 
 template <int NR>
@@ -307,47 +402,48 @@ __device__ void bwd_item(const DevPtrs &d, const SolveItem &it, double *__restri
     auto &xs = S.xs;
     auto &v = S.v;
     auto &xo = S.xo;
+    auto &part = S.part;
     const FrontDev F = d.fronts[it.s];
     const int f = F.f, p = F.p;
     const double *Lb = d.L + F.lofs;
     const int32_t *frows = d.rows + F.rofs;
     const int tid = threadIdx.x, rl = tid & 63, g = tid >> 6;
-    TriRegs R;
-    if (it.tkb > 0) {
-        tri_prefetch(R, Lb, f, it.tk, it.tkb, rl, g);
-        if (it.kb == 0)
-            for (int idx = tid; idx < kSB * NR; idx += kSThreads) {
-                const int t = idx % kSB, r = idx / kSB;
-                v[t][r] = (t < it.tkb && r < nrhs) ? y[F.col0 + it.tk + t + static_cast<int64_t>(r) * n] : 0.0;
-            }
-    }
-    if (it.kb > 0)
-        bwd_update<NR>(Lb, frows, f, p, F.col0, it.k, it.k + it.kb, it.a0, it.a1, (it.flags & 1) != 0, xs, v, it.tk,
-                       it.tkb, y, n, nrhs);
-    if (it.tkb <= 0) return;
-    // the triangle, second diagonal block first:
-    // x_b = inv(L_b)^T v_b; v_a -= L_ba^T x_b; x_a = inv(L_a)^T v_a
+    double Ra[8], Rb[8], Rc[8];
     const int na = min(kSD, it.tkb), nb = it.tkb - kSD;
-    if (nb > 0) {
-        put_block(Dg, R.c, rl, g);
-        __syncthreads();
-        tri_bwd<NR>(Dg, v + kSD, xo + kSD, nb, nrhs);
-        __syncthreads();
-        put_block(Dg, R.b, rl, g);  // Dg[t][c] = L_ba[t][c]
-        __syncthreads();
-        {
-            const int c = tid & 63, r = tid >> 6;
-            if (r < NR && r < nrhs && c < na) {
-                double s = 0.0;
-                for (int t = 0; t < nb; ++t) s += Dg[t][c] * xo[kSD + t][r];
-                v[c][r] -= s;
-            }
+    if (it.tkb > 0) {
+        if (nb > 0) tri_load<2>(Rc, Lb, f, it.tk, it.tkb, rl, g);
+        else tri_load<0>(Ra, Lb, f, it.tk, it.tkb, rl, g);
+        for (int idx = tid; idx < kSB * NR; idx += kSThreads) {
+            const int t = idx % kSB, r = idx / kSB;
+            v[t][r] = (it.kb == 0 && t < it.tkb && r < nrhs) ? y[F.col0 + it.tk + t + static_cast<int64_t>(r) * n] : 0.0;
         }
         __syncthreads();
     }
-    put_block(Dg, R.a, rl, g);
+    if (it.kb > 0)
+        bwd_update<NR>(Lb, frows, f, p, F.col0, it.k, it.k + it.kb, it.a0, it.a1, (it.flags & 1) != 0, xs, part, v,
+                       it.tk, it.tkb, y, n, nrhs);
+    if (it.tkb <= 0) return;
+    // the triangle, second diagonal block first:
+    // x_b = inv(L_b)^T v_b; v_a -= L_ba^T x_b; x_a = inv(L_a)^T v_a
+    if (nb > 0) {
+        tri_load<1>(Rb, Lb, f, it.tk, it.tkb, rl, g);
+        tri_load<0>(Ra, Lb, f, it.tk, it.tkb, rl, g);
+        put_diag(Dg, Rc, rl, g, nb);
+        __syncthreads();
+        block_times<NR, false>(Dg, v + kSD, part);
+        __syncthreads();
+        add_halves<NR, false>(xo + kSD, part, nb);
+        put_block(Dg, Rb, rl, g);  // Dg[t][c] = L_ba[t][c]
+        __syncthreads();
+        block_times<NR, true>(Dg, xo + kSD, part);
+        __syncthreads();
+        add_halves<NR, true>(v, part, na);
+    }
+    put_diag(Dg, Ra, rl, g, na);
     __syncthreads();
-    tri_bwd<NR>(Dg, v, xo, na, nrhs);
+    block_times<NR, false>(Dg, v, part);
+    __syncthreads();
+    add_halves<NR, false>(xo, part, na);
     __syncthreads();
     for (int idx = tid; idx < it.tkb * nrhs; idx += kSThreads) {
         const int t = idx % it.tkb, r = idx / it.tkb;
@@ -356,7 +452,7 @@ __device__ void bwd_item(const DevPtrs &d, const SolveItem &it, double *__restri
 }
 
 template <int NR>
-__global__ __launch_bounds__(kSThreads) void k_bwd_step(DevPtrs d, const SolveItem *__restrict__ items,
+__global__ __launch_bounds__(kSThreads, NR == 1 ? 4 : 1) void k_bwd_step(DevPtrs d, const SolveItem *__restrict__ items,
                                                        double *__restrict__ y, int32_t n, int32_t nrhs) {
     __shared__ BwdLds<NR> S;
     bwd_item<NR>(d, items[blockIdx.x], y, n, nrhs, S);
@@ -447,20 +543,6 @@ __device__ __forceinline__ double lane_value(double v, int l) {
 // halves of the wavefront (v_permlane32_swap: {a.lo, b.lo}, {a.hi, b.hi}),
 // 16: rows of 16 lanes, 8 and 4: inside a row (rotation by 8, mirror of 8
 // lanes); the lanes that share e are then added.
-template <int ROW>
-__device__ __forceinline__ double swap_add(double a, double b) {
-    typedef unsigned u2 __attribute__((ext_vector_type(2)));
-    const unsigned al = __double2loint(a), ah = __double2hiint(a), bl = __double2loint(b), bh = __double2hiint(b);
-    u2 l, h;
-    if constexpr (ROW == 32) {
-        l = __builtin_amdgcn_permlane32_swap(al, bl, false, false);
-        h = __builtin_amdgcn_permlane32_swap(ah, bh, false, false);
-    } else {
-        l = __builtin_amdgcn_permlane16_swap(al, bl, false, false);
-        h = __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
-    }
-    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
-}
 template <int CTRL>
 __device__ __forceinline__ double dpp_move(double v) {
     return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, false),
@@ -916,11 +998,11 @@ void launch_sweep(hipStream_t st, const DevPtrs &d, bool forward, const SolveIte
     if (forward) {
         if (nrhs == 1) k_sweep<1, true><<<grid, kSThreads, 0, st>>>(d, items, step_of, step_cnt, ctr, err, y, n, nrhs);
         else if (nrhs <= 4) k_sweep<4, true><<<grid, kSThreads, 0, st>>>(d, items, step_of, step_cnt, ctr, err, y, n, nrhs);
-        else k_sweep<8, true><<<grid, kSThreads, 0, st>>>(d, items, step_of, step_cnt, ctr, err, y, n, nrhs);
+        else k_sweep<16, true><<<grid, kSThreads, 0, st>>>(d, items, step_of, step_cnt, ctr, err, y, n, nrhs);
     } else {
         if (nrhs == 1) k_sweep<1, false><<<grid, kSThreads, 0, st>>>(d, items, step_of, step_cnt, ctr, err, y, n, nrhs);
         else if (nrhs <= 4) k_sweep<4, false><<<grid, kSThreads, 0, st>>>(d, items, step_of, step_cnt, ctr, err, y, n, nrhs);
-        else k_sweep<8, false><<<grid, kSThreads, 0, st>>>(d, items, step_of, step_cnt, ctr, err, y, n, nrhs);
+        else k_sweep<16, false><<<grid, kSThreads, 0, st>>>(d, items, step_of, step_cnt, ctr, err, y, n, nrhs);
     }
 }
 
@@ -930,7 +1012,7 @@ void launch_fwd_step(hipStream_t st, const DevPtrs &d, const SolveItem *items, i
         const dim3 grid(static_cast<unsigned>(std::min(kMaxLaunchGroups, count - o)));
         if (nrhs == 1) k_fwd_step<1><<<grid, kSThreads, 0, st>>>(d, items + o, y, n, nrhs);
         else if (nrhs <= 4) k_fwd_step<4><<<grid, kSThreads, 0, st>>>(d, items + o, y, n, nrhs);
-        else k_fwd_step<8><<<grid, kSThreads, 0, st>>>(d, items + o, y, n, nrhs);
+        else k_fwd_step<16><<<grid, kSThreads, 0, st>>>(d, items + o, y, n, nrhs);
     }
 }
 
@@ -940,7 +1022,7 @@ void launch_bwd_step(hipStream_t st, const DevPtrs &d, const SolveItem *items, i
         const dim3 grid(static_cast<unsigned>(std::min(kMaxLaunchGroups, count - o)));
         if (nrhs == 1) k_bwd_step<1><<<grid, kSThreads, 0, st>>>(d, items + o, y, n, nrhs);
         else if (nrhs <= 4) k_bwd_step<4><<<grid, kSThreads, 0, st>>>(d, items + o, y, n, nrhs);
-        else k_bwd_step<8><<<grid, kSThreads, 0, st>>>(d, items + o, y, n, nrhs);
+        else k_bwd_step<16><<<grid, kSThreads, 0, st>>>(d, items + o, y, n, nrhs);
     }
 }
 

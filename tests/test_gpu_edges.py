@@ -12,6 +12,7 @@ if not gpu_available():
     pytest.skip("no GPU", allow_module_level=True)
 
 from opt_solver_amd import generators as g  # noqa: E402
+from opt_solver_amd._lib import TUNE_SOLVE_FUSE_ROWS  # noqa: E402
 from opt_solver_amd.solver import Plan, analyse  # noqa: E402
 from tests.test_gpu_spd import block_rel_err  # noqa: E402
 
@@ -78,3 +79,28 @@ def test_indefinite_sweep_edges(p, q):
     for nr in (1, 2, 3, 7):
         xs = fac.solve(B[:, :nr] if nr > 1 else B[:, 0]).reshape(n, nr)
         assert np.abs(xs - X[:, :nr]).max() < 1e-13 * max(n, 10)
+
+
+@pytest.mark.parametrize("p,q", [(1, 0), (1, 1), (3, 1), (63, 66), (64, 511), (64, 513), (65, 2), (127, 129),
+                                 (128, 0), (129, 640), (191, 1), (192, 257), (193, 256), (256, 255), (320, 1100)])
+def test_cholesky_sweep_edges(p, q):
+    """Sweeps of a Cholesky factor whose first front has p pivots and q rows
+    below them: 64-pivot blocks, 128-pivot steps, 64- and 128-row groups,
+    odd row counts (pairs of rows), 256-row stages, 512-row segments, and 1,
+    4, 16 and more right-hand sides. Condition number about 5."""
+    n = p + q
+    print("case cholesky sweep", p, q, flush=True)
+    rng = np.random.default_rng([p, q, 1])
+    G = rng.standard_normal((n, n))
+    M = G @ G.T / n + np.eye(n)
+    A, arrays = dense_front_problem(M, p)
+    plan = Plan(arrays, posdef=True)
+    fac = plan.factor(A[3])
+    assert fac.status == 0
+    X = rng.uniform(-1, 1, (n, 18))
+    B = M @ X
+    for fuse in (512, 0, 1 << 20):
+        plan.tune(TUNE_SOLVE_FUSE_ROWS, fuse)
+        for nr in (1, 3, 4, 5, 16, 18):
+            xs = fac.solve(B[:, :nr] if nr > 1 else B[:, 0]).reshape(n, nr)
+            assert np.abs(xs - X[:, :nr]).max() < 1e-14 * max(n, 100), (fuse, nr)
