@@ -149,18 +149,23 @@ struct FV {
 // without the explicit grouping every element waits out a full memory
 // latency.
 constexpr int kU = 4;
+// A one-wavefront workgroup's front has at most 48 rows, in LDS: one load
+// covers a sweep.
+template <int ST>
+constexpr int sweep_loads = ST == 64 ? 1 : kU;
 
-// f(i, v) for v = ld(i), i = lo, lo + st, ... < hi, in increasing i per
+// f(i, v) for v = ld(i), i = lo, lo + ST, ... < hi, in increasing i per
 // thread
-template <class Ld, class Fn>
-__device__ __forceinline__ void sweep(int lo, int hi, int st, Ld &&ld, Fn &&fn) {
-    for (int i0 = lo; i0 < hi; i0 += kU * st) {
-        double v[kU];
+template <int ST, class Ld, class Fn>
+__device__ __forceinline__ void sweep(int lo, int hi, Ld &&ld, Fn &&fn) {
+    constexpr int U = sweep_loads<ST>;
+    for (int i0 = lo; i0 < hi; i0 += U * ST) {
+        double v[U];
 #pragma unroll
-        for (int u = 0; u < kU; ++u) v[u] = ld(min(i0 + u * st, hi - 1));
+        for (int u = 0; u < U; ++u) v[u] = ld(min(i0 + u * ST, hi - 1));
 #pragma unroll
-        for (int u = 0; u < kU; ++u)
-            if (i0 + u * st < hi) fn(i0 + u * st, v[u]);
+        for (int u = 0; u < U; ++u)
+            if (i0 + u * ST < hi) fn(i0 + u * ST, v[u]);
     }
 }
 
@@ -214,21 +219,22 @@ __device__ __forceinline__ void col_copy(double *dst, const double *src, int lo,
 
 // exchange a[i] and b[i] (different columns, or a row and a column that
 // share no element over the range)
-template <class PA, class PB>
-__device__ __forceinline__ void swap_range(PA &&pa, PB &&pb, int lo, int hi, int st) {
-    for (int i0 = lo; i0 < hi; i0 += kU * st) {
-        double x[kU], y[kU];
+template <int ST, class PA, class PB>
+__device__ __forceinline__ void swap_range(PA &&pa, PB &&pb, int lo, int hi) {
+    constexpr int U = sweep_loads<ST>;
+    for (int i0 = lo; i0 < hi; i0 += U * ST) {
+        double x[U], y[U];
 #pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            const int i = min(i0 + u * st, hi - 1);
+        for (int u = 0; u < U; ++u) {
+            const int i = min(i0 + u * ST, hi - 1);
             x[u] = *pa(i);
             y[u] = *pb(i);
         }
 #pragma unroll
-        for (int u = 0; u < kU; ++u)
-            if (i0 + u * st < hi) {
-                *pa(i0 + u * st) = y[u];
-                *pb(i0 + u * st) = x[u];
+        for (int u = 0; u < U; ++u)
+            if (i0 + u * ST < hi) {
+                *pa(i0 + u * ST) = y[u];
+                *pb(i0 + u * ST) = x[u];
             }
     }
 }
@@ -285,7 +291,7 @@ __device__ void select_pivot_wg(const FV &A, int k, int ne, int limit, const Prm
         if (a0 >= prm.eff_small) {
             double m = 0.0;
             const double *ck = &A.at(0, k);
-            sweep(k + 1 + tid, f, NT, [&](int i) { return ck[i]; }, [&](int, double v) { m = fmax(m, fabs(v)); });
+            sweep<NT>(k + 1 + tid, f, [&](int i) { return ck[i]; }, [&](int, double v) { m = fmax(m, fabs(v)); });
             const double colmax = red_max(rs, m);
             if (!(prm.u * colmax > a0) && !(a0 < kWeakPivotRatio * colmax)) {
                 kind = 1;
@@ -320,13 +326,13 @@ __device__ void select_pivot_wg(const FV &A, int k, int ne, int limit, const Prm
         // increasing order
         const double *cc = &A.at(0, cand);
         const int k1 = k + tid;
-        sweep(k1, min(cand, ne), NT, [&](int i) { return A.at(cand, i); }, top2);
+        sweep<NT>(k1, min(cand, ne), [&](int i) { return A.at(cand, i); }, top2);
         {
             // first index of this thread's sequence past cand
             const int c1 = cand + 1 + (((k1 - (cand + 1)) % NT) + NT) % NT;
-            sweep(c1, ne, NT, [&](int i) { return cc[i]; }, top2);
+            sweep<NT>(c1, ne, [&](int i) { return cc[i]; }, top2);
             const int e1 = ext0 + (((k1 - ext0) % NT) + NT) % NT;
-            sweep(e1, f, NT, [&](int i) { return cc[i]; }, [&](int, double x) { mel = fmax(mel, fabs(x)); });
+            sweep<NT>(e1, f, [&](int i) { return cc[i]; }, [&](int, double x) { mel = fmax(mel, fabs(x)); });
         }
         double m1;
         int r_best;
@@ -367,8 +373,8 @@ __device__ void select_pivot_wg(const FV &A, int k, int ne, int limit, const Prm
             if (i != cand) o1 = fmax(o1, v);
         };
         const double *cr = &A.at(0, r_best);
-        sweep(k + tid, r_best, NT, [&](int i) { return A.at(r_best, i); }, part);
-        sweep(r_best + 1 + (((k + tid - (r_best + 1)) % NT) + NT) % NT, f, NT, [&](int i) { return cr[i]; }, part);
+        sweep<NT>(k + tid, r_best, [&](int i) { return A.at(r_best, i); }, part);
+        sweep<NT>(r_best + 1 + (((k + tid - (r_best + 1)) % NT) + NT) % NT, f, [&](int i) { return cr[i]; }, part);
         const double om2 = red_max(rs, o2);
         const double off1 = red_max(rs, o1);
         // two_by_two_ok (ldlt_kernel.cpp:97-122)
@@ -438,7 +444,7 @@ __device__ int partner_pairs_wg(const FV &A, int k, int pl, int ne, int nb, cons
         double bv = 0.0;
         int bi = -1;
         const double *cp = &A.at(0, pos);
-        sweep(pl + tid, ne, NT, [&](int i) { return cp[i]; }, [&](int i, double x) {
+        sweep<NT>(pl + tid, ne, [&](int i) { return cp[i]; }, [&](int i, double x) {
             const double v = fabs(x);
             if (v > bv) {
                 bv = v;
@@ -495,11 +501,11 @@ __device__ void sym_swap_wg(const FV &A, int p, int q, int32_t *rows, double *W,
     }
     // rows p and q of the columns before p; column p and row q between
     // them; columns p and q below q
-    swap_range([&](int m) { return &A.at(p, m); }, [&](int m) { return &A.at(q, m); }, c_lo + tid, p, NT);
-    swap_range([&](int m) { return &A.at(m, p); }, [&](int m) { return &A.at(q, m); }, p + 1 + tid, q, NT);
-    swap_range([&](int m) { return &A.at(m, p); }, [&](int m) { return &A.at(m, q); }, q + 1 + tid, f, NT);
-    swap_range([&](int idx) { return &W[static_cast<int64_t>(idx) * wld + p]; },
-               [&](int idx) { return &W[static_cast<int64_t>(idx) * wld + q]; }, tid, w_cols, NT);
+    swap_range<NT>([&](int m) { return &A.at(p, m); }, [&](int m) { return &A.at(q, m); }, c_lo + tid, p);
+    swap_range<NT>([&](int m) { return &A.at(m, p); }, [&](int m) { return &A.at(q, m); }, p + 1 + tid, q);
+    swap_range<NT>([&](int m) { return &A.at(m, p); }, [&](int m) { return &A.at(m, q); }, q + 1 + tid, f);
+    swap_range<NT>([&](int idx) { return &W[static_cast<int64_t>(idx) * wld + p]; },
+               [&](int idx) { return &W[static_cast<int64_t>(idx) * wld + q]; }, tid, w_cols);
     __syncthreads();
 }
 
@@ -532,12 +538,41 @@ __device__ void place_rows_wg(const FV &A, int k, int ne, int np, const int32_t 
 // eliminate_1x1 (ldlt_kernel.cpp:350-432): columns (k, ucol_end) get the
 // rank-1 update c_j[i] -= c_k[i] * (c_k[j] / d) (multiply, then subtract),
 // the unscaled column is saved in W column w_col, then c_k is scaled.
+// One wavefront (at most 48 rows, in LDS): lane i keeps its unscaled entries
+// of the pivot columns, the scaled columns go back at once, and the updates
+// of kCU columns at a time have their LDS reads in flight together (a column
+// at a time every one waited out the LDS latency, twice).
+constexpr int kCU = 8;
+
 template <int NT = kLT>
 __device__ void elim1_wg(const FV &A, int k, int ucol_end, double *W, int wld, int w_col) {
     const int tid = threadIdx.x;
     const int f = A.f;
     const double inv_d = 1.0 / A.at(k, k);
     double *ck = &A.at(0, k);
+    if constexpr (NT == 64) {
+        const bool in = tid > k && tid < f;
+        const int i = min(tid, f - 1);
+        const double u = ck[i];
+        if (in) ck[i] = __dmul_rn(u, inv_d);
+        __syncthreads();
+        for (int j0 = k + 1; j0 < ucol_end; j0 += kCU) {
+            double l[kCU], c[kCU];
+#pragma unroll
+            for (int e = 0; e < kCU; ++e) {
+                const int j = min(j0 + e, ucol_end - 1);
+                l[e] = ck[j];
+                c[e] = A.at(i, j);
+            }
+#pragma unroll
+            for (int e = 0; e < kCU; ++e) {
+                const int j = j0 + e;
+                if (j < ucol_end && in && i >= j && l[e] != 0.0) A.at(i, j) = __dsub_rn(c[e], __dmul_rn(u, l[e]));
+            }
+        }
+        __syncthreads();
+        return;
+    }
     if (W) col_copy(W + static_cast<int64_t>(w_col) * wld, ck, k + 1 + tid, f, NT);
     if (ucol_end > k + 1) {
         const int lg = lg_rows<NT>(f - (k + 1));
@@ -567,6 +602,35 @@ __device__ void elim2_wg(const FV &A, int k, int ucol_end, double *W, int wld, i
     const double inv = 1.0 / __dmul_rn(__dsub_rn(__dmul_rn(a, c), __dmul_rn(b, b)), s);
     const double i00 = __dmul_rn(c, inv), i10 = __dmul_rn(-b, inv), i11 = __dmul_rn(a, inv);
     double *ck0 = &A.at(0, k), *ck1 = &A.at(0, k + 1);
+    if constexpr (NT == 64) {
+        const bool in = tid > k + 1 && tid < f;
+        const int i = min(tid, f - 1);
+        const double u0 = ck0[i], u1 = ck1[i];
+        __syncthreads();
+        if (in) {
+            ck0[i] = __dadd_rn(__dmul_rn(i00, u0), __dmul_rn(i10, u1));
+            ck1[i] = __dadd_rn(__dmul_rn(i10, u0), __dmul_rn(i11, u1));
+        }
+        __syncthreads();
+        for (int j0 = k + 2; j0 < ucol_end; j0 += kCU) {
+            double l0[kCU], l1[kCU], cv[kCU];
+#pragma unroll
+            for (int e = 0; e < kCU; ++e) {
+                const int j = min(j0 + e, ucol_end - 1);
+                l0[e] = ck0[j];
+                l1[e] = ck1[j];
+                cv[e] = A.at(i, j);
+            }
+#pragma unroll
+            for (int e = 0; e < kCU; ++e) {
+                const int j = j0 + e;
+                if (j < ucol_end && in && i >= j && !(l0[e] == 0.0 && l1[e] == 0.0))
+                    A.at(i, j) = __dsub_rn(cv[e], __dadd_rn(__dmul_rn(u0, l0[e]), __dmul_rn(u1, l1[e])));
+            }
+        }
+        __syncthreads();
+        return;
+    }
     if (W) {
         col_copy(W + static_cast<int64_t>(w_col) * wld, ck0, k + 2 + tid, f, NT);
         col_copy(W + static_cast<int64_t>(w_col + 1) * wld, ck1, k + 2 + tid, f, NT);
@@ -649,8 +713,8 @@ __device__ int force_static_wg(const FV &A, int k, int ne, double sp, const Prm 
     for (int cand = k; cand < search_end; ++cand) {
         double m = 0.0;
         const double *cc = &A.at(0, cand);
-        sweep(k + tid, cand, NT, [&](int i) { return A.at(cand, i); }, [&](int, double v) { m = fmax(m, fabs(v)); });
-        sweep(cand + 1 + tid, f, NT, [&](int i) { return cc[i]; }, [&](int, double v) { m = fmax(m, fabs(v)); });
+        sweep<NT>(k + tid, cand, [&](int i) { return A.at(cand, i); }, [&](int, double v) { m = fmax(m, fabs(v)); });
+        sweep<NT>(cand + 1 + tid, f, [&](int i) { return cc[i]; }, [&](int, double v) { m = fmax(m, fabs(v)); });
         const double colmax = red_max(rs, m);
         const double a = fabs(A.at(cand, cand));
         const double ratio = colmax > 0.0 ? a / colmax : a;
