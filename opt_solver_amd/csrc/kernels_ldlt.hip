@@ -67,6 +67,37 @@ __device__ __forceinline__ void max_step(double &v) {
     if (b > v) v = b;
 }
 
+// The largest of the lanes' values (none NaN), on every lane: the rows of
+// 16 as above, then the rows' results into the last one.
+__device__ __forceinline__ double wave_max(double v) {
+    const auto carry = [&](auto ctrl, auto rows) {
+        const long long b = __double_as_longlong(v);
+        const int l0 = static_cast<int>(b), h0 = static_cast<int>(b >> 32);
+        const int lo = __builtin_amdgcn_update_dpp(l0, l0, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+        const int hi = __builtin_amdgcn_update_dpp(h0, h0, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+        v = fmax(v, __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo)));
+    };
+    v = fmax(v, dpp_d<kDppXor1>(v));
+    v = fmax(v, dpp_d<kDppXor2>(v));
+    v = fmax(v, dpp_d<kDppHalfMirror>(v));
+    v = fmax(v, dpp_d<kDppMirror>(v));
+    carry(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});  // lane 15 of a row to the next
+    carry(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});  // lane 31 to rows 2, 3
+    return lane_d(v, 63);
+}
+
+// What __syncthreads gives a workgroup, for NT threads; one wavefront's LDS
+// accesses happen in its own order.
+template <int NT>
+__device__ __forceinline__ void wg_sync() {
+    if constexpr (NT == 64) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        __syncthreads();
+    }
+}
+
 template <int NT>
 __device__ __forceinline__ void red_maxfirst(RedScratchT<NT> &rs, double v, int idx, double &outv, int &outi) {
     if constexpr (NT == 64) {
@@ -289,11 +320,20 @@ __device__ void select_pivot_wg(const FV &A, int k, int ne, int limit, const Prm
     if (k < limit) {
         const double a0 = fabs(A.at(k, k));
         if (a0 >= prm.eff_small) {
-            double m = 0.0;
             const double *ck = &A.at(0, k);
-            sweep<NT>(k + 1 + tid, f, [&](int i) { return ck[i]; }, [&](int, double v) { m = fmax(m, fabs(v)); });
-            const double colmax = red_max(rs, m);
-            if (!(prm.u * colmax > a0) && !(a0 < kWeakPivotRatio * colmax)) {
+            bool good;
+            if constexpr (NT == 64) {
+                // a row per lane; u * colmax and kWeakPivotRatio * colmax are
+                // the largest of the rows' products (rounding is monotone)
+                const double v = fabs(ck[min(tid, f - 1)]);
+                good = __ballot(tid > k && tid < f && (prm.u * v > a0 || a0 < kWeakPivotRatio * v)) == 0;
+            } else {
+                double m = 0.0;
+                sweep<NT>(k + 1 + tid, f, [&](int i) { return ck[i]; }, [&](int, double v) { m = fmax(m, fabs(v)); });
+                const double colmax = red_max(rs, m);
+                good = !(prm.u * colmax > a0) && !(a0 < kWeakPivotRatio * colmax);
+            }
+            if (good) {
                 kind = 1;
                 pa = k;
                 return;
@@ -309,40 +349,53 @@ __device__ void select_pivot_wg(const FV &A, int k, int ne, int limit, const Prm
         // rows [ne, f). The thread holding the overall first argmax then
         // contributes its second value to m2, every other thread its first.
         const int ext0 = max(ne, cand + 1);
-        double bv = -1.0, b2 = 0.0, mel = 0.0;
-        int bi = -1;
-        const auto top2 = [&](int i, double x) {
-            const double v = fabs(x);
-            if (v > bv) {
-                b2 = fmax(b2, bv);
-                bv = v;
-                bi = i;
-            } else {
-                b2 = fmax(b2, v);
-            }
-        };
-        // rows [k, cand) of the candidate's row, then rows (cand, ne) and
-        // [ext0, f) of its column: each thread still meets its indices in
-        // increasing order
-        const double *cc = &A.at(0, cand);
-        const int k1 = k + tid;
-        sweep<NT>(k1, min(cand, ne), [&](int i) { return A.at(cand, i); }, top2);
-        {
-            // first index of this thread's sequence past cand
-            const int c1 = cand + 1 + (((k1 - (cand + 1)) % NT) + NT) % NT;
-            sweep<NT>(c1, ne, [&](int i) { return cc[i]; }, top2);
-            const int e1 = ext0 + (((k1 - ext0) % NT) + NT) % NT;
-            sweep<NT>(e1, f, [&](int i) { return cc[i]; }, [&](int, double x) { mel = fmax(mel, fabs(x)); });
-        }
-        double m1;
+        double m1, m2, m_ext;
         int r_best;
-        red_maxfirst(rs, bv, bi, m1, r_best);
-        if (!(m1 > 0.0)) {
-            m1 = 0.0;
+        if constexpr (NT == 64) {
+            // a row per lane, NaN entries not counted
+            const int r = min(tid, f - 1);
+            const double v = fabs(tid < cand ? A.at(cand, r) : A.at(r, cand));
+            const bool elig = v >= 0.0 && tid >= k && tid < ne && tid != cand;
+            m1 = wave_max(elig ? v : -1.0);
+            m_ext = wave_max(v >= 0.0 && tid >= ext0 && tid < f ? v : 0.0);
             r_best = -1;
+            if (m1 > 0.0) r_best = __builtin_ctzll(__ballot(elig && v == m1));
+            else m1 = 0.0;
+            m2 = wave_max(elig && tid != r_best ? v : 0.0);
+        } else {
+            double bv = -1.0, b2 = 0.0, mel = 0.0;
+            int bi = -1;
+            const auto top2 = [&](int i, double x) {
+                const double v = fabs(x);
+                if (v > bv) {
+                    b2 = fmax(b2, bv);
+                    bv = v;
+                    bi = i;
+                } else {
+                    b2 = fmax(b2, v);
+                }
+            };
+            // rows [k, cand) of the candidate's row, then rows (cand, ne) and
+            // [ext0, f) of its column: each thread still meets its indices in
+            // increasing order
+            const double *cc = &A.at(0, cand);
+            const int k1 = k + tid;
+            sweep<NT>(k1, min(cand, ne), [&](int i) { return A.at(cand, i); }, top2);
+            {
+                // first index of this thread's sequence past cand
+                const int c1 = cand + 1 + (((k1 - (cand + 1)) % NT) + NT) % NT;
+                sweep<NT>(c1, ne, [&](int i) { return cc[i]; }, top2);
+                const int e1 = ext0 + (((k1 - ext0) % NT) + NT) % NT;
+                sweep<NT>(e1, f, [&](int i) { return cc[i]; }, [&](int, double x) { mel = fmax(mel, fabs(x)); });
+            }
+            red_maxfirst(rs, bv, bi, m1, r_best);
+            if (!(m1 > 0.0)) {
+                m1 = 0.0;
+                r_best = -1;
+            }
+            m2 = red_max(rs, (r_best >= 0 && bi == r_best) ? b2 : fmax(bv, 0.0));
+            m_ext = red_max(rs, mel);
         }
-        const double m2 = red_max(rs, (r_best >= 0 && bi == r_best) ? b2 : fmax(bv, 0.0));
-        const double m_ext = red_max(rs, mel);
         bool weak = false;
         double weak_growth = 0.0;
         if (a_cand >= prm.eff_small && !(prm.u * m1 > a_cand)) {
@@ -366,17 +419,26 @@ __device__ void select_pivot_wg(const FV &A, int k, int ne, int limit, const Prm
             continue;
         }
         // partner column: max excluding r_best, and excluding cand too
-        double o2 = 0.0, o1 = 0.0;
-        const auto part = [&](int i, double x) {
-            const double v = fabs(x);
-            o2 = fmax(o2, v);
-            if (i != cand) o1 = fmax(o1, v);
-        };
-        const double *cr = &A.at(0, r_best);
-        sweep<NT>(k + tid, r_best, [&](int i) { return A.at(r_best, i); }, part);
-        sweep<NT>(r_best + 1 + (((k + tid - (r_best + 1)) % NT) + NT) % NT, f, [&](int i) { return cr[i]; }, part);
-        const double om2 = red_max(rs, o2);
-        const double off1 = red_max(rs, o1);
+        double om2, off1;
+        if constexpr (NT == 64) {
+            const int r = min(tid, f - 1);
+            const double v = fabs(tid < r_best ? A.at(r_best, r) : A.at(r, r_best));
+            const bool in = v >= 0.0 && tid >= k && tid < f && tid != r_best;
+            om2 = wave_max(in ? v : 0.0);
+            off1 = wave_max(in && tid != cand ? v : 0.0);
+        } else {
+            double o2 = 0.0, o1 = 0.0;
+            const auto part = [&](int i, double x) {
+                const double v = fabs(x);
+                o2 = fmax(o2, v);
+                if (i != cand) o1 = fmax(o1, v);
+            };
+            const double *cr = &A.at(0, r_best);
+            sweep<NT>(k + tid, r_best, [&](int i) { return A.at(r_best, i); }, part);
+            sweep<NT>(r_best + 1 + (((k + tid - (r_best + 1)) % NT) + NT) % NT, f, [&](int i) { return cr[i]; }, part);
+            om2 = red_max(rs, o2);
+            off1 = red_max(rs, o1);
+        }
         // two_by_two_ok (ldlt_kernel.cpp:97-122)
         bool ok2 = false;
         double growth2 = 0.0;
@@ -398,7 +460,7 @@ __device__ void select_pivot_wg(const FV &A, int k, int ne, int limit, const Prm
                         const double bound1 = __dadd_rn(__dmul_rn(fabs(b), off0), __dmul_rn(fabs(a), off1)) / s2;
                         const double bm = bound0 > bound1 ? bound0 : bound1;
                         if (prm.u * bm > fabs(det_s)) ok2 = false;
-                        else growth2 = bm / fabs(det_s);
+                        else if (weak) growth2 = bm / fabs(det_s);
                     }
                 }
             }
@@ -490,7 +552,7 @@ __device__ void sym_swap_wg(const FV &A, int p, int q, int32_t *rows, double *W,
     }
     const int tid = threadIdx.x;
     const int f = A.f;
-    __syncthreads();
+    wg_sync<NT>();
     if (tid == 0) {
         const double t = A.at(p, p);
         A.at(p, p) = A.at(q, q);
@@ -506,7 +568,7 @@ __device__ void sym_swap_wg(const FV &A, int p, int q, int32_t *rows, double *W,
     swap_range<NT>([&](int m) { return &A.at(m, p); }, [&](int m) { return &A.at(m, q); }, q + 1 + tid, f);
     swap_range<NT>([&](int idx) { return &W[static_cast<int64_t>(idx) * wld + p]; },
                [&](int idx) { return &W[static_cast<int64_t>(idx) * wld + q]; }, tid, w_cols);
-    __syncthreads();
+    wg_sync<NT>();
 }
 
 // Brings the rows order[0..np) to positions k, k + 1, ... in turn with
@@ -538,10 +600,15 @@ __device__ void place_rows_wg(const FV &A, int k, int ne, int np, const int32_t 
 // eliminate_1x1 (ldlt_kernel.cpp:350-432): columns (k, ucol_end) get the
 // rank-1 update c_j[i] -= c_k[i] * (c_k[j] / d) (multiply, then subtract),
 // the unscaled column is saved in W column w_col, then c_k is scaled.
-// One wavefront (at most 48 rows, in LDS): lane i keeps its unscaled entries
-// of the pivot columns, the scaled columns go back at once, and the updates
-// of kCU columns at a time have their LDS reads in flight together (a column
-// at a time every one waited out the LDS latency, twice).
+// One wavefront (at most 48 rows, in LDS, in columns of a fixed length with
+// kCU spare ones behind): what bounds it is the number of instructions of a
+// single wavefront. Lane i keeps its unscaled entries of the pivot columns,
+// the scaled columns go back at once, and the updates of kCU columns at a
+// time, their LDS reads in flight together, take every lane and every column
+// of the group, without a test: what they leave above the diagonal and in
+// the spare columns is read by nothing, and a lane past the last row repeats
+// that row. Tested lanes and columns were three times the instructions
+// (about 4000 of 4500 cycles a pivot of a front of 24 rows).
 constexpr int kCU = 8;
 
 template <int NT = kLT>
@@ -551,26 +618,24 @@ __device__ void elim1_wg(const FV &A, int k, int ucol_end, double *W, int wld, i
     const double inv_d = 1.0 / A.at(k, k);
     double *ck = &A.at(0, k);
     if constexpr (NT == 64) {
-        const bool in = tid > k && tid < f;
         const int i = min(tid, f - 1);
         const double u = ck[i];
-        if (in) ck[i] = __dmul_rn(u, inv_d);
-        __syncthreads();
+        ck[i] = i > k ? __dmul_rn(u, inv_d) : u;
+        wg_sync<NT>();
         for (int j0 = k + 1; j0 < ucol_end; j0 += kCU) {
             double l[kCU], c[kCU];
 #pragma unroll
             for (int e = 0; e < kCU; ++e) {
-                const int j = min(j0 + e, ucol_end - 1);
-                l[e] = ck[j];
-                c[e] = A.at(i, j);
+                l[e] = ck[j0 + e];
+                c[e] = A.at(i, j0 + e);
             }
 #pragma unroll
             for (int e = 0; e < kCU; ++e) {
-                const int j = j0 + e;
-                if (j < ucol_end && in && i >= j && l[e] != 0.0) A.at(i, j) = __dsub_rn(c[e], __dmul_rn(u, l[e]));
+                const double v = __dsub_rn(c[e], __dmul_rn(u, l[e]));
+                A.at(i, j0 + e) = l[e] != 0.0 ? v : c[e];
             }
         }
-        __syncthreads();
+        wg_sync<NT>();
         return;
     }
     if (W) col_copy(W + static_cast<int64_t>(w_col) * wld, ck, k + 1 + tid, f, NT);
@@ -603,32 +668,29 @@ __device__ void elim2_wg(const FV &A, int k, int ucol_end, double *W, int wld, i
     const double i00 = __dmul_rn(c, inv), i10 = __dmul_rn(-b, inv), i11 = __dmul_rn(a, inv);
     double *ck0 = &A.at(0, k), *ck1 = &A.at(0, k + 1);
     if constexpr (NT == 64) {
-        const bool in = tid > k + 1 && tid < f;
         const int i = min(tid, f - 1);
         const double u0 = ck0[i], u1 = ck1[i];
-        __syncthreads();
-        if (in) {
-            ck0[i] = __dadd_rn(__dmul_rn(i00, u0), __dmul_rn(i10, u1));
-            ck1[i] = __dadd_rn(__dmul_rn(i10, u0), __dmul_rn(i11, u1));
-        }
-        __syncthreads();
+        const double s0 = __dadd_rn(__dmul_rn(i00, u0), __dmul_rn(i10, u1));
+        const double s1 = __dadd_rn(__dmul_rn(i10, u0), __dmul_rn(i11, u1));
+        wg_sync<NT>();
+        ck0[i] = i > k + 1 ? s0 : u0;
+        ck1[i] = i > k + 1 ? s1 : u1;
+        wg_sync<NT>();
         for (int j0 = k + 2; j0 < ucol_end; j0 += kCU) {
             double l0[kCU], l1[kCU], cv[kCU];
 #pragma unroll
             for (int e = 0; e < kCU; ++e) {
-                const int j = min(j0 + e, ucol_end - 1);
-                l0[e] = ck0[j];
-                l1[e] = ck1[j];
-                cv[e] = A.at(i, j);
+                l0[e] = ck0[j0 + e];
+                l1[e] = ck1[j0 + e];
+                cv[e] = A.at(i, j0 + e);
             }
 #pragma unroll
             for (int e = 0; e < kCU; ++e) {
-                const int j = j0 + e;
-                if (j < ucol_end && in && i >= j && !(l0[e] == 0.0 && l1[e] == 0.0))
-                    A.at(i, j) = __dsub_rn(cv[e], __dadd_rn(__dmul_rn(u0, l0[e]), __dmul_rn(u1, l1[e])));
+                const double v = __dsub_rn(cv[e], __dadd_rn(__dmul_rn(u0, l0[e]), __dmul_rn(u1, l1[e])));
+                A.at(i, j0 + e) = l0[e] == 0.0 && l1[e] == 0.0 ? cv[e] : v;
             }
         }
-        __syncthreads();
+        wg_sync<NT>();
         return;
     }
     if (W) {
@@ -681,11 +743,13 @@ __device__ void inertia_2x2(double d00, double d10, double d11, double small, in
         cnt[2] += 2;
         return;
     }
-    const double tr_s = __dadd_rn(d00 / s, d11 / s);
     if (det_s < -small) {
         ++cnt[0];
         ++cnt[1];
-    } else if (fabs(det_s) <= small) {
+        return;
+    }
+    const double tr_s = __dadd_rn(d00 / s, d11 / s);
+    if (fabs(det_s) <= small) {
         ++cnt[2];
         if (tr_s > small) ++cnt[0];
         else if (tr_s < -small) ++cnt[1];
@@ -724,22 +788,23 @@ __device__ int force_static_wg(const FV &A, int k, int ne, double sp, const Prm 
             best_colmax = colmax;
         }
     }
-    __syncthreads();
+    wg_sync<NT>();
     double dv = A.at(best, best);
     raised = 0;
     if (!(fabs(dv) >= sp)) {
         raised = (isfinite(dv) && fabs(dv) >= prm.eff_small) ? 1 : 2;
         dv = dv < 0.0 ? -sp : sp;
         ++nstatic;
-        __syncthreads();
+        wg_sync<NT>();
         if (tid == 0) A.at(best, best) = dv;
     }
     if (best_colmax > 0.0 && fabs(dv) > 0.0) growth = fmax(growth, best_colmax / fabs(dv));
-    __syncthreads();
+    wg_sync<NT>();
     return best;
 }
 
-// apply_pivot (ldlt_kernel.cpp:665-698). Thread 0 keeps the counters.
+// apply_pivot (ldlt_kernel.cpp:665-698). Thread 0 keeps the counters; one wavefront's
+// lanes all keep them (cnt is then each lane's own).
 template <int NT = kLT>
 __device__ void apply_pivot_wg(const FV &A, int kind, int pa, int pb, int &k, int32_t *rows, int8_t *tags, double *W,
                                int wld, int w_cols, int ucol_end, const Prm &prm, int *cnt, double &flops, int c_lo,
@@ -747,7 +812,7 @@ __device__ void apply_pivot_wg(const FV &A, int kind, int pa, int pb, int &k, in
     const int f = A.f;
     if (kind == 1) {
         sym_swap_wg<NT>(A, k, pa, rows, W, wld, w_cols, c_lo);
-        if (threadIdx.x == 0) {
+        if (NT == 64 || threadIdx.x == 0) {
             if (as_zero) ++cnt[2];
             else inertia_1x1(A.at(k, k), prm.eff_small, cnt);
             tags[k] = 1;
@@ -764,12 +829,12 @@ __device__ void apply_pivot_wg(const FV &A, int kind, int pa, int pb, int &k, in
         if (partner == k) partner = pa;
     }
     if (partner != k + 1) sym_swap_wg<NT>(A, k + 1, partner, rows, W, wld, w_cols, c_lo);
-    if (threadIdx.x == 0) {
+    if (NT == 64 || threadIdx.x == 0) {
         inertia_2x2(A.at(k, k), A.at(k + 1, k), A.at(k + 1, k + 1), prm.small_pivot, cnt);
         tags[k] = 2;
         tags[k + 1] = -1;
     }
-    __syncthreads();
+    wg_sync<NT>();
     elim2_wg<NT>(A, k, ucol_end, W, wld, w_cols);
     const double rem = static_cast<double>(f - (k + 2));
     flops += 6.0 * rem + 2.0 * rem * (rem + 1.0);
@@ -2218,20 +2283,21 @@ void launch_ldlt_assemble(hipStream_t st, const LdltDev &d, const AsmTask *tasks
 // to the strict upper slot (c, c+1), zeros elsewhere above the diagonal
 // and in a zero pivot's column; the square itself is left as it is (its
 // trailing part is the contribution block).
-__device__ __forceinline__ double stored_entry(const double *G, int f, int c, int i, int8_t tg) {
-    if (i < c) return (tg == -1 && i == c - 1) ? G[static_cast<int64_t>(c - 1) * f + c] : 0.0;
-    if (tg == 0 || (tg == 2 && i == c + 1)) return 0.0;
-    return G[static_cast<int64_t>(c) * f + i];
+__device__ __forceinline__ double stored_entry(const double *G, int ld, int c, int i, int8_t tg) {
+    const bool up = i < c;
+    const bool zero = up ? !(tg == -1 && i == c - 1) : (tg == 0 || (tg == 2 && i == c + 1));
+    const double v = G[up ? static_cast<int64_t>(c > 0 ? c - 1 : 0) * ld + c : static_cast<int64_t>(c) * ld + i];
+    return zero ? 0.0 : v;
 }
 
-// The epilogue of one front whose square (leading dimension f) is at G, in
-// global memory or LDS; store: also write its stored factor columns.
+// The epilogue of one front whose square (leading dimension ld) and pivot tags
+// are at G and tags, in global memory or LDS; store: also write its stored
+// factor columns, a column per wavefront at a time.
 template <int NT = kLT>
-__device__ void finish_front_wg(const LdltDev &d, FrontLd &F, const double *G, bool store) {
+__device__ void finish_front_wg(const LdltDev &d, FrontLd &F, const double *G, int ld, int8_t *tags, bool store) {
     __shared__ int n2;
     const int f = F.f;
     int p = F.p;
-    int8_t *tags = d.tags + F.rofs;
     const int tid = threadIdx.x;
     const bool root = F.root != 0;
     int ps = p;
@@ -2239,28 +2305,28 @@ __device__ void finish_front_wg(const LdltDev &d, FrontLd &F, const double *G, b
         for (int c = p + tid; c < F.ne; c += NT) tags[c] = 0;
         ps = F.ne;
     }
-    __syncthreads();
+    wg_sync<NT>();
     if (tid == 0) {
         F.pstore = ps;
         if (root && p < F.ne) F.nzero += F.ne - p;
         F.delayed = root ? 0 : F.ne - p;
         n2 = 0;
     }
-    __syncthreads();
+    wg_sync<NT>();
     int mine = 0;
     for (int c = tid; c < ps; c += NT) mine += tags[c] == 2;
     if (mine) atomicAdd(&n2, mine);
-    __syncthreads();
+    wg_sync<NT>();
     if (tid == 0) F.n2x2 = n2;
     for (int c = tid; c < ps; c += NT) {
-        const double *Lc = G + static_cast<int64_t>(c) * f;
+        const double *Lc = G + static_cast<int64_t>(c) * ld;
         const int8_t tg = tags[c];
         const double d00 = Lc[c];
         double *dv = d.dinv + 3 * (F.dofs + c);
         int8_t *dk = d.dkind + F.dofs + c;
         if (tg == 2) {
             const double d10 = Lc[c + 1];
-            const double d11 = G[static_cast<int64_t>(c + 1) * f + c + 1];
+            const double d11 = G[static_cast<int64_t>(c + 1) * ld + c + 1];
             double sc = fabs(d00);
             if (sc < fabs(d10)) sc = fabs(d10);
             if (sc < fabs(d11)) sc = fabs(d11);
@@ -2288,167 +2354,216 @@ __device__ void finish_front_wg(const LdltDev &d, FrontLd &F, const double *G, b
     }
     if (!store) return;
     double *O = d.fac + F.lofs;
-    const int64_t tot = static_cast<int64_t>(ps) * f;
-    for (int64_t idx = tid; idx < tot; idx += NT) {
-        const int c = static_cast<int>(idx / f), i = static_cast<int>(idx - static_cast<int64_t>(c) * f);
-        O[idx] = stored_entry(G, f, c, i, tags[c]);
+    for (int c = tid >> 6; c < ps; c += NT / 64) {
+        const int8_t tg = tags[c];
+        for (int i = tid & 63; i < f; i += 64) O[static_cast<int64_t>(c) * f + i] = stored_entry(G, ld, c, i, tg);
     }
 }
 
 __global__ __launch_bounds__(kLT) void k_ldlt_epilogue(LdltDev d, const int32_t *__restrict__ flist,
                                                        int32_t n_inline) {
     FrontLd &F = d.fronts[flist[blockIdx.x]];
-    finish_front_wg(d, F, d.arena + F.fofs, static_cast<int>(blockIdx.x) < n_inline);
+    finish_front_wg(d, F, d.arena + F.fofs, F.f, d.tags + F.rofs, static_cast<int>(blockIdx.x) < n_inline);
 }
 
 // ---------------------------------------------------------------------------
 // Levels of small fronts laid out on the device.
 //
-// Layout: one thread per front. Its size follows from the children's
-// results (nd = their delayed columns, f = nd + symbolic rows, ne = nd +
-// symbolic pivots, as the host layout); its four offsets are a workgroup
-// scan plus one bump of each counter. A front larger than L.fmax, or a
-// bump past the room, refuses the level (atomicMin of the level index).
-__global__ __launch_bounds__(kLT) void k_dev_layout(LdltDev d, DevLevel L, const int32_t *__restrict__ flist,
-                                                    int32_t nf, int32_t lv) {
-    __shared__ long long sc[4][kLT];
-    __shared__ unsigned long long base[4];
-    __shared__ int refuse;
-    // after a refused level nothing more is laid out
-    if (__atomic_load_n(&L.ctr[kDcLevel], __ATOMIC_RELAXED) < static_cast<unsigned long long>(lv)) return;
-    const int tid = threadIdx.x;
-    const int i = blockIdx.x * kLT + tid;
-    FrontLd F{};
-    long long sz[4] = {0, 0, 0, 0};
-    bool big = false;
-    if (tid == 0) refuse = 0;
-    if (i < nf) {
-        const int s = flist[i];
-        const FrontDev Sy = L.sym[s];
-        int nd = 0;
-        for (int c = L.child_ptr[s]; c < L.child_ptr[s + 1]; ++c) nd += d.fronts[L.child_idx[c]].delayed;
+// One wavefront's fronts, in columns of a fixed length (odd: a row's entries
+// lie in different banks) with kCU spare columns behind.
+constexpr int kDevWaveMax = 48, kDevWaveLd = kDevWaveMax + 1;
+constexpr int kDevKids = 16;  // children whose records are kept in LDS
+
+struct DevChild {
+    int64_t cb, rows, cmap;  // contribution block, its row ids, its symbolic rows' positions in the parent
+    int32_t f, q, del;       // leading dimension, size, delayed columns
+};
+
+template <int FMAX>
+struct DevLds {
+    double Fs[FMAX == kDevWaveMax ? kDevWaveLd * (kDevWaveMax + kCU) : FMAX * FMAX];
+    int32_t rows[FMAX], cpos[FMAX], cptr[FMAX + 1];
+    int8_t tags[FMAX];
+    int cnt[3];
+    FrontLd F;
+    DevChild kid[kDevKids];
+    bool ok;
+};
+
+__device__ __forceinline__ DevChild dev_child(const LdltDev &d, const DevLevel &L, int ch) {
+    const FrontLd &C = d.fronts[ch];
+    DevChild K;
+    K.cb = C.fofs + static_cast<int64_t>(C.p) * C.f + C.p;
+    K.rows = C.rofs + C.p;
+    K.cmap = L.sym_cmofs[ch];
+    K.f = C.f;
+    K.q = C.f - C.p;
+    K.del = C.delayed;
+    return K;
+}
+
+// Layout: a front's size follows from its children's results (nd = their
+// delayed columns, f = nd + symbolic rows, ne = nd + symbolic pivots, as the
+// host layout); its four offsets are bumps of the counters. A front larger
+// than L.fmax, or a bump past the room, refuses the level (atomicMin of the
+// level index); the level is then laid out again whole, from its children,
+// which nothing of it has changed. By the first wavefront of the front's
+// workgroup: a child per lane, the front's record and the first children's
+// to LDS. laid: the record is there already, only the children are read
+// (the second launch of a level, for its fronts above kDevWaveMax rows).
+template <int FMAX>
+__device__ void dev_layout(const DevLevel &L, const LdltDev &d, int s, int32_t lv, bool laid, DevLds<FMAX> &S) {
+    const int lane = threadIdx.x & 63;
+    // a refused level is left whole to the host (a front of it may be
+    // refusing it right now: one reading decides for the workgroup)
+    const unsigned long long refused = __atomic_load_n(&L.ctr[kDcLevel], __ATOMIC_RELAXED);
+    const FrontDev Sy = L.sym[s];
+    const int32_t parent = L.parent[s];
+    const int c0 = L.child_ptr[s], nc = L.child_ptr[s + 1] - c0;
+    int nd = 0;
+    for (int o = 0; o < nc; o += 64) {
+        int del = 0;
+        if (o + lane < nc) {
+            const DevChild K = dev_child(d, L, L.child_idx[c0 + o + lane]);
+            if (o + lane < kDevKids) S.kid[o + lane] = K;
+            del = K.del;
+        }
+        del += dpp_i<kDppXor1>(del);
+        del += dpp_i<kDppXor2>(del);
+        del += dpp_i<kDppHalfMirror>(del);
+        del += dpp_i<kDppMirror>(del);
+        for (int r = 0; r < 64; r += 16) nd += __builtin_amdgcn_readlane(del, r);
+    }
+    if (__ballot(refused <= static_cast<unsigned long long>(lv)) != 0) {
+        if (lane == 0) S.ok = false;
+        return;
+    }
+    if (laid) {
+        if (lane == 0) {
+            S.F = d.fronts[s];
+            S.ok = S.F.f > kDevWaveMax;  // the others are done
+        }
+        return;
+    }
+    const long long f = nd + Sy.f, ne = nd + Sy.p;
+    bool over = f > L.fmax;
+    unsigned long long why = kDevWhySize;
+    long long at = 0;
+    if (!over) {
+        // lane k bumps counter k
+        static_assert(kDcSq == 0 && kDcFac == 1 && kDcRows == 2 && kDcDinv == 3, "counter order");
+        const long long sz = lane == 0 ? (f * f + 63) / 64 * 64 : (lane == 1 ? f * ne : (lane == 2 ? f : ne));
+        if (lane < 4) at = static_cast<long long>(atomicAdd(&L.ctr[lane], static_cast<unsigned long long>(sz)));
+        over = __ballot(lane < 4 && at + sz > L.cap[lane & 3]) != 0;
+        why = kDevWhyRoom;
+    }
+    const long long o1 = __shfl(at, 1, 64), o2 = __shfl(at, 2, 64), o3 = __shfl(at, 3, 64);
+    if (lane == 0) {
+        S.ok = !over;
+        if (over) {
+            atomicMin(&L.ctr[kDcLevel], static_cast<unsigned long long>(lv));
+            atomicOr(&L.ctr[kDcWhy], why);
+        }
+        FrontLd F{};
         F.nd = nd;
         F.psym = Sy.p;
         F.col0 = Sy.col0;
-        F.f = nd + Sy.f;
-        F.ne = nd + Sy.p;
-        F.root = L.parent[s] < 0 ? 1 : 0;
+        F.f = static_cast<int32_t>(f);
+        F.ne = static_cast<int32_t>(ne);
+        F.root = parent < 0 ? 1 : 0;
         F.dev = 1;
-        big = F.f > L.fmax;
-        const long long f = F.f;
-        sz[0] = (f * f + 63) / 64 * 64;
-        sz[1] = f * F.ne;
-        sz[2] = f;
-        sz[3] = F.ne;
+        F.fofs = at;
+        F.lofs = o1;
+        F.rofs = o2;
+        F.dofs = o3;
+        S.F = F;
     }
-    for (int k = 0; k < 4; ++k) sc[k][tid] = sz[k];
-    __syncthreads();
-    // inclusive scan (Hillis-Steele)
-    for (int w = 1; w < kLT; w <<= 1) {
-        long long v[4];
-        for (int k = 0; k < 4; ++k) v[k] = tid >= w ? sc[k][tid - w] : 0;
-        __syncthreads();
-        for (int k = 0; k < 4; ++k) sc[k][tid] += v[k];
-        __syncthreads();
-    }
-    if (tid == 0) {
-        for (int k = 0; k < 4; ++k) {
-            const unsigned long long tot = static_cast<unsigned long long>(sc[k][kLT - 1]);
-            base[k] = atomicAdd(&L.ctr[k], tot);
-            if (static_cast<long long>(base[k] + tot) > L.cap[k]) refuse = 1;
-        }
-    }
-    __syncthreads();
-    if (refuse && tid == 0) {
-        atomicMin(&L.ctr[kDcLevel], static_cast<unsigned long long>(lv));
-        atomicOr(&L.ctr[kDcWhy], kDevWhyRoom);
-    }
-    if (i >= nf) return;
-    if (big) {
-        atomicMin(&L.ctr[kDcLevel], static_cast<unsigned long long>(lv));
-        atomicOr(&L.ctr[kDcWhy], kDevWhySize);
-    }
-    F.fofs = static_cast<int64_t>(base[0] + (sc[0][tid] - sz[0]));
-    F.lofs = static_cast<int64_t>(base[1] + (sc[1][tid] - sz[1]));
-    F.rofs = static_cast<int64_t>(base[2] + (sc[2][tid] - sz[2]));
-    F.dofs = static_cast<int64_t>(base[3] + (sc[3][tid] - sz[3]));
-    d.fronts[flist[i]] = F;
 }
 
-void launch_dev_layout(hipStream_t st, const LdltDev &d, const DevLevel &L, const int32_t *flist, int32_t nf,
-                       int32_t lv) {
-    if (nf <= 0) return;
-    k_dev_layout<<<dim3((nf + kLT - 1) / kLT), kLT, 0, st>>>(d, L, flist, nf, lv);
-}
-
-// One front per workgroup, the square in LDS: row list (children's delayed
+// One front by NT threads, the square in LDS: row list (children's delayed
 // columns in child order, then the symbolic rows), assembly (zero, the
 // front's original entries, each child's contribution block in child
 // order: per entry the host layout's order of sums), the unblocked
 // factorization, the epilogue, and the contribution block written back to
-// the front's square for the parent.
-template <int NT, int FMIN, int FMAX>
-__global__ __launch_bounds__(NT) void k_dev_fronts(LdltDev d, DevLevel L, const int32_t *__restrict__ flist, int32_t lv,
-                                                   Prm prm) {
-    __shared__ double Fs[FMAX * FMAX];
-    __shared__ RedScratchT<NT> rs;
-    __shared__ int cnt[3];
-    __shared__ int32_t cpos[FMAX];
-    __shared__ int32_t cptr[FMAX + 1];
-    // a refused level is left whole to the host
-    if (__atomic_load_n(&L.ctr[kDcLevel], __ATOMIC_RELAXED) <= static_cast<unsigned long long>(lv)) return;
-    const int s = flist[blockIdx.x];
-    FrontLd &Fd = d.fronts[s];
-    const FrontLd F = Fd;
+// the front's square for the parent. Row ids and tags stay in LDS until the
+// end: a store to memory in a pivot step is waited for at its next barrier
+// (about 2000 cycles a pivot).
+// A level is as slow as its slowest front, one wavefront's instructions and
+// memory latencies in turn: a level of the 121-level stage chain (fronts of
+// 24-31 rows) takes 28.7 us (44 with row ids and tags in memory, a layout
+// launch before and tested eliminations), one of 64 chains' 401 levels 37.7
+// (57).
+template <int NT, int FMAX>
+__device__ void dev_front(const LdltDev &d, const DevLevel &L, int s, const Prm &prm, DevLds<FMAX> &S,
+                          RedScratchT<NT> &rs) {
+    double *Fs = S.Fs;
     const FrontDev Sy = L.sym[s];
+    const FrontLd F = S.F;
     const int f = F.f, ne = F.ne, nd = F.nd;
-    if (f <= FMIN || f > FMAX) return;  // the other size class's launch
-    int32_t *rows = d.rows + F.rofs;
-    int8_t *tags = d.tags + F.rofs;
-    const int tid = threadIdx.x;
-    for (int idx = tid; idx < f * f; idx += NT) Fs[idx] = 0.0;
-    for (int t = tid; t < f; t += NT) tags[t] = 0;
-    for (int t = tid; t < Sy.f; t += NT) rows[nd + t] = L.sym_rows[Sy.rofs + t];
-    if (tid < 3) cnt[tid] = 0;
-    __syncthreads();
+    const int ld = NT == 64 ? kDevWaveLd : f;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     // original entries of the own pivot columns (one per row and column):
     // the columns' entries are contiguous; their pointers go to LDS once and
     // each lane finds the column of its entries there
-    for (int t = tid; t <= F.psym; t += NT) cptr[t] = d.pcol_ptr[F.col0 + t];
-    __syncthreads();
+    for (int t = tid; t <= F.psym; t += NT) S.cptr[t] = d.pcol_ptr[F.col0 + t];
+    for (int t = tid; t < Sy.f; t += NT) S.rows[nd + t] = L.sym_rows[Sy.rofs + t];
+    for (int idx = tid; idx < f * ld; idx += NT) Fs[idx] = 0.0;
+    for (int t = tid; t < f; t += NT) S.tags[t] = 0;
+    if (tid < 3) S.cnt[tid] = 0;
+    wg_sync<NT>();
     {
-        const int e0 = cptr[0], e1 = cptr[F.psym];
+        const int e0 = S.cptr[0], e1 = S.cptr[F.psym];
         for (int e = e0 + tid; e < e1; e += NT) {
+            const int r = d.amap[e];
+            const double a = d.av[e];
             int lo = 0, hi = F.psym;  // the column oc with cptr[oc] <= e < cptr[oc + 1]
             while (hi - lo > 1) {
                 const int mid = (lo + hi) >> 1;
-                if (cptr[mid] <= e) lo = mid;
+                if (S.cptr[mid] <= e) lo = mid;
                 else hi = mid;
             }
-            Fs[(nd + lo) * f + nd + d.amap[e]] += d.av[e];
+            Fs[(nd + lo) * ld + nd + r] += a;
         }
     }
-    __syncthreads();
+    wg_sync<NT>();
     int dp = 0;
-    for (int c = L.child_ptr[s]; c < L.child_ptr[s + 1]; ++c) {
-        const int ch = L.child_idx[c];
-        const FrontLd C = d.fronts[ch];
-        const int q = C.f - C.p, del = C.delayed;
-        const int32_t *crow = d.rows + C.rofs + C.p;
-        const int32_t *sm = L.sym_cmap + L.sym_cmofs[ch];
-        for (int ii = tid; ii < q; ii += NT) cpos[ii] = ii < del ? dp + ii : nd + sm[ii - del];
-        for (int t = tid; t < del; t += NT) rows[dp + t] = crow[t];
-        __syncthreads();
-        const double *cb = d.arena + C.fofs + static_cast<int64_t>(C.p) * C.f + C.p;
-        for (int idx = tid; idx < q * q; idx += NT) {
-            const int jj = idx / q, ii = idx - jj * q;
-            if (ii >= jj) Fs[cpos[jj] * f + cpos[ii]] += cb[static_cast<int64_t>(jj) * C.f + ii];
+    const int c0 = L.child_ptr[s], nc = L.child_ptr[s + 1] - c0;
+    for (int c = 0; c < nc; ++c) {
+        const DevChild C = c < kDevKids ? S.kid[c] : dev_child(d, L, L.child_idx[c0 + c]);
+        const int q = C.q, del = C.del;
+        for (int ii = tid; ii < q; ii += NT) S.cpos[ii] = ii < del ? dp + ii : nd + L.sym_cmap[C.cmap + ii - del];
+        for (int t = tid; t < del; t += NT) S.rows[dp + t] = d.rows[C.rows + t];
+        wg_sync<NT>();
+        // lane = row of the child's block; each wavefront's columns 8 at a
+        // time, their loads in flight together
+        const double *cb = d.arena + C.cb;
+        constexpr int kG = 8, kW = NT / 64;
+        for (int i0 = 0; i0 < q; i0 += 64) {
+            const int ii = i0 + lane, ic = min(ii, q - 1);
+            const int pi = S.cpos[ic];
+            for (int j0 = w; j0 < min(q, i0 + 64); j0 += kG * kW) {
+                double v[kG], x[kG];
+                int at[kG];
+#pragma unroll
+                for (int u = 0; u < kG; ++u) {
+                    const int jj = min(j0 + kW * u, q - 1);
+                    v[u] = cb[static_cast<int64_t>(jj) * C.f + max(ic, jj)];
+                    at[u] = S.cpos[jj] * ld + pi;
+                }
+#pragma unroll
+                for (int u = 0; u < kG; ++u) x[u] = Fs[at[u]];
+#pragma unroll
+                for (int u = 0; u < kG; ++u)
+                    if (j0 + kW * u <= ii && ii < q) Fs[at[u]] = x[u] + v[u];
+            }
         }
-        __syncthreads();
+        wg_sync<NT>();
         dp += del;
     }
-    FV A{Fs, f, f};
+    FV A{Fs, ld, f};
     int k = 0;
+    int own[3] = {0, 0, 0};
+    int *cnt = NT == 64 ? own : S.cnt;
     double flops = 0.0;
     Prm fp;
     const double sp = front_prm(prm, F, fp);
@@ -2465,50 +2580,82 @@ __global__ __launch_bounds__(NT) void k_dev_fronts(LdltDev d, DevLevel L, const 
             kind = 1;
             az = static_as_zero(raised, fp, F);
         }
-        apply_pivot_wg<NT>(A, kind, pa, pb, k, rows, tags, nullptr, 0, 0, f, fp, cnt, flops, 0, az);
+        apply_pivot_wg<NT>(A, kind, pa, pb, k, S.rows, S.tags, nullptr, 0, 0, f, fp, cnt, flops, 0, az);
     }
-    __syncthreads();
+    wg_sync<NT>();
     if (tid == 0) {
-        Fd.p = k;
-        Fd.npos = cnt[0];
-        Fd.nneg = cnt[1];
-        Fd.nzero = cnt[2];
-        Fd.flops = flops;
-        Fd.nstatic = nstatic;
-        Fd.growth = growth;
-        Fd.stalls = Fd.pulls = Fd.rotated = Fd.searches = 0;  // unblocked: no panels
+        S.F.p = k;
+        S.F.npos = cnt[0];
+        S.F.nneg = cnt[1];
+        S.F.nzero = cnt[2];
+        S.F.flops = flops;
+        S.F.nstatic = nstatic;
+        S.F.growth = growth;  // stalls to searches stay 0: unblocked, no panels
     }
-    __syncthreads();
-    finish_front_wg<NT>(d, Fd, Fs, true);
-    if (F.root) return;
     // contribution block (lower part of columns [k, f)) for the parent
-    double *G = d.arena + F.fofs;
-    const int q = f - k;
-    for (int idx = tid; idx < q * q; idx += NT) {
-        const int jj = idx / q, ii = idx - jj * q;
-        if (ii >= jj) G[static_cast<int64_t>(k + jj) * f + k + ii] = Fs[(k + jj) * f + k + ii];
+    if (!F.root) {
+        double *G = d.arena + F.fofs;
+        for (int j = k + w; j < f; j += NT / 64)
+            for (int i = j + lane; i < f; i += 64) G[static_cast<int64_t>(j) * f + i] = Fs[j * ld + i];
+    }
+    wg_sync<NT>();
+    finish_front_wg<NT>(d, S.F, Fs, ld, S.tags, true);
+    wg_sync<NT>();
+    if (tid == 0) d.fronts[s] = S.F;
+    for (int t = tid; t < f; t += NT) {
+        d.rows[F.rofs + t] = S.rows[t];
+        d.tags[F.rofs + t] = S.tags[t];
     }
 }
+
+// A level's fronts, one workgroup each.
+// CLASS 0 (64 threads): layout, then the fronts of at most 48 rows (one
+// wavefront and 23 KB of LDS: many fronts per CU); a larger one keeps its
+// layout for the CLASS 1 launch (256 threads). CLASS 2 (256 threads): layout,
+// then the first wavefront alone or the whole workgroup, by the same line:
+// one launch where a level has few fronts. CLASS 3: layout and 256 threads
+// whatever the size.
+template <int CLASS>
+__global__ __launch_bounds__(CLASS == 0 ? 64 : kLT) void k_dev_fronts(LdltDev d, DevLevel L,
+                                                                     const int32_t *__restrict__ flist, int32_t lv,
+                                                                     Prm prm) {
+    __shared__ DevLds<CLASS == 0 ? kDevWaveMax : kDevFrontMax> S;
+    __shared__ RedScratchT<CLASS == 0 ? 64 : kLT> rs;
+    const int s = flist[blockIdx.x];
+    if (threadIdx.x < 64) dev_layout(L, d, s, lv, CLASS == 1, S);
+    __syncthreads();
+    if (!S.ok) return;
+    const bool one_wave = CLASS != 1 && CLASS != 3 && S.F.f <= kDevWaveMax;
+    if constexpr (CLASS == 0) {
+        if (one_wave) dev_front<64>(d, L, s, prm, S, rs);
+        else if (threadIdx.x == 0) d.fronts[s] = S.F;
+    } else if (!one_wave) {
+        dev_front<kLT>(d, L, s, prm, S, rs);
+    } else if constexpr (CLASS == 2) {
+        // (the reductions of one wavefront use no scratch)
+        if (threadIdx.x < 64) dev_front<64>(d, L, s, prm, S, *reinterpret_cast<RedScratchT<64> *>(&rs));
+    }
+}
+
+// fronts of a level up to which one launch takes both sizes (two 256-thread
+// workgroups of 76 KB per CU)
+constexpr int32_t kDevOneLaunch = 512;
 
 void launch_dev_fronts(hipStream_t st, const LdltDev &d, const DevLevel &L, const int32_t *flist, int32_t nf,
                        int32_t lv, double u, double eff_small, double small_pivot, const StaticPrm &S, bool wave) {
     if (nf <= 0) return;
     Prm prm{u, eff_small, small_pivot, 0.0, S};
-    if (!wave) {
-        // every front on kLT threads (shorter per-front latency where a
-        // level has few fronts)
-        for (int64_t o = 0; o < nf; o += kMaxLaunchGroups)
-            k_dev_fronts<kLT, 0, 95><<<dim3(static_cast<unsigned>(std::min<int64_t>(kMaxLaunchGroups, nf - o))), kLT, 0,
-                                        st>>>(d, L, flist + o, lv, prm);
-        return;
-    }
-    // two size classes: one wavefront and a 48 x 48 square (many fronts per
-    // CU), a workgroup of kLT and the largest square
-    static_assert(kDevFrontMax == 95, "size classes");
     for (int64_t o = 0; o < nf; o += kMaxLaunchGroups) {
         const dim3 grid(static_cast<unsigned>(std::min<int64_t>(kMaxLaunchGroups, nf - o)));
-        k_dev_fronts<64, 0, 48><<<grid, 64, 0, st>>>(d, L, flist + o, lv, prm);
-        k_dev_fronts<kLT, 48, 95><<<grid, kLT, 0, st>>>(d, L, flist + o, lv, prm);
+        if (!wave) {
+            // every front on kLT threads (tuning)
+            k_dev_fronts<3><<<grid, kLT, 0, st>>>(d, L, flist + o, lv, prm);
+        } else if (nf <= kDevOneLaunch) {
+            k_dev_fronts<2><<<grid, kLT, 0, st>>>(d, L, flist + o, lv, prm);
+        } else {
+            k_dev_fronts<0><<<grid, 64, 0, st>>>(d, L, flist + o, lv, prm);
+            k_dev_fronts<1><<<grid, kLT, 0, st>>>(d, L, flist + o, lv, prm);
+        }
     }
 }
 

@@ -154,8 +154,8 @@ int ldlt_plan_build(smfgpu_plan_s *P, const smfgpu_analysis_desc *D) {
 
 // Levels of small fronts on the device, from lv0 through the run of levels
 // whose symbolic fronts are all small: room for the run (an estimate that
-// allows some delays) is reserved, the layout and front kernels of every
-// level are launched, and the counters and the done fronts are read back
+// allows some delays) is reserved, the front kernels of every level are
+// launched, and the counters and the done fronts are read back
 // once. A level refused for room is retried with twice the room; one
 // refused for a front too large is left to the host layout (hold).
 // next: the first level not done.
@@ -210,7 +210,6 @@ static int ldlt_dev_levels(smfgpu_plan_s *P, int32_t lv0, double u, double eff_s
         for (int32_t l = next; l < end; ++l) {
             const int32_t *fl = P->d_flist.p + P->lv_flist_ofs[l];
             const int32_t nf = static_cast<int32_t>(P->lv_flist_ofs[l + 1] - P->lv_flist_ofs[l]);
-            launch_dev_layout(st, d, L, fl, nf, l);
             launch_dev_fronts(st, d, L, fl, nf, l, u, eff_small, small, S, P->dev_wave != 0);
         }
         HIP_OK(hipGetLastError());

@@ -130,14 +130,14 @@ __host__ __device__ inline double front_static_value(const StaticPrm &S, int32_t
     return (S.fallback > 0.0 && (root != 0 || nd > psym)) ? S.fallback : S.sp;
 }
 
-// Levels of small fronts laid out on the device: per level, a layout
-// kernel (each front's size from its children's delays, offsets by a bump
-// of the counters below) and one workgroup per front that builds the row
-// list, assembles, factors (the unblocked kernel's steps) and stores the
-// front with the square in LDS. A level whose fronts do not all fit is
-// refused as a whole before any of it is factored: the counters record the
-// first refused level and the reason, and the launches of later levels
-// return at once.
+// Levels of small fronts laid out on the device: one workgroup per front that
+// lays it out (its size from its children's delays, offsets by a bump of the
+// counters below), builds the row list, assembles, factors (the unblocked
+// kernel's steps) and stores the front with the square in LDS. A level whose
+// fronts do not all fit is refused: the counters record the first refused
+// level and the reason, the launches of later levels return at once, and the
+// refused level is laid out again whole (the fronts of it that ran changed
+// nothing of their children).
 constexpr int32_t kDevFrontMax = 95;   // largest realized front of a device level (blocked_min_front - 1)
 constexpr int32_t kDevSymMax = 64;     // largest symbolic front of a level laid out on the device
 enum : int32_t { kDcSq = 0, kDcFac = 1, kDcRows = 2, kDcDinv = 3, kDcLevel = 4, kDcWhy = 5, kDcN = 6 };
@@ -152,8 +152,6 @@ struct DevLevel {
     int64_t cap[4];             // ends of the room for the four offsets
     int32_t fmax;               // largest realized front taken
 };
-void launch_dev_layout(hipStream_t st, const LdltDev &d, const DevLevel &L, const int32_t *flist, int32_t nf,
-                       int32_t lv);
 void launch_dev_fronts(hipStream_t st, const LdltDev &d, const DevLevel &L, const int32_t *flist, int32_t nf,
                        int32_t lv, double u, double eff_small, double small_pivot, const StaticPrm &S, bool wave);
 
