@@ -2488,11 +2488,10 @@ __device__ void dev_layout(const DevLevel &L, const LdltDev &d, int s, int32_t l
 // the front's square for the parent. Row ids and tags stay in LDS until the
 // end: a store to memory in a pivot step is waited for at its next barrier
 // (about 2000 cycles a pivot).
-// A level is as slow as its slowest front, one wavefront's instructions and
-// memory latencies in turn: a level of the 121-level stage chain (fronts of
-// 24-31 rows) takes 28.7 us (44 with row ids and tags in memory, a layout
-// launch before and tested eliminations), one of 64 chains' 401 levels 37.7
-// (57).
+// A chain is one wavefront's instructions and memory latencies in turn: 28.4
+// us a front of 24-31 rows (121-level stage chain; 44 with row ids and tags
+// in memory, a layout launch before and tested eliminations). 192 such chains
+// of 401 levels: 11.9 ms in one launch, 15.1 in a launch a level.
 template <int NT, int FMAX>
 __device__ void dev_front(const LdltDev &d, const DevLevel &L, int s, const Prm &prm, DevLds<FMAX> &S,
                           RedScratchT<NT> &rs) {
@@ -2613,7 +2612,9 @@ __device__ void dev_front(const LdltDev &d, const DevLevel &L, int s, const Prm 
 // wavefront and 23 KB of LDS: many fronts per CU); a larger one keeps its
 // layout for the CLASS 1 launch (256 threads). CLASS 2 (256 threads): layout,
 // then the first wavefront alone or the whole workgroup, by the same line:
-// one launch where a level has few fronts. CLASS 3: layout and 256 threads
+// one launch where a level has few fronts (kDevOneLaunch: the workgroups of
+// 77 KB that the card holds at a time), and for a whole band of levels, each
+// workgroup going up its chain of fronts. CLASS 3: layout and 256 threads
 // whatever the size.
 template <int CLASS>
 __global__ __launch_bounds__(CLASS == 0 ? 64 : kLT) void k_dev_fronts(LdltDev d, DevLevel L,
@@ -2621,25 +2622,29 @@ __global__ __launch_bounds__(CLASS == 0 ? 64 : kLT) void k_dev_fronts(LdltDev d,
                                                                      Prm prm) {
     __shared__ DevLds<CLASS == 0 ? kDevWaveMax : kDevFrontMax> S;
     __shared__ RedScratchT<CLASS == 0 ? 64 : kLT> rs;
-    const int s = flist[blockIdx.x];
-    if (threadIdx.x < 64) dev_layout(L, d, s, lv, CLASS == 1, S);
-    __syncthreads();
-    if (!S.ok) return;
-    const bool one_wave = CLASS != 1 && CLASS != 3 && S.F.f <= kDevWaveMax;
-    if constexpr (CLASS == 0) {
-        if (one_wave) dev_front<64>(d, L, s, prm, S, rs);
-        else if (threadIdx.x == 0) d.fronts[s] = S.F;
-    } else if (!one_wave) {
-        dev_front<kLT>(d, L, s, prm, S, rs);
-    } else if constexpr (CLASS == 2) {
-        // (the reductions of one wavefront use no scratch)
-        if (threadIdx.x < 64) dev_front<64>(d, L, s, prm, S, *reinterpret_cast<RedScratchT<64> *>(&rs));
+    for (int s = flist[blockIdx.x];;) {
+        if (threadIdx.x < 64) dev_layout(L, d, s, lv, CLASS == 1, S);
+        __syncthreads();
+        if (!S.ok) return;
+        const bool one_wave = CLASS != 1 && CLASS != 3 && S.F.f <= kDevWaveMax;
+        if constexpr (CLASS == 0) {
+            if (one_wave) dev_front<64>(d, L, s, prm, S, rs);
+            else if (threadIdx.x == 0) d.fronts[s] = S.F;
+        } else if (!one_wave) {
+            dev_front<kLT>(d, L, s, prm, S, rs);
+        } else if constexpr (CLASS == 2) {
+            // (the reductions of one wavefront use no scratch)
+            if (threadIdx.x < 64) dev_front<64>(d, L, s, prm, S, *reinterpret_cast<RedScratchT<64> *>(&rs));
+        }
+        if constexpr (CLASS != 2) return;
+        // on to the parent: this front is its only child in the band
+        s = L.parent[s];
+        if (s < 0) return;
+        lv = L.lev[s];
+        if (lv >= L.end) return;
+        __syncthreads();
     }
 }
-
-// fronts of a level up to which one launch takes both sizes (two 256-thread
-// workgroups of 76 KB per CU)
-constexpr int32_t kDevOneLaunch = 512;
 
 void launch_dev_fronts(hipStream_t st, const LdltDev &d, const DevLevel &L, const int32_t *flist, int32_t nf,
                        int32_t lv, double u, double eff_small, double small_pivot, const StaticPrm &S, bool wave) {

@@ -702,7 +702,8 @@ SMFGPU_API int smfgpu_plan_stats(smfgpu_plan_t P, double *out) {
     bytes += P->d_fl.bytes() + P->d_arena.bytes() + P->d_work.bytes() + P->d_dinv.bytes() + P->d_fac.bytes() +
              P->d_lrows.bytes() + P->d_lcmap.bytes() + P->d_flist.bytes() + P->d_ltags.bytes() +
              P->d_dkind.bytes() + P->d_stage.bytes() + P->d_child_ptr.bytes() + P->d_child_idx.bytes() +
-             P->d_parent.bytes() + P->d_xpl.bytes();
+             P->d_parent.bytes() + P->d_xpl.bytes() + P->d_level.bytes() + P->d_chain.bytes() +
+             P->d_chain_ptr.bytes();
     out[0] = bytes;
     out[1] = static_cast<double>(P->level_fronts.size());
     out[2] = static_cast<double>(P->launches.size());

@@ -129,7 +129,17 @@ int ldlt_plan_build(smfgpu_plan_s *P, const smfgpu_analysis_desc *D) {
             r[3] += pe;
         }
     }
-    if ((rc = P->d_flist.upload(lf)) || (rc = P->d_fl.alloc(std::max(ns, 1))) ||
+    P->lv_join.assign(nlev, -1);
+    for (int32_t s = 0; s < ns; ++s) {
+        int32_t hi = -1, second = -1;
+        for (int32_t c = P->child_ptr[s]; c < P->child_ptr[s + 1]; ++c) {
+            const int32_t l = P->level[P->child_idx[c]];
+            second = std::max(second, std::min(hi, l));
+            hi = std::max(hi, l);
+        }
+        P->lv_join[P->level[s]] = std::max(P->lv_join[P->level[s]], second);
+    }
+    if ((rc = P->d_level.upload(P->level)) || (rc = P->d_flist.upload(lf)) || (rc = P->d_fl.alloc(std::max(ns, 1))) ||
         (rc = P->d_child_ptr.upload(P->child_ptr)) || (rc = P->d_child_idx.upload(P->child_idx)) ||
         (rc = P->d_parent.upload(P->sn_parent)) || (rc = P->d_dctr.alloc(kDcN)))
         return rc;
@@ -206,10 +216,14 @@ static int ldlt_dev_levels(smfgpu_plan_s *P, int32_t lv0, double u, double eff_s
         L.cap[kDcRows] = P->rows_used + e_rows;
         L.cap[kDcDinv] = P->dinv_used + e_dinv;
         L.fmax = P->dev_fmax;
+        L.lev = P->d_level.p;
         const LdltDev d = ldlt_dev(P);
-        for (int32_t l = next; l < end; ++l) {
+        for (int32_t l = next; l < end; l = L.end) {
             const int32_t *fl = P->d_flist.p + P->lv_flist_ofs[l];
             const int32_t nf = static_cast<int32_t>(P->lv_flist_ofs[l + 1] - P->lv_flist_ofs[l]);
+            // a band of levels in one launch
+            L.end = l + 1;
+            while (P->dev_wave != 0 && nf <= kDevOneLaunch && L.end < end && P->lv_join[L.end] < l) ++L.end;
             launch_dev_fronts(st, d, L, fl, nf, l, u, eff_small, small, S, P->dev_wave != 0);
         }
         HIP_OK(hipGetLastError());
@@ -551,6 +565,46 @@ static int ldlt_solve_lists(smfgpu_plan_s *P) {
     // written in place into pinned staging and uploaded once
     // a step's wide triangles and its other items are two launches
     const auto slot = [](int32_t t, const SolveItem &it) { return 2 * t + ((it.flags & kItemWide) ? 0 : 1); };
+    // bands of levels whose fronts form chains (each has one child in the
+    // band) and all fit: one step, a chain's fronts in order
+    std::vector<int32_t> band_end(nlev, 0), chain_lv, chain_ptr{0};  // 0: not in a band
+    std::vector<std::pair<int64_t, int64_t>> band_step(nlev);
+    {
+        std::vector<char> fits(nlev, 1);
+        for (size_t s = 0; s < ns; ++s)
+            if (lf[s] > kChainRows) fits[P->level[s]] = 0;
+        int64_t tot = 0;
+        for (int32_t l = 0, e; l < nlev; l = e) {
+            e = l + 1;
+            while (fits[l] && e < nlev && fits[e] && P->lv_join[e] < l) ++e;
+            if (e == l + 1) continue;
+            for (int32_t k = l; k < e; ++k) {
+                band_end[k] = e;
+                tot += static_cast<int64_t>(P->level_fronts[k].size());
+            }
+        }
+        int rc;
+        if (tot > 0 && (rc = P->h_chain.reserve(static_cast<size_t>(tot)))) return rc;
+        int64_t at = 0;
+        for (int32_t l = 0; l < nlev; l = std::max(l + 1, band_end[l])) {
+            if (band_end[l] == 0) continue;
+            band_step[l] = {static_cast<int64_t>(chain_ptr.size()) - 1, static_cast<int64_t>(P->level_fronts[l].size())};
+            for (int32_t s0 : P->level_fronts[l]) {
+                for (int32_t s = s0; s >= 0 && P->level[s] < band_end[l]; s = P->sn_parent[s])
+                    if (lp[s] > 0) P->h_chain[at++] = ChainFront{P->fl[s].lofs, P->fl[s].rofs, lf[s], lp[s]};
+                chain_ptr.push_back(static_cast<int32_t>(at));
+            }
+        }
+        if (tot > 0) {
+            if ((rc = ensure(P->d_chain, static_cast<size_t>(tot), false, "chain fronts")) ||
+                (rc = ensure(P->d_chain_ptr, chain_ptr.size(), false, "chains")))
+                return rc;
+            HIP_OK(hipMemcpyAsync(P->d_chain.p, P->h_chain.data(), static_cast<size_t>(at) * sizeof(ChainFront),
+                                  hipMemcpyHostToDevice, P->stream));
+            HIP_OK(hipMemcpyAsync(P->d_chain_ptr.p, chain_ptr.data(), chain_ptr.size() * sizeof(int32_t),
+                                  hipMemcpyHostToDevice, P->stream));
+        }
+    }
     auto build = [&](bool bwd, PinnedArr<SolveItem> &items, DBuf<SolveItem> &dev,
                      std::vector<std::pair<int64_t, int64_t>> &steps, std::vector<uint8_t> &wide,
                      std::vector<int32_t> &lvs) -> int {
@@ -561,18 +615,25 @@ static int ldlt_solve_lists(smfgpu_plan_s *P) {
         for (int32_t lv = 0; lv < nlev; ++lv) {
             lvs[lv] = static_cast<int32_t>(steps.size());
             cnt.clear();
+            lv_t0[lv] = static_cast<int64_t>(tfirst.size());
+            if (band_end[lv] != 0) {
+                if (band_step[lv].second > 0) {
+                    steps.push_back(band_step[lv]);
+                    wide.push_back(kStepChains);
+                }
+                continue;
+            }
             for (int32_t s : P->level_fronts[lv])
                 front_solve_items(lf[s], lp[s], s, bwd, [&](int32_t t, const SolveItem &it) {
                     const size_t e = slot(t, it);
                     if (cnt.size() <= e) cnt.resize(e + 1, 0);
                     ++cnt[e];
                 });
-            lv_t0[lv] = static_cast<int64_t>(tfirst.size());
             for (size_t t = 0; t < cnt.size(); ++t) {
                 tfirst.push_back(total);  // first item of step index t (none if cnt[t] == 0)
                 if (cnt[t] > 0) {
                     steps.emplace_back(total, cnt[t]);
-                    wide.push_back(t % 2 == 0);
+                    wide.push_back(t % 2 == 0 ? kStepWide : 0);
                     total += cnt[t];
                 }
             }
@@ -582,6 +643,7 @@ static int ldlt_solve_lists(smfgpu_plan_s *P) {
         int rc;
         if ((rc = items.reserve(static_cast<size_t>(std::max<int64_t>(total, 1))))) return rc;
         for (int32_t lv = 0; lv < nlev; ++lv) {
+            if (band_end[lv] != 0) continue;
             // the first item of each of the level's step indices, from the
             // counting pass
             pos.assign(tfirst.begin() + lv_t0[lv], tfirst.begin() + lv_t0[lv] + lv_nstep[lv]);
@@ -1001,11 +1063,19 @@ int ldlt_solve(smfgpu_plan_s *P, const double *b_dev, int64_t ldb, double *out_d
             HIP_OK(hipMemcpy2DAsync(y, n * sizeof(double), b_dev + r0 * ldb, ldb * sizeof(double),
                                     n * sizeof(double), nr, hipMemcpyDeviceToDevice, st));
         if (tm) HIP_OK(hipEventRecord(P->sev[0], st));
+        const auto step = [&](bool up, int32_t i) {
+            const auto [first, count] = up ? P->fwd_steps[i] : P->bwd_steps[i];
+            const uint8_t kind = up ? P->fwd_wide[i] : P->bwd_wide[i];
+            if (kind == kStepChains)
+                launch_ldlt_chains(st, d, up, P->d_chain_ptr.p + first, P->d_chain.p, count, y, n, nr);
+            else if (up)
+                launch_ldlt_fwd_step(st, d, P->d_fwd_items.p + first, count, kind == kStepWide, y, n, nr);
+            else
+                launch_ldlt_bwd_step(st, d, P->d_bwd_items.p + first, count, kind == kStepWide, y, n, nr);
+        };
         if (fwd)
             for (int32_t lv = 0; lv < nl; ++lv)
-                for (int32_t i = P->fwd_lv[lv]; i < P->fwd_lv[lv + 1]; ++i)
-                    launch_ldlt_fwd_step(st, d, P->d_fwd_items.p + P->fwd_steps[i].first, P->fwd_steps[i].second,
-                                         P->fwd_wide[i] != 0, y, n, nr);
+                for (int32_t i = P->fwd_lv[lv]; i < P->fwd_lv[lv + 1]; ++i) step(true, i);
         if (job == 2) launch_ldlt_diag_div(st, d, P->d_flist.p, static_cast<int32_t>(P->lv_flist_ofs[nl]), y, n, nr);
         if (job == 1 || job == 2) {
             // the permuted-order result
@@ -1017,9 +1087,7 @@ int ldlt_solve(smfgpu_plan_s *P, const double *b_dev, int64_t ldb, double *out_d
             launch_ldlt_diag(st, d, P->d_flist.p, static_cast<int32_t>(P->lv_flist_ofs[nl]), P->max_pstore, y, n, nr);
         if (tm) HIP_OK(hipEventRecord(P->sev[1], st));
         for (int32_t lv = nl - 1; lv >= 0; --lv)
-            for (int32_t i = P->bwd_lv[lv]; i < P->bwd_lv[lv + 1]; ++i)
-                launch_ldlt_bwd_step(st, d, P->d_bwd_items.p + P->bwd_steps[i].first, P->bwd_steps[i].second,
-                                     P->bwd_wide[i] != 0, y, n, nr);
+            for (int32_t i = P->bwd_lv[lv]; i < P->bwd_lv[lv + 1]; ++i) step(false, i);
         if (tm) {
             HIP_OK(hipEventRecord(P->sev[2], st));
             HIP_OK(hipStreamSynchronize(st));

@@ -130,7 +130,9 @@ __host__ __device__ inline double front_static_value(const StaticPrm &S, int32_t
     return (S.fallback > 0.0 && (root != 0 || nd > psym)) ? S.fallback : S.sp;
 }
 
-// Levels of small fronts laid out on the device: one workgroup per front that
+// Levels of small fronts laid out on the device: one workgroup per front (of
+// the lowest level of a band: levels whose fronts all have one child in the
+// band, so each workgroup goes up its own chain of fronts) that
 // lays it out (its size from its children's delays, offsets by a bump of the
 // counters below), builds the row list, assembles, factors (the unblocked
 // kernel's steps) and stores the front with the square in LDS. A level whose
@@ -151,9 +153,13 @@ struct DevLevel {
     unsigned long long *ctr;    // kDcN counters: next free square / factor / row / D^-1 offsets, refused level, reason
     int64_t cap[4];             // ends of the room for the four offsets
     int32_t fmax;               // largest realized front taken
+    const int32_t *lev;         // level per front
+    int32_t end;                // a workgroup goes on from a front to its parent while that lies below this level
 };
 void launch_dev_fronts(hipStream_t st, const LdltDev &d, const DevLevel &L, const int32_t *flist, int32_t nf,
                        int32_t lv, double u, double eff_small, double small_pivot, const StaticPrm &S, bool wave);
+// fronts of a level up to which one launch takes both sizes, and a band
+constexpr int32_t kDevOneLaunch = 512;
 
 void launch_ldlt_small(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, double u, double eff_small,
                        double small_pivot, const StaticPrm &S);
@@ -179,6 +185,17 @@ constexpr int32_t kItemWide = 8;    // a triangle of more than 64 pivots
 // one step of the blocked forward / backward sweep (items of all fronts of
 // a level); wide: the step's triangles of more than 64 pivots, else its
 // other items (the two are independent)
+constexpr uint8_t kStepWide = 1, kStepChains = 2;
+// a front of a chain: at most kChainRows rows
+constexpr int32_t kChainRows = 64;
+struct ChainFront {
+    int64_t lofs, rofs;
+    int32_t f, p;
+};
+// a band of levels in one launch: chain c is the fronts [ptr[c], ptr[c + 1])
+// from the lowest level up
+void launch_ldlt_chains(hipStream_t st, const LdltDev &d, bool fwd, const int32_t *ptr, const ChainFront *fronts,
+                        int64_t count, double *y, int32_t n, int32_t nrhs);
 void launch_ldlt_fwd_step(hipStream_t st, const LdltDev &d, const SolveItem *items, int64_t count, bool wide,
                           double *y, int32_t n, int32_t nrhs);
 void launch_ldlt_bwd_step(hipStream_t st, const LdltDev &d, const SolveItem *items, int64_t count, bool wide,

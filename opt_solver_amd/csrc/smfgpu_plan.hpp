@@ -238,7 +238,7 @@ struct smfgpu_plan_s {
     std::vector<std::pair<int64_t, int64_t>> fwd_steps, bwd_steps;
     std::vector<int32_t> fwd_lv, bwd_lv;
     int32_t max_pstore = 0;                   // LDL^T: most stored pivots of a front
-    std::vector<uint8_t> fwd_wide, bwd_wide;  // LDL^T: per step, whether its items are wide triangles
+    std::vector<uint8_t> fwd_wide, bwd_wide;  // LDL^T: per step, kStepWide (wide triangles), kStepChains (first chain, chains) or 0
     // SPD sweeps as one persistent launch each: the items in the order the
     // sweep takes them (forward: as stored; backward: levels from the root
     // down), the step of each, the item count of each step, and the
@@ -325,6 +325,14 @@ struct smfgpu_plan_s {
     int64_t fac_used = 0, rows_used = 0, dinv_used = 0;
     std::vector<int64_t> lv_flist_ofs;              // per level: offset of its fronts in d_flist (solve)
     std::vector<int32_t> lv_fsym_max;               // per level: largest symbolic front
+    // per level: the largest level of any front's second-highest child (-1:
+    // none). Levels (l, e] continue the band that starts at l while theirs
+    // lies below l: every front then has exactly one child in the band.
+    std::vector<int32_t> lv_join;
+    DBuf<int32_t> d_level;
+    PinnedArr<ChainFront> h_chain;                  // sweeps: fronts of the bands' chains
+    DBuf<ChainFront> d_chain;
+    DBuf<int32_t> d_chain_ptr;
     std::vector<int64_t> lv_room;                   // prefix over levels of the device-level room estimates (4 per level)
     int32_t dev_fmax = kDevFrontMax;                // largest realized front of a device level (0: host layout only)
     int32_t dev_levels = 0;                         // levels the last factorization ran on the device

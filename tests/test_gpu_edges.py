@@ -104,3 +104,39 @@ def test_cholesky_sweep_edges(p, q):
         for nr in (1, 3, 4, 5, 16, 18):
             xs = fac.solve(B[:, :nr] if nr > 1 else B[:, 0]).reshape(n, nr)
             assert np.abs(xs - X[:, :nr]).max() < 1e-14 * max(n, 100), (fuse, nr)
+
+
+def block_chains(s, seed):
+    """Blocks of s columns: a chain of seven, then two chains of four and
+    two that meet in a third of three. Dense blocks on the diagonal and
+    between neighbours, diagonal of alternating sign twice the row sums."""
+    links = [(i, i + 1) for i in range(6)] + [(7, 8), (8, 9), (9, 10), (10, 13), (11, 12), (12, 13), (13, 14), (14, 15)]
+    nb, rng = 16, np.random.default_rng([s, seed])
+    M = np.zeros((nb * s, nb * s))
+    for i, j in links + [(i, i) for i in range(nb)]:
+        M[j * s:(j + 1) * s, i * s:(i + 1) * s] = rng.uniform(0.1, 1, (s, s))
+    M = np.tril(M, -1)
+    M = M + M.T
+    n = nb * s
+    return M + np.diag(np.where(np.arange(n) % 3 == 0, -2.0, 2.0) * (M.sum(1) + 1.0))
+
+
+@pytest.mark.parametrize("s", [1, 2, 8, 15, 16, 17, 24, 31, 32, 33])
+def test_chain_bands(s):
+    """Chains of fronts of 2 s rows: one launch a band while the rows are at
+    most 64, columns in groups of 16 with 32 read ahead, one wavefront up to
+    48 rows and a workgroup above, chains of one front and more, every number
+    of right-hand sides a pass holds. Strictly diagonally dominant by a factor
+    of two: the solution is known to a few n eps."""
+    print("case chains", s, flush=True)
+    M = block_chains(s, 0)
+    n = M.shape[0]
+    r, c = np.nonzero(np.tril(M))
+    A = g.coo_lower_to_csc(n, r, c, M[r, c])
+    fac = Plan(analyse(A, perm=np.arange(n), nemin=1), posdef=False).factor(A[3])
+    assert fac.status == 0
+    X = np.random.default_rng(s).uniform(-1, 1, (n, 18))
+    B = M @ X
+    for nr in (1, 2, 3, 16, 18):
+        xs = fac.solve(B[:, :nr] if nr > 1 else B[:, 0]).reshape(n, nr)
+        assert np.abs(xs - X[:, :nr]).max() < 1e-13 * max(n, 10), nr
