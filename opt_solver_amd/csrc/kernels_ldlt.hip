@@ -67,25 +67,6 @@ __device__ __forceinline__ void max_step(double &v) {
     if (b > v) v = b;
 }
 
-// The largest of the lanes' values (none NaN), on every lane: the rows of
-// 16 as above, then the rows' results into the last one.
-__device__ __forceinline__ double wave_max(double v) {
-    const auto carry = [&](auto ctrl, auto rows) {
-        const long long b = __double_as_longlong(v);
-        const int l0 = static_cast<int>(b), h0 = static_cast<int>(b >> 32);
-        const int lo = __builtin_amdgcn_update_dpp(l0, l0, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
-        const int hi = __builtin_amdgcn_update_dpp(h0, h0, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
-        v = fmax(v, __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo)));
-    };
-    v = fmax(v, dpp_d<kDppXor1>(v));
-    v = fmax(v, dpp_d<kDppXor2>(v));
-    v = fmax(v, dpp_d<kDppHalfMirror>(v));
-    v = fmax(v, dpp_d<kDppMirror>(v));
-    carry(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});  // lane 15 of a row to the next
-    carry(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});  // lane 31 to rows 2, 3
-    return lane_d(v, 63);
-}
-
 // What __syncthreads gives a workgroup, for NT threads; one wavefront's LDS
 // accesses happen in its own order.
 template <int NT>
@@ -299,6 +280,31 @@ __device__ __forceinline__ bool static_as_zero(int raised, const Prm &prm, const
     return (prm.S.flags & kStaticAsZero) || (raised == 2 && stays);
 }
 
+// two_by_two_ok (ldlt_kernel.cpp:97-122): the block of columns c0 and c1,
+// off0 and off1 their largest entries outside it.
+__device__ __forceinline__ bool two_by_two_ok(const FV &A, int c0, int c1, double off0, double off1, const Prm &prm,
+                                              double &growth) {
+    growth = 0.0;
+    const double d00 = A.at(c0, c0);
+    const double d10 = A.sym(c1, c0);
+    const double d11 = A.at(c1, c1);
+    double s2 = fabs(d00);
+    if (s2 < fabs(d10)) s2 = fabs(d10);
+    if (s2 < fabs(d11)) s2 = fabs(d11);
+    if (!(s2 >= prm.eff_small && isfinite(s2))) return false;
+    const double a = d00 / s2, b = d10 / s2, c = d11 / s2;
+    const double det_s = __dsub_rn(__dmul_rn(a, c), __dmul_rn(b, b));
+    if (!(fabs(det_s) > prm.small_pivot)) return false;
+    if (off0 > 0.0 || off1 > 0.0) {
+        const double bound0 = __dadd_rn(__dmul_rn(fabs(c), off0), __dmul_rn(fabs(b), off1)) / s2;
+        const double bound1 = __dadd_rn(__dmul_rn(fabs(b), off0), __dmul_rn(fabs(a), off1)) / s2;
+        const double bm = bound0 > bound1 ? bound0 : bound1;
+        if (prm.u * bm > fabs(det_s)) return false;
+        growth = bm / fabs(det_s);
+    }
+    return true;
+}
+
 // select_pivot (ldlt_kernel.cpp:127-275) with workgroup reductions. Every
 // thread returns the same choice.
 template <int NT>
@@ -321,19 +327,10 @@ __device__ void select_pivot_wg(const FV &A, int k, int ne, int limit, const Prm
         const double a0 = fabs(A.at(k, k));
         if (a0 >= prm.eff_small) {
             const double *ck = &A.at(0, k);
-            bool good;
-            if constexpr (NT == 64) {
-                // a row per lane; u * colmax and kWeakPivotRatio * colmax are
-                // the largest of the rows' products (rounding is monotone)
-                const double v = fabs(ck[min(tid, f - 1)]);
-                good = __ballot(tid > k && tid < f && (prm.u * v > a0 || a0 < kWeakPivotRatio * v)) == 0;
-            } else {
-                double m = 0.0;
-                sweep<NT>(k + 1 + tid, f, [&](int i) { return ck[i]; }, [&](int, double v) { m = fmax(m, fabs(v)); });
-                const double colmax = red_max(rs, m);
-                good = !(prm.u * colmax > a0) && !(a0 < kWeakPivotRatio * colmax);
-            }
-            if (good) {
+            double m = 0.0;
+            sweep<NT>(k + 1 + tid, f, [&](int i) { return ck[i]; }, [&](int, double v) { m = fmax(m, fabs(v)); });
+            const double colmax = red_max(rs, m);
+            if (!(prm.u * colmax > a0) && !(a0 < kWeakPivotRatio * colmax)) {
                 kind = 1;
                 pa = k;
                 return;
@@ -349,53 +346,40 @@ __device__ void select_pivot_wg(const FV &A, int k, int ne, int limit, const Prm
         // rows [ne, f). The thread holding the overall first argmax then
         // contributes its second value to m2, every other thread its first.
         const int ext0 = max(ne, cand + 1);
-        double m1, m2, m_ext;
-        int r_best;
-        if constexpr (NT == 64) {
-            // a row per lane, NaN entries not counted
-            const int r = min(tid, f - 1);
-            const double v = fabs(tid < cand ? A.at(cand, r) : A.at(r, cand));
-            const bool elig = v >= 0.0 && tid >= k && tid < ne && tid != cand;
-            m1 = wave_max(elig ? v : -1.0);
-            m_ext = wave_max(v >= 0.0 && tid >= ext0 && tid < f ? v : 0.0);
-            r_best = -1;
-            if (m1 > 0.0) r_best = __builtin_ctzll(__ballot(elig && v == m1));
-            else m1 = 0.0;
-            m2 = wave_max(elig && tid != r_best ? v : 0.0);
-        } else {
-            double bv = -1.0, b2 = 0.0, mel = 0.0;
-            int bi = -1;
-            const auto top2 = [&](int i, double x) {
-                const double v = fabs(x);
-                if (v > bv) {
-                    b2 = fmax(b2, bv);
-                    bv = v;
-                    bi = i;
-                } else {
-                    b2 = fmax(b2, v);
-                }
-            };
-            // rows [k, cand) of the candidate's row, then rows (cand, ne) and
-            // [ext0, f) of its column: each thread still meets its indices in
-            // increasing order
-            const double *cc = &A.at(0, cand);
-            const int k1 = k + tid;
-            sweep<NT>(k1, min(cand, ne), [&](int i) { return A.at(cand, i); }, top2);
-            {
-                // first index of this thread's sequence past cand
-                const int c1 = cand + 1 + (((k1 - (cand + 1)) % NT) + NT) % NT;
-                sweep<NT>(c1, ne, [&](int i) { return cc[i]; }, top2);
-                const int e1 = ext0 + (((k1 - ext0) % NT) + NT) % NT;
-                sweep<NT>(e1, f, [&](int i) { return cc[i]; }, [&](int, double x) { mel = fmax(mel, fabs(x)); });
+        double bv = -1.0, b2 = 0.0, mel = 0.0;
+        int bi = -1;
+        const auto top2 = [&](int i, double x) {
+            const double v = fabs(x);
+            if (v > bv) {
+                b2 = fmax(b2, bv);
+                bv = v;
+                bi = i;
+            } else {
+                b2 = fmax(b2, v);
             }
-            red_maxfirst(rs, bv, bi, m1, r_best);
-            if (!(m1 > 0.0)) {
-                m1 = 0.0;
-                r_best = -1;
-            }
-            m2 = red_max(rs, (r_best >= 0 && bi == r_best) ? b2 : fmax(bv, 0.0));
-            m_ext = red_max(rs, mel);
+        };
+        // rows [k, cand) of the candidate's row, then rows (cand, ne) and
+        // [ext0, f) of its column: each thread still meets its indices in
+        // increasing order
+        const double *cc = &A.at(0, cand);
+        const int k1 = k + tid;
+        sweep<NT>(k1, min(cand, ne), [&](int i) { return A.at(cand, i); }, top2);
+        {
+            // first index of this thread's sequence past cand
+            const int c1 = cand + 1 + (((k1 - (cand + 1)) % NT) + NT) % NT;
+            sweep<NT>(c1, ne, [&](int i) { return cc[i]; }, top2);
+            const int e1 = ext0 + (((k1 - ext0) % NT) + NT) % NT;
+            sweep<NT>(e1, f, [&](int i) { return cc[i]; }, [&](int, double x) { mel = fmax(mel, fabs(x)); });
         }
+        double m1;
+        int r_best;
+        red_maxfirst(rs, bv, bi, m1, r_best);
+        if (!(m1 > 0.0)) {
+            m1 = 0.0;
+            r_best = -1;
+        }
+        const double m2 = red_max(rs, (r_best >= 0 && bi == r_best) ? b2 : fmax(bv, 0.0));
+        const double m_ext = red_max(rs, mel);
         bool weak = false;
         double weak_growth = 0.0;
         if (a_cand >= prm.eff_small && !(prm.u * m1 > a_cand)) {
@@ -419,52 +403,19 @@ __device__ void select_pivot_wg(const FV &A, int k, int ne, int limit, const Prm
             continue;
         }
         // partner column: max excluding r_best, and excluding cand too
-        double om2, off1;
-        if constexpr (NT == 64) {
-            const int r = min(tid, f - 1);
-            const double v = fabs(tid < r_best ? A.at(r_best, r) : A.at(r, r_best));
-            const bool in = v >= 0.0 && tid >= k && tid < f && tid != r_best;
-            om2 = wave_max(in ? v : 0.0);
-            off1 = wave_max(in && tid != cand ? v : 0.0);
-        } else {
-            double o2 = 0.0, o1 = 0.0;
-            const auto part = [&](int i, double x) {
-                const double v = fabs(x);
-                o2 = fmax(o2, v);
-                if (i != cand) o1 = fmax(o1, v);
-            };
-            const double *cr = &A.at(0, r_best);
-            sweep<NT>(k + tid, r_best, [&](int i) { return A.at(r_best, i); }, part);
-            sweep<NT>(r_best + 1 + (((k + tid - (r_best + 1)) % NT) + NT) % NT, f, [&](int i) { return cr[i]; }, part);
-            om2 = red_max(rs, o2);
-            off1 = red_max(rs, o1);
-        }
-        // two_by_two_ok (ldlt_kernel.cpp:97-122)
-        bool ok2 = false;
-        double growth2 = 0.0;
-        if (k + 1 < limit) {
-            const double d00 = A.at(cand, cand);
-            const double d10 = A.sym(r_best, cand);
-            const double d11 = A.at(r_best, r_best);
-            double s2 = fabs(d00);
-            if (s2 < fabs(d10)) s2 = fabs(d10);
-            if (s2 < fabs(d11)) s2 = fabs(d11);
-            if (s2 >= prm.eff_small && isfinite(s2)) {
-                const double a = d00 / s2, b = d10 / s2, c = d11 / s2;
-                const double det_s = __dsub_rn(__dmul_rn(a, c), __dmul_rn(b, b));
-                if (fabs(det_s) > prm.small_pivot) {
-                    const double off0 = fmax(m2, m_ext);
-                    ok2 = true;
-                    if (off0 > 0.0 || off1 > 0.0) {
-                        const double bound0 = __dadd_rn(__dmul_rn(fabs(c), off0), __dmul_rn(fabs(b), off1)) / s2;
-                        const double bound1 = __dadd_rn(__dmul_rn(fabs(b), off0), __dmul_rn(fabs(a), off1)) / s2;
-                        const double bm = bound0 > bound1 ? bound0 : bound1;
-                        if (prm.u * bm > fabs(det_s)) ok2 = false;
-                        else if (weak) growth2 = bm / fabs(det_s);
-                    }
-                }
-            }
-        }
+        double o2 = 0.0, o1 = 0.0;
+        const auto part = [&](int i, double x) {
+            const double v = fabs(x);
+            o2 = fmax(o2, v);
+            if (i != cand) o1 = fmax(o1, v);
+        };
+        const double *cr = &A.at(0, r_best);
+        sweep<NT>(k + tid, r_best, [&](int i) { return A.at(r_best, i); }, part);
+        sweep<NT>(r_best + 1 + (((k + tid - (r_best + 1)) % NT) + NT) % NT, f, [&](int i) { return cr[i]; }, part);
+        const double om2 = red_max(rs, o2);
+        const double off1 = red_max(rs, o1);
+        double growth2;
+        const bool ok2 = k + 1 < limit && two_by_two_ok(A, cand, r_best, fmax(m2, m_ext), off1, prm, growth2);
         if (ok2 && (!weak || growth2 < weak_growth)) {
             kind = 2;
             pa = cand;
@@ -600,44 +551,12 @@ __device__ void place_rows_wg(const FV &A, int k, int ne, int np, const int32_t 
 // eliminate_1x1 (ldlt_kernel.cpp:350-432): columns (k, ucol_end) get the
 // rank-1 update c_j[i] -= c_k[i] * (c_k[j] / d) (multiply, then subtract),
 // the unscaled column is saved in W column w_col, then c_k is scaled.
-// One wavefront (at most 48 rows, in LDS, in columns of a fixed length with
-// kCU spare ones behind): what bounds it is the number of instructions of a
-// single wavefront. Lane i keeps its unscaled entries of the pivot columns,
-// the scaled columns go back at once, and the updates of kCU columns at a
-// time, their LDS reads in flight together, take every lane and every column
-// of the group, without a test: what they leave above the diagonal and in
-// the spare columns is read by nothing, and a lane past the last row repeats
-// that row. Tested lanes and columns were three times the instructions
-// (about 4000 of 4500 cycles a pivot of a front of 24 rows).
-constexpr int kCU = 8;
-
 template <int NT = kLT>
 __device__ void elim1_wg(const FV &A, int k, int ucol_end, double *W, int wld, int w_col) {
     const int tid = threadIdx.x;
     const int f = A.f;
     const double inv_d = 1.0 / A.at(k, k);
     double *ck = &A.at(0, k);
-    if constexpr (NT == 64) {
-        const int i = min(tid, f - 1);
-        const double u = ck[i];
-        ck[i] = i > k ? __dmul_rn(u, inv_d) : u;
-        wg_sync<NT>();
-        for (int j0 = k + 1; j0 < ucol_end; j0 += kCU) {
-            double l[kCU], c[kCU];
-#pragma unroll
-            for (int e = 0; e < kCU; ++e) {
-                l[e] = ck[j0 + e];
-                c[e] = A.at(i, j0 + e);
-            }
-#pragma unroll
-            for (int e = 0; e < kCU; ++e) {
-                const double v = __dsub_rn(c[e], __dmul_rn(u, l[e]));
-                A.at(i, j0 + e) = l[e] != 0.0 ? v : c[e];
-            }
-        }
-        wg_sync<NT>();
-        return;
-    }
     if (W) col_copy(W + static_cast<int64_t>(w_col) * wld, ck, k + 1 + tid, f, NT);
     if (ucol_end > k + 1) {
         const int lg = lg_rows<NT>(f - (k + 1));
@@ -667,32 +586,6 @@ __device__ void elim2_wg(const FV &A, int k, int ucol_end, double *W, int wld, i
     const double inv = 1.0 / __dmul_rn(__dsub_rn(__dmul_rn(a, c), __dmul_rn(b, b)), s);
     const double i00 = __dmul_rn(c, inv), i10 = __dmul_rn(-b, inv), i11 = __dmul_rn(a, inv);
     double *ck0 = &A.at(0, k), *ck1 = &A.at(0, k + 1);
-    if constexpr (NT == 64) {
-        const int i = min(tid, f - 1);
-        const double u0 = ck0[i], u1 = ck1[i];
-        const double s0 = __dadd_rn(__dmul_rn(i00, u0), __dmul_rn(i10, u1));
-        const double s1 = __dadd_rn(__dmul_rn(i10, u0), __dmul_rn(i11, u1));
-        wg_sync<NT>();
-        ck0[i] = i > k + 1 ? s0 : u0;
-        ck1[i] = i > k + 1 ? s1 : u1;
-        wg_sync<NT>();
-        for (int j0 = k + 2; j0 < ucol_end; j0 += kCU) {
-            double l0[kCU], l1[kCU], cv[kCU];
-#pragma unroll
-            for (int e = 0; e < kCU; ++e) {
-                l0[e] = ck0[j0 + e];
-                l1[e] = ck1[j0 + e];
-                cv[e] = A.at(i, j0 + e);
-            }
-#pragma unroll
-            for (int e = 0; e < kCU; ++e) {
-                const double v = __dsub_rn(cv[e], __dadd_rn(__dmul_rn(u0, l0[e]), __dmul_rn(u1, l1[e])));
-                A.at(i, j0 + e) = l0[e] == 0.0 && l1[e] == 0.0 ? cv[e] : v;
-            }
-        }
-        wg_sync<NT>();
-        return;
-    }
     if (W) {
         col_copy(W + static_cast<int64_t>(w_col) * wld, ck0, k + 2 + tid, f, NT);
         col_copy(W + static_cast<int64_t>(w_col + 1) * wld, ck1, k + 2 + tid, f, NT);
@@ -803,8 +696,7 @@ __device__ int force_static_wg(const FV &A, int k, int ne, double sp, const Prm 
     return best;
 }
 
-// apply_pivot (ldlt_kernel.cpp:665-698). Thread 0 keeps the counters; one wavefront's
-// lanes all keep them (cnt is then each lane's own).
+// apply_pivot (ldlt_kernel.cpp:665-698). Thread 0 keeps the counters.
 template <int NT = kLT>
 __device__ void apply_pivot_wg(const FV &A, int kind, int pa, int pb, int &k, int32_t *rows, int8_t *tags, double *W,
                                int wld, int w_cols, int ucol_end, const Prm &prm, int *cnt, double &flops, int c_lo,
@@ -812,7 +704,7 @@ __device__ void apply_pivot_wg(const FV &A, int kind, int pa, int pb, int &k, in
     const int f = A.f;
     if (kind == 1) {
         sym_swap_wg<NT>(A, k, pa, rows, W, wld, w_cols, c_lo);
-        if (NT == 64 || threadIdx.x == 0) {
+        if (threadIdx.x == 0) {
             if (as_zero) ++cnt[2];
             else inertia_1x1(A.at(k, k), prm.eff_small, cnt);
             tags[k] = 1;
@@ -829,7 +721,7 @@ __device__ void apply_pivot_wg(const FV &A, int kind, int pa, int pb, int &k, in
         if (partner == k) partner = pa;
     }
     if (partner != k + 1) sym_swap_wg<NT>(A, k + 1, partner, rows, W, wld, w_cols, c_lo);
-    if (NT == 64 || threadIdx.x == 0) {
+    if (threadIdx.x == 0) {
         inertia_2x2(A.at(k, k), A.at(k + 1, k), A.at(k + 1, k + 1), prm.small_pivot, cnt);
         tags[k] = 2;
         tags[k + 1] = -1;
@@ -2293,7 +2185,8 @@ __device__ __forceinline__ double stored_entry(const double *G, int ld, int c, i
 // The epilogue of one front whose square (leading dimension ld) and pivot tags
 // are at G and tags, in global memory or LDS; store: also write its stored
 // factor columns, a column per wavefront at a time.
-template <int NT = kLT>
+// LANES: at most 64 rows.
+template <int NT = kLT, bool LANES = false>
 __device__ void finish_front_wg(const LdltDev &d, FrontLd &F, const double *G, int ld, int8_t *tags, bool store) {
     __shared__ int n2;
     const int f = F.f;
@@ -2313,11 +2206,16 @@ __device__ void finish_front_wg(const LdltDev &d, FrontLd &F, const double *G, i
         n2 = 0;
     }
     wg_sync<NT>();
-    int mine = 0;
-    for (int c = tid; c < ps; c += NT) mine += tags[c] == 2;
-    if (mine) atomicAdd(&n2, mine);
-    wg_sync<NT>();
-    if (tid == 0) F.n2x2 = n2;
+    if constexpr (LANES) {
+        const int c2 = __popcll(__ballot(tid < ps && tags[min(tid, f - 1)] == 2));
+        if (tid == 0) F.n2x2 = c2;
+    } else {
+        int mine = 0;
+        for (int c = tid; c < ps; c += NT) mine += tags[c] == 2;
+        if (mine) atomicAdd(&n2, mine);
+        wg_sync<NT>();
+        if (tid == 0) F.n2x2 = n2;
+    }
     for (int c = tid; c < ps; c += NT) {
         const double *Lc = G + static_cast<int64_t>(c) * ld;
         const int8_t tg = tags[c];
@@ -2354,6 +2252,19 @@ __device__ void finish_front_wg(const LdltDev &d, FrontLd &F, const double *G, i
     }
     if (!store) return;
     double *O = d.fac + F.lofs;
+    if constexpr (LANES) {
+        // a row per lane, 8 columns' reads in flight
+        const int lane = tid & 63, i = min(lane, f - 1);
+        for (int c0 = 8 * (tid >> 6); c0 < ps; c0 += NT / 8) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = stored_entry(G, ld, min(c0 + u, ps - 1), i, tags[min(c0 + u, ps - 1)]);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (c0 + u < ps && lane < f) O[static_cast<int64_t>(c0 + u) * f + lane] = v[u];
+        }
+        return;
+    }
     for (int c = tid >> 6; c < ps; c += NT / 64) {
         const int8_t tg = tags[c];
         for (int i = tid & 63; i < f; i += 64) O[static_cast<int64_t>(c) * f + i] = stored_entry(G, ld, c, i, tg);
@@ -2367,12 +2278,316 @@ __global__ __launch_bounds__(kLT) void k_ldlt_epilogue(LdltDev d, const int32_t 
 }
 
 // ---------------------------------------------------------------------------
+// A front of at most 64 rows in LDS by NW wavefronts, the unblocked steps
+// with a row per lane: columns of a fixed odd length kLd (a row's entries lie
+// in different banks), kCU spare columns behind the last. What bounds a front
+// is the number of instructions that its wavefronts go through one after the
+// other. So
+// - a wavefront takes kCU columns at a time, every lane and every column of
+//   the group, without a test: what that leaves above the diagonal and in
+//   the spare columns is read by nothing, a lane past the last row repeats
+//   that row (tested lanes and columns were three times the instructions);
+// - each wavefront scales the pivot columns for itself (lcol); the columns
+//   are scaled in place after the step's barrier, by the first wavefront,
+//   which also swaps rows: no other reads a finished column;
+// - the pivot test is a ballot, the search looks at all candidates at once.
+constexpr int kCU = 8;
+constexpr int kLaneRows = 64;  // rows at most
+
+struct LanePick {
+    int cand, take, partner;
+};
+template <int NW>
+struct LaneLds {
+    double lcol[NW][2][kLaneRows + kCU];
+    LanePick pick[NW];
+};
+
+// select_pivot's search over the candidates [k, limit): 2^lg lanes per
+// candidate, each meeting its rows in increasing order, so the lanes of a
+// candidate find what a sequential scan finds; the first candidate that a
+// test accepts is the choice. (One candidate after the other by one
+// wavefront took about 2500 cycles each, and badly pivoted fronts look at
+// many.)
+template <int NW>
+__device__ __forceinline__ void lane_search(const FV &A, int k, int ne, const Prm &prm, LaneLds<NW> &S, int &kind,
+                                            int &pa, int &pb) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int f = A.f, ld = A.ld;
+    const int nc = ne - k;
+    if (nc <= 0) return;
+    // lanes per candidate: all candidates in one go, at most 8 lanes each
+    int lg = 0;
+    while (lg < 3 && nc << (lg + 1) <= 64 * NW) ++lg;
+    const int g = 1 << lg, slice = lane & (g - 1);
+    const int cl = w * (64 >> lg) + (lane >> lg);
+    const bool live = cl < nc;
+    const int cand = k + min(cl, nc - 1);
+    // fn(row, |entry|) for the lane's rows of [lo, hi) in column c of the
+    // symmetric matrix; NaN entries, row c and rows out of range as -1
+    constexpr int kR = NW == 1 ? 8 : 4;
+    const auto rows = [&](int c, int lo, int hi, auto &&fn) {
+        for (int i0 = lo + slice; i0 - slice < hi; i0 += g * kR) {
+            double v[kR];
+#pragma unroll
+            for (int u = 0; u < kR; ++u) {
+                const int i = min(i0 + g * u, f - 1);
+                v[u] = A.F[i < c ? i * ld + c : c * ld + i];
+            }
+#pragma unroll
+            for (int u = 0; u < kR; ++u) {
+                const int i = i0 + g * u;
+                fn(i, i < hi && i != c ? fmax(fabs(v[u]), -1.0) : -1.0);
+            }
+        }
+    };
+    const double a_cand = fabs(A.at(cand, cand));
+    // largest entry over the eligible rows [k, ne) other than cand (first
+    // index on ties), the largest of the rest, the largest of rows [ne, f)
+    double m1 = -1.0, m2 = 0.0, m_ext = 0.0;
+    int r_best = -1;
+    rows(cand, k, ne, [&](int i, double v) {
+        m2 = fmax(m2, fmin(v, m1));
+        if (v > m1) {
+            m1 = v;
+            r_best = i;
+        }
+    });
+    rows(cand, ne, f, [&](int, double v) { m_ext = fmax(m_ext, v); });
+    const auto join = [&](auto ctrl) {
+        constexpr int C = decltype(ctrl)::value;
+        const double n1 = dpp_d<C>(m1), n2 = dpp_d<C>(m2);
+        const int rb = dpp_i<C>(r_best);
+        m_ext = fmax(m_ext, dpp_d<C>(m_ext));
+        m2 = fmax(fmax(m2, n2), fmin(m1, n1));
+        if (better_first(n1, rb, m1, r_best)) {
+            m1 = n1;
+            r_best = rb;
+        }
+    };
+    if (lg > 0) join(std::integral_constant<int, kDppXor1>{});
+    if (lg > 1) join(std::integral_constant<int, kDppXor2>{});
+    if (lg > 2) join(std::integral_constant<int, kDppHalfMirror>{});
+    if (!(m1 > 0.0)) {
+        m1 = 0.0;
+        r_best = -1;
+    }
+    // 0: refused, 1: alone, 2: with its partner, 3: its partner alone
+    int take = 0;
+    bool weak = false;
+    double weak_growth = 0.0;
+    if (live && a_cand >= prm.eff_small && !(prm.u * m1 > a_cand) && !(prm.u * m_ext > a_cand)) {
+        const double colmax = fmax(m1, m_ext);
+        if (!(a_cand < kWeakPivotRatio * colmax)) {
+            take = 1;
+        } else {
+            weak = true;
+            weak_growth = colmax / a_cand;
+        }
+    }
+    const bool pair = live && take == 0 && r_best >= k;
+    if (weak && !pair) take = 1;
+    const unsigned long long sure = __ballot(take != 0);
+    // candidates before the first one taken already may still pair up
+    if (__ballot(pair && (sure == 0 || lane < __builtin_ctzll(sure))) != 0) {
+        // partner column: max excluding r_best, and excluding cand too
+        const int r = pair ? r_best : cand;
+        double om2 = 0.0, off1 = 0.0;
+        rows(r, k, f, [&](int i, double v) {
+            om2 = fmax(om2, v);
+            off1 = fmax(off1, i != cand ? v : 0.0);
+        });
+        const auto join2 = [&](auto ctrl) {
+            constexpr int C = decltype(ctrl)::value;
+            om2 = fmax(om2, dpp_d<C>(om2));
+            off1 = fmax(off1, dpp_d<C>(off1));
+        };
+        if (lg > 0) join2(std::integral_constant<int, kDppXor1>{});
+        if (lg > 1) join2(std::integral_constant<int, kDppXor2>{});
+        if (lg > 2) join2(std::integral_constant<int, kDppHalfMirror>{});
+        if (pair) {
+            double growth2;
+            const bool ok2 = k + 1 < ne && two_by_two_ok(A, cand, r, fmax(m2, m_ext), off1, prm, growth2);
+            const double a_r = fabs(A.at(r, r));
+            if (ok2 && (!weak || growth2 < weak_growth)) take = 2;
+            else if (weak) take = 1;
+            else if (a_r >= prm.eff_small && (om2 == 0.0 || a_r >= prm.u * om2)) take = 3;
+        }
+    }
+    const unsigned long long taken = __ballot(take != 0);
+    LanePick P{-1, 0, -1};
+    if (taken != 0) {
+        const int l = __builtin_ctzll(taken);
+        P.cand = __builtin_amdgcn_readlane(cand, l);
+        P.take = __builtin_amdgcn_readlane(take, l);
+        P.partner = __builtin_amdgcn_readlane(r_best, l);
+    }
+    if constexpr (NW > 1) {
+        // the wavefronts' candidates follow each other
+        if (lane == 0) S.pick[w] = P;
+        __syncthreads();
+        for (int v = NW - 1; v >= 0; --v)
+            if (S.pick[v].take != 0) P = S.pick[v];
+    }
+    if (P.take == 0) return;
+    kind = P.take == 2 ? 2 : 1;
+    pa = P.take == 3 ? P.partner : P.cand;
+    if (P.take == 2) pb = P.partner;
+}
+
+// select_pivot: the same choice as select_pivot_wg with limit = ne.
+template <int NW>
+__device__ __forceinline__ void lane_select(const FV &A, int k, int ne, const Prm &prm, LaneLds<NW> &S, int &kind,
+                                            int &pa, int &pb) {
+    const int lane = threadIdx.x & 63;
+    const int f = A.f;
+    kind = 0;
+    pa = pb = -1;
+    const double d0 = A.at(k, k), a0 = fabs(d0);
+    if (prm.min_abs > 0.0) {
+        // in order, no search: column k or nothing (then the static path)
+        if (isfinite(d0) && a0 >= prm.min_abs) {
+            kind = 1;
+            pa = k;
+        }
+        return;
+    }
+    if (a0 >= prm.eff_small) {
+        // u * colmax and kWeakPivotRatio * colmax are the largest of the
+        // rows' products (rounding is monotone)
+        const double v = fabs(A.at(min(lane, f - 1), k));
+        if (__ballot(lane > k && lane < f && (prm.u * v > a0 || a0 < kWeakPivotRatio * v)) == 0) {
+            kind = 1;
+            pa = k;
+            return;
+        }
+    }
+    lane_search<NW>(A, k, ne, prm, S, kind, pa, pb);
+}
+
+// sym_swap by the first wavefront, a row per lane: the lane's pair of
+// entries, itself twice where nothing moves
+template <int NW>
+__device__ __forceinline__ void lane_swap(const FV &A, int p, int q, int32_t *rows) {
+    if (p == q) return;
+    if (p > q) {
+        const int t = p;
+        p = q;
+        q = t;
+    }
+    wg_sync<64 * NW>();
+    if (threadIdx.x < 64) {
+        const int m = min(static_cast<int>(threadIdx.x), A.f - 1), ld = A.ld;
+        const int ia = m < p ? m * ld + p : p * ld + m;
+        int ib = m == p ? q * ld + q : (m < q ? m * ld + q : q * ld + m);
+        if (m == q) ib = ia;
+        const double x = A.F[ia], y = A.F[ib];
+        const int32_t rp = rows[p], rq = rows[q];
+        wg_sync<64>();
+        A.F[ia] = y;
+        A.F[ib] = x;
+        rows[p] = rq;
+        rows[q] = rp;
+    }
+    wg_sync<64 * NW>();
+}
+
+// columns (k + np - 1, f) minus the pivot columns' products: lane i's
+// unscaled entries u0 (u1), the scaled columns in l0 (l1)
+template <int NW, int NP>
+__device__ __forceinline__ void lane_update(const FV &A, int j1, int i, double u0, double u1, const double *l0,
+                                            const double *l1) {
+    for (int j0 = j1 + kCU * (threadIdx.x >> 6); j0 < A.f; j0 += kCU * NW) {
+        double a[kCU], b[kCU], c[kCU];
+#pragma unroll
+        for (int e = 0; e < kCU; ++e) {
+            a[e] = l0[j0 + e];
+            if (NP == 2) b[e] = l1[j0 + e];
+            c[e] = A.at(i, j0 + e);
+        }
+#pragma unroll
+        for (int e = 0; e < kCU; ++e) {
+            // eliminate_1x1 and eliminate_2x2 skip columns of zero factors
+            const double v = NP == 2 ? __dsub_rn(c[e], __dadd_rn(__dmul_rn(u0, a[e]), __dmul_rn(u1, b[e])))
+                                     : __dsub_rn(c[e], __dmul_rn(u0, a[e]));
+            const bool skip = NP == 2 ? a[e] == 0.0 && b[e] == 0.0 : a[e] == 0.0;
+            A.at(i, j0 + e) = skip ? c[e] : v;
+        }
+    }
+}
+
+// apply_pivot (ldlt_kernel.cpp:665-698); every thread keeps the counters
+template <int NW>
+__device__ __forceinline__ void lane_apply(const FV &A, int kind, int pa, int pb, int &k, int32_t *rows, int8_t *tags,
+                                           const Prm &prm, LaneLds<NW> &S, int (&cnt)[3], double &flops,
+                                           bool as_zero) {
+    const int f = A.f;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i = min(lane, f - 1);
+    double *l0 = S.lcol[w][0], *l1 = S.lcol[w][1];
+    if (kind == 1) {
+        lane_swap<NW>(A, k, pa, rows);
+        const double dk = A.at(k, k), u = A.at(i, k);
+        if (as_zero) ++cnt[2];
+        else inertia_1x1(dk, prm.eff_small, cnt);
+        const double s = __dmul_rn(u, 1.0 / dk);
+        l0[lane] = s;
+        wg_sync<64>();
+        lane_update<NW, 1>(A, k + 1, i, u, 0.0, l0, l1);
+        wg_sync<64 * NW>();
+        if (w == 0) {
+            tags[k] = 1;
+            A.at(i, k) = i > k ? s : u;
+            wg_sync<64>();
+        }
+        const double rem = static_cast<double>(f - (k + 1));
+        flops += rem + rem * (rem + 1.0);
+        k += 1;
+        return;
+    }
+    int partner = pb;
+    if (pa != k) {
+        lane_swap<NW>(A, k, pa, rows);
+        if (partner == k) partner = pa;
+    }
+    if (partner != k + 1) lane_swap<NW>(A, k + 1, partner, rows);
+    const double d00 = A.at(k, k), d10 = A.at(k + 1, k), d11 = A.at(k + 1, k + 1);
+    const double u0 = A.at(i, k), u1 = A.at(i, k + 1);
+    inertia_2x2(d00, d10, d11, prm.small_pivot, cnt);
+    double s = fabs(d00);
+    if (s < fabs(d10)) s = fabs(d10);
+    if (s < fabs(d11)) s = fabs(d11);
+    const double a = d00 / s, b = d10 / s, c = d11 / s;
+    const double inv = 1.0 / __dmul_rn(__dsub_rn(__dmul_rn(a, c), __dmul_rn(b, b)), s);
+    const double i00 = __dmul_rn(c, inv), i10 = __dmul_rn(-b, inv), i11 = __dmul_rn(a, inv);
+    const double s0 = __dadd_rn(__dmul_rn(i00, u0), __dmul_rn(i10, u1));
+    const double s1 = __dadd_rn(__dmul_rn(i10, u0), __dmul_rn(i11, u1));
+    l0[lane] = s0;
+    l1[lane] = s1;
+    wg_sync<64>();
+    lane_update<NW, 2>(A, k + 2, i, u0, u1, l0, l1);
+    wg_sync<64 * NW>();
+    if (w == 0) {
+        tags[k] = 2;
+        tags[k + 1] = -1;
+        A.at(i, k) = i > k + 1 ? s0 : u0;
+        A.at(i, k + 1) = i > k + 1 ? s1 : u1;
+        wg_sync<64>();
+    }
+    const double rem = static_cast<double>(f - (k + 2));
+    flops += 6.0 * rem + 2.0 * rem * (rem + 1.0);
+    k += 2;
+}
+
+// ---------------------------------------------------------------------------
 // Levels of small fronts laid out on the device.
 //
-// One wavefront's fronts, in columns of a fixed length (odd: a row's entries
-// lie in different banks) with kCU spare columns behind.
-constexpr int kDevWaveMax = 48, kDevWaveLd = kDevWaveMax + 1;
-constexpr int kDevKids = 16;  // children whose records are kept in LDS
+// One wavefront's fronts have at most kDevWaveMax rows (their squares of 23 KB
+// let seven workgroups share a CU), several wavefronts' kLaneRows.
+constexpr int kDevWaveMax = 48;
+template <int ROWS>
+constexpr int lane_square = (ROWS + 1) * (ROWS + kCU);
+constexpr int kDevKids = 8;   // children whose records are kept in LDS
 
 struct DevChild {
     int64_t cb, rows, cmap;  // contribution block, its row ids, its symbolic rows' positions in the parent
@@ -2381,10 +2596,11 @@ struct DevChild {
 
 template <int FMAX>
 struct DevLds {
-    double Fs[FMAX == kDevWaveMax ? kDevWaveLd * (kDevWaveMax + kCU) : FMAX * FMAX];
+    double Fs[FMAX == kDevWaveMax ? lane_square<kDevWaveMax> : FMAX * FMAX];
     int32_t rows[FMAX], cpos[FMAX], cptr[FMAX + 1];
     int8_t tags[FMAX];
     int cnt[3];
+    LaneLds<FMAX == kDevWaveMax ? 1 : kLT / 64> lane;
     FrontLd F;
     DevChild kid[kDevKids];
     bool ok;
@@ -2488,18 +2704,23 @@ __device__ void dev_layout(const DevLevel &L, const LdltDev &d, int s, int32_t l
 // the front's square for the parent. Row ids and tags stay in LDS until the
 // end: a store to memory in a pivot step is waited for at its next barrier
 // (about 2000 cycles a pivot).
-// A chain is one wavefront's instructions and memory latencies in turn: 28.4
-// us a front of 24-31 rows (121-level stage chain; 44 with row ids and tags
-// in memory, a layout launch before and tested eliminations). 192 such chains
-// of 401 levels: 11.9 ms in one launch, 15.1 in a launch a level.
-template <int NT, int FMAX>
+// A chain is one workgroup's instructions and memory latencies in turn: a
+// front of 24-31 rows (121-level stage chain) takes 21.1 us by four
+// wavefronts, 28 by one (44 with row ids and tags in memory, a layout launch
+// before and tested eliminations). 192 such chains of up to 401 levels: 8.9
+// ms by four wavefronts, 11.6 by one.
+// ROWS: the unblocked steps with a row per lane, a front of at most ROWS
+// rows; 0: by workgroup reductions.
+template <int NT, int ROWS, int FMAX>
 __device__ void dev_front(const LdltDev &d, const DevLevel &L, int s, const Prm &prm, DevLds<FMAX> &S,
                           RedScratchT<NT> &rs) {
     double *Fs = S.Fs;
     const FrontDev Sy = L.sym[s];
     const FrontLd F = S.F;
     const int f = F.f, ne = F.ne, nd = F.nd;
-    const int ld = NT == 64 ? kDevWaveLd : f;
+    constexpr bool kLanes = ROWS > 0;
+    static_assert(!kLanes || (ROWS <= kLaneRows && lane_square<ROWS> <= sizeof(S.Fs) / sizeof(double)), "fits");
+    const int ld = kLanes ? ROWS + 1 : f;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     // original entries of the own pivot columns (one per row and column):
     // the columns' entries are contiguous; their pointers go to LDS once and
@@ -2512,16 +2733,29 @@ __device__ void dev_front(const LdltDev &d, const DevLevel &L, int s, const Prm 
     wg_sync<NT>();
     {
         const int e0 = S.cptr[0], e1 = S.cptr[F.psym];
-        for (int e = e0 + tid; e < e1; e += NT) {
-            const int r = d.amap[e];
-            const double a = d.av[e];
-            int lo = 0, hi = F.psym;  // the column oc with cptr[oc] <= e < cptr[oc + 1]
-            while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (S.cptr[mid] <= e) lo = mid;
-                else hi = mid;
+        constexpr int kE = 4;
+        for (int e = e0 + tid; e < e1; e += kE * NT) {
+            int r[kE], lo[kE], hi[kE];
+            double a[kE];
+#pragma unroll
+            for (int u = 0; u < kE; ++u) {
+                const int eu = min(e + u * NT, e1 - 1);
+                r[u] = d.amap[eu];
+                a[u] = d.av[eu];
+                lo[u] = 0;
+                hi[u] = F.psym;
             }
-            Fs[(nd + lo) * ld + nd + r] += a;
+            // the column oc with cptr[oc] <= e < cptr[oc + 1]
+            for (int w2 = F.psym; w2 > 1; w2 = (w2 + 1) >> 1)
+#pragma unroll
+                for (int u = 0; u < kE; ++u) {
+                    const int mid = (lo[u] + hi[u]) >> 1;
+                    if (S.cptr[mid] <= min(e + u * NT, e1 - 1)) lo[u] = mid;
+                    else hi[u] = mid;
+                }
+#pragma unroll
+            for (int u = 0; u < kE; ++u)
+                if (e + u * NT < e1) Fs[(nd + lo[u]) * ld + nd + r[u]] += a[u];
         }
     }
     wg_sync<NT>();
@@ -2533,10 +2767,10 @@ __device__ void dev_front(const LdltDev &d, const DevLevel &L, int s, const Prm 
         for (int ii = tid; ii < q; ii += NT) S.cpos[ii] = ii < del ? dp + ii : nd + L.sym_cmap[C.cmap + ii - del];
         for (int t = tid; t < del; t += NT) S.rows[dp + t] = d.rows[C.rows + t];
         wg_sync<NT>();
-        // lane = row of the child's block; each wavefront's columns 8 at a
-        // time, their loads in flight together
+        // lane = row of the child's block; each wavefront's columns kG at
+        // a time, their loads in flight together
         const double *cb = d.arena + C.cb;
-        constexpr int kG = 8, kW = NT / 64;
+        constexpr int kG = NT == 64 ? 16 : 8, kW = NT / 64;
         for (int i0 = 0; i0 < q; i0 += 64) {
             const int ii = i0 + lane, ic = min(ii, q - 1);
             const int pi = S.cpos[ic];
@@ -2562,7 +2796,7 @@ __device__ void dev_front(const LdltDev &d, const DevLevel &L, int s, const Prm 
     FV A{Fs, ld, f};
     int k = 0;
     int own[3] = {0, 0, 0};
-    int *cnt = NT == 64 ? own : S.cnt;
+    int *cnt = kLanes ? own : S.cnt;
     double flops = 0.0;
     Prm fp;
     const double sp = front_prm(prm, F, fp);
@@ -2570,7 +2804,8 @@ __device__ void dev_front(const LdltDev &d, const DevLevel &L, int s, const Prm 
     double growth = 0.0;
     while (k < ne) {
         int kind, pa, pb;
-        select_pivot_wg(A, k, ne, ne, fp, rs, kind, pa, pb);
+        if constexpr (kLanes) lane_select<NT / 64>(A, k, ne, fp, S.lane, kind, pa, pb);
+        else select_pivot_wg(A, k, ne, ne, fp, rs, kind, pa, pb);
         bool az = false;
         if (kind == 0) {
             if (!(sp > 0.0)) break;
@@ -2579,7 +2814,8 @@ __device__ void dev_front(const LdltDev &d, const DevLevel &L, int s, const Prm 
             kind = 1;
             az = static_as_zero(raised, fp, F);
         }
-        apply_pivot_wg<NT>(A, kind, pa, pb, k, S.rows, S.tags, nullptr, 0, 0, f, fp, cnt, flops, 0, az);
+        if constexpr (kLanes) lane_apply<NT / 64>(A, kind, pa, pb, k, S.rows, S.tags, fp, S.lane, own, flops, az);
+        else apply_pivot_wg<NT>(A, kind, pa, pb, k, S.rows, S.tags, nullptr, 0, 0, f, fp, cnt, flops, 0, az);
     }
     wg_sync<NT>();
     if (tid == 0) {
@@ -2594,11 +2830,23 @@ __device__ void dev_front(const LdltDev &d, const DevLevel &L, int s, const Prm 
     // contribution block (lower part of columns [k, f)) for the parent
     if (!F.root) {
         double *G = d.arena + F.fofs;
-        for (int j = k + w; j < f; j += NT / 64)
-            for (int i = j + lane; i < f; i += 64) G[static_cast<int64_t>(j) * f + i] = Fs[j * ld + i];
+        if constexpr (kLanes) {
+            const int i = min(lane, f - 1);
+            for (int j0 = k + 8 * w; j0 < f; j0 += NT / 8) {
+                double v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = Fs[min(j0 + u, f - 1) * ld + i];
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (lane >= j0 + u && lane < f) G[static_cast<int64_t>(j0 + u) * f + lane] = v[u];
+            }
+        } else {
+            for (int j = k + w; j < f; j += NT / 64)
+                for (int i = j + lane; i < f; i += 64) G[static_cast<int64_t>(j) * f + i] = Fs[j * ld + i];
+        }
     }
     wg_sync<NT>();
-    finish_front_wg<NT>(d, S.F, Fs, ld, S.tags, true);
+    finish_front_wg<NT, kLanes>(d, S.F, Fs, ld, S.tags, true);
     wg_sync<NT>();
     if (tid == 0) d.fronts[s] = S.F;
     for (int t = tid; t < f; t += NT) {
@@ -2609,13 +2857,12 @@ __device__ void dev_front(const LdltDev &d, const DevLevel &L, int s, const Prm 
 
 // A level's fronts, one workgroup each.
 // CLASS 0 (64 threads): layout, then the fronts of at most 48 rows (one
-// wavefront and 23 KB of LDS: many fronts per CU); a larger one keeps its
-// layout for the CLASS 1 launch (256 threads). CLASS 2 (256 threads): layout,
-// then the first wavefront alone or the whole workgroup, by the same line:
-// one launch where a level has few fronts (kDevOneLaunch: the workgroups of
-// 77 KB that the card holds at a time), and for a whole band of levels, each
-// workgroup going up its chain of fronts. CLASS 3: layout and 256 threads
-// whatever the size.
+// wavefront and 25 KB of LDS: many fronts per CU); a larger one keeps its
+// layout for the CLASS 1 launch (256 threads). CLASS 2 (256 threads): layout
+// and any front, four wavefronts each: where a level has few fronts
+// (kDevOneLaunch: the workgroups of 80 KB that the card holds at a time),
+// and for a whole band of levels, each workgroup going up its chain of
+// fronts. CLASS 3: layout and workgroup reductions whatever the size.
 template <int CLASS>
 __global__ __launch_bounds__(CLASS == 0 ? 64 : kLT) void k_dev_fronts(LdltDev d, DevLevel L,
                                                                      const int32_t *__restrict__ flist, int32_t lv,
@@ -2626,15 +2873,13 @@ __global__ __launch_bounds__(CLASS == 0 ? 64 : kLT) void k_dev_fronts(LdltDev d,
         if (threadIdx.x < 64) dev_layout(L, d, s, lv, CLASS == 1, S);
         __syncthreads();
         if (!S.ok) return;
-        const bool one_wave = CLASS != 1 && CLASS != 3 && S.F.f <= kDevWaveMax;
         if constexpr (CLASS == 0) {
-            if (one_wave) dev_front<64>(d, L, s, prm, S, rs);
+            if (S.F.f <= kDevWaveMax) dev_front<64, kDevWaveMax>(d, L, s, prm, S, rs);
             else if (threadIdx.x == 0) d.fronts[s] = S.F;
-        } else if (!one_wave) {
-            dev_front<kLT>(d, L, s, prm, S, rs);
-        } else if constexpr (CLASS == 2) {
-            // (the reductions of one wavefront use no scratch)
-            if (threadIdx.x < 64) dev_front<64>(d, L, s, prm, S, *reinterpret_cast<RedScratchT<64> *>(&rs));
+        } else if (CLASS != 3 && S.F.f <= kLaneRows) {
+            dev_front<kLT, kLaneRows>(d, L, s, prm, S, rs);
+        } else {
+            dev_front<kLT, 0>(d, L, s, prm, S, rs);
         }
         if constexpr (CLASS != 2) return;
         // on to the parent: this front is its only child in the band
