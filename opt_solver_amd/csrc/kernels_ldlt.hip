@@ -1039,59 +1039,60 @@ __device__ __forceinline__ void super_block_tile(int nrb, int ncb, int tile, int
 // MFMAs). Modes 1-3 accumulate in FP32 over the panel and subtract the
 // result from the FP64 entries.
 constexpr int kBigKcBf = 32;  // panel columns per LDS stage of the BF16 tiles (FP64 operands in registers)
-template <int MODE>
+template <int MODE, int TILE = kT>
 __host__ __device__ constexpr int big_lds_bytes() {
-    return MODE <= 1 ? 4 * 16 * kT * static_cast<int>(sizeof(double)) : bf_lds_bytes<MODE == 3, kBigKcBf>();
+    return MODE <= 1 ? 4 * 16 * TILE * static_cast<int>(sizeof(double)) : bf_lds_bytes<MODE == 3, kBigKcBf, TILE>();
 }
-template <int MODE>
+template <int MODE, int TILE = kT>
 __device__ __forceinline__ void big_tile(const LdltDev &d, const FrontLd &F, const double *Bm, int boff, int c0, int c1, int t0,
                          int t1, int tile, unsigned char *smem) {
     typedef typename std::conditional<MODE == 0, double, float>::type E;
     typedef SyrkMfma<E> M;
     const int f = F.f;
     int ib, jb;
-    super_block_tile((f - c0 + kT - 1) / kT, (c1 - c0 + kT - 1) / kT, tile, ib, jb);
-    const int i0 = c0 + ib * kT, j0 = c0 + jb * kT;
+    super_block_tile((f - c0 + TILE - 1) / TILE, (c1 - c0 + TILE - 1) / TILE, tile, ib, jb);
+    constexpr int kNB = TILE / 32, kW = TILE / 2;  // MFMA blocks of a wave each way, its rows
+    const int i0 = c0 + ib * TILE, j0 = c0 + jb * TILE;
     double *G = d.arena + F.fofs;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int wr = w >> 1, wc = w & 1;
-    const bool active = (i0 + wr * 64 + 63) >= (j0 + wc * 64);
-    typename M::acc_t acc[4][4];
+    const bool active = (i0 + wr * kW + kW - 1) >= (j0 + wc * kW);
+    typename M::acc_t acc[kNB][kNB];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < kNB; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = M::zero();
+        for (int b = 0; b < kNB; ++b) acc[a][b] = M::zero();
     if constexpr (MODE <= 1) {
-        if (active) tile_loop<E, true, 16, 2, double>(G, Bm, f, boff, i0, j0, f, c1, t0, t1, smem, acc);
-        else tile_loop<E, false, 16, 2, double>(G, Bm, f, boff, i0, j0, f, c1, t0, t1, smem, acc);
+        if (active) tile_loop<E, true, 16, 2, double, TILE>(G, Bm, f, boff, i0, j0, f, c1, t0, t1, smem, acc);
+        else tile_loop<E, false, 16, 2, double, TILE>(G, Bm, f, boff, i0, j0, f, c1, t0, t1, smem, acc);
     } else {
-        if (active) tile_loop_bf16<MODE == 3, true, kBigKcBf, double>(G, Bm, f, boff, i0, j0, f, c1, t0, t1, smem, acc);
-        else tile_loop_bf16<MODE == 3, false, kBigKcBf, double>(G, Bm, f, boff, i0, j0, f, c1, t0, t1, smem, acc);
+        if (active) tile_loop_bf16<MODE == 3, true, kBigKcBf, double, TILE>(G, Bm, f, boff, i0, j0, f, c1, t0, t1, smem, acc);
+        else tile_loop_bf16<MODE == 3, false, kBigKcBf, double, TILE>(G, Bm, f, boff, i0, j0, f, c1, t0, t1, smem, acc);
     }
     if (!active) return;
     double *junk = d.junk + threadIdx.x;
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        double *dst[4][4];
-        double old[4][4];
+    for (int m = 0; m < kNB; ++m) {
+        double *dst[kNB][4];
+        double old[kNB][4];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int j = j0 + wc * 64 + m * 16 + M::row(v, lane);
+            const int j = j0 + wc * kW + m * 16 + M::row(v, lane);
             double *col = G + static_cast<int64_t>(min(j, c1 - 1)) * f;
 #pragma unroll
-            for (int nn = 0; nn < 4; ++nn) {
-                const int i = i0 + wr * 64 + nn * 16 + (lane & 15);
+            for (int nn = 0; nn < kNB; ++nn) {
+                const int i = i0 + wr * kW + nn * 16 + (lane & 15);
                 dst[nn][v] = (i < f && j < c1 && i >= j) ? col + i : junk;
             }
         }
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
-            for (int nn = 0; nn < 4; ++nn) old[nn][v] = *dst[nn][v];
+            for (int nn = 0; nn < kNB; ++nn) old[nn][v] = *dst[nn][v];
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
-            for (int nn = 0; nn < 4; ++nn) *dst[nn][v] = old[nn][v] - acc[m][nn][v];
+            for (int nn = 0; nn < kNB; ++nn) *dst[nn][v] = old[nn][v] - acc[m][nn][v];
     }
 }
 
@@ -1110,9 +1111,10 @@ __device__ __forceinline__ XcdRange xcd_range(const BigPart &g, int nt) {
     return XcdRange{lo + (g.part >> 3), hi, per};
 }
 
+template <int TILE = kT>
 __device__ __forceinline__ int big_tiles(int f, int c0, int c1) {
     if (c1 <= c0) return 0;
-    const int nr = (f - c0 + kT - 1) / kT, nc = (c1 - c0 + kT - 1) / kT;
+    const int nr = (f - c0 + TILE - 1) / TILE, nc = (c1 - c0 + TILE - 1) / TILE;
     return nc * nr - nc * (nc - 1) / 2;
 }
 
@@ -1782,25 +1784,38 @@ __global__ __launch_bounds__(kLT) void k_big_panel(LdltDev d, const BigLd *__res
 }
 
 // The requested update and flush of every front, its tiles by stride over
-// its workgroups.
-template <int MODE>
+// its workgroups. The update (a group's 64 columns applied to the rest of
+// their outer block) has few tiles and little depth: 64 x 64 tiles while that
+// is at most two of them a workgroup (the chip's share of the front: more
+// read their operands too often): 15.9 us an update and flush against 22.4
+// with 128 x 128 tiles (fronts of up to 1700 rows), 36.7 against 42.5 (8216
+// rows). SMALL: the updates of fronts whose flush is
+// k_big_wide's, all in 64 x 64 tiles (LDS of three workgroups a CU, not
+// one): 22.1 against 23.8 us (23348 rows; 19 us its traffic).
+template <int MODE, bool SMALL>
 __global__ __launch_bounds__(kLT, 2) void k_big_update(LdltDev d, const BigLd *__restrict__ states,
                                                        const BigPart *__restrict__ grid) {
-    __shared__ __attribute__((aligned(16))) unsigned char smem[big_lds_bytes<MODE>()];
+    constexpr int kS = 64;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[SMALL ? big_lds_bytes<MODE, kS>() : big_lds_bytes<MODE>()];
     const BigPart g = grid[blockIdx.x];
     const BigLd B = states[g.front];
     if (B.prec != MODE) return;  // another precision's launch
     const FrontLd F = d.fronts[B.s];
     const double *W = d.work + F.wofs;
-    const int t1 = (B.u_p1 > B.u_p0) ? big_tiles(F.f, B.u_c0, B.u_c1) : 0;
-    // BF16 modes on planes: the flush is k_big_wide's
-    const bool wide = MODE >= 2 && d.xpl != nullptr;
-    const int t2 = (!wide && B.x_p1 > B.x_p0) ? big_tiles(F.f, B.x_c0, F.ne) : 0;
+    const bool u = B.u_p1 > B.u_p0;
+    int t1 = u ? big_tiles<kS>(F.f, B.u_c0, B.u_c1) : 0;
+    const bool small = SMALL || (MODE <= 1 && t1 <= 2 * g.parts);
+    if (!small) t1 = big_tiles(F.f, B.u_c0, B.u_c1);
+    const int t2 = (!SMALL && B.x_p1 > B.x_p0) ? big_tiles(F.f, B.x_c0, F.ne) : 0;
     const XcdRange xr = xcd_range(g, t1 + t2);
     for (int tile = xr.lo; tile < xr.hi; tile += xr.step) {
-        const bool u = tile < t1;
-        big_tile<MODE>(d, F, W, B.w_base, u ? B.u_c0 : B.x_c0, u ? B.u_c1 : F.ne, u ? B.u_p0 : B.x_p0,
-                    u ? B.u_p1 : B.x_p1, u ? tile : tile - t1, smem);
+        if ((SMALL || MODE <= 1) && small && tile < t1) {
+            big_tile<MODE, kS>(d, F, W, B.w_base, B.u_c0, B.u_c1, B.u_p0, B.u_p1, tile, smem);
+        } else if constexpr (!SMALL) {
+            const bool up = tile < t1;
+            big_tile<MODE>(d, F, W, B.w_base, up ? B.u_c0 : B.x_c0, up ? B.u_c1 : F.ne, up ? B.u_p0 : B.x_p0,
+                           up ? B.u_p1 : B.x_p1, up ? tile : tile - t1, smem);
+        }
         __syncthreads();
     }
 }
@@ -2059,10 +2074,16 @@ void launch_big_update(hipStream_t st, const LdltDev &d, const BigLd *states, co
                        const int32_t *nmode) {
     const dim3 nt(g.ntiles);
     if (d.xpl != nullptr && nmode[2] + nmode[3] > 0) k_big_pack<false><<<nt, kLT, 0, st>>>(d, states, g.tiles, 0, 0);
-    if (nmode[0] > 0) k_big_update<0><<<nt, kLT, 0, st>>>(d, states, g.tiles);
-    if (nmode[1] > 0) k_big_update<1><<<nt, kLT, 0, st>>>(d, states, g.tiles);
-    if (nmode[2] > 0) k_big_update<2><<<nt, kLT, 0, st>>>(d, states, g.tiles);
-    if (nmode[3] > 0) k_big_update<3><<<nt, kLT, 0, st>>>(d, states, g.tiles);
+    if (nmode[0] > 0) k_big_update<0, false><<<nt, kLT, 0, st>>>(d, states, g.tiles);
+    if (nmode[1] > 0) k_big_update<1, false><<<nt, kLT, 0, st>>>(d, states, g.tiles);
+    // BF16 modes on planes: the flush is k_big_wide's
+    if (d.xpl != nullptr) {
+        if (nmode[2] > 0) k_big_update<2, true><<<nt, kLT, 0, st>>>(d, states, g.tiles);
+        if (nmode[3] > 0) k_big_update<3, true><<<nt, kLT, 0, st>>>(d, states, g.tiles);
+    } else {
+        if (nmode[2] > 0) k_big_update<2, false><<<nt, kLT, 0, st>>>(d, states, g.tiles);
+        if (nmode[3] > 0) k_big_update<3, false><<<nt, kLT, 0, st>>>(d, states, g.tiles);
+    }
     if (d.xpl != nullptr) {
         if (nmode[2] > 0) k_big_wide<2, false><<<dim3(g.nwide), kWideThreads, 0, st>>>(d, states, g.wide, 0, 0);
         if (nmode[3] > 0) k_big_wide<3, false><<<dim3(g.nwide), kWideThreads, 0, st>>>(d, states, g.wide, 0, 0);

@@ -207,8 +207,8 @@ typedef __bf16 v8bf_t __attribute__((ext_vector_type(8)));
 template <int kKc>
 __host__ __device__ constexpr int bf_lds_ld() { return kKc + 8; }
 // LDS bytes: 2 stages x 2 operands (x 2 for hi / lo) of kT rows
-template <bool SPLIT, int kKc>
-__host__ __device__ constexpr int bf_lds_bytes() { return (SPLIT ? 2 : 1) * 2 * 2 * kT * bf_lds_ld<kKc>() * 2; }
+template <bool SPLIT, int kKc, int TILE = kT>
+__host__ __device__ constexpr int bf_lds_bytes() { return (SPLIT ? 2 : 1) * 2 * 2 * TILE * bf_lds_ld<kKc>() * 2; }
 
 __device__ __forceinline__ v4f_t mfma_bf16(v8bf_t a, v8bf_t b, v4f_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -221,22 +221,27 @@ __device__ __forceinline__ v4f_t mfma_bf16(v8bf_t a, v8bf_t b, v4f_t c) {
 // descriptor). Each thread loads one row's 8 consecutive k-values per group
 // (the 256 threads cover 128 rows x kKc columns of each operand), converts
 // them and writes one 16-byte LDS vector per operand (two with SPLIT).
-template <bool SPLIT, bool ACTIVE, int kKc, typename GE>
+// TILE: 128, or 64 as for tile_loop (four threads a row).
+template <bool SPLIT, bool ACTIVE, int kKc, typename GE, int TILE = kT>
 __device__ __forceinline__ void tile_loop_bf16(const GE *Ab, const GE *Bb, int ld, int boff, int i0, int j0, int f,
-                                               int j1, int t0, int t1, unsigned char *smem, v4f_t (&acc)[4][4]) {
+                                               int j1, int t0, int t1, unsigned char *smem,
+                                               v4f_t (&acc)[TILE / 32][TILE / 32]) {
     constexpr int kLd = bf_lds_ld<kKc>();
-    constexpr int kGroups = kKc / 16;  // 8-column groups per thread and operand
+    constexpr int kNB = TILE / 32, kW = TILE / 2;  // MFMA blocks of a wave each way, its rows
+    constexpr int kPer = kTileThreads / TILE;      // threads of a row
+    constexpr int kGroups = kKc / (8 * kPer);      // 8-column groups per thread and operand
+    static_assert(kGroups >= 1, "a thread takes at least a group");
     constexpr int kLoads = 8 * kGroups;
-    constexpr int kPlane = 2 * kT * kLd;  // one operand's two stages, in bf16 elements
+    constexpr int kPlane = 2 * TILE * kLd;  // one operand's two stages, in bf16 elements
     __bf16 *lds = reinterpret_cast<__bf16 *>(smem);
     // planes: A (hi), B (hi), then with SPLIT A (lo), B (lo); stage s of a
-    // plane starts at s * kT * kLd
+    // plane starts at s * TILE * kLd
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int w = tid >> 6;
     const int wr = w >> 1, wc = w & 1;
     constexpr uint32_t kOut = 0x80000000u;
-    const int rl = tid & (kT - 1), th = tid >> 7;
+    const int rl = tid % TILE, th = tid / TILE;
     const uint32_t colb = static_cast<uint32_t>(ld) * static_cast<uint32_t>(sizeof(GE));
     const uint32_t voa = (i0 + rl < f) ? static_cast<uint32_t>(i0 + rl) * sizeof(GE) : kOut;
     const uint32_t vob = (j0 + rl < j1) ? static_cast<uint32_t>(j0 + rl) * sizeof(GE) : kOut;
@@ -251,7 +256,7 @@ __device__ __forceinline__ void tile_loop_bf16(const GE *Ab, const GE *Bb, int l
         for (int e = 0; e < kGroups; ++e)
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                const uint32_t co = static_cast<uint32_t>(8 * (th + 2 * e) + u) * colb;
+                const uint32_t co = static_cast<uint32_t>(8 * (th + kPer * e) + u) * colb;
                 ra[8 * e + u] = buffer_load<GE>(sa, voa + co);
                 rb[8 * e + u] = buffer_load<GE>(sb, vob + co);
             }
@@ -259,7 +264,7 @@ __device__ __forceinline__ void tile_loop_bf16(const GE *Ab, const GE *Bb, int l
     auto sstore = [&](const Regs &ra, const Regs &rb, int stg) {
 #pragma unroll
         for (int e = 0; e < kGroups; ++e) {
-            const int o = stg * kT * kLd + rl * kLd + 8 * (th + 2 * e);
+            const int o = stg * TILE * kLd + rl * kLd + 8 * (th + kPer * e);
             v8bf_t ha, hb, la, lb;
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
@@ -282,40 +287,40 @@ __device__ __forceinline__ void tile_loop_bf16(const GE *Ab, const GE *Bb, int l
     };
     auto mfma_stage = [&](int stg) {
         if (!ACTIVE) return;
-        const __bf16 *As = lds + stg * kT * kLd;
-        const __bf16 *Bs = lds + kPlane + stg * kT * kLd;
+        const __bf16 *As = lds + stg * TILE * kLd;
+        const __bf16 *Bs = lds + kPlane + stg * TILE * kLd;
 #pragma unroll
         for (int kk = 0; kk < kKc; kk += 32) {
             const int ko = kk + 8 * (lane >> 4);
-            v8bf_t a[4], b[4];
+            v8bf_t a[kNB], b[kNB];
 #pragma unroll
-            for (int m = 0; m < 4; ++m)
-                a[m] = *reinterpret_cast<const v8bf_t *>(Bs + (wc * 64 + m * 16 + (lane & 15)) * kLd + ko);
+            for (int m = 0; m < kNB; ++m)
+                a[m] = *reinterpret_cast<const v8bf_t *>(Bs + (wc * kW + m * 16 + (lane & 15)) * kLd + ko);
 #pragma unroll
-            for (int nn = 0; nn < 4; ++nn)
-                b[nn] = *reinterpret_cast<const v8bf_t *>(As + (wr * 64 + nn * 16 + (lane & 15)) * kLd + ko);
+            for (int nn = 0; nn < kNB; ++nn)
+                b[nn] = *reinterpret_cast<const v8bf_t *>(As + (wr * kW + nn * 16 + (lane & 15)) * kLd + ko);
             if (SPLIT) {
-                v8bf_t al[4], bl[4];
+                v8bf_t al[kNB], bl[kNB];
 #pragma unroll
-                for (int m = 0; m < 4; ++m)
-                    al[m] = *reinterpret_cast<const v8bf_t *>(Bs + 2 * kPlane + (wc * 64 + m * 16 + (lane & 15)) * kLd + ko);
+                for (int m = 0; m < kNB; ++m)
+                    al[m] = *reinterpret_cast<const v8bf_t *>(Bs + 2 * kPlane + (wc * kW + m * 16 + (lane & 15)) * kLd + ko);
 #pragma unroll
-                for (int nn = 0; nn < 4; ++nn)
-                    bl[nn] = *reinterpret_cast<const v8bf_t *>(As + 2 * kPlane + (wr * 64 + nn * 16 + (lane & 15)) * kLd + ko);
+                for (int nn = 0; nn < kNB; ++nn)
+                    bl[nn] = *reinterpret_cast<const v8bf_t *>(As + 2 * kPlane + (wr * kW + nn * 16 + (lane & 15)) * kLd + ko);
                 // small terms first
 #pragma unroll
-                for (int m = 0; m < 4; ++m)
+                for (int m = 0; m < kNB; ++m)
 #pragma unroll
-                    for (int nn = 0; nn < 4; ++nn) {
+                    for (int nn = 0; nn < kNB; ++nn) {
                         acc[m][nn] = mfma_bf16(al[m], bl[nn], acc[m][nn]);
                         acc[m][nn] = mfma_bf16(al[m], b[nn], acc[m][nn]);
                         acc[m][nn] = mfma_bf16(a[m], bl[nn], acc[m][nn]);
                     }
             }
 #pragma unroll
-            for (int m = 0; m < 4; ++m)
+            for (int m = 0; m < kNB; ++m)
 #pragma unroll
-                for (int nn = 0; nn < 4; ++nn) acc[m][nn] = mfma_bf16(a[m], b[nn], acc[m][nn]);
+                for (int nn = 0; nn < kNB; ++nn) acc[m][nn] = mfma_bf16(a[m], b[nn], acc[m][nn]);
         }
     };
     // one register set: the loads of chunk c+1 are in flight during the
