@@ -2125,67 +2125,167 @@ void launch_big_finish(hipStream_t st, const LdltDev &d, const BigLd *states, in
 }
 
 // ---------------------------------------------------------------------------
-// Assembly of the level's fronts (f x f squares in the arena, lower
-// triangle). One workgroup per front column, rows from the diagonal down:
-// zero, original entries of the front's own pivot columns, then each
-// child's CB column in child order; the CB of a child is the trailing
-// (f_c - p_c) square of its own front.
-constexpr int kAsmChunkL = 2048;
-
-__device__ __forceinline__ int lbound(const int32_t *a, int lo, int hi, int32_t key) {
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (a[mid] < key) lo = mid + 1;
-        else hi = mid;
+// Rows of a level laid out on the host: the fronts' records, their row ids
+// (children's delayed rows in child order, then the symbolic rows) and
+// cleared tags; a workgroup per front.
+__global__ __launch_bounds__(kLT) void k_ldlt_rows(LdltDev d, LdltAsm A, const FrontLd *__restrict__ patch,
+                                                  const int32_t *__restrict__ ids) {
+    const int s = ids[blockIdx.x];
+    const FrontLd F = patch[blockIdx.x];
+    const int tid = threadIdx.x;
+    if (tid == 0) d.fronts[s] = F;
+    int32_t *rows = d.rows + F.rofs;
+    int dp = 0;
+    for (int c = A.child_ptr[s]; c < A.child_ptr[s + 1]; ++c) {
+        const FrontLd &K = d.fronts[A.child_idx[c]];
+        const int del = K.delayed;
+        const int32_t *crow = d.rows + K.rofs + K.p;
+        for (int t = tid; t < del; t += kLT) rows[dp + t] = crow[t];
+        dp += del;
     }
-    return lo;
+    const int32_t *sr = A.sym_rows + A.sym[s].rofs;
+    for (int t = tid; t < F.f - F.nd; t += kLT) rows[F.nd + t] = sr[t];
+    for (int t = tid; t < F.f; t += kLT) d.tags[F.rofs + t] = 0;
 }
 
-__global__ __launch_bounds__(kLT) void k_ldlt_assemble(LdltDev d, const AsmTask *__restrict__ tasks,
-                                                      const ChildCol *__restrict__ cc) {
-    __shared__ double buf[kAsmChunkL];
-    const AsmTask t = tasks[blockIdx.x];
-    const FrontLd F = d.fronts[t.s];
-    const int c = t.c;
-    const int f = F.f;
+void launch_ldlt_rows(hipStream_t st, const LdltDev &d, const LdltAsm &A, const FrontLd *patch, const int32_t *ids,
+                      int32_t nf) {
+    for (int64_t o = 0; o < nf; o += kMaxLaunchGroups)
+        k_ldlt_rows<<<dim3(static_cast<unsigned>(std::min<int64_t>(kMaxLaunchGroups, nf - o))), kLT, 0, st>>>(
+            d, A, patch + o, ids + o);
+}
+
+// Assembly of the level's fronts (f x f squares in the arena, lower
+// triangle), column by column, rows from the diagonal down: zero, original
+// entries of the front's own pivot columns, then each child's CB column in
+// child order; the CB of a child is the trailing (f_c - p_c) square of its
+// own front, its first rows and columns the delayed ones. Which child columns
+// meet in a column is known from the symbolic fronts (A.col_ptr), and where
+// their rows go too: delayed ones to the child's place among the front's
+// first nd rows, symbolic ones by their map, nd further. Fronts of up to
+// kAsmWaveRows rows take a wavefront per column (its LDS accesses happen in
+// its own order, no barriers), larger ones a workgroup per column in chunks
+// of kAsmChunkL rows. Bound by memory, and by the chain of loads to a
+// column's first entry: a column's loads go out four per thread at a time. 5.7 ms
+// for 23348 columns of a root and sixteen fronts of 8900 (20 GB; 6.4 ms with
+// per-column task lists made and uploaded by the host, 5 ms of host time).
+constexpr int kAsmChunkL = 2048;
+
+template <int NT>
+__device__ void assemble_column(const LdltDev &d, const LdltAsm &A, int s, const FrontLd &F, int64_t srow, int c,
+                                double *buf) {
+    constexpr int kChunk = NT == 64 ? kAsmWaveRows : kAsmChunkL;
+    constexpr int kCur = 16;  // children whose place in the column is kept
+    __shared__ int cur[kCur];
+    const int tid = NT == 64 ? threadIdx.x & 63 : threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int f = F.f, nd = F.nd;
     double *colp = d.arena + F.fofs + static_cast<int64_t>(c) * f;
-    const int tid = threadIdx.x;
     // the strict upper triangle is never read: left as it is
-    const int oc = c - F.nd;  // own pivot column index, when in [0, psym)
-    for (int r0 = c; r0 < f; r0 += kAsmChunkL) {
-        const int r1 = min(f, r0 + kAsmChunkL);
-        for (int r = r0 + tid; r < r1; r += kLT) buf[r - r0] = 0.0;
-        __syncthreads();
+    const int oc = c - nd;  // symbolic column (own pivot column when in [0, psym))
+    for (int r0 = c; r0 < f; r0 += kChunk) {
+        const int r1 = min(f, r0 + kChunk);
+        for (int r = r0 + tid; r < r1; r += NT) buf[r - r0] = 0.0;
+        wg_sync<NT>();
         if (oc >= 0 && oc < F.psym) {
             const int j = F.col0 + oc;
             const int k0 = d.pcol_ptr[j], k1 = d.pcol_ptr[j + 1];
-            for (int k = k0 + tid; k < k1; k += kLT) {
-                const int lr = F.nd + d.amap[k];
+            for (int k = k0 + tid; k < k1; k += NT) {
+                const int lr = nd + d.amap[k];
                 if (lr >= r0 && lr < r1) buf[lr - r0] += d.av[k];
             }
-            __syncthreads();
+            wg_sync<NT>();
         }
-        for (int e = t.cc0; e < t.cc1; ++e) {
-            const ChildCol ch = cc[e];
-            const FrontLd C = d.fronts[ch.ch];
-            const int q = C.f - C.p;
-            const int32_t *cm = d.cmap + C.cmofs;
-            const double *cbcol = d.arena + C.fofs + static_cast<int64_t>(C.p + ch.jj) * C.f + C.p;
-            const int lo = lbound(cm, ch.jj, q, r0);
-            const int hi = lbound(cm, lo, q, r1);
-            for (int ii = lo + tid; ii < hi; ii += kLT) buf[cm[ii] - r0] += cbcol[ii];
-            __syncthreads();
+        // column jj of child ch, its delayed rows at dp; e: its number here
+        const auto add = [&](int e, int ch, int jj, int dp) {
+            const FrontLd &C = d.fronts[ch];
+            const int cp = C.p, cf = C.f, q = cf - cp, del = C.delayed;
+            // (without a branch: some valid address where no map is read)
+            const int32_t *sm = q > del ? A.sym_cmap + A.sym_cmofs[ch] : A.sym_rows;
+            const double *cbcol = d.arena + C.fofs + static_cast<int64_t>(cp + jj) * cf + cp;
+            const auto place = [&](int ii) {
+                const int m = sm[max(ii - del, 0)];
+                return ii < del ? dp + ii : nd + m;
+            };
+            // first row at or past key: 64 places at a time
+            const auto lbound = [&](int lo, int hi, int key) {
+                while (lo < hi) {
+                    const int step = (hi - lo + 63) >> 6;
+                    const int i = min(lo + lane * step, hi - 1);
+                    const int below = __popcll(__ballot(lo + lane * step < hi && place(i) < key));
+                    if (below == 0) return lo;
+                    hi = min(hi, lo + below * step);
+                    lo += (below - 1) * step + 1;
+                }
+                return lo;
+            };
+            // the rows of the chunk: they follow the chunk before's, no more
+            // than the chunk has places
+            const int lo = r0 == c ? jj : (e < kCur ? cur[e] : lbound(jj, q, r0));
+            const int hi = r1 == f ? q : lbound(lo, min(q, lo + r1 - r0), r1);
+            for (int i0 = lo + tid; i0 < hi; i0 += 4 * NT) {
+                int x[4];
+                double v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int ii = min(i0 + u * NT, hi - 1);
+                    x[u] = place(ii);
+                    v[u] = cbcol[ii];
+                }
+                // (a column's places differ: read all, then write)
+                double b[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) b[u] = buf[x[u] - r0];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (i0 + u * NT < hi) buf[x[u] - r0] = b[u] + v[u];
+            }
+            wg_sync<NT>();
+            if (NT > 64 && e < kCur && tid == 0) cur[e] = hi;
+        };
+        if (oc >= 0) {
+            const int e0 = A.col_ptr[srow + oc], e1 = A.col_ptr[srow + oc + 1];
+            for (int e = e0; e < e1; ++e) {
+                const ChildCol k = A.cc[e];
+                add(e - e0, k.ch, k.jj + d.fronts[k.ch].delayed, 0);
+            }
+        } else {
+            // a delayed column: one child's
+            int dp = 0;
+            for (int e = A.child_ptr[s]; e < A.child_ptr[s + 1]; ++e) {
+                const int ch = A.child_idx[e];
+                const int del = d.fronts[ch].delayed;
+                if (c < dp + del) {
+                    add(0, ch, c - dp, dp);
+                    break;
+                }
+                dp += del;
+            }
         }
-        for (int r = r0 + tid; r < r1; r += kLT) colp[r] = buf[r - r0];
-        __syncthreads();
+        for (int r = r0 + tid; r < r1; r += NT) colp[r] = buf[r - r0];
+        wg_sync<NT>();
     }
 }
 
-void launch_ldlt_assemble(hipStream_t st, const LdltDev &d, const AsmTask *tasks, int64_t ntasks, const ChildCol *cc) {
-    if (ntasks <= 0) return;
-    for (int64_t o = 0; o < ntasks; o += kMaxLaunchGroups)
-        k_ldlt_assemble<<<dim3(static_cast<unsigned>(std::min(kMaxLaunchGroups, ntasks - o))), kLT, 0, st>>>(
-            d, tasks + o, cc);
+template <int NT>
+__global__ __launch_bounds__(kLT) void k_ldlt_assemble(LdltDev d, LdltAsm A, const AsmPart *__restrict__ parts) {
+    __shared__ double buf[NT == 64 ? kAsmWaveRows * (kLT / 64) : kAsmChunkL];
+    constexpr int kW = kLT / NT, kPer = kAsmCols / kW;  // columns of a workgroup, workgroups of a part
+    const AsmPart t = parts[blockIdx.x / kPer];
+    const FrontLd F = d.fronts[t.s];
+    const int w = threadIdx.x / NT;
+    const int c = t.c + kW * (blockIdx.x % kPer) + w;
+    if (c < F.f) assemble_column<NT>(d, A, t.s, F, A.sym[t.s].rofs, c, buf + w * kAsmWaveRows);
+}
+
+void launch_ldlt_assemble(hipStream_t st, const LdltDev &d, const LdltAsm &A, const AsmPart *parts, int64_t nwave,
+                          int64_t nwg) {
+    constexpr int64_t kMax = kMaxLaunchGroups / kAsmCols;
+    const auto grid = [=](int64_t n, int64_t per) { return dim3(static_cast<unsigned>(std::min<int64_t>(kMax, n) * per)); };
+    for (int64_t o = 0; o < nwave; o += kMax)
+        k_ldlt_assemble<64><<<grid(nwave - o, kAsmCols / (kLT / 64)), kLT, 0, st>>>(d, A, parts + o);
+    for (int64_t o = 0; o < nwg; o += kMax)
+        k_ldlt_assemble<kLT><<<grid(nwg - o, kAsmCols), kLT, 0, st>>>(d, A, parts + nwave + o);
 }
 
 // ---------------------------------------------------------------------------
@@ -2943,11 +3043,6 @@ __global__ __launch_bounds__(kLT) void k_ldlt_store(LdltDev d, const int32_t *__
     }
 }
 
-__global__ void k_front_patch(FrontLd *fronts, const FrontLd *patch, const int32_t *ids, int32_t np) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < np) fronts[ids[i]] = patch[i];
-}
-
 __global__ void k_front_gather(const FrontLd *fronts, FrontLd *out, const int32_t *ids, int32_t np) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < np) out[i] = fronts[ids[i]];
@@ -2956,11 +3051,6 @@ __global__ void k_front_gather(const FrontLd *fronts, FrontLd *out, const int32_
 void launch_front_gather(hipStream_t st, const FrontLd *fronts, FrontLd *out, const int32_t *ids, int32_t np) {
     if (np <= 0) return;
     k_front_gather<<<dim3((np + 127) / 128), 128, 0, st>>>(fronts, out, ids, np);
-}
-
-void launch_front_patch(hipStream_t st, FrontLd *fronts, const FrontLd *patch, const int32_t *ids, int32_t np) {
-    if (np <= 0) return;
-    k_front_patch<<<dim3((np + 127) / 128), 128, 0, st>>>(fronts, patch, ids, np);
 }
 
 void launch_ldlt_epilogue(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, int32_t n_inline) {

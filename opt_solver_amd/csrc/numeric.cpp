@@ -455,6 +455,36 @@ int plan_build(smfgpu_plan_s *P, const smfgpu_analysis_desc *D) {
     std::vector<ChildCol> cc;
     std::vector<int64_t> asm_first(nlev + 1, 0);
     std::vector<std::vector<ChildCol>> bucket;
+    if (!P->posdef) {
+        // LDL^T: the children's symbolic columns per symbolic row, in child
+        // order (a counting sort; delayed columns shift both by counts)
+        if (cmofs[ns] > INT32_MAX) return set_error(SMFGPU_ERR_ALLOC, "plan: too many child columns");
+        std::vector<int32_t> col_ptr(static_cast<size_t>(P->rows_total) + 1, 0);
+        for (int pass = 0; pass < 2; ++pass) {
+            for (int32_t s = 0; s < ns; ++s) {
+                const int32_t r0 = P->fronts[s].rofs;
+                for (int32_t c = D->child_ptr[s]; c < D->child_ptr[s + 1]; ++c) {
+                    const int32_t ch = D->child_idx[c];
+                    const int32_t *cm = cmap.data() + cmofs[ch];
+                    for (int jj = 0; jj < P->fronts[ch].q; ++jj) {
+                        int32_t &at = col_ptr[r0 + cm[jj] + (pass == 0 ? 1 : 0)];
+                        if (pass == 1) cc[at] = ChildCol{ch, jj};
+                        ++at;
+                    }
+                }
+            }
+            if (pass == 0) {
+                cc.resize(static_cast<size_t>(cmofs[ns]));
+                for (size_t r = 0; r + 1 < col_ptr.size(); ++r) col_ptr[r + 1] += col_ptr[r];
+            }
+        }
+        // the second pass moved every entry to the next one's start
+        for (size_t r = col_ptr.size() - 1; r > 0; --r) col_ptr[r] = col_ptr[r - 1];
+        col_ptr[0] = 0;
+        int rc;
+        if ((rc = P->d_col_ptr.upload(col_ptr)) || (rc = P->d_col_cc.upload(cc))) return rc;
+        cc.clear();
+    }
     if (P->posdef) {
     for (int32_t lv = 0; lv < nlev; ++lv) {
         asm_first[lv] = static_cast<int64_t>(tasks.size());
@@ -700,7 +730,7 @@ SMFGPU_API int smfgpu_plan_stats(smfgpu_plan_t P, double *out) {
              P->d_av_ref.bytes();
     // LDL^T fronts, factor store and staging
     bytes += P->d_fl.bytes() + P->d_arena.bytes() + P->d_work.bytes() + P->d_dinv.bytes() + P->d_fac.bytes() +
-             P->d_lrows.bytes() + P->d_lcmap.bytes() + P->d_flist.bytes() + P->d_ltags.bytes() +
+             P->d_lrows.bytes() + P->d_col_ptr.bytes() + P->d_col_cc.bytes() + P->d_flist.bytes() + P->d_ltags.bytes() +
              P->d_dkind.bytes() + P->d_stage.bytes() + P->d_child_ptr.bytes() + P->d_child_idx.bytes() +
              P->d_parent.bytes() + P->d_xpl.bytes() + P->d_level.bytes() + P->d_chain.bytes() +
              P->d_chain_ptr.bytes();

@@ -54,7 +54,6 @@ LdltDev ldlt_dev(smfgpu_plan_s *P) {
     d.work = P->d_work.p;
     d.dinv = P->d_dinv.p;
     d.dkind = P->d_dkind.p;
-    d.cmap = P->d_lcmap.p;
     d.pcol_ptr = P->d_pcol_ptr.p;
     d.amap = P->d_amap.p;
     d.av = P->d_av.p;
@@ -62,13 +61,17 @@ LdltDev ldlt_dev(smfgpu_plan_s *P) {
     return d;
 }
 
-// staging layout helper: appends a vector's bytes (8-aligned), returns offset
+// staging layout helper: room for a vector's bytes (8-aligned) behind `end`,
+// returns its offset
 template <class T>
-size_t stage(std::vector<unsigned char> &buf, const std::vector<T> &v) {
-    size_t off = (buf.size() + 7) & ~size_t{7};
-    buf.resize(off + v.size() * sizeof(T));
-    if (!v.empty()) std::memcpy(buf.data() + off, v.data(), v.size() * sizeof(T));
+size_t stage(size_t &end, const std::vector<T> &v) {
+    const size_t off = (end + 7) & ~size_t{7};
+    end = off + v.size() * sizeof(T);
     return off;
+}
+template <class T>
+void put(PinnedArr<unsigned char> &buf, size_t off, const std::vector<T> &v) {
+    if (!v.empty()) std::memcpy(buf.data() + off, v.data(), v.size() * sizeof(T));
 }
 
 // Peak of the square pool over a factorization without delays: each level
@@ -98,8 +101,6 @@ int ldlt_plan_build(smfgpu_plan_s *P, const smfgpu_analysis_desc *D) {
     P->sn_parent.assign(D->sn_parent, D->sn_parent + ns);
     P->child_ptr.assign(D->child_ptr, D->child_ptr + ns + 1);
     P->child_idx.assign(D->child_idx, D->child_idx + P->child_ptr[ns]);
-    P->front_row_ptr.assign(D->front_row_ptr, D->front_row_ptr + ns + 1);
-    P->front_row_idx.assign(D->front_row_idx, D->front_row_idx + P->front_row_ptr[ns]);
     int rc;
     if ((rc = P->fl.assign(ns, FrontLd{}))) return rc;
     // level front lists (all fronts) for the solves
@@ -252,10 +253,6 @@ static int ldlt_dev_levels(smfgpu_plan_s *P, int32_t lv0, double u, double eff_s
                         dinv_end = std::max(dinv_end, F.dofs + F.ne);
                     }
             }
-            P->rows_h.resize(rows_end);
-            HIP_OK(hipMemcpyAsync(P->rows_h.data() + P->rows_used, P->d_lrows.p + P->rows_used,
-                                  (rows_end - P->rows_used) * sizeof(int32_t), hipMemcpyDeviceToHost, st));
-            HIP_OK(hipStreamSynchronize(st));
             P->fac_used = fac_end;
             P->rows_used = rows_end;
             P->dinv_used = dinv_end;
@@ -701,15 +698,10 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
     P->sq_pool.reset();
     P->ldlt_prec.assign(P->nsup, 0);
     P->sel_cand.clear();
-    std::vector<int32_t> pos(n, -1);
-    std::vector<int32_t> cmap;
-    std::vector<AsmTask> tasks;
-    std::vector<ChildCol> cc;
-    std::vector<int32_t> colstart, colfill;
-    std::vector<int32_t> ids, small_list, blocked_list, big_list, ep_list, store_list;
+    std::vector<AsmPart> parts, wg_parts;
+    std::vector<int32_t> small_list, blocked_list, big_list, ep_list, store_list;
     std::vector<BigLd> big_h;
     std::vector<FrontLd> patch;
-    std::vector<int32_t> lrows;
     const int32_t nlev = static_cast<int32_t>(P->level_fronts.size());
     int rc;
     int32_t levels_done = 0, reduced = 0;
@@ -739,7 +731,6 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
     }
     int32_t cur = 0, stop_s = -1;
     int64_t work_prefix = 0, neg_prefix = 0;
-    P->rows_h.resize(0);
     P->dev_levels = 0;
     for (double &t : P->t_ldlt_host) t = 0.0;
     // levels of small fronts run on the device unless a limit needs the
@@ -759,18 +750,14 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
             dev_hold = lv;
         }
         const auto &fr = P->level_fronts[lv];
-        cmap.clear();
-        tasks.clear();
-        cc.clear();
-        ids.clear();
+        parts.clear();
+        wg_parts.clear();
         patch.clear();
-        lrows.clear();
         small_list.clear();
         blocked_list.clear();
         big_list.clear();
         ep_list.clear();
         store_list.clear();
-        const int64_t rows_start = P->rows_used;
         int64_t work_used = 0;
         for (int32_t s : fr) {
             const FrontDev &Sy = P->fronts[s];
@@ -819,60 +806,9 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
             else ep_list.push_back(s);
             P->rows_used += F.f;
             P->dinv_used += F.ne;
-            // rows: children's delayed columns in child order, then the
-            // symbolic rows
-            int32_t at = 0;
-            const size_t r0 = lrows.size();
-            for (int32_t c = P->child_ptr[s]; c < P->child_ptr[s + 1]; ++c) {
-                const FrontLd &C = P->fl[P->child_idx[c]];
-                const int32_t *cr = P->rows_h.data() + C.rofs;
-                for (int32_t t = 0; t < C.delayed; ++t) {
-                    lrows.push_back(cr[C.p + t]);
-                    pos[cr[C.p + t]] = at++;
-                }
-            }
-            for (int32_t t = P->front_row_ptr[s]; t < P->front_row_ptr[s + 1]; ++t) {
-                lrows.push_back(P->front_row_idx[t]);
-                pos[P->front_row_idx[t]] = at++;
-            }
-            // child maps (increasing: delayed rows come first in both) and
-            // the contributions per parent column
-            const size_t cm0 = cmap.size();
-            for (int32_t c = P->child_ptr[s]; c < P->child_ptr[s + 1]; ++c) {
-                const int32_t ch = P->child_idx[c];
-                FrontLd &C = P->fl[ch];
-                const int32_t q = C.f - C.p;
-                C.cmofs = static_cast<int64_t>(cmap.size());
-                const int32_t *cr = P->rows_h.data() + C.rofs + C.p;
-                int32_t prev = -1;
-                for (int32_t ii = 0; ii < q; ++ii) {
-                    const int32_t l = pos[cr[ii]];
-                    if (l < 0 || l <= prev)
-                        return set_error(SMFGPU_ERR_INVALID_ARG, "factor: child row outside its parent front");
-                    cmap.push_back(l);
-                    prev = l;
-                }
-                ids.push_back(ch);
-                patch.push_back(C);
-            }
-            // per parent column, its children's columns in child order (a
-            // counting sort over the maps just built)
-            colstart.assign(static_cast<size_t>(F.f) + 1, 0);
-            for (size_t e = cm0; e < cmap.size(); ++e) ++colstart[cmap[e] + 1];
-            for (int32_t c = 0; c < F.f; ++c) colstart[c + 1] += colstart[c];
-            const int32_t cc0 = static_cast<int32_t>(cc.size());
-            cc.resize(cc.size() + (cmap.size() - cm0));
-            colfill.assign(colstart.begin(), colstart.end() - 1);
-            for (int32_t c = P->child_ptr[s]; c < P->child_ptr[s + 1]; ++c) {
-                const int32_t ch = P->child_idx[c];
-                const FrontLd &C = P->fl[ch];
-                const int32_t q = C.f - C.p;
-                for (int32_t jj = 0; jj < q; ++jj) cc[cc0 + colfill[cmap[C.cmofs + jj]]++] = ChildCol{ch, jj};
-            }
-            for (int32_t c = 0; c < F.f; ++c) tasks.push_back(AsmTask{s, c, cc0 + colstart[c], cc0 + colstart[c + 1]});
-            for (size_t t = r0; t < lrows.size(); ++t) pos[lrows[t]] = -1;
+            auto &pt = F.f <= kAsmWaveRows ? parts : wg_parts;
+            for (int32_t c = 0; c < F.f; c += kAsmCols) pt.push_back(AsmPart{s, c});
             P->fl[s] = F;
-            ids.push_back(s);
             patch.push_back(F);
         }
         // the next front in order is in this level and its work crosses the
@@ -883,7 +819,6 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
             work_prefix += fwork[cur];
             break;
         }
-        if (cc.size() > static_cast<size_t>(INT32_MAX)) return set_error(SMFGPU_ERR_ALLOC, "factor: level too large");
         // capacities (arena contents stay: offsets are relative)
         if ((rc = ensure(P->d_arena, static_cast<size_t>(P->sq_pool.end), true, "front squares")) ||
             (rc = ensure(P->d_fac, static_cast<size_t>(P->fac_used), true, "factor store")) ||
@@ -891,41 +826,38 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
             (rc = ensure(P->d_ltags, static_cast<size_t>(P->rows_used), true, "pivot tags")) ||
             (rc = ensure(P->d_dinv, static_cast<size_t>(3 * P->dinv_used), true, "D^-1 table")) ||
             (rc = ensure(P->d_dkind, static_cast<size_t>(P->dinv_used), true, "D^-1 kinds")) ||
-            (rc = ensure(P->d_work, static_cast<size_t>(std::max<int64_t>(work_used, 1)), false, "panel workspace")) ||
-            (rc = ensure(P->d_lcmap, std::max<size_t>(cmap.size(), 1), false, "child maps")))
+            (rc = ensure(P->d_work, static_cast<size_t>(std::max<int64_t>(work_used, 1)), false, "panel workspace")))
             return rc;
-        // one staged upload: patch, ids, rows, cmap, tasks, contributions,
-        // front lists
-        P->h_stage.clear();
-        const size_t o_patch = stage(P->h_stage, patch);
-        const size_t o_ids = stage(P->h_stage, ids);
-        const size_t o_rows = stage(P->h_stage, lrows);
-        const size_t o_cmap = stage(P->h_stage, cmap);
-        const size_t o_tasks = stage(P->h_stage, tasks);
-        const size_t o_cc = stage(P->h_stage, cc);
-        const size_t o_small = stage(P->h_stage, small_list);
-        const size_t o_blk = stage(P->h_stage, blocked_list);
-        const size_t o_fr = stage(P->h_stage, fr);
         const int32_t n_inline = static_cast<int32_t>(ep_list.size());
         int32_t max_store_cols = 0;
         for (int32_t s : store_list) max_store_cols = std::max(max_store_cols, P->fl[s].ne);
         ep_list.insert(ep_list.end(), store_list.begin(), store_list.end());
-        const size_t o_ep = stage(P->h_stage, ep_list);
-        const size_t o_back = (P->h_stage.size() + 7) & ~size_t{7};
-        P->h_stage.resize(o_back + fr.size() * sizeof(FrontLd));
-        if ((rc = ensure(P->d_stage, P->h_stage.size(), false, "level staging"))) return rc;
+        // one staged upload: the fronts' records, the assembly's workgroups,
+        // the kernels' front lists (pinned: the level before has been read
+        // back, nothing of it is in flight)
+        const int64_t nwave = static_cast<int64_t>(parts.size());
+        parts.insert(parts.end(), wg_parts.begin(), wg_parts.end());
+        size_t end = 0;
+        const size_t o_patch = stage(end, patch), o_parts = stage(end, parts), o_small = stage(end, small_list),
+                     o_blk = stage(end, blocked_list), o_ep = stage(end, ep_list);
+        const size_t o_back = (end + 7) & ~size_t{7};
+        end = o_back + fr.size() * sizeof(FrontLd);
+        if ((rc = P->h_stage.reserve(end)) || (rc = ensure(P->d_stage, end, false, "level staging"))) return rc;
+        put(P->h_stage, o_patch, patch);
+        put(P->h_stage, o_parts, parts);
+        put(P->h_stage, o_small, small_list);
+        put(P->h_stage, o_blk, blocked_list);
+        put(P->h_stage, o_ep, ep_list);
         unsigned char *S = P->d_stage.p;
         HIP_OK(hipMemcpyAsync(S, P->h_stage.data(), o_back, hipMemcpyHostToDevice, st));
-        HIP_OK(hipMemcpyAsync(P->d_lrows.p + rows_start, S + o_rows, lrows.size() * sizeof(int32_t),
-                              hipMemcpyDeviceToDevice, st));
-        HIP_OK(hipMemsetAsync(P->d_ltags.p + rows_start, 0, lrows.size(), st));
-        if (!cmap.empty())
-            HIP_OK(hipMemcpyAsync(P->d_lcmap.p, S + o_cmap, cmap.size() * sizeof(int32_t), hipMemcpyDeviceToDevice, st));
-        launch_front_patch(st, P->d_fl.p, reinterpret_cast<const FrontLd *>(S + o_patch),
-                           reinterpret_cast<const int32_t *>(S + o_ids), static_cast<int32_t>(ids.size()));
         LdltDev d = ldlt_dev(P);
-        launch_ldlt_assemble(st, d, reinterpret_cast<const AsmTask *>(S + o_tasks), static_cast<int64_t>(tasks.size()),
-                             reinterpret_cast<const ChildCol *>(S + o_cc));
+        const LdltAsm A{P->d_fronts.p,    P->d_rows.p,      P->d_cmap.p,    P->d_cmofs.p,
+                        P->d_child_ptr.p, P->d_child_idx.p, P->d_col_ptr.p, P->d_col_cc.p};
+        const int32_t *d_fr = P->d_flist.p + P->lv_flist_ofs[lv];
+        launch_ldlt_rows(st, d, A, reinterpret_cast<const FrontLd *>(S + o_patch), d_fr,
+                         static_cast<int32_t>(fr.size()));
+        launch_ldlt_assemble(st, d, A, reinterpret_cast<const AsmPart *>(S + o_parts), nwave,
+                             static_cast<int64_t>(wg_parts.size()));
         // the children's squares are free for the launches that follow
         for (int32_t s : fr)
             for (int32_t c = P->child_ptr[s]; c < P->child_ptr[s + 1]; ++c) {
@@ -944,17 +876,15 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
                           static_cast<int32_t>(store_list.size()), max_store_cols);
         for (int32_t s : fr)
             if (P->fl[s].root) P->sq_pool.give(P->fl[s].fofs, static_cast<int64_t>(P->fl[s].f) * P->fl[s].f);
-        launch_front_gather(st, P->d_fl.p, reinterpret_cast<FrontLd *>(S + o_back),
-                            reinterpret_cast<const int32_t *>(S + o_fr), static_cast<int32_t>(fr.size()));
+        launch_front_gather(st, P->d_fl.p, reinterpret_cast<FrontLd *>(S + o_back), d_fr,
+                            static_cast<int32_t>(fr.size()));
         HIP_OK(hipGetLastError());
-        // read back the level's fronts and final row orders
-        std::vector<FrontLd> back(fr.size());
-        HIP_OK(hipMemcpyAsync(back.data(), S + o_back, back.size() * sizeof(FrontLd), hipMemcpyDeviceToHost, st));
-        P->rows_h.resize(P->rows_used);
-        HIP_OK(hipMemcpyAsync(P->rows_h.data() + rows_start, P->d_lrows.p + rows_start, lrows.size() * sizeof(int32_t),
+        // read back the level's fronts
+        HIP_OK(hipMemcpyAsync(P->h_stage.data() + o_back, S + o_back, fr.size() * sizeof(FrontLd),
                               hipMemcpyDeviceToHost, st));
         HIP_OK(hipStreamSynchronize(st));
-        for (size_t i = 0; i < fr.size(); ++i) P->fl[fr[i]] = back[i];
+        for (size_t i = 0; i < fr.size(); ++i)
+            std::memcpy(&P->fl[fr[i]], P->h_stage.data() + o_back + i * sizeof(FrontLd), sizeof(FrontLd));
         levels_done = lv + 1;
         if (!fdone.empty()) {
             for (int32_t s : fr) fdone[s] = 1;
@@ -1122,7 +1052,9 @@ int ldlt_export(smfgpu_plan_s *P, int64_t *sizes, int64_t *steps, double *fv, in
         sizes[3] = nt;
     }
     int64_t fo = 0, ro = 0, to = 0;
-    std::vector<int8_t> tg;
+    std::vector<int32_t> lrows(rows ? static_cast<size_t>(P->rows_used) : 0);
+    if (!lrows.empty())
+        HIP_OK(hipMemcpy(lrows.data(), P->d_lrows.p, lrows.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
     for (int32_t s = 0; s < ns; ++s) {
         const FrontLd &F = P->fl[s];
         if (steps) {
@@ -1134,7 +1066,7 @@ int ldlt_export(smfgpu_plan_s *P, int64_t *sizes, int64_t *steps, double *fv, in
         if (fv && F.pstore > 0)
             HIP_OK(hipMemcpy(fv + fo, P->d_fac.p + F.lofs, static_cast<size_t>(F.f) * F.pstore * sizeof(double),
                              hipMemcpyDeviceToHost));
-        if (rows) std::memcpy(rows + ro, P->rows_h.data() + F.rofs, static_cast<size_t>(F.f) * sizeof(int32_t));
+        if (rows) std::memcpy(rows + ro, lrows.data() + F.rofs, static_cast<size_t>(F.f) * sizeof(int32_t));
         if (tags && F.pstore > 0) HIP_OK(hipMemcpy(tags + to, P->d_ltags.p + F.rofs, F.pstore, hipMemcpyDeviceToHost));
         fo += static_cast<int64_t>(F.f) * F.pstore;
         ro += F.f;

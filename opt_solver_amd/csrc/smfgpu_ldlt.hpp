@@ -34,7 +34,6 @@ struct FrontLd {
     int64_t rofs;             // offset of the row ids / tags
     int64_t wofs;             // offset of the panel workspace W (blocked fronts)
     int64_t dofs;             // offset of the pivots' D^-1 entries
-    int64_t cmofs;            // offset of this front's CB-row map into its parent
 };
 
 struct LdltDev {
@@ -46,7 +45,6 @@ struct LdltDev {
     double *work;
     double *dinv;             // 3 per pivot
     int8_t *dkind;            // 1, 2, 0 per pivot
-    const int32_t *cmap;      // CB-row maps
     const int32_t *pcol_ptr;
     const int32_t *amap;      // per permuted entry: position among its front's symbolic rows
     const double *av;
@@ -165,7 +163,28 @@ void launch_ldlt_small(hipStream_t st, const LdltDev &d, const int32_t *flist, i
                        double small_pivot, const StaticPrm &S);
 void launch_ldlt_blocked(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, double u,
                          double eff_small, double small_pivot, int32_t nb, const StaticPrm &S);
-void launch_ldlt_assemble(hipStream_t st, const LdltDev &d, const AsmTask *tasks, int64_t ntasks, const ChildCol *cc);
+// Assembly of a level laid out on the host: its plan-time tables, and groups
+// of kAsmCols columns from c of front s, those of fronts of up to
+// kAsmWaveRows rows (a wavefront per column) before those of larger ones (a
+// workgroup per column).
+struct LdltAsm {
+    const FrontDev *sym;        // symbolic fronts
+    const int32_t *sym_rows;    // symbolic row ids
+    const int32_t *sym_cmap;    // as DevLevel
+    const int64_t *sym_cmofs;
+    const int32_t *child_ptr, *child_idx;
+    const int32_t *col_ptr;     // per symbolic row of every front: its children's symbolic columns there,
+    const ChildCol *cc;         // in child order
+};
+struct AsmPart {
+    int32_t s, c;
+};
+constexpr int32_t kAsmCols = 8, kAsmWaveRows = 1024;
+// records, row ids and cleared tags of the level's fronts (patch[i]: front ids[i])
+void launch_ldlt_rows(hipStream_t st, const LdltDev &d, const LdltAsm &A, const FrontLd *patch, const int32_t *ids,
+                      int32_t nf);
+void launch_ldlt_assemble(hipStream_t st, const LdltDev &d, const LdltAsm &A, const AsmPart *parts, int64_t nwave,
+                          int64_t nwg);
 // epilogue (pivot counts, D^-1) of the fronts in flist; it also stores the
 // factor columns of the first n_inline fronts, launch_ldlt_store those of
 // the rest (many workgroups per front)
@@ -176,7 +195,6 @@ void launch_ldlt_diag(hipStream_t st, const LdltDev &d, const int32_t *flist, in
 // the diagonal-only solve job: D from the stored columns, by division
 void launch_ldlt_diag_div(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, double *y, int32_t n,
                           int32_t nrhs);
-void launch_front_patch(hipStream_t st, FrontLd *fronts, const FrontLd *patch, const int32_t *ids, int32_t np);
 // flags of the LDL^T sweeps' items
 constexpr int32_t kItemAtomic = 1;  // backward chunk: several items add to its columns
 constexpr int32_t kItemTri = 2;     // a block's triangle, else a chunk

@@ -309,19 +309,20 @@ struct smfgpu_plan_s {
     std::set<smfgpu_factor_s *> issued;             // every factor handle of this plan not yet freed
     double max_abs = 0.0;
     // ---- LDL^T (posdef = 0) ----
-    std::vector<int32_t> sn_parent, child_ptr, child_idx, front_row_ptr, front_row_idx;
+    std::vector<int32_t> sn_parent, child_ptr, child_idx;
     std::vector<int32_t> amap_h;                    // host copy of the symbolic-position map
     PinnedArr<FrontLd> fl;                          // host mirror of the fronts of the last factorization
-    std::vector<int32_t> rows_h;                    // host mirror of the final row ids (rofs offsets)
     std::vector<int8_t> tags_h;
     DBuf<FrontLd> d_fl;
     DBuf<double> d_arena, d_work, d_dinv;
     DBuf<double> d_fac;                             // stored factor columns (f x ne per front)
     RangePool sq_pool;                              // live front squares in d_arena
-    DBuf<int32_t> d_lrows, d_lcmap, d_flist;
+    DBuf<int32_t> d_lrows, d_flist;
+    DBuf<int32_t> d_col_ptr;                        // per symbolic row: first of its children's columns in d_col_cc
+    DBuf<ChildCol> d_col_cc;
     DBuf<int8_t> d_ltags, d_dkind;
     DBuf<unsigned char> d_stage;                    // per-level upload staging
-    std::vector<unsigned char> h_stage;
+    PinnedArr<unsigned char> h_stage;
     int64_t fac_used = 0, rows_used = 0, dinv_used = 0;
     std::vector<int64_t> lv_flist_ofs;              // per level: offset of its fronts in d_flist (solve)
     std::vector<int32_t> lv_fsym_max;               // per level: largest symbolic front
