@@ -964,7 +964,7 @@ __global__ __launch_bounds__(kLThreads) void k_ldlt_bwd_step(LdltDev d, const So
 // its pivots' steps one after the other. So the next front's row ids and
 // first kChainCols columns are loaded during the front before, and accesses
 // of one wavefront to the same y need no wait between them. 121 fronts of
-// 24-31 rows: 111 us forward, 172 us backward (a launch a level: 640 and 590
+// 24-31 rows: 114 us forward, 227 us backward (a launch a level: 640 and 590
 // us).
 constexpr int kChainCols = 32;
 
@@ -1003,6 +1003,7 @@ __global__ __launch_bounds__(64) void k_ldlt_fwd_chain(LdltDev d, const int32_t 
             const double v = y_load(yr + static_cast<int64_t>(min(r, nr - 1)) * n + x.g);
             yv[r] = lane < c.p ? v : 0.0;
         }
+        double acc[4][NR] = {};  // the rows below: four sums, as they round less than one
         const ChainFront cnn = fronts[min(j + 2, j1 - 1)];
         xn.load(d, cn);
         const double *L = d.fac + c.lofs + min(lane, c.f - 1);
@@ -1019,14 +1020,18 @@ __global__ __launch_bounds__(64) void k_ldlt_fwd_chain(LdltDev d, const int32_t 
 #pragma unroll
             for (int u = 0; u < 16; ++u)
 #pragma unroll
-                for (int r = 0; r < NR; ++r) yv[r] -= t[u] * lane_value(yv[r], c0 + u);
+                for (int r = 0; r < NR; ++r) {
+                    const double v = lane_value(yv[r], c0 + u);
+                    yv[r] -= t[u] * v;
+                    acc[u & 3][r] -= t[u] * v;
+                }
         }
 #pragma unroll
         for (int r = 0; r < NR; ++r)
             if (r < nr) {
                 double *dst = yr + static_cast<int64_t>(r) * n + x.g;
                 if (lane < c.p) *dst = yv[r];
-                else if (lane < c.f) unsafeAtomicAdd(dst, yv[r]);
+                else if (lane < c.f) unsafeAtomicAdd(dst, (acc[0][r] + acc[1][r]) + (acc[2][r] + acc[3][r]));
             }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         c = cn;
@@ -1075,14 +1080,33 @@ __global__ __launch_bounds__(64) void k_ldlt_bwd_chain(LdltDev d, const int32_t 
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        // the rows below the pivots: four sums of their own, then taken off
+        // (off the right-hand side one by one, each would round at its size)
+        double acc[4][NR] = {};
 #pragma unroll
         for (int i0 = kChainRows - 16; i0 >= 0; i0 -= 16) {
-            if (i0 >= c.f) continue;
+            if (i0 >= c.f || i0 + 16 <= c.p) continue;
             double t[16];
 #pragma unroll
             for (int u = 0; u < 16; ++u) {
                 t[u] = T[lane][i0 + u];
-                if (lane >= c.p) t[u] = 0.0;
+                if (lane >= c.p || i0 + u < c.p) t[u] = 0.0;
+            }
+#pragma unroll
+            for (int u = 15; u >= 0; --u)
+#pragma unroll
+                for (int r = 0; r < NR; ++r) acc[u & 3][r] += t[u] * lane_value(yv[r], i0 + u);
+        }
+#pragma unroll
+        for (int r = 0; r < NR; ++r) yv[r] -= (acc[0][r] + acc[1][r]) + (acc[2][r] + acc[3][r]);
+#pragma unroll
+        for (int i0 = kChainRows - 16; i0 >= 0; i0 -= 16) {
+            if (i0 >= c.p) continue;
+            double t[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                t[u] = T[lane][i0 + u];
+                if (lane >= c.p || i0 + u >= c.p) t[u] = 0.0;
             }
 #pragma unroll
             for (int u = 15; u >= 0; --u)
