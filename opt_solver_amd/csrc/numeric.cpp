@@ -423,6 +423,10 @@ int plan_build(smfgpu_plan_s *P, const smfgpu_analysis_desc *D) {
     std::vector<int64_t> cmofs(ns + 1, 0);
     for (int32_t s = 0; s < ns; ++s) cmofs[s + 1] = cmofs[s] + P->fronts[s].q;
     std::vector<int32_t> cmap(cmofs[ns]);
+    // LDL^T: per symbolic row of every front, first the number, then the
+    // first of its children's symbolic columns there
+    std::vector<int32_t> col_ptr(P->posdef ? 0 : static_cast<size_t>(P->rows_total) + 1, 0);
+    if (!P->posdef && cmofs[ns] > INT32_MAX) return set_error(SMFGPU_ERR_ALLOC, "plan: too many child columns");
     for (int32_t s = 0; s < ns; ++s) {
         const FrontDev &F = P->fronts[s];
         const int32_t *fr = D->front_row_idx + F.rofs;
@@ -444,6 +448,7 @@ int plan_build(smfgpu_plan_s *P, const smfgpu_analysis_desc *D) {
                 const int32_t r = pos[cr[ii]];
                 if (r < 0 || r <= prev) return set_error(SMFGPU_ERR_INVALID_ARG, "plan: child row outside parent front");
                 cmap[cmofs[ch] + ii] = r;
+                if (!P->posdef) ++col_ptr[F.rofs + r + 1];
                 prev = r;
             }
         }
@@ -458,27 +463,16 @@ int plan_build(smfgpu_plan_s *P, const smfgpu_analysis_desc *D) {
     if (!P->posdef) {
         // LDL^T: the children's symbolic columns per symbolic row, in child
         // order (a counting sort; delayed columns shift both by counts)
-        if (cmofs[ns] > INT32_MAX) return set_error(SMFGPU_ERR_ALLOC, "plan: too many child columns");
-        std::vector<int32_t> col_ptr(static_cast<size_t>(P->rows_total) + 1, 0);
-        for (int pass = 0; pass < 2; ++pass) {
-            for (int32_t s = 0; s < ns; ++s) {
-                const int32_t r0 = P->fronts[s].rofs;
-                for (int32_t c = D->child_ptr[s]; c < D->child_ptr[s + 1]; ++c) {
-                    const int32_t ch = D->child_idx[c];
-                    const int32_t *cm = cmap.data() + cmofs[ch];
-                    for (int jj = 0; jj < P->fronts[ch].q; ++jj) {
-                        int32_t &at = col_ptr[r0 + cm[jj] + (pass == 0 ? 1 : 0)];
-                        if (pass == 1) cc[at] = ChildCol{ch, jj};
-                        ++at;
-                    }
-                }
+        cc.resize(static_cast<size_t>(cmofs[ns]));
+        for (size_t r = 0; r + 1 < col_ptr.size(); ++r) col_ptr[r + 1] += col_ptr[r];
+        for (int32_t s = 0; s < ns; ++s)
+            for (int32_t c = D->child_ptr[s]; c < D->child_ptr[s + 1]; ++c) {
+                const int32_t ch = D->child_idx[c];
+                const int32_t *cm = cmap.data() + cmofs[ch];
+                int32_t *at = col_ptr.data() + P->fronts[s].rofs;
+                for (int jj = 0; jj < P->fronts[ch].q; ++jj) cc[at[cm[jj]]++] = ChildCol{ch, jj};
             }
-            if (pass == 0) {
-                cc.resize(static_cast<size_t>(cmofs[ns]));
-                for (size_t r = 0; r + 1 < col_ptr.size(); ++r) col_ptr[r + 1] += col_ptr[r];
-            }
-        }
-        // the second pass moved every entry to the next one's start
+        // every entry has moved to the next one's start
         for (size_t r = col_ptr.size() - 1; r > 0; --r) col_ptr[r] = col_ptr[r - 1];
         col_ptr[0] = 0;
         int rc;
