@@ -423,8 +423,10 @@ SMFGPU_API int smfgpu_factor_solve(smfgpu_plan_t plan, const double *values, int
  * workgroups share a CU. */
 #define SMFGPU_TUNE_ASM_CHUNK 9
 /* SMFGPU_TUNE_LDLT_DEVICE_WAVE: 1 (default) factors the device levels'
- * fronts of at most 48 rows with one wavefront each (many fronts per CU),
- * 0 gives every front of a device level a 256-thread workgroup. */
+ * fronts of at most 64 rows with a row per lane (one wavefront each, up to 48
+ * rows, on levels of more than 512 fronts; four on smaller levels, where a
+ * band of levels whose fronts form chains is one launch), 0 gives every
+ * front of a device level a 256-thread workgroup, a launch per level. */
 #define SMFGPU_TUNE_LDLT_DEVICE_WAVE 10
 /* SMFGPU_TUNE_SOLVE_PERSISTENT: 1 runs each SPD sweep as one launch, a
  * workgroup per item taking its item by ticket in step order and waiting

@@ -33,7 +33,7 @@ TUNED_DIR = os.path.join(HERE, "tuned")
 
 # (bucket, knob name, candidate values, library default, workloads it acts on)
 KNOBS = [
-    ("LDL^T device levels, fronts of <= 48 rows: one wavefront (1) or one workgroup (0) per front",
+    ("LDL^T device levels: a row per lane and bands in one launch (1) or workgroup reductions, a launch per level (0)",
      "LDLT_DEVICE_WAVE", [1, 0], 1, ("batch", "kkt")),
     ("LDL^T device levels: largest symbolic front laid out on the device (rows)",
      "LDLT_DEVICE_FRONTS", [95, 64, 48], 95, ("batch", "kkt")),

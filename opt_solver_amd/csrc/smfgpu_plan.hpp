@@ -337,7 +337,7 @@ struct smfgpu_plan_s {
     std::vector<int64_t> lv_room;                   // prefix over levels of the device-level room estimates (4 per level)
     int32_t dev_fmax = kDevFrontMax;                // largest realized front of a device level (0: host layout only)
     int32_t dev_levels = 0;                         // levels the last factorization ran on the device
-    int32_t dev_wave = 1;                           // device levels: one wavefront per front of <= 48 rows
+    int32_t dev_wave = 1;                           // device levels: a row per lane up to 64 rows, bands in one launch
     double t_ldlt_host[4] = {0, 0, 0, 0};           // s: device levels (run), their read-back, statistics, solve lists
     DBuf<int32_t> d_child_ptr, d_child_idx, d_parent;
     DBuf<unsigned long long> d_dctr;                // device-level counters
