@@ -140,3 +140,31 @@ def test_chain_bands(s):
     for nr in (1, 2, 3, 16, 18):
         xs = fac.solve(B[:, :nr] if nr > 1 else B[:, 0]).reshape(n, nr)
         assert np.abs(xs - X[:, :nr]).max() < 1e-13 * max(n, 10), nr
+
+
+@pytest.mark.parametrize("delayed", [False, True])
+@pytest.mark.parametrize("p,q", [(1, 96), (3, 1021), (3, 1024), (3, 1025), (2, 2047), (3, 2049), (70, 960)])
+def test_indefinite_assembly_edges(p, q, delayed):
+    """A root of q rows (p more with the child's delayed columns) assembled
+    from one child: a wavefront per column up to 1024 rows, a workgroup with
+    2048-row chunks above, groups of 8 columns, and the root's updates in 64 x
+    64 tiles. delayed: the child's block is zero, so all its columns reach the
+    root; the matrix is then [0 B; B^T D] with D = 2 n I, B uniform in [-1,
+    1], of condition number about 12 n, solved to well below 1e-13 n."""
+    n = p + q
+    print("case assembly", p, q, delayed, flush=True)
+    rng = np.random.default_rng([p, q, 3])
+    M = rng.uniform(-1, 1, (n, n))
+    M = M + M.T
+    d = np.full(n, 2.0 * n) if delayed else 2.0 * n * np.where(np.arange(n) % 3 == 0, -1.0, 1.0)
+    M += np.diag(d)
+    if delayed:
+        M[:p, :p] = 0.0
+        M[p:, p:] = np.diag(d[p:])
+    A, arrays = dense_front_problem(M, p)
+    fac = Plan(arrays, posdef=False).factor(A[3])
+    assert fac.status == 0
+    neg = p if delayed else int((d < 0).sum())
+    assert fac.inertia == (n - neg, neg, 0)
+    x = rng.uniform(-1, 1, n)
+    assert np.abs(fac.solve(M @ x) - x).max() < 1e-13 * max(n, 10)
