@@ -626,12 +626,15 @@ __device__ __forceinline__ void load_unit_triangle(const double *L, int f, int c
 }
 
 // One wavefront's substitution with the unit triangle T (zero on and above
-// the diagonal and past the block): lane l holds y_l. Bound by the 64
-// dependent steps; T's values are read 16 steps ahead of the chain, the
-// solved value is broadcast through scalar registers (through LDS a step
-// took about 150 cycles, here about 30).
-__device__ __forceinline__ double unit_forward(const double (*T)[kLB + 1], double yv, int nc) {
+// the diagonal and past the block): lane l holds y_l (0 past the block). Bound
+// by the 64 dependent steps; T's values are read 16 steps ahead of the chain,
+// the solved value is broadcast through scalar registers (through LDS a step
+// took about 150 cycles, here about 30). T's zeros times a value that is not
+// finite would be NaN in the lanes solved before it: such a block is solved
+// again with a test on the lane.
+__device__ __forceinline__ double unit_forward(const double (*T)[kLB + 1], double y0, int nc) {
     const int l = threadIdx.x & 63;
+    double yv = y0;
 #pragma unroll
     for (int c0 = 0; c0 < kLB; c0 += 16) {
         if (c0 >= nc) break;
@@ -641,10 +644,18 @@ __device__ __forceinline__ double unit_forward(const double (*T)[kLB + 1], doubl
 #pragma unroll
         for (int u = 0; u < 16; ++u) yv -= t[u] * lane_value(yv, c0 + u);
     }
+    if (__ballot(!isfinite(yv)) != 0) {
+        yv = y0;
+        for (int c = 0; c < min(nc, kLB); ++c) {
+            const double v = lane_value(yv, c);
+            if (l > c && l < nc) yv -= T[c][l] * v;
+        }
+    }
     return yv;
 }
-__device__ __forceinline__ double unit_backward(const double (*T)[kLB + 1], double yv, int nc) {
+__device__ __forceinline__ double unit_backward(const double (*T)[kLB + 1], double y0, int nc) {
     const int l = threadIdx.x & 63;
+    double yv = y0;
 #pragma unroll
     for (int c0 = kLB - 16; c0 >= 0; c0 -= 16) {
         if (c0 >= nc) continue;
@@ -653,6 +664,13 @@ __device__ __forceinline__ double unit_backward(const double (*T)[kLB + 1], doub
         for (int u = 0; u < 16; ++u) t[u] = T[l][c0 + u];
 #pragma unroll
         for (int u = 15; u >= 0; --u) yv -= t[u] * lane_value(yv, c0 + u);
+    }
+    if (__ballot(!isfinite(yv)) != 0) {
+        yv = y0;
+        for (int c = min(nc, kLB) - 1; c > 0; --c) {
+            const double v = lane_value(yv, c);
+            if (l < c) yv -= T[l][c] * v;
+        }
     }
     return yv;
 }
@@ -1026,6 +1044,32 @@ __global__ __launch_bounds__(64) void k_ldlt_fwd_chain(LdltDev d, const int32_t 
                     acc[u & 3][r] -= t[u] * v;
                 }
         }
+        bool finite = true;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) finite = finite && isfinite(yv[r]);
+        if (__ballot(!finite) != 0) {
+            // as in unit_forward: again, with a test on the lane
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                const double v = y_load(yr + static_cast<int64_t>(min(r, nr - 1)) * n + x.g);
+                yv[r] = lane < c.p ? v : 0.0;
+                for (int k = 0; k < 4; ++k) acc[k][r] = 0.0;
+            }
+            for (int c0 = 0; c0 < c.p; c0 += 4)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (c0 + u >= c.p) break;
+                    const double t = L[static_cast<int64_t>(c0 + u) * c.f];
+#pragma unroll
+                    for (int r = 0; r < NR; ++r) {
+                        const double v = lane_value(yv[r], c0 + u);
+                        if (lane > c0 + u) {
+                            yv[r] -= t * v;
+                            acc[u][r] -= t * v;
+                        }
+                    }
+                }
+        }
 #pragma unroll
         for (int r = 0; r < NR; ++r)
             if (r < nr) {
@@ -1112,6 +1156,33 @@ __global__ __launch_bounds__(64) void k_ldlt_bwd_chain(LdltDev d, const int32_t 
             for (int u = 15; u >= 0; --u)
 #pragma unroll
                 for (int r = 0; r < NR; ++r) yv[r] -= t[u] * lane_value(yv[r], i0 + u);
+        }
+        bool finite = true;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) finite = finite && (isfinite(yv[r]) || lane >= c.p);
+        if (__ballot(!finite) != 0) {
+            // as in unit_backward: again, with a test on the lane
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                yv[r] = y_load(yr + static_cast<int64_t>(min(r, nr - 1)) * n + x.g);
+                for (int k = 0; k < 4; ++k) acc[k][r] = 0.0;
+            }
+            const int lc = min(lane, c.p - 1);
+            for (int i0 = (c.f - 1) / 4 * 4; i0 + 4 > c.p; i0 -= 4)
+#pragma unroll
+                for (int u = 3; u >= 0; --u) {
+                    if (i0 + u >= c.f || i0 + u < c.p) continue;
+#pragma unroll
+                    for (int r = 0; r < NR; ++r) acc[u][r] += T[lc][i0 + u] * lane_value(yv[r], i0 + u);
+                }
+#pragma unroll
+            for (int r = 0; r < NR; ++r) yv[r] -= (acc[0][r] + acc[1][r]) + (acc[2][r] + acc[3][r]);
+            for (int i = c.p - 1; i > 0; --i)
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    const double v = lane_value(yv[r], i);
+                    if (lane < i) yv[r] -= T[lane][i] * v;
+                }
         }
 #pragma unroll
         for (int r = 0; r < NR; ++r)
