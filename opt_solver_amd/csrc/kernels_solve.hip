@@ -76,6 +76,12 @@ struct Acc {
             if ((threadIdx.x & 48) == 0) part[col][r] = q;
         }
     }
+    __device__ __forceinline__ bool finite() const {
+        bool f = true;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) f = f && isfinite(a[r]);
+        return f;
+    }
 };
 template <>
 struct Acc<16> {
@@ -88,6 +94,9 @@ struct Acc<16> {
         const int lk = (threadIdx.x & 63) >> 4;
 #pragma unroll
         for (int v = 0; v < 4; ++v) part[col][4 * v + lk] = a[v];
+    }
+    __device__ __forceinline__ bool finite() const {
+        return isfinite(a[0]) && isfinite(a[1]) && isfinite(a[2]) && isfinite(a[3]);
     }
 };
 
@@ -141,8 +150,11 @@ __device__ __forceinline__ void put_diag(double (*Dg)[kSD + 1], const double (&v
 }
 
 // part[h][i][r] = sum over half h of k of D(i, k) v[k][r], D(i, k) =
-// TR ? Dg[k][i] : Dg[i][k], 64 x 64; wave w: 16 of i (w % 4), half w / 4
-template <int NR, bool TR>
+// TR ? Dg[k][i] : Dg[i][k], 64 x 64; wave w: 16 of i (w % 4), half w / 4.
+// TRI: a diagonal block, D zero for k > i (TR) or k < i. Its zeros times a
+// value that is not finite would be NaN in entries that do not depend on it:
+// a wavefront that meets one takes those sums again over the triangle only.
+template <int NR, bool TR, bool TRI>
 __device__ __forceinline__ void block_times(const double (*Dg)[kSD + 1], const double (*v)[NR],
                                             double (*part)[kSD][NR]) {
     const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4, w = threadIdx.x >> 6;
@@ -154,6 +166,16 @@ __device__ __forceinline__ void block_times(const double (*Dg)[kSD + 1], const d
         acc.add(v, k, TR ? Dg[k][i] : Dg[i][k]);
     }
     acc.put(part[h], i);
+    if (TRI && __ballot(!acc.finite()) != 0) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        for (int r = lk; r < NR; r += 4) {
+            if (isfinite(part[h][i][r])) continue;
+            double s = 0.0;
+            for (int k = 32 * h; k < 32 * h + 32; ++k)
+                if (TR ? k <= i : k >= i) s += (TR ? Dg[k][i] : Dg[i][k]) * v[k][r];
+            part[h][i][r] = s;
+        }
+    }
 }
 
 // Forward update of rows [lo, hi): y[row] -= sum_{t < kb} L[row][k + t] zs[t]
@@ -263,18 +285,18 @@ __device__ void fwd_item(const DevPtrs &d, const SolveItem &it, double *__restri
     }
     put_diag(Dg, Ra, rl, g, na);
     __syncthreads();
-    block_times<NR, true>(Dg, yb, part);
+    block_times<NR, true, true>(Dg, yb, part);
     __syncthreads();
     add_halves<NR, false>(zs, part, na);
     if (nb > 0) put_block(Dg, Rb, rl, g);
     __syncthreads();
     if (nb > 0) {
-        block_times<NR, false>(Dg, zs, part);
+        block_times<NR, false, false>(Dg, zs, part);
         __syncthreads();
         add_halves<NR, true>(yb + kSD, part, nb);
         put_diag(Dg, Rc, rl, g, nb);
         __syncthreads();
-        block_times<NR, true>(Dg, yb + kSD, part);
+        block_times<NR, true, true>(Dg, yb + kSD, part);
         __syncthreads();
         add_halves<NR, false>(zs + kSD, part, nb);
         __syncthreads();
@@ -430,18 +452,18 @@ __device__ void bwd_item(const DevPtrs &d, const SolveItem &it, double *__restri
         tri_load<0>(Ra, Lb, f, it.tk, it.tkb, rl, g);
         put_diag(Dg, Rc, rl, g, nb);
         __syncthreads();
-        block_times<NR, false>(Dg, v + kSD, part);
+        block_times<NR, false, true>(Dg, v + kSD, part);
         __syncthreads();
         add_halves<NR, false>(xo + kSD, part, nb);
         put_block(Dg, Rb, rl, g);  // Dg[t][c] = L_ba[t][c]
         __syncthreads();
-        block_times<NR, true>(Dg, xo + kSD, part);
+        block_times<NR, true, false>(Dg, xo + kSD, part);
         __syncthreads();
         add_halves<NR, true>(v, part, na);
     }
     put_diag(Dg, Ra, rl, g, na);
     __syncthreads();
-    block_times<NR, false>(Dg, v, part);
+    block_times<NR, false, true>(Dg, v, part);
     __syncthreads();
     add_halves<NR, false>(xo, part, na);
     __syncthreads();

@@ -41,7 +41,7 @@ def substitute(e, y, unit, backward):
 
 def check(fac, perm, unit, at, seed):
     n = perm.size
-    assert fac.status == 0 and fac.info.two_by_two_pivots == 0
+    assert fac.status == 0 and fac.info.two_by_two_pivots == 0  # entry by entry: 1x1 pivots
     e = fac.export()
     inv = np.empty(n, np.int64)
     inv[perm] = np.arange(n)
@@ -90,3 +90,15 @@ def test_indefinite_chains(s):
     for at in (3 * s + s // 2, 9 * s + s - 2, n - 2):
         print("case chains", s, at, flush=True)
         check(fac, an.arrays()["perm"], True, at, s)
+
+
+@pytest.mark.parametrize("p,q", [(20, 30), (64, 600), (100, 40), (128, 30), (200, 60)])
+def test_cholesky_dense(p, q):
+    """Pivots inside the 64-pivot diagonal blocks that are applied as stored
+    inverses, on the vector unit (up to four right-hand sides) and on MFMA;
+    condition number about 1."""
+    A, arrays = dense_front_problem(dominant(p + q, 2, True), p)
+    fac = Plan(arrays, posdef=True).factor(A[3])
+    for at in (p // 2, p - 3):
+        print("case", p, q, at, flush=True)
+        check(fac, arrays["perm"], False, at, p)
