@@ -1246,8 +1246,9 @@ __device__ void big_stall_wg(const LdltDev &d, BigLd &B, int32_t nb, RedScratch 
     FV A{d.arena + Fd.fofs, f, f};
     const int tid = threadIdx.x;
     const int k = B.k, pl = B.pl;
-    const int live = B.live;
-    if (k != B.k_paired) {
+    const int live = B.live, k_paired = B.k_paired;
+    __syncthreads();  // every thread has read the state before thread 0 changes it
+    if (k != k_paired) {
         const int np = partner_pairs_wg(A, k, pl, ne, nb, rows, order, rs);
         if (np > 0) {
             place_rows_wg(A, k, ne, np, order, rows, rs);
@@ -1288,6 +1289,7 @@ __global__ __launch_bounds__(kLT) void k_big_region(LdltDev d, BigLd *__restrict
     __shared__ double dd[64], invd[64];
     __shared__ RedScratch rs;
     __shared__ int32_t order[128];
+    // (every wavefront has read it when big_stall_wg changes it)
     if (states[blockIdx.x].pass == 0 && states[blockIdx.x].stalled) {
         big_stall_wg(d, states[blockIdx.x], nb, rs, order);
         __syncthreads();

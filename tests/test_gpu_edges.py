@@ -168,3 +168,33 @@ def test_indefinite_assembly_edges(p, q, delayed):
     assert fac.inertia == (n - neg, neg, 0)
     x = rng.uniform(-1, 1, n)
     assert np.abs(fac.solve(M @ x) - x).max() < 1e-13 * max(n, 10)
+
+
+@pytest.mark.parametrize("p,q", [(17, 100), (18, 78), (20, 201), (32, 300)])
+def test_panel_stalls_with_no_live_column_left(oracle_lib, p, q):
+    """A first front of p eligible columns, none of which is an acceptable
+    pivot (entries of 1 between them, of 1e6 below them): its first panel
+    stalls, pulls the partners from behind it, stalls at the same position and
+    is rotated away, and what was pulled stalls there again as the last live
+    columns, with nothing to exchange. Counters, delays and inertia are the
+    oracle's."""
+    n = p + q
+    print("case last live columns", p, q, flush=True)
+    rng = np.random.default_rng([p, q, 5])
+    M = np.zeros((n, n))
+    for j in range(16, p):
+        M[j, j - 16] = 1.0
+    M[p:, :p] = 1e6 * rng.uniform(0.5, 1, (q, p))
+    M = M + M.T
+    M[p:, p:] = np.diag(2e6 * n * np.where(np.arange(q) % 3 == 0, -1.0, 1.0))
+    A, arrays = dense_front_problem(M, p)
+    fac = Plan(arrays, posdef=False).factor(A[3])
+    orc = oracle_lib.Factor(arrays, A[3], posdef=False)
+    front = oracle_lib.ldlt_front(M, p)[3]
+    assert (front["stalls"], front["pulls"], front["rotated"]) == (3, min(p - 16, 8), p), front  # 16 / 2 pairs at most
+    assert fac.status == orc.status == 0 and fac.inertia == orc.inertia
+    assert tuple(fac.stall_stats()[0]) == (front["stalls"], front["pulls"], front["rotated"], front["searches"])
+    assert fac.info.delayed_pivots == orc.delayed == p
+    x = rng.uniform(-1, 1, n)
+    eta, _ = oracle_lib.backward_error(A, M @ x, fac.solve(M @ x))
+    assert eta < 1e-13  # n eps
