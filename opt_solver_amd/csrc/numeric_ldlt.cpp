@@ -359,7 +359,7 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
     if (P->ldlt_planes != 0 && (nmode[2] + nmode[3] > 0 || (collect && !sf.empty()))) {
         int64_t planes = 0;
         for (int32_t s : big)
-            planes = std::max(planes, 4 * (P->fl[s].wofs + static_cast<int64_t>(P->fl[s].f) * big_work(P->fl[s].ne)));
+            planes = std::max(planes, 4 * (P->fl[s].wofs + work_room(P->fl[s].f, big_work(P->fl[s].ne))));
         if ((rc = ensure(P->d_xpl, static_cast<size_t>(planes), false, "update planes"))) return rc;
         d.xpl = P->d_xpl.p;
     }
@@ -790,11 +790,11 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
             const bool stat = front_static_value(spr, F.root, F.nd, F.psym) > 0.0;
             if (F.f >= P->ldlt_big_min && F.ne > 0 && !stat) {
                 F.wofs = work_used;
-                work_used += static_cast<int64_t>(F.f) * big_work(F.ne);
+                work_used += work_room(F.f, big_work(F.ne));
                 big_list.push_back(s);
             } else if (F.f >= kBlockedMinFront) {
                 F.wofs = work_used;
-                work_used += static_cast<int64_t>(F.f) * nb;
+                work_used += work_room(F.f, nb);
                 blocked_list.push_back(s);
             } else {
                 small_list.push_back(s);

@@ -72,9 +72,18 @@ constexpr int32_t kBigOuter = 512;
 constexpr int32_t kBigOuterMax = 1024;
 // W columns of a front with ne eligible columns: an outer block's pivots
 // (L*D chunks of the final update), then a speculative group's final
-// entries, from column big_spec on
-__host__ __device__ constexpr int32_t big_spec(int32_t ne) { return ne < kBigOuterMax ? ne : kBigOuterMax; }
+// entries, from column big_spec on. A multiple of 8 columns: an operand
+// plane of as many bf16 columns then keeps its reader's 16-byte alignment.
+__host__ __device__ constexpr int32_t big_spec(int32_t ne) {
+    return ne < kBigOuterMax ? (ne + 7) / 8 * 8 : kBigOuterMax;
+}
 __host__ __device__ constexpr int32_t big_work(int32_t ne) { return big_spec(ne) + 64; }
+// Workspace entries of a front of f rows and `cols` W columns: a multiple of
+// 8, so that the next front's planes, at 4 bf16 entries per entry, start on 16
+// bytes too.
+__host__ __device__ constexpr int64_t work_room(int32_t f, int32_t cols) {
+    return (static_cast<int64_t>(f) * cols + 7) / 8 * 8;
+}
 static_assert(kBigOuterMax >= kBigOuter, "W holds the pivots of an outer block");
 struct BigLd {
     int32_t s;                  // supernode

@@ -1,0 +1,58 @@
+"""Offsets and launch shapes that the host code computes for the device, from
+the library's own headers, compiled here for the CPU."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "opt_solver_amd", "csrc")
+ROCM = "/opt/rocm/include"
+
+if not os.path.isdir(ROCM) or shutil.which("g++") is None:
+    pytest.skip("no HIP headers or no g++", allow_module_level=True)
+
+
+def run(tmp_path, body):
+    """The output of a program around `body` with the internal headers."""
+    src, exe = tmp_path / "t.cpp", tmp_path / "t"
+    src.write_text('#include <cstdio>\n#include "smfgpu_ldlt.hpp"\nusing namespace smfgpu;\nint main() {\n'
+                   + body + "\n    return 0;\n}\n")
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I", CSRC, "-I", ROCM, str(src), "-o", str(exe)],
+                   check=True)
+    return subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
+
+
+def test_operand_planes_start_on_16_bytes(tmp_path):
+    """A plane of bf16 operands holds big_work(ne) columns of f entries; the
+    four planes of a front follow each other and are read 16 bytes at a
+    time, so a plane's length is a multiple of 8 entries for any f and ne."""
+    out = run(tmp_path, """
+    int bad = 0;
+    for (int ne = 1; ne <= 1200; ++ne)
+        for (int f = ne; f < ne + 16; ++f) {
+            const long long plane = static_cast<long long>(big_work(ne)) * f;
+            if (plane % 8 != 0 || big_work(ne) < big_spec(ne) + kGroupCols || big_spec(ne) < (ne < 1024 ? ne : 1024)) ++bad;
+        }
+    std::printf("%d", bad);""")
+    assert out == "0"
+
+
+def test_panel_workspaces_start_on_even_entries(tmp_path):
+    """A front's planes lie at four bf16 entries per entry of its panel
+    workspace: the workspaces of a level's fronts, of any number of rows and
+    columns, start on even entries."""
+    out = run(tmp_path, """
+    int bad = 0;
+    long long at = 0;
+    for (int f = 96; f < 400; f += 7)
+        for (int cols = 2; cols < 40; ++cols) {
+            const long long room = work_room(f, cols);
+            if (room < static_cast<long long>(f) * cols || room >= static_cast<long long>(f) * cols + 8) ++bad;
+            at += room;
+            if (4 * at % 8 != 0) ++bad;
+        }
+    if (work_room(2000000, 1088) != 2176000000ll) ++bad;
+    std::printf("%d", bad);""")
+    assert out == "0"

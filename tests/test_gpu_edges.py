@@ -198,3 +198,33 @@ def test_panel_stalls_with_no_live_column_left(oracle_lib, p, q):
     x = rng.uniform(-1, 1, n)
     eta, _ = oracle_lib.backward_error(A, M @ x, fac.solve(M @ x))
     assert eta < 1e-13  # n eps
+
+
+@pytest.mark.parametrize("prec", ["bf16x3", "bf16"])
+def test_odd_fronts_on_planes_bitwise(prec):
+    """Several large fronts of odd row and column counts below 1024 in one
+    level, so that no front's operand planes have a round length: the same
+    factor, bit for bit, as with the operands rounded inside every tile."""
+    from opt_solver_amd import batch
+    from opt_solver_amd._lib import TUNE_LDLT_OUTER_WIDE, TUNE_LDLT_PLANES
+    from opt_solver_amd.solver import PREC_BF16, PREC_BF16X3
+    print("case odd planes", prec, flush=True)
+    rng = np.random.default_rng(11)
+    systems, vals = [], []
+    for f, ne in ((901, 301), (1301, 901), (777, 535), (1175, 1023)):
+        M = rng.uniform(-1, 1, (f, f))
+        M = M + M.T + np.diag(4.0 * f * np.where(np.arange(f) % 3 == 0, -1.0, 1.0))
+        A, arrays = dense_front_problem(M, ne)
+        systems.append(arrays)
+        vals.append(A[3])
+    plan = Plan(batch.union_arrays(systems)[0], posdef=False)
+    plan.tune(TUNE_LDLT_OUTER_WIDE, 512)
+    ex = []
+    for planes in (1, 0):
+        plan.tune(TUNE_LDLT_PLANES, planes)
+        fac = plan.factor(np.concatenate(vals), precision={"bf16x3": PREC_BF16X3, "bf16": PREC_BF16}[prec],
+                          mixed_min_front=512)
+        assert fac.status == 0 and fac.info.fronts_reduced >= 4
+        ex.append(fac.export())
+    for key in ("steps", "row_indices", "pivot_types", "factor_values"):
+        assert np.array_equal(ex[0][key], ex[1][key]), key
