@@ -19,6 +19,13 @@ constexpr int kBlockedMinFront = 96;  // ldlt_kernel.hpp:15 (blocked_min_front)
 // stored entries from which a front gets the store kernel (one workgroup
 // stores about 30 GB/s: 16 us for a front at the limit)
 constexpr int64_t kStoreWide = int64_t{1} << 15;
+// A level's large fronts run together, up to 1 GiB (in doubles) of panel
+// workspaces and group buffers, or kBigTogether fronts where those take more:
+// the levels of one system (KKT 260^2: 1024 fronts at most) are one list,
+// and many systems' fronts of 96 rows (187 KB of scratch each beside a square
+// of 74 KB) come in lists that fill the card many times over.
+constexpr int64_t kBigScratch = int64_t{1} << 27;
+constexpr size_t kBigTogether = 1024;
 
 namespace {
 
@@ -699,7 +706,8 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
     P->ldlt_prec.assign(P->nsup, 0);
     P->sel_cand.clear();
     std::vector<AsmPart> parts, wg_parts;
-    std::vector<int32_t> small_list, blocked_list, big_list, ep_list, store_list;
+    std::vector<int32_t> small_list, blocked_list, ep_list, store_list;
+    std::vector<std::vector<int32_t>> big_lists;  // large fronts that run together
     std::vector<BigLd> big_h;
     std::vector<FrontLd> patch;
     const int32_t nlev = static_cast<int32_t>(P->level_fronts.size());
@@ -755,10 +763,12 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
         patch.clear();
         small_list.clear();
         blocked_list.clear();
-        big_list.clear();
+        big_lists.clear();
         ep_list.clear();
         store_list.clear();
-        int64_t work_used = 0;
+        // panel workspaces: the blocked fronts' and each list of large fronts'
+        // run one after the other in the same room
+        int64_t blocked_work = 0, big_used = 0, work_used = 0;
         for (int32_t s : fr) {
             const FrontDev &Sy = P->fronts[s];
             FrontLd F{};
@@ -789,12 +799,21 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
             // front takes the one-workgroup blocked kernel
             const bool stat = front_static_value(spr, F.root, F.nd, F.psym) > 0.0;
             if (F.f >= P->ldlt_big_min && F.ne > 0 && !stat) {
-                F.wofs = work_used;
-                work_used += work_room(F.f, big_work(F.ne));
-                big_list.push_back(s);
+                const int64_t room = work_room(F.f, big_work(F.ne));
+                if (big_lists.empty() || (big_lists.back().size() >= kBigTogether &&
+                                          big_used + room + kGroupBuf * static_cast<int64_t>(big_lists.back().size() + 1) >
+                                              kBigScratch)) {
+                    big_lists.emplace_back();
+                    big_used = 0;
+                }
+                F.wofs = big_used;
+                big_used += room;
+                work_used = std::max(work_used, big_used);
+                big_lists.back().push_back(s);
             } else if (F.f >= kBlockedMinFront) {
-                F.wofs = work_used;
-                work_used += work_room(F.f, nb);
+                F.wofs = blocked_work;
+                blocked_work += work_room(F.f, nb);
+                work_used = std::max(work_used, blocked_work);
                 blocked_list.push_back(s);
             } else {
                 small_list.push_back(s);
@@ -868,8 +887,10 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
                           opt.pivot_u, eff_small, small, spr);
         launch_ldlt_blocked(st, d, reinterpret_cast<const int32_t *>(S + o_blk),
                             static_cast<int32_t>(blocked_list.size()), opt.pivot_u, eff_small, small, nb, spr);
-        if (!big_list.empty() && (rc = ldlt_big_fronts(P, d, big_list, opt, eff_small, small, nb, big_h, reduced)))
-            return rc;
+        for (size_t i = 0; i < big_lists.size(); ++i) {
+            if (i > 0) HIP_OK(hipStreamSynchronize(st));  // the list before has used its states' host copy
+            if ((rc = ldlt_big_fronts(P, d, big_lists[i], opt, eff_small, small, nb, big_h, reduced))) return rc;
+        }
         launch_ldlt_epilogue(st, d, reinterpret_cast<const int32_t *>(S + o_ep), static_cast<int32_t>(ep_list.size()),
                              n_inline);
         launch_ldlt_store(st, d, reinterpret_cast<const int32_t *>(S + o_ep) + n_inline,
