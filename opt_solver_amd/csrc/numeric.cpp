@@ -1334,7 +1334,8 @@ int solve_device(smfgpu_plan_s *P, const double *b_dev, int64_t ldb, double *out
     for (int32_t r0 = 0; r0 < nrhs; r0 += group) {
         const int32_t nr = std::min(group, nrhs - r0);
         if (!ybuf && P->d_y.n < static_cast<size_t>(n) * nr) {
-            const int rc = P->d_y.alloc(static_cast<size_t>(n) * nr);
+            // the whole group at the first solve: no later one frees it
+            const int rc = P->d_y.alloc(static_cast<size_t>(n) * kGroup);
             if (rc) return rc;
         }
         double *y = ybuf ? ybuf : P->d_y.p;

@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 
 from tests.conftest import gpu_available
-from tests.helpers import dense_front_problem
+from tests.helpers import dense_front_problem, matvec
 
 pytestmark = pytest.mark.gpu
 
@@ -13,7 +13,8 @@ if not gpu_available():
 import torch  # noqa: E402
 
 from opt_solver_amd import batch  # noqa: E402
-from opt_solver_amd.solver import Plan  # noqa: E402
+from opt_solver_amd import generators as g  # noqa: E402
+from opt_solver_amd.solver import Plan, analyse  # noqa: E402
 
 
 def many_fronts(count, f):
@@ -51,3 +52,22 @@ def test_level_of_many_large_fronts(f, count):
     print("grown", grown, flush=True)
     assert err < 1e-13 * f
     assert grown < 2**30 + 4096 * count
+
+
+def test_solve_buffer_settles_at_the_first_call():
+    """A plan's right-hand-side block is sized by its first solve: no later
+    call with more right-hand sides frees and allocates it again."""
+    for posdef in (True, False):
+        A = g.laplace7_3d(9)
+        plan = Plan(analyse(A), posdef=posdef)
+        fac = plan.factor(A[3])
+        X = np.random.default_rng(3).uniform(-1, 1, (A[0], 33))
+        B = torch.from_numpy(np.ascontiguousarray(matvec(A, X).T)).cuda()
+        sizes = []
+        for nr in (1, 2, 5, 16, 33):
+            x = B[:nr].clone()
+            torch.cuda.synchronize()
+            fac.solve_device(x.data_ptr(), nr)
+            assert np.abs(x.cpu().numpy().T - X[:, :nr]).max() < 1e-11
+            sizes.append(plan.stats()["device_bytes"])
+        assert len(set(sizes)) == 1, (posdef, sizes)
