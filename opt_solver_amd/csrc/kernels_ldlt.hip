@@ -3066,9 +3066,10 @@ void launch_ldlt_epilogue(hipStream_t st, const LdltDev &d, const int32_t *flist
 
 void launch_ldlt_store(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, int32_t max_cols) {
     if (nf <= 0 || max_cols <= 0) return;
-    // about 8192 workgroups over the launch's fronts, at least 16 a front
-    const int32_t per = std::min(max_cols, std::max(16, 8192 / nf));
-    k_ldlt_store<<<dim3(per, nf), kLT, 0, st>>>(d, flist);
+    for (int32_t o = 0; o < nf; o += kStoreFronts) {
+        const StoreGrid g = store_grid(nf - o, max_cols);
+        k_ldlt_store<<<dim3(g.per, g.fronts), kLT, 0, st>>>(d, flist + o);
+    }
 }
 
 // ---------------------------------------------------------------------------

@@ -199,6 +199,18 @@ void launch_ldlt_assemble(hipStream_t st, const LdltDev &d, const LdltAsm &A, co
 // the rest (many workgroups per front)
 void launch_ldlt_epilogue(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, int32_t n_inline);
 void launch_ldlt_store(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, int32_t max_cols);
+// A store launch: `per` workgroups for each of the next `fronts` fronts, which
+// are the grid's rows (65536 at most): about 8192 workgroups, at least 16 a
+// front.
+constexpr int32_t kStoreFronts = 32768;
+struct StoreGrid {
+    int32_t per, fronts;
+};
+inline StoreGrid store_grid(int32_t nf, int32_t max_cols) {
+    const int32_t m = nf < kStoreFronts ? nf : kStoreFronts;
+    const int32_t per = 8192 / m > 16 ? 8192 / m : 16;
+    return StoreGrid{per < max_cols ? per : max_cols, m};
+}
 void launch_ldlt_diag(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, int32_t max_p, double *y,
                       int32_t n, int32_t nrhs);
 // the diagonal-only solve job: D from the stored columns, by division

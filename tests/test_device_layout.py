@@ -56,3 +56,23 @@ def test_panel_workspaces_start_on_even_entries(tmp_path):
     if (work_room(2000000, 1088) != 2176000000ll) ++bad;
     std::printf("%d", bad);""")
     assert out == "0"
+
+
+def test_store_launches_stay_within_the_grid(tmp_path):
+    """The store launches of a level's fronts cover every front once, each
+    within the device's 65536 rows of workgroups and 2^22 workgroups."""
+    out = run(tmp_path, """
+    int bad = 0;
+    for (int nf : {1, 2, 511, 512, 65535, 65536, 65537, 131072, 200000, 1000000})
+        for (int cols : {1, 15, 128, 9000}) {
+            long long done = 0;
+            for (int o = 0; o < nf; o += kStoreFronts) {
+                const StoreGrid g = store_grid(nf - o, cols);
+                if (g.fronts < 1 || g.fronts > 65536 || g.per < 1 || g.per > cols) ++bad;
+                if (static_cast<long long>(g.fronts) * g.per > (1ll << 22)) ++bad;
+                done += g.fronts;
+            }
+            if (done != nf) ++bad;
+        }
+    std::printf("%d", bad);""")
+    assert out == "0"
