@@ -64,8 +64,9 @@ extern "C" {
 #define SMFGPU_STATUS_INERTIA_EXCEEDED 4
 
 /* Precision of the Schur-complement updates of large fronts (fronts of at
- * least mixed_min_front rows). Pivot tests, D, inertia, residuals and the
- * refined solution are always FP64. */
+ * least mixed_min_front rows; LDL^T: and at least 256, or
+ * SMFGPU_TUNE_LDLT_BIG_MIN where that has been set). Pivot tests, D, inertia,
+ * residuals and the refined solution are always FP64. */
 #define SMFGPU_PREC_FP64 0
 #define SMFGPU_PREC_FP32 1   /* FP32 MFMA, FP32 accumulation */
 #define SMFGPU_PREC_BF16 2   /* BF16 MFMA (operands rounded to bf16), FP32 accumulation */
@@ -399,7 +400,9 @@ SMFGPU_API int smfgpu_factor_solve(smfgpu_plan_t plan, const double *values, int
  * workgroups (speculative panel groups, pivot logic per panel in one
  * workgroup, MFMA updates); smaller blocked fronts take one workgroup
  * (about 1.3 ms a level; KKT 40^2 6.1 ms per factor + solve with the line
- * at 256 rows and 4.0 ms at 96, 150^2 37.1 and 34.1 ms). */
+ * at 256 rows and 4.0 ms at 96, 150^2 37.1 and 34.1 ms; a level of 1500
+ * fronts of 96 rows 2.1 and 1.1 ms, of 250 rows 19.2 and 4.8 ms). Once set, it
+ * is also the size from which fronts may run below FP64 (256 before). */
 #define SMFGPU_TUNE_LDLT_BIG_MIN 5
 /* SMFGPU_TUNE_LDLT_GROUP: 1 (default) lets the large-front LDL^T path try
  * groups of four first-pass panels at once (accepted when every pivot

@@ -779,7 +779,7 @@ SMFGPU_API int smfgpu_plan_tune(smfgpu_plan_t P, int32_t key, int64_t value) {
         return P->posdef ? dense_schedule(P) : SMFGPU_OK;
     case SMFGPU_TUNE_LDLT_BIG_MIN:
         if (value < 96 || value > (int64_t{1} << 30)) return set_error(SMFGPU_ERR_INVALID_ARG, "tune: bad front size");
-        P->ldlt_big_min = static_cast<int32_t>(value);
+        P->ldlt_big_min = P->ldlt_red_min = static_cast<int32_t>(value);
         return SMFGPU_OK;
     case SMFGPU_TUNE_LDLT_GROUP:
         if (value != 0 && value != 1) return set_error(SMFGPU_ERR_INVALID_ARG, "tune: group must be 0 or 1");

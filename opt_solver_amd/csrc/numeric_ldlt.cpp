@@ -297,6 +297,7 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
     const bool group = P->ldlt_group != 0 && nb == 16;
     const bool autosel = opt.precision == SMFGPU_PREC_AUTO;
     const bool collect = opt.collect != 0;
+    const int32_t red_min = std::max(opt.mixed_min_front, P->ldlt_red_min);  // smaller fronts stay FP64
     h.assign(nbig, BigLd{});
     int64_t cap = 64;
     int32_t nmode[4] = {0, 0, 0, 0};
@@ -312,7 +313,7 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
         int64_t cs = 0;
         for (int32_t b = 0; b < nbig; ++b) {
             const FrontLd &F = P->fl[big[b]];
-            if (F.f < opt.mixed_min_front) continue;
+            if (F.f < red_min) continue;
             sf.push_back(SelFront{big[b], F.f, F.ne, F.nd, cs, F.fofs, snap_total});
             sf_big.push_back(b);
             cs += F.ne;
@@ -347,10 +348,10 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
         B.k_paired = -1;
         B.spec = group ? 1 : 0;
         // mixed precision: reduced-precision MFMA updates on the fronts of
-        // at least mixed_min_front rows (the pivot logic stays FP64), the
+        // at least red_min rows (the pivot logic stays FP64), the
         // requested one or the selector's choice
-        if (autosel) B.prec = F.f >= opt.mixed_min_front ? P->ldlt_prec[big[b]] : 0;
-        else B.prec = code > 0 && F.f >= opt.mixed_min_front ? code : 0;
+        if (autosel) B.prec = F.f >= red_min ? P->ldlt_prec[big[b]] : 0;
+        else B.prec = code > 0 && F.f >= red_min ? code : 0;
         B.outer = (P->ldlt_planes != 0 && B.prec >= 2) ? P->ldlt_outer_wide : kBigOuter;
         B.oe = std::min(F.ne, B.outer);
         P->ldlt_prec[big[b]] = static_cast<int8_t>(B.prec);

@@ -254,6 +254,7 @@ struct smfgpu_plan_s {
     std::vector<int64_t> asm_first;                // SPD: first assembly task of each level
     int32_t cb_seg = 4096;                         // SPD: pivot columns per contribution-block update
     int32_t ldlt_big_min = 96;                     // LDL^T: fronts with at least this many rows take the large-front path
+    int32_t ldlt_red_min = 256;                    // LDL^T: smaller fronts never run below FP64 (ldlt_big_min once that is set)
     DBuf<BigLd> d_big;                             // LDL^T: large-front states of the level
     DBuf<BigPart> d_parts;                         // the level's launches: workgroup -> front
     int32_t ldlt_planes = 1;                       // LDL^T: bf16 operand planes for the large fronts' outer-block updates

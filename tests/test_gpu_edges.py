@@ -228,3 +228,29 @@ def test_odd_fronts_on_planes_bitwise(prec):
         ex.append(fac.export())
     for key in ("steps", "row_indices", "pivot_types", "factor_values"):
         assert np.array_equal(ex[0][key], ex[1][key]), key
+
+
+@pytest.mark.parametrize("ne,f", [(60, 96), (150, 200), (100, 255), (100, 256), (200, 300)])
+def test_reduced_precision_starts_at_256_rows(ne, f):
+    """An indefinite factorization below FP64 keeps fronts of fewer than 256
+    rows in FP64 whatever mixed_min_front says, and takes no training pair
+    from them, unless the plan's large-front line is set lower."""
+    from opt_solver_amd._lib import TUNE_LDLT_BIG_MIN
+    from opt_solver_amd.solver import PREC_FP32, PREC_FP64
+    print("case reduced", ne, f, flush=True)
+    rng = np.random.default_rng([ne, f])
+    M = rng.uniform(-1, 1, (f, f))
+    M = M + M.T + np.diag(4.0 * f * np.where(np.arange(f) % 3 == 0, -1.0, 1.0))
+    A, arrays = dense_front_problem(M, ne)
+    plan = Plan(arrays, posdef=False)
+    want = 1 if f >= 256 else 0
+    fac = plan.factor(A[3], precision=PREC_FP32, mixed_min_front=64)
+    # (the root has f - ne < 256 rows)
+    assert fac.info.fronts_reduced == want and (fac.precisions()[0] != PREC_FP64) == bool(want)
+    if not want:
+        low = fac.export()["factor_values"]
+        assert np.array_equal(low, plan.factor(A[3]).export()["factor_values"])
+    fac = plan.factor(A[3], collect=True, mixed_min_front=64)
+    assert list(fac.selector_pairs()[2]) == [0] * want
+    plan.tune(TUNE_LDLT_BIG_MIN, 96)
+    assert plan.factor(A[3], precision=PREC_FP32, mixed_min_front=64).precisions()[0] == PREC_FP32
