@@ -392,7 +392,10 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
         return static_cast<int32_t>(std::min<int64_t>(cap, (m * (m + 1) / 2 + 7) / 8 * 8));
     };
     BigGrid grid{};
-    grid.nrows = add_parts([&](int32_t f) { return (f + kGroupRows - 1) / kGroupRows; });
+    std::vector<int32_t> chunks(nbig);
+    for (int32_t b = 0; b < nbig; ++b) chunks[b] = (P->fl[big[b]].f + kGroupRows - 1) / kGroupRows;
+    row_parts(chunks, parts);
+    grid.nrows = static_cast<int32_t>(parts.size());
     grid.ntiles = add_parts([&](int32_t f) { return tile_parts(f, 128, per_front); });
     grid.nwide = add_parts([&](int32_t f) { return tile_parts(f, 256, wide_per_front); });
     if ((rc = ensure(P->d_parts, parts.size(), false, "large-front workgroups"))) return rc;

@@ -6,6 +6,8 @@
 
 #include "smfgpu_internal.hpp"
 
+#include <vector>
+
 namespace smfgpu {
 
 // Front s of the current factorization. Its f x f square (column-major,
@@ -118,6 +120,22 @@ struct BigGrid {
     const BigPart *wide;    // 256 x 256 update tiles, likewise
     int32_t nrows, ntiles, nwide;
 };
+// The list of row chunks, chunks[b] of front b: every front's first chunk, then
+// every front's second one, and so on. A front's first workgroup does its
+// pivot logic; workgroups go to the 8 XCDs in turn, so lists front by front
+// put the pivot logic of equal fronts of 2, 4 or 8 chunks on 4, 2 or one
+// of them.
+inline void row_parts(const std::vector<int32_t> &chunks, std::vector<BigPart> &out) {
+    bool more = true;
+    for (int32_t i = 0; more; ++i) {
+        more = false;
+        for (size_t b = 0; b < chunks.size(); ++b)
+            if (i < chunks[b]) {
+                out.push_back(BigPart{static_cast<int32_t>(b), i, chunks[b]});
+                more = true;
+            }
+    }
+}
 constexpr int32_t kGroupCols = 64;   // columns of a speculative group (four panels of 16)
 constexpr int32_t kGroupRows = 64;   // rows per workgroup below a group's diagonal region
 static_assert(big_work(1) - big_spec(1) == kGroupCols, "W holds a group's speculative columns");

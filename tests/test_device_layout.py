@@ -76,3 +76,27 @@ def test_store_launches_stay_within_the_grid(tmp_path):
         }
     std::printf("%d", bad);""")
     assert out == "0"
+
+
+def test_row_chunks_begin_with_every_front(tmp_path):
+    """A level's row chunks: each of every front once, the fronts' first
+    chunks (their pivot logic) ahead of all others, so that they spread over
+    the device's XCDs whatever the fronts' sizes."""
+    out = run(tmp_path, """
+    int bad = 0;
+    for (int same = 0; same < 10; ++same) {
+        std::vector<int32_t> chunks(301);
+        for (int b = 0; b < 301; ++b) chunks[b] = same > 0 ? same : 1 + b * b % 37;
+        std::vector<BigPart> p;
+        row_parts(chunks, p);
+        std::vector<int> seen(301 * 64, 0);
+        size_t total = 0;
+        for (int c : chunks) total += c;
+        if (p.size() != total) ++bad;
+        for (size_t i = 0; i < p.size(); ++i) {
+            if (p[i].parts != chunks[p[i].front] || p[i].part >= p[i].parts || seen[64 * p[i].front + p[i].part]++) ++bad;
+            if ((p[i].part == 0) != (i < 301)) ++bad;
+        }
+    }
+    std::printf("%d", bad);""")
+    assert out == "0"
