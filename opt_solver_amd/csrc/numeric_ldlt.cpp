@@ -294,8 +294,12 @@ static int ldlt_big_fronts(smfgpu_plan_s *P, const LdltDev &d0, const std::vecto
     LdltDev d = d0;
     d.xpl = nullptr;
     const int32_t nbig = static_cast<int32_t>(big.size());
-    const bool group = P->ldlt_group != 0 && nb == 16;
     const bool autosel = opt.precision == SMFGPU_PREC_AUTO;
+    // a panel lies inside its outer block: W holds no more columns, and the
+    // flush past the block would update a wider panel's pivots again
+    nb = std::min(nb, kBigOuter);
+    if (P->ldlt_planes != 0 && (autosel || prec_code(opt.precision) >= 2)) nb = std::min(nb, P->ldlt_outer_wide);
+    const bool group = P->ldlt_group != 0 && nb == 16;
     const bool collect = opt.collect != 0;
     const int32_t red_min = std::max(opt.mixed_min_front, P->ldlt_red_min);  // smaller fronts stay FP64
     h.assign(nbig, BigLd{});
@@ -699,7 +703,7 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
     // eff_small (factor_indef.cpp:633-636)
     const double small = opt.small_pivot;
     const double eff_small = (max_abs > 0.0 && max_abs < small) ? small * max_abs : small;
-    const int32_t nb = std::max(2, opt.panel);
+    const int32_t nb = std::max(2, std::min(opt.panel, n));  // (no front has more columns)
     // static pivoting values (factor_indef.cpp:642-645)
     StaticPrm spr{};
     spr.sp = opt.static_pivot_tol > 0.0 ? opt.static_pivot_tol * max_abs : 0.0;

@@ -254,3 +254,29 @@ def test_reduced_precision_starts_at_256_rows(ne, f):
     assert list(fac.selector_pairs()[2]) == [0] * want
     plan.tune(TUNE_LDLT_BIG_MIN, 96)
     assert plan.factor(A[3], precision=PREC_FP32, mixed_min_front=64).precisions()[0] == PREC_FP32
+
+
+@pytest.mark.parametrize("panel,wide", [(511, 1024), (513, 1024), (700, 1024), (2000, 1024), (2**31 - 1, 1024), (100, 64)])
+def test_panels_wider_than_the_outer_block(panel, wide):
+    """Panel widths up to and past the large fronts' outer block of 512
+    columns (and past its workspace), or of 64 where the plan's planes are
+    tuned to it: the solution is known to about n eps."""
+    from opt_solver_amd._lib import TUNE_LDLT_OUTER_WIDE
+    from opt_solver_amd.solver import PREC_BF16X3, PREC_FP64
+    print("case panel", panel, wide, flush=True)
+    ne, n = 1300, 1400
+    rng = np.random.default_rng(panel % 1000)
+    M = rng.uniform(-1, 1, (n, n))
+    M = M + M.T + np.diag(4.0 * n * np.where(np.arange(n) % 3 == 0, -1.0, 1.0))
+    A, arrays = dense_front_problem(M, ne)
+    plan = Plan(arrays, posdef=False)
+    plan.tune(TUNE_LDLT_OUTER_WIDE, wide)
+    x = rng.uniform(-1, 1, n)
+    fac = plan.factor(A[3], panel=panel)
+    assert fac.status == 0 and fac.inertia == (n - (n + 2) // 3, (n + 2) // 3, 0)
+    assert np.abs(fac.solve(M @ x) - x).max() < 1e-13 * n
+    # split BF16 products are within 2^-16 of the entries', which are at most
+    # 1 / (2 n) of the diagonal
+    fac = plan.factor(A[3], panel=panel, precision=PREC_BF16X3, mixed_min_front=1024)
+    assert fac.precisions()[0] != PREC_FP64
+    assert np.abs(fac.solve(M @ x) - x).max() < 1e-6
