@@ -1141,13 +1141,6 @@ __device__ __forceinline__ int big_tiles(int f, int c0, int c1) {
 // (inputs are finite: the factorization rejects non-finite values).
 __device__ __forceinline__ double masked(double v, bool keep) { return v * (keep ? 1.0 : 0.0); }
 
-__device__ __forceinline__ double rdlane(double v, int l) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane(static_cast<int>(b), l);
-    const int hi = __builtin_amdgcn_readlane(static_cast<int>(b >> 32), l);
-    return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
-}
-
 // Columns of the group the one-panel path would factor next if no panel
 // stalled: panels of nb from k, each ending at min(live, start + nb), the
 // group ending after the panel whose end triggers the outer block's flush.
@@ -1409,8 +1402,9 @@ __device__ __forceinline__ double wave_max8(double (&v)[8]) {
 // earlier panels' update on FP64 MFMA (operands and result through LDS, which
 // turns the tile's layout into rows per lane), then the panel's 16 pivots,
 // their multipliers broadcast inside each row of 16 lanes by DPP. Bound by
-// latency: the columns' loads, then wavefront-serial work (384 MFMAs of 64
-// cycles' issue, 480 FMAs with a broadcast each). 58 us with separate
+// latency: the columns' loads, then one wavefront's work in turn (96 MFMAs of
+// 64 cycles' issue, 480 FMAs with a broadcast each, and the panels' trips
+// through LDS between them). 58 us with separate
 // multiplies and subtracts, multipliers from LDS and 256 rows a workgroup;
 // 32 us with all 2016 FMAs of a row on the vector unit; 16.8 us now.
 constexpr int kGLd = 80;  // LDS column stride: the two lane rows of a half wavefront fall on different banks
@@ -1537,7 +1531,9 @@ __global__ __launch_bounds__(kGroupRows) void k_big_group(LdltDev d, const BigLd
 
 // Leading panels of a group that pass the first test: the number of accepted
 // columns, from the pivots and column maxima the region and rows launches
-// left (lane c of every wavefront tests column c). A NaN maximum fails.
+// left (lane c of every wavefront tests column c). A NaN pivot fails; a NaN
+// below it (only an overflow makes one, the input is finite) is passed over by
+// the maxima, as by select_pivot's.
 __device__ __forceinline__ int group_accepted(const double *gp, int gcols, const Prm &prm, double &piv) {
     const int c = threadIdx.x & 63;
     bool ok = true;
@@ -2705,8 +2701,9 @@ __device__ __forceinline__ void lane_apply(const FV &A, int kind, int pa, int pb
 // ---------------------------------------------------------------------------
 // Levels of small fronts laid out on the device.
 //
-// One wavefront's fronts have at most kDevWaveMax rows (their squares of 23 KB
-// let seven workgroups share a CU), several wavefronts' kLaneRows.
+// One wavefront's fronts have at most kDevWaveMax rows (their squares of 21 KB,
+// 24 KB with the rest, let six workgroups share a CU), several wavefronts'
+// kLaneRows.
 constexpr int kDevWaveMax = 48;
 template <int ROWS>
 constexpr int lane_square = (ROWS + 1) * (ROWS + kCU);
@@ -2983,9 +2980,8 @@ __device__ void dev_front(const LdltDev &d, const DevLevel &L, int s, const Prm 
 // wavefront and 25 KB of LDS: many fronts per CU); a larger one keeps its
 // layout for the CLASS 1 launch (256 threads). CLASS 2 (256 threads): layout
 // and any front, four wavefronts each: where a level has few fronts
-// (kDevOneLaunch: the workgroups of 80 KB that the card holds at a time),
-// and for a whole band of levels, each workgroup going up its chain of
-// fronts. CLASS 3: layout and workgroup reductions whatever the size.
+// (kDevOneLaunch), and for a whole band of levels, each workgroup going up its
+// chain of fronts. CLASS 3: layout and workgroup reductions whatever the size.
 template <int CLASS>
 __global__ __launch_bounds__(CLASS == 0 ? 64 : kLT) void k_dev_fronts(LdltDev d, DevLevel L,
                                                                      const int32_t *__restrict__ flist, int32_t lv,

@@ -1,9 +1,10 @@
-// Host driver of the indefinite (LDL^T) numeric phase: level by level, the
-// host lays out the level's fronts from its children's results (delayed
-// columns first, as process_front, solver/src/multifrontal_serial.cpp:510-545
-// of the reference), uploads the row lists, child maps and assembly tasks,
-// launches assembly, the front kernels and the epilogue, and reads back the
-// pivot counts and final row orders the next level needs.
+// Host driver of the indefinite (LDL^T) numeric phase. Levels of small fronts
+// run on the device without it. For the others, level by level, the host lays
+// out the level's fronts from its children's results (delayed columns first,
+// as process_front, solver/src/multifrontal_serial.cpp:510-545 of the
+// reference), uploads the fronts' records, the assembly's workgroups and the
+// kernels' front lists, launches the row lists, assembly, front kernels and
+// epilogue, and reads back the records, whose pivot counts size the next level.
 #include "smfgpu_plan.hpp"
 
 #include <algorithm>
@@ -278,8 +279,8 @@ static int ldlt_dev_levels(smfgpu_plan_s *P, int32_t lv0, double u, double eff_s
     return SMFGPU_OK;
 }
 
-// Large fronts of one level (multi-workgroup blocked LDL^T): the panel,
-// update and stall kernels in turn until every front is done, then the
+// Large fronts of one level (multi-workgroup blocked LDL^T): the region,
+// group, panel and update kernels in turn until every front is done, then the
 // contribution blocks' update in chunks of an outer block's pivots and the
 // fronts' results. The state is read back after as many rounds as the
 // fronts need when every panel group is accepted (a round then takes 64
@@ -720,7 +721,7 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
     std::vector<FrontLd> patch;
     const int32_t nlev = static_cast<int32_t>(P->level_fronts.size());
     int rc;
-    int32_t levels_done = 0, reduced = 0;
+    int32_t reduced = 0;
     bool inertia_exceeded = false, work_exceeded = false;
     // Early stops (multifrontal_serial.cpp:653-671, 1196-1205, 1612-1622).
     // The reference takes the fronts one by one in supernode order (its
@@ -757,7 +758,6 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
         if (dev_on && lv != dev_hold && P->lv_fsym_max[lv] <= std::min(kDevSymMax, P->dev_fmax)) {
             int32_t next = lv, hold = -1;
             if ((rc = ldlt_dev_levels(P, lv, opt.pivot_u, eff_small, small, spr, next, hold))) return rc;
-            levels_done = next;
             dev_hold = hold;
             if (next > lv) {
                 lv = next - 1;
@@ -914,7 +914,6 @@ int ldlt_factor(smfgpu_plan_s *P, const double *dv, int64_t nvalues, const smfgp
         HIP_OK(hipStreamSynchronize(st));
         for (size_t i = 0; i < fr.size(); ++i)
             std::memcpy(&P->fl[fr[i]], P->h_stage.data() + o_back + i * sizeof(FrontLd), sizeof(FrontLd));
-        levels_done = lv + 1;
         if (!fdone.empty()) {
             for (int32_t s : fr) fdone[s] = 1;
             while (cur < P->nsup && fdone[cur]) {

@@ -95,7 +95,7 @@ struct BigLd {
     int32_t stalled;            // first pass: the last panel stalled
     int32_t ps, pl;             // the last panel
     int32_t oe;                 // outer block end
-    int32_t outer;              // outer block width (kBigOuter, or kBigOuterWide on planes)
+    int32_t outer;              // outer block width (kBigOuter, or the plan's ldlt_outer_wide on planes)
     int32_t pend0;              // pivots [pend0, k) held back for the columns >= oe; W column 0
     int32_t u_c0, u_c1, u_p0, u_p1;  // update request: columns [u_c0, u_c1), rows [u_c0, f), pivots [u_p0, u_p1)
     int32_t x_c0, x_p0, x_p1;        // flush request: columns [x_c0, ne), rows [x_c0, f), pivots [x_p0, x_p1)
@@ -183,7 +183,12 @@ struct DevLevel {
 };
 void launch_dev_fronts(hipStream_t st, const LdltDev &d, const DevLevel &L, const int32_t *flist, int32_t nf,
                        int32_t lv, double u, double eff_small, double small_pivot, const StaticPrm &S, bool wave);
-// fronts of a level up to which one launch takes both sizes, and a band
+// Fronts of a level up to which one launch takes both sizes, and a band: the
+// four-wavefront workgroups (80 KB of LDS) that the card holds at a time. More
+// of them wait for a place, and a launch a level with a wavefront a front is
+// the faster one: 1536 trajectory systems of horizons up to 200 31.1 ms in
+// one launch and 26.1 in a launch a level, 1024 22.2 and 20.9, 640 15.5 and
+// 14.4; 520 still 11.8 and 12.1.
 constexpr int32_t kDevOneLaunch = 512;
 
 void launch_ldlt_small(hipStream_t st, const LdltDev &d, const int32_t *flist, int32_t nf, double u, double eff_small,
@@ -239,9 +244,8 @@ constexpr int32_t kItemAtomic = 1;  // backward chunk: several items add to its 
 constexpr int32_t kItemTri = 2;     // a block's triangle, else a chunk
 constexpr int32_t kItemFused = 4;   // forward: the triangle, then the rows [a0, a1) below it in the same workgroup
 constexpr int32_t kItemWide = 8;    // a triangle of more than 64 pivots
-// one step of the blocked forward / backward sweep (items of all fronts of
-// a level); wide: the step's triangles of more than 64 pivots, else its
-// other items (the two are independent)
+// kinds of a sweep's steps: wide triangles, a band of chains, or (0) the other
+// items
 constexpr uint8_t kStepWide = 1, kStepChains = 2;
 // a front of a chain: at most kChainRows rows
 constexpr int32_t kChainRows = 64;
@@ -253,22 +257,26 @@ struct ChainFront {
 // from the lowest level up
 void launch_ldlt_chains(hipStream_t st, const LdltDev &d, bool fwd, const int32_t *ptr, const ChainFront *fronts,
                         int64_t count, double *y, int32_t n, int32_t nrhs);
+// one step of the blocked forward / backward sweep (items of all fronts of
+// a level); wide: the step's triangles of more than 64 pivots, else its
+// other items (the two are independent)
 void launch_ldlt_fwd_step(hipStream_t st, const LdltDev &d, const SolveItem *items, int64_t count, bool wide,
                           double *y, int32_t n, int32_t nrhs);
 void launch_ldlt_bwd_step(hipStream_t st, const LdltDev &d, const SolveItem *items, int64_t count, bool wide,
                           double *y, int32_t n, int32_t nrhs);
 // one round of the level's large fronts: the states of the round and,
 // written by the panel launch, the next ones; gpart: the group buffers (null:
-// one panel per round)
+// one panel per round); nmode[m]: fronts whose updates run in precision code m
+// (0 FP64, 1 FP32, 2 BF16, 3 split BF16), a launch per code in use
 void launch_big_round(hipStream_t st, const LdltDev &d, BigLd *states, BigLd *next, int32_t nbig, const BigGrid &g,
                       double u, double eff_small, double small_pivot, int32_t nb, double *gpart,
                       const int32_t *nmode);
-// nmode[m]: fronts of the level whose updates run in precision code m
-// (0 FP64, 1 FP32, 2 BF16, 3 split BF16); a launch per code in use
 // final contribution-block update with pivots [c0, c0 + width) of every
-// front (L*D of the chunk into W first); then the fronts' results
+// front (L*D of the chunk into W first); wide: the fronts on bf16 planes, else
+// the others
 void launch_big_cb(hipStream_t st, const LdltDev &d, const BigLd *states, const BigGrid &g, int32_t c0, int32_t width,
                    const int32_t *nmode, bool wide);
+// the finished fronts' results, from their states to their records
 void launch_big_finish(hipStream_t st, const LdltDev &d, const BigLd *states, int32_t nbig);
 
 }  // namespace smfgpu

@@ -311,9 +311,7 @@ struct smfgpu_plan_s {
     double max_abs = 0.0;
     // ---- LDL^T (posdef = 0) ----
     std::vector<int32_t> sn_parent, child_ptr, child_idx;
-    std::vector<int32_t> amap_h;                    // host copy of the symbolic-position map
     PinnedArr<FrontLd> fl;                          // host mirror of the fronts of the last factorization
-    std::vector<int8_t> tags_h;
     DBuf<FrontLd> d_fl;
     DBuf<double> d_arena, d_work, d_dinv;
     DBuf<double> d_fac;                             // stored factor columns (f x ne per front)
