@@ -401,8 +401,12 @@ SMFGPU_API int smfgpu_factor_solve(smfgpu_plan_t plan, const double *values, int
  * workgroup, MFMA updates); smaller blocked fronts take one workgroup
  * (about 1.3 ms a level; KKT 40^2 6.1 ms per factor + solve with the line
  * at 256 rows and 4.0 ms at 96, 150^2 37.1 and 34.1 ms; a level of 1500
- * fronts of 96 rows 2.1 and 1.1 ms, of 250 rows 19.2 and 4.8 ms). Once set, it
- * is also the size from which fronts may run below FP64 (256 before). */
+ * fronts of 96 rows 2.1 and 1.1 ms, of 250 rows 19.2 and 3.9 ms). Where no
+ * column is an acceptable pivot and every panel stalls, one workgroup is the
+ * faster one up to about 150 rows (96 rows: 2.2 against 2.6 ms, 1500 such
+ * fronts 5.6 against 10.5; 250 rows: 9.1 against 7.0, 1500 30.5 against 37).
+ * Once set, it is also the size from which fronts may run below FP64 (256
+ * before). */
 #define SMFGPU_TUNE_LDLT_BIG_MIN 5
 /* SMFGPU_TUNE_LDLT_GROUP: 1 (default) lets the large-front LDL^T path try
  * groups of four first-pass panels at once (accepted when every pivot
